@@ -73,14 +73,24 @@ CK_HD uint32_t mid_sq(uint32_t x, uint32_t land) { return ((x + land + 1u) >> 1)
 // ------------------------------------------------------------------------------------------
 // Philox4x32-10 (Salmon, Moraes, Dror, Shaw, SC'11)
 // ------------------------------------------------------------------------------------------
+// Exclusive or of three words: one v_bitop3_b32 on the device (the compiler makes two v_xor_b32 of
+// a ^ b ^ c; a Philox block has twenty of them).
+CK_HD uint32_t xor3(uint32_t a, uint32_t b, uint32_t c) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return __builtin_amdgcn_bitop3_b32(a, b, c, 0x96);
+#else
+  return a ^ b ^ c;
+#endif
+}
+
 CK_HD void philox(uint32_t c0, uint32_t c1, uint32_t c2, uint32_t c3, uint32_t k0, uint32_t k1,
                   uint32_t out[4]) {
 #pragma unroll
   for (int round = 0; round < 10; round++) {
     uint64_t a = (uint64_t)0xD2511F53u * c0;
     uint64_t b = (uint64_t)0xCD9E8D57u * c2;
-    uint32_t n0 = (uint32_t)(b >> 32) ^ c1 ^ k0;
-    uint32_t n2 = (uint32_t)(a >> 32) ^ c3 ^ k1;
+    uint32_t n0 = xor3((uint32_t)(b >> 32), c1, k0);
+    uint32_t n2 = xor3((uint32_t)(a >> 32), c3, k1);
     c1 = (uint32_t)b;
     c3 = (uint32_t)a;
     c0 = n0;
@@ -274,34 +284,114 @@ CK_HD uint32_t perm(uint32_t hi, uint32_t lo, uint32_t sel) {
 #endif
 }
 
-// k-th move (0-based) of the slot masks in square-major, slot-minor order.  The four masks are
-// transposed by bytes, so that word x_b holds squares 8b..8b+7 of slot t in its byte t; the
-// group of eight squares holding the k-th move is found from the four words' popcounts, and the
-// square inside it by a 3-step search that counts the group's moves below a square with one
-// popcount (the square's low-bit mask copied into every byte).
-CK_HD void select_slot(const uint32_t s[4], uint32_t k, uint32_t &sq, uint32_t &sl) {
+// The four slot masks transposed by bytes: word b holds squares 8b..8b+7 of slot t in its byte t.
+// n01 counts the moves of words 0 and 1, n all moves.
+struct SlotWords {
+  uint32_t x0, x1, x2, x3;
+  uint32_t n0, n01, n;
+};
+
+CK_HD SlotWords slot_words(const uint32_t s[4]) {
   const uint32_t a_lo = perm(s[1], s[0], 0x05010400u), a_hi = perm(s[1], s[0], 0x07030602u);
   const uint32_t b_lo = perm(s[3], s[2], 0x05010400u), b_hi = perm(s[3], s[2], 0x07030602u);
-  const uint32_t x0 = perm(b_lo, a_lo, 0x05040100u), x1 = perm(b_lo, a_lo, 0x07060302u);
-  const uint32_t x2 = perm(b_hi, a_hi, 0x05040100u), x3 = perm(b_hi, a_hi, 0x07060302u);
-  const uint32_t p1 = popc(x0), p2 = p1 + popc(x1), p3 = p2 + popc(x2);
-  const bool g1 = k >= p1, g2 = k >= p2, g3 = k >= p3;
-  const uint32_t x = g3 ? x3 : g2 ? x2 : g1 ? x1 : x0;
-  const uint32_t base = g3 ? p3 : g2 ? p2 : g1 ? p1 : 0u;
-  const uint32_t kk = k - base;
-  auto below = [x](uint32_t j) { return popc(x & perm(0u, bit(j) - 1u, 0u)); };
-  uint32_t lo = 0;
-#pragma unroll
-  for (uint32_t stride = 4; stride >= 1; stride >>= 1)
-    if (below(lo + stride) <= kk) lo += stride;
-  uint32_t j = kk - below(lo);
-  const uint32_t y = (x >> lo) & 0x01010101u;
-  uint32_t here = (y | (y >> 7) | (y >> 14) | (y >> 21)) & 15u;
+  SlotWords w;
+  w.x0 = perm(b_lo, a_lo, 0x05040100u);
+  w.x1 = perm(b_lo, a_lo, 0x07060302u);
+  w.x2 = perm(b_hi, a_hi, 0x05040100u);
+  w.x3 = perm(b_hi, a_hi, 0x07060302u);
+  w.n0 = popc(w.x0);
+  w.n01 = popc(w.x1) + w.n0;
+  w.n = popc(w.x3) + (popc(w.x2) + w.n01);
+  return w;
+}
+
+// k - c when k >= c, else k (k, c < 2^31): the unsigned difference wraps to above k.
+CK_HD uint32_t sub_if(uint32_t k, uint32_t c) {
+  const uint32_t d = k - c;
+  return d < k ? d : k;
+}
+
+// What the lane logic looks up.  Direct computes every entry where it is used; the playout kernels
+// hold them in LDS (playout_kernels.hip), where a read costs one issue slot.
+//   mod(r, n)      r mod n, 1 <= n <= kModMax (the moves of four slot masks)
+//   nth(y, j)      the slot of the j-th move of one square: bit 8t of y is set where slot t has one
+//   move(i, f, r)  masks of a move: i = square | slot << 5 | king << 7 | capture << 8; f flips the
+//                  squares it leaves and enters, r holds the piece it removes
+constexpr uint32_t kModMax = 128;
+
+CK_HD uint32_t nth_slot(uint32_t nibble, uint32_t j) {  // the j-th set bit of four
+  uint32_t here = nibble;
   if (j >= 1u) here &= here - 1u;
   if (j >= 2u) here &= here - 1u;
   if (j >= 3u) here &= here - 1u;
-  sq = 8u * (uint32_t)(g1 + g2 + g3) + lo;
-  sl = ctz(here);
+  return here ? ctz(here) : 0u;
+}
+
+// Bits 0, 8, 16 and 24 of y to bits 2..5 (the product's partial terms fall on distinct bits).
+CK_HD uint32_t gather4(uint32_t y) { return (y * 0x10204080u) >> 26; }
+
+// A step in direction d from square x moves base_d - (x's row parity) squares, base = {5, 4, -3,
+// -4}; a jump is two steps from rows of opposite parity, 2 base_d - 1 squares, over the square one
+// step away.  Slots name directions 0..3 but for a man's captures, whose slot 0 is direction 1.
+// Entries off the board are never read.
+CK_HD void move_masks(uint32_t i, uint32_t &flip, uint32_t &removed) {
+  const uint32_t sq = i & 31u, sl = (i >> 5) & 3u, king = (i >> 7) & 1u, capture = (i >> 8) & 1u;
+  const uint32_t d = (capture && !king && sl < 2u) ? sl ^ 1u : sl;
+  const uint32_t one = step_to(sq, d), two = (uint32_t)((int)sq + jump_off(d));
+  flip = bit(sq) | bit((capture ? two : one) & 31u);
+  removed = capture ? bit(one & 31u) : 0u;
+}
+
+struct Direct {
+  CK_HD uint32_t mod(uint32_t r, uint32_t n) const { return mod_small(r, n); }
+  CK_HD uint32_t nth(uint32_t y, uint32_t j) const { return nth_slot(gather4(y) >> 2, j); }
+  CK_HD void move(uint32_t i, uint32_t &flip, uint32_t &removed) const {
+    move_masks(i, flip, removed);
+  }
+};
+
+// r mod n from m = floor((2^32 - 1) / n): the quotient floor(r m / 2^32) is at most one too small,
+// since 2^32 / n - m <= 1 and so r / n - r m / 2^32 <= r / 2^32 < 1; the remainder is r - q n or
+// that less n.
+CK_HD uint32_t mod_by(uint32_t r, uint32_t n, uint32_t m) {
+  const uint32_t q = (uint32_t)(((uint64_t)r * m) >> 32);
+  const uint32_t rem = r - q * n;
+  return rem < rem - n ? rem : rem - n;
+}
+CK_HD uint32_t mod_factor(uint32_t n) { return 0xFFFFFFFFu / (n ? n : 1u); }
+
+// k-th move (0-based) in square-major, slot-minor order.  The word of eight squares that holds it
+// is found from the words' move counts; inside it three steps halve the squares, each counting the
+// moves of the lower half with one popcount and shifting the upper half down where the move lies
+// there.  What is left in bits 0, 8, 16 and 24 are the moves of one square.
+template <class TAB>
+CK_HD void select_move(const SlotWords &w, uint32_t k, uint32_t &sq, uint32_t &sl,
+                       const TAB &tab) {
+  const bool g2 = k >= w.n01;
+  const uint32_t lo = g2 ? w.x2 : w.x0, hi = g2 ? w.x3 : w.x1;
+  k = sub_if(k, w.n01);
+  const uint32_t c = popc(lo);
+  const bool g1 = k >= c;
+  uint32_t x = g1 ? hi : lo;
+  k = sub_if(k, c);
+  const uint32_t c4 = popc(x & 0x0F0F0F0Fu);
+  const uint32_t s4 = k >= c4 ? 4u : 0u;
+  x >>= s4;
+  k = sub_if(k, c4);
+  const uint32_t c2 = popc(x & 0x03030303u);
+  const uint32_t s2 = k >= c2 ? 2u : 0u;
+  x >>= s2;
+  k = sub_if(k, c2);
+  const uint32_t c1 = popc(x & 0x01010101u);
+  const uint32_t s1 = k >= c1 ? 1u : 0u;
+  x >>= s1;
+  k = sub_if(k, c1);
+  sq = ((g2 ? 16u : 0u) | (g1 ? 8u : 0u)) | (s4 | s2 | s1);
+  sl = tab.nth(x & 0x01010101u, k);
+}
+
+CK_HD void select_slot(const uint32_t s[4], uint32_t k, uint32_t &sq, uint32_t &sl) {
+  select_move(slot_words(s), k, sq, sl, Direct());
 }
 
 // ------------------------------------------------------------------------------------------
@@ -370,6 +460,24 @@ CK_HD void apply(Lane &L, uint32_t from, uint32_t to, uint32_t removed) {
   uint32_t kings = L.kings & ~removed;
   kings = was_king ? (kings ^ (fb | tb)) : (kings | ((to >= FAR_ROW_FIRST) ? tb : 0u));
   L.counter = removed ? 0u : L.counter + 1u;
+  L.own = brev(opp);
+  L.opp = brev(own);
+  L.kings = brev(kings);
+  L.turn ^= 1u;
+}
+
+// The move of slot choice (square sq, slot sl), applied (a king is a piece on sq with its bit set:
+// own holds sq).  A man's entered square on the far row becomes a king; kings hold no empty square,
+// so flipping sets it.
+template <class TAB>
+CK_HD void play_slot(Lane &L, uint32_t capture, uint32_t sq, uint32_t sl, const TAB &tab) {
+  const uint32_t km = 0u - ((L.kings >> sq) & 1u);  // all ones: the piece is a king
+  uint32_t flip, removed;
+  tab.move((sq | (sl << 5) | (km & 128u)) + (capture ? 256u : 0u), flip, removed);
+  const uint32_t own = L.own ^ flip;
+  const uint32_t opp = L.opp & ~removed;
+  const uint32_t kings = (L.kings & ~removed) ^ (flip & (km | ROW7));
+  L.counter = capture ? 0u : L.counter + 1u;
   L.own = brev(opp);
   L.opp = brev(own);
   L.kings = brev(kings);
@@ -944,8 +1052,9 @@ CK_HD PlyResult ply_random(Lane &L, uint32_t r, uint32_t *list_dig) {
 // The common part of a random ply: plays it unless it is a capture ply with a multi-jump origin,
 // in which case the position is left untouched and `deferred` is returned set (the caller plays
 // it later with ply_random_given, the same word and the analysis left in g).
-template <bool TRACE>
-CK_HD PlyResult ply_random_fast(Lane &L, uint32_t r, uint32_t *list_dig, bool &deferred, Gen &g) {
+template <bool TRACE, class TAB = Direct>
+CK_HD PlyResult ply_random_fast(Lane &L, uint32_t r, uint32_t *list_dig, bool &deferred, Gen &g,
+                                const TAB &tab = TAB()) {
   analyse(L, g);
   PlyResult res;
   deferred = g.multi != 0u;
@@ -956,7 +1065,8 @@ CK_HD PlyResult ply_random_fast(Lane &L, uint32_t r, uint32_t *list_dig, bool &d
     res.winner = 0;
     return res;
   }
-  const uint32_t n = slot_count(g.slot);
+  const SlotWords w = slot_words(g.slot);
+  const uint32_t n = w.n;
   res.n = n;
   if (TRACE) *list_dig = list_digest(L, g, n);
   if (n == 0u || L.counter >= 50u) {
@@ -965,21 +1075,21 @@ CK_HD PlyResult ply_random_fast(Lane &L, uint32_t r, uint32_t *list_dig, bool &d
     res.winner = L.counter < 50u ? (int32_t)(L.turn ^ 1u) : -1;
     return res;
   }
-  const uint32_t k = mod_small(r, n);
+  const uint32_t k = tab.mod(r, n);
   res.chosen = k;
   res.over = 0u;
   res.winner = 0;
   uint32_t sq, sl;
-  select_slot(g.slot, L.turn ? n - 1u - k : k, sq, sl);
-  const Choice c = slot_choice(L, g, sq, sl);
-  apply(L, c.from, c.to, c.removed);
+  select_move(w, L.turn ? n - 1u - k : k, sq, sl, tab);
+  play_slot(L, g.capture, sq, sl, tab);
   return res;
 }
 
 // The heuristic ply after analyse.  WALK = false promises that no capture sequence is longer
 // than one jump (the caller deferred such plies), which drops the tree walks from the code.
-template <bool TRACE, bool WALK>
-CK_HD PlyResult heuristic_body(Lane &L, const Gen &g, uint32_t r, uint32_t *list_dig) {
+template <bool TRACE, bool WALK, class TAB = Direct>
+CK_HD PlyResult heuristic_body(Lane &L, const Gen &g, uint32_t r, uint32_t *list_dig,
+                               const TAB &tab = TAB()) {
   PlyResult res;
   const uint32_t sm = material(L.own, L.kings);
   const uint32_t so = material(L.opp, L.kings);
@@ -1035,7 +1145,6 @@ CK_HD PlyResult heuristic_body(Lane &L, const Gen &g, uint32_t r, uint32_t *list
         }
       }
     }
-    ties = slot_count(tslot);
   } else if (g.capture) {
     uint32_t o = g.origins;
     uint32_t king = 0;
@@ -1069,7 +1178,11 @@ CK_HD PlyResult heuristic_body(Lane &L, const Gen &g, uint32_t r, uint32_t *list
     tslot[1] = promo ? pb : g.slot[1];
     tslot[2] = promo ? 0u : g.slot[2];
     tslot[3] = promo ? 0u : g.slot[3];
-    ties = slot_count(tslot);
+  }
+  SlotWords tw;
+  if (!walked) {
+    tw = slot_words(tslot);
+    ties = tw.n;
   }
   res.n = n;
   if (TRACE) *list_dig = list_digest(L, g, n);
@@ -1079,7 +1192,7 @@ CK_HD PlyResult heuristic_body(Lane &L, const Gen &g, uint32_t r, uint32_t *list
     res.winner = L.counter < 50u ? (int32_t)(L.turn ^ 1u) : -1;
     return res;
   }
-  uint32_t k = mod_small(r, ties);
+  uint32_t k = walked ? mod_small(r, ties) : tab.mod(r, ties);
   uint32_t km = L.turn ? ties - 1u - k : k;
   res.over = 0u;
   res.winner = 0;
@@ -1114,8 +1227,7 @@ CK_HD PlyResult heuristic_body(Lane &L, const Gen &g, uint32_t r, uint32_t *list
     res.chosen = L.turn ? n - 1u - idx : idx;
   } else {
     uint32_t sq, sl;
-    select_slot(tslot, km, sq, sl);
-    c = slot_choice(L, g, sq, sl);
+    select_move(tw, km, sq, sl, tab);
     if (TRACE) {
       // reference index: rank of (sq, sl) in the full slot order
       uint32_t below = bit(sq) - 1u;
@@ -1126,6 +1238,8 @@ CK_HD PlyResult heuristic_body(Lane &L, const Gen &g, uint32_t r, uint32_t *list
     } else {
       res.chosen = 0u;
     }
+    play_slot(L, g.capture, sq, sl, tab);
+    return res;
   }
   apply(L, c.from, c.to, c.removed);
   return res;
@@ -1149,9 +1263,9 @@ CK_HD PlyResult ply_heuristic_given(Lane &L, const Gen &g, uint32_t r, uint32_t 
 // The common part of a heuristic ply: plays it unless it is a capture ply with a sequence
 // longer than one jump, which is left untouched with `deferred` set (the caller plays it later
 // with ply_heuristic_given, the same word and the analysis left in g).
-template <bool TRACE>
+template <bool TRACE, class TAB = Direct>
 CK_HD PlyResult ply_heuristic_fast(Lane &L, uint32_t r, uint32_t *list_dig, bool &deferred,
-                                   Gen &g) {
+                                   Gen &g, const TAB &tab = TAB()) {
   analyse(L, g);
   deferred = g.capture && g.multi;
   if (deferred) {
@@ -1162,7 +1276,7 @@ CK_HD PlyResult ply_heuristic_fast(Lane &L, uint32_t r, uint32_t *list_dig, bool
     res.winner = 0;
     return res;
   }
-  return heuristic_body<TRACE, false>(L, g, r, list_dig);
+  return heuristic_body<TRACE, false>(L, g, r, list_dig, tab);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1435,11 +1549,13 @@ CK_HD PlyResult ply_noisy_given(Lane &L, const Gen &g, uint32_t r, uint32_t *lis
 // The common part of a noisy heuristic ply: plays it when its moves all weigh the same (and no
 // capture sequence is longer than one jump), else leaves it untouched with `deferred` set, for
 // ply_noisy_given with the same word and the analysis left in g.
-template <bool TRACE>
-CK_HD PlyResult ply_noisy_fast(Lane &L, uint32_t r, uint32_t *list_dig, bool &deferred, Gen &g) {
+template <bool TRACE, class TAB = Direct>
+CK_HD PlyResult ply_noisy_fast(Lane &L, uint32_t r, uint32_t *list_dig, bool &deferred, Gen &g,
+                               const TAB &tab = TAB()) {
   PlyResult res;
   analyse(L, g);
-  const uint32_t n = slot_count(g.slot);
+  const SlotWords w = slot_words(g.slot);
+  const uint32_t n = w.n;
   bool inf = false;
   deferred = (g.capture && g.multi) ||
              (n != 0u && L.counter < 50u &&
@@ -1459,14 +1575,13 @@ CK_HD PlyResult ply_noisy_fast(Lane &L, uint32_t r, uint32_t *list_dig, bool &de
     res.winner = L.counter < 50u ? (int32_t)(L.turn ^ 1u) : -1;
     return res;
   }
-  const uint32_t k = inf ? 0u : mod_small(r, n);  // reference index
+  const uint32_t k = inf ? 0u : tab.mod(r, n);  // reference index
   uint32_t sq, sl;
-  select_slot(g.slot, L.turn ? n - 1u - k : k, sq, sl);
-  const Choice c = slot_choice(L, g, sq, sl);
+  select_move(w, L.turn ? n - 1u - k : k, sq, sl, tab);
   res.over = 0u;
   res.winner = 0;
   res.chosen = k;
-  apply(L, c.from, c.to, c.removed);
+  play_slot(L, g.capture, sq, sl, tab);
   return res;
 }
 

@@ -2,10 +2,14 @@
 //
 // k_playouts is a persistent kernel: each lane of a wave64 runs one playout at a time with the
 // position in VGPRs (ck::Lane) and, when its game ends, takes the next playout index.  New
-// playouts start only on wave iterations that are multiples of four, so every active lane is at
-// a ply index that is a multiple of four on those iterations and the Philox4x32-10 call that
-// yields the next four words is wave-uniform (one call per four plies instead of a divergent
-// call on almost every iteration).  Refill policy MI_REFILL_QUEUE claims playout indices for the
+// playouts start only on wave iterations that are multiples of four, where the Philox4x32-10 call
+// that yields the next four words runs for the whole wave (one call per four plies instead of a
+// divergent call on almost every iteration).  The kernel is bound by the issue of vector
+// instructions (every integer instruction, multiplications included, takes four cycles of a SIMD;
+// only reciprocals take longer), so what a ply would compute from small operands -- the factor of
+// r mod n, the j-th slot of a square, a move's masks -- and its Philox words are read from LDS,
+// one issue slot each, and flags of the lanes are wave masks in scalar registers: 355 -> 269
+// vector instructions per wave iteration on random-1024x1024, 0.778 -> 0.615 ms.  Refill policy MI_REFILL_QUEUE claims playout indices for the
 // whole wave in multiples of kChunk from its slab's device counter (one atomic per claim,
 // broadcast with a lane read; slabs are described in kernels.h), MI_REFILL_STATIC strides lanes
 // over the index space without atomics.
@@ -31,6 +35,11 @@ constexpr uint32_t kChunk = 16;
 __device__ __forceinline__ uint32_t lane_rank(uint64_t mask) {
   return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),
                                    __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+}
+
+// Whether this lane is in a wave mask.
+__device__ __forceinline__ bool lane_in(uint64_t mask) {
+  return __builtin_amdgcn_inverse_ballot_w64(mask);
 }
 
 __global__ void k_reset(WorkWords *work) {
@@ -78,28 +87,40 @@ __device__ __forceinline__ void locate(const PlayoutArgs &a, uint32_t g, uint32_
   }
 }
 
-// Philox words of a lane: `cur` holds block `blk` of its stream (words 4*blk .. 4*blk+3),
-// `nxt` block blk+1 when nxt_ok.  Blocks are generated only on wave iterations that are
-// multiples of four (wave-uniform work); since a lane consumes at most one word per iteration,
-// holding the current and the next block always covers the next four iterations.
-struct Words {
-  uint32_t c0, c1, c2, c3, n0, n1, n2, n3;
-  uint32_t blk;
-  bool cur_ok, nxt_ok;
+// The lane logic's lookups (ck::Direct's functions) from LDS, filled once per workgroup.
+struct LdsTables {
+  uint32_t factor[ck::kModMax + 1];
+  uint8_t nth[64];
+  uint2 move[512];
+
+  __device__ void fill() {
+    for (uint32_t i = threadIdx.x; i < 512u; i += blockDim.x) {
+      uint2 m;
+      ck::move_masks(i, m.x, m.y);
+      move[i] = m;
+    }
+    for (uint32_t i = threadIdx.x; i <= ck::kModMax; i += blockDim.x) factor[i] = ck::mod_factor(i);
+    if (threadIdx.x < 64u) nth[threadIdx.x] = (uint8_t)ck::nth_slot(threadIdx.x >> 2, threadIdx.x & 3u);
+  }
 };
 
-__device__ __forceinline__ uint32_t take_word(Words &w, uint32_t ply) {
-  if ((ply >> 2) != w.blk) {
-    w.c0 = w.n0;
-    w.c1 = w.n1;
-    w.c2 = w.n2;
-    w.c3 = w.n3;
-    w.blk++;
-    w.nxt_ok = false;
+struct Lookup {
+  const LdsTables &t;
+  __device__ uint32_t mod(uint32_t r, uint32_t n) const { return ck::mod_by(r, n, t.factor[n]); }
+  __device__ uint32_t nth(uint32_t y, uint32_t j) const { return t.nth[ck::gather4(y) + j]; }
+  __device__ void move(uint32_t i, uint32_t &flip, uint32_t &removed) const {
+    const uint2 m = t.move[i];
+    flip = m.x;
+    removed = m.y;
   }
-  const uint32_t q = ply & 3u;
-  return q == 0u ? w.c0 : q == 1u ? w.c1 : q == 2u ? w.c2 : w.c3;
-}
+};
+
+// Philox words of a wave's lanes, two blocks of four per lane: word w of a lane's stream sits in
+// row w & 7 (64 lanes wide, so that the lanes' reads fall on different banks whatever rows they
+// are at).  Blocks are generated on wave iterations that are multiples of four (wave-uniform
+// work): the one that holds word ply + 3, so that with the words left from the block before it
+// the lane has the next four -- it consumes at most one word per iteration.
+constexpr uint32_t kWordRows = 8;
 
 template <uint32_t POLICY, bool TRACE, uint32_t REFILL>
 __global__ void __launch_bounds__(1024) k_playouts(PlayoutArgs a) {
@@ -115,12 +136,22 @@ __global__ void __launch_bounds__(1024) k_playouts(PlayoutArgs a) {
     if (d->offs_at) a.offs = (const uint32_t *)(base + d->offs_at);
     a.keys = d->keys_at ? (const uint32_t *)(base + d->keys_at) : nullptr;
   }
+  __shared__ LdsTables tables;
+  extern __shared__ uint32_t wave_words[];  // kWordRows x 64 words per wave
+  tables.fill();
+  __syncthreads();
+  const Lookup tab = {tables};
   const uint32_t lane = threadIdx.x & 63u;
+  uint32_t *const words = wave_words + (threadIdx.x >> 6) * (kWordRows * 64u) + lane;
   const uint32_t nthreads = gridDim.x * blockDim.x;
-  bool active = false, deferred = false;
+  // Lanes that hold a game, and those of them whose ply waits for the walk phase.  Wave masks (in
+  // scalar registers) rather than per-lane flags: flags changed on divergent paths are kept in
+  // vector registers, a dozen instructions per ply.
+  uint64_t active = 0, deferred = 0;
+  // ply counts in units of kPly, the row stride of `words`: a word's row offset is one mask away
+  constexpr uint32_t kPly = 64u;
   uint32_t g = 0, p = 0, j = 0, ply = 0, h = 0, maxn = 0;
-  Words w = {0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u, false, false};
-  uint64_t plies_acc = 0;
+  uint32_t plies_acc = 0;  // a lane's plies of a launch stay far below 2^32 (2^31 playouts in all)
   ck::Lane L = {0u, 0u, 0u, 0u, 0u};
   ck::Gen gd;  // the analysis of a deferred ply, kept for its walk (saves a second analyse)
   // wave-uniform refill and deferral state: the reservation [res_next, res_end) is slab-local in
@@ -132,138 +163,127 @@ __global__ void __launch_bounds__(1024) k_playouts(PlayoutArgs a) {
   uint32_t static_next = blockIdx.x * blockDim.x + threadIdx.x;
   const uint32_t defer_min = a.defer_min;
 
+  // Plies were decided on the lanes `on`: their game is over, or its move has been played.
+  auto decided = [&](bool on, const ck::PlyResult &res, uint32_t ld) {
+    if (on) {
+      if (TRACE) h = ck::hash_step(h, ck::ply_record(ld, res.n, res.chosen));
+      maxn = res.n > maxn ? res.n : maxn;
+    }
+    const bool over = on && res.over;
+    if (over) {
+      a.winners[g] = (int8_t)res.winner;
+      if (TRACE) {
+        if (a.plies) a.plies[g] = ply / kPly;
+        if (a.hashes) a.hashes[g] = h;
+      }
+      plies_acc += ply / kPly;
+    }
+    if (on) ply += kPly;  // (of no account once the game is over)
+    active &= ~__ballot(over);
+  };
+
   for (uint32_t iter = 0;; iter++) {
     if ((iter & 3u) == 0u) {
       bool start = false;
       if (REFILL == MI_REFILL_STATIC) {
-        if (!active && static_next < a.total) {
+        if (!lane_in(active) && static_next < a.total) {
           g = static_next;
           static_next += nthreads;
           start = true;
         }
-      } else if (!exhausted) {
-        const uint64_t idle = __ballot(!active);
-        if (idle) {
-          const uint32_t cnt = (uint32_t)__popcll(idle);
-          const uint32_t rank = lane_rank(idle);  // of an idle lane among the idle lanes
-          const uint32_t avail = res_end - res_next;
-          uint32_t c = 0;
-          // the new claim covers every idle lane that the old one cannot
-          const uint32_t want = avail < cnt ? ((cnt - avail + kChunk - 1u) / kChunk) * kChunk : 0u;
-          if (avail < cnt) {
-            if (lane == 0u) c = atomicAdd(&a.work->queue[slab].next, want);
-            c = __shfl(c, 0);
-          }
-          if (!active) {
-            const uint32_t idx =
-                slab_index(rank < avail ? res_next + rank : c + (rank - avail), slab, nslabs);
-            if (idx < a.total) {
-              g = idx;
-              start = true;
-            }
-          }
-          if (avail < cnt) {
-            res_next = c + (cnt - avail);
-            res_end = c + want;
-          } else {
-            res_next += cnt;
-          }
-          if (slab_index(res_next, slab, nslabs) >= a.total) exhausted = true;  // slab dry
+      } else if (!exhausted && ~active) {
+        const uint64_t idle = ~active;
+        const uint32_t cnt = (uint32_t)__popcll(idle);
+        const uint32_t rank = lane_rank(idle);  // of an idle lane among the idle lanes
+        const uint32_t avail = res_end - res_next;
+        uint32_t c = 0;
+        // the new claim covers every idle lane that the old one cannot
+        const uint32_t want = avail < cnt ? ((cnt - avail + kChunk - 1u) / kChunk) * kChunk : 0u;
+        if (avail < cnt) {
+          if (lane == 0u) c = atomicAdd(&a.work->queue[slab].next, want);
+          c = __builtin_amdgcn_readfirstlane(c);
         }
+        if (lane_in(idle)) {
+          const uint32_t idx =
+              slab_index(rank < avail ? res_next + rank : c + (rank - avail), slab, nslabs);
+          if (idx < a.total) {
+            g = idx;
+            start = true;
+          }
+        }
+        if (avail < cnt) {
+          res_next = c + (cnt - avail);
+          res_end = c + want;
+        } else {
+          res_next += cnt;
+        }
+        if (slab_index(res_next, slab, nslabs) >= a.total) exhausted = true;  // slab dry
       }
       if (start) {
-        active = true;
-        deferred = false;
         mi_pos q;
         locate(a, g, p, j, g, q);  // from here on g is the playout's result slot
         if (a.keys) p = a.keys[p];  // from here on p is the stream key
         L = ck::lane_from_abs(q.p1, q.p2, q.kings, q.turn, q.counter);
         ply = 0;
         h = 0;
-        w.cur_ok = false;
-        w.nxt_ok = false;
       }
-      if (!__any(active)) break;
-      if (active && (!w.cur_ok || !w.nxt_ok)) {
-        const uint32_t b = w.cur_ok ? w.blk + 1u : (ply >> 2);
+      active |= __ballot(start);
+      if (!active) break;
+      if (lane_in(active)) {
+        const uint32_t b = (ply / kPly + 3u) >> 2;
         uint32_t o[4];
         ck::philox(b, j, ck::TAG_PLAYOUT, a.epoch, a.seed, p, o);
-        if (w.cur_ok) {
-          w.n0 = o[0];
-          w.n1 = o[1];
-          w.n2 = o[2];
-          w.n3 = o[3];
-          w.nxt_ok = true;
-        } else {
-          w.c0 = o[0];
-          w.c1 = o[1];
-          w.c2 = o[2];
-          w.c3 = o[3];
-          w.blk = b;
-          w.cur_ok = true;
-        }
+        uint32_t *const row = words + (b & 1u) * (4u * 64u);
+#pragma unroll
+        for (uint32_t w = 0; w < 4u; w++) row[w * 64u] = o[w];
       }
     }
-    // common part of the ply; multi-jump plies of the random policy wait for the walk phase
-    bool play = false;
-    ck::PlyResult res;
-    uint32_t ld = 0;
-    if (active && !deferred) {
-      const uint32_t r = take_word(w, ply);
-      // a deferred ply takes the same word again in the walk phase (take_word is idempotent
-      // for a given ply)
-      bool d = false;
-      if (POLICY == MI_POLICY_RANDOM) res = ck::ply_random_fast<TRACE>(L, r, &ld, d, gd);
-      else if (POLICY == MI_POLICY_HEURISTIC) res = ck::ply_heuristic_fast<TRACE>(L, r, &ld, d, gd);
-      else res = ck::ply_noisy_fast<TRACE>(L, r, &ld, d, gd);
-      deferred = d;
-      play = !d;
-    }
+    // common part of the ply; plies with longer captures (for the noisy heuristic also those whose
+    // moves weigh differently) wait for the walk phase, where they take the same word again
     {
-      const uint64_t dm = __ballot(deferred);
-      if (dm) {
-        const uint32_t nd = (uint32_t)__popcll(dm);
-        const uint32_t na = (uint32_t)__popcll(__ballot(active));
-        if (nd >= defer_min || nd == na || since_walk >= 8u) {
-          since_walk = 0;
-          if (deferred) {
-            const uint32_t r = take_word(w, ply);
-            if (POLICY == MI_POLICY_RANDOM) {
-              // capture trees in closed form; the walk only for king trees past two jumps
-              bool deep = false;
-              res = ck::ply_random_trees<TRACE>(L, gd, r, &ld, deep);
-              if (deep) res = ck::ply_random_given<TRACE>(L, gd, r, &ld);
-            }
-            else if (POLICY == MI_POLICY_HEURISTIC) res = ck::ply_heuristic_given<TRACE>(L, gd, r, &ld);
-            else res = ck::ply_noisy_given<TRACE>(L, gd, r, &ld);
-            deferred = false;
-            play = true;
-          }
-        } else {
-          since_walk++;
-        }
+      const bool on = lane_in(active & ~deferred);
+      bool d = false;
+      ck::PlyResult res = {0u, 0u, 0u, 0};
+      uint32_t ld = 0;
+      if (on) {
+        const uint32_t r = words[ply & ((kWordRows - 1u) * kPly)];
+        if (POLICY == MI_POLICY_RANDOM) res = ck::ply_random_fast<TRACE>(L, r, &ld, d, gd, tab);
+        else if (POLICY == MI_POLICY_HEURISTIC) res = ck::ply_heuristic_fast<TRACE>(L, r, &ld, d, gd, tab);
+        else res = ck::ply_noisy_fast<TRACE>(L, r, &ld, d, gd, tab);
       }
+      deferred |= __ballot(on && d);
+      decided(on && !d, res, ld);
     }
-    if (play) {
-      if (TRACE) h = ck::hash_step(h, ck::ply_record(ld, res.n, res.chosen));
-      maxn = res.n > maxn ? res.n : maxn;
-      if (res.over) {
-        a.winners[g] = (int8_t)res.winner;
-        if (TRACE) {
-          if (a.plies) a.plies[g] = ply;
-          if (a.hashes) a.hashes[g] = h;
+    if (deferred) {
+      const uint32_t nd = (uint32_t)__popcll(deferred);
+      if (nd >= defer_min || deferred == active || since_walk >= 8u) {
+        since_walk = 0;
+        const bool on = lane_in(deferred);
+        ck::PlyResult res = {0u, 0u, 0u, 0};
+        uint32_t ld = 0;
+        if (on) {
+          const uint32_t r = words[ply & ((kWordRows - 1u) * kPly)];
+          if (POLICY == MI_POLICY_RANDOM) {
+            // capture trees in closed form; the walk only for king trees past two jumps
+            bool deep = false;
+            res = ck::ply_random_trees<TRACE>(L, gd, r, &ld, deep);
+            if (deep) res = ck::ply_random_given<TRACE>(L, gd, r, &ld);
+          }
+          else if (POLICY == MI_POLICY_HEURISTIC) res = ck::ply_heuristic_given<TRACE>(L, gd, r, &ld);
+          else res = ck::ply_noisy_given<TRACE>(L, gd, r, &ld);
         }
-        plies_acc += ply;
-        active = false;
+        deferred = 0;
+        decided(on, res, ld);
       } else {
-        ply++;
+        since_walk++;
       }
     }
   }
   // statistics: per wave, then per workgroup in LDS, then one device atomic each (device atomics
   // travel to memory as 32-byte requests)
+  unsigned long long wave_plies = plies_acc;
   for (int off = 32; off >= 1; off >>= 1) {
-    plies_acc += __shfl_xor(plies_acc, off);
+    wave_plies += __shfl_xor(wave_plies, off);
     uint32_t m = __shfl_xor(maxn, off);
     maxn = m > maxn ? m : maxn;
   }
@@ -275,7 +295,7 @@ __global__ void __launch_bounds__(1024) k_playouts(PlayoutArgs a) {
   }
   __syncthreads();
   if (lane == 0u) {
-    atomicAdd(&wg_plies, (unsigned long long)plies_acc);
+    atomicAdd(&wg_plies, wave_plies);
     atomicMax(&wg_maxn, maxn);
   }
   __syncthreads();
@@ -435,15 +455,21 @@ __global__ void __launch_bounds__(256) k_valu_rate(uint32_t iters, uint32_t salt
 }
 #undef VALU_STEP
 
+}  // namespace
+
+uint32_t playout_lds(uint32_t block) { return block / 64u * (kWordRows * 64u * sizeof(uint32_t)); }
+
+namespace {
+
 template <uint32_t POLICY, bool TRACE>
 hipError_t launch_refill(const PlayoutArgs &args, uint32_t refill, uint32_t grid, uint32_t block,
                          hipStream_t stream) {
   if (refill == MI_REFILL_STATIC)
-    hipLaunchKernelGGL((k_playouts<POLICY, TRACE, MI_REFILL_STATIC>), dim3(grid), dim3(block), 0,
-                       stream, args);
+    hipLaunchKernelGGL((k_playouts<POLICY, TRACE, MI_REFILL_STATIC>), dim3(grid), dim3(block),
+                       playout_lds(block), stream, args);
   else
-    hipLaunchKernelGGL((k_playouts<POLICY, TRACE, MI_REFILL_QUEUE>), dim3(grid), dim3(block), 0,
-                       stream, args);
+    hipLaunchKernelGGL((k_playouts<POLICY, TRACE, MI_REFILL_QUEUE>), dim3(grid), dim3(block),
+                       playout_lds(block), stream, args);
   return hipGetLastError();
 }
 
