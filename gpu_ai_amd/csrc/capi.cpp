@@ -66,6 +66,27 @@ int ensure_host(mi_ctx *ctx, HostBuf &b, size_t bytes) {
   return MI_OK;
 }
 
+uint32_t tune_bucket(uint64_t total) {
+  const uint32_t b = total ? 63u - (uint32_t)__builtin_clzll(total) : 0u;
+  return b < kTuneBuckets ? b : kTuneBuckets - 1u;
+}
+
+// Whether a batch of `total` playouts runs with one wave per game (k_playouts_wave).  A small batch
+// lasts as long as its longest game: 0.41-0.66 us per ply with a wave of its own (random, noisy)
+// against 1.0-2.3 us in a wave of 64 games, but a game costs a whole wave's instructions, so from
+// some size on the lanes win.  Kernel ms, one wave per game / one lane per game, 256 CUs:
+//   playouts       256          4,096        8,192        16,384       32,768
+//   random     .060 / .140  .088 / .148  .120 / .144  .170 / .146  .278 / .166
+//   heuristic  .062 / .213  .105 / .206  .145 / .199  .217 / .202  .352 / .208
+//   noisy      .079 / .395  .124 / .331  .174 / .319  .238 / .330  .393 / .333
+// A context that was given a launch shape, or has measured one for the batch's size, uses it.
+bool wave_batch(const mi_ctx *ctx, uint32_t policy, uint64_t total) {
+  if (ctx->shaped || total > (uint64_t)ctx->cus * (policy == MI_POLICY_HEURISTIC_NOISY ? 64u : 32u))
+    return false;
+  const TuneEntry *e = ctx->tune_table[policy][tune_bucket(total)];
+  return e[0].kernel_ms < 0.f && e[1].kernel_ms < 0.f;
+}
+
 }  // namespace ctxutil
 }  // namespace gpuai
 
@@ -74,6 +95,8 @@ using gpuai::ctxutil::ensure;
 using gpuai::ctxutil::ensure_host;
 using gpuai::ctxutil::fail;
 using gpuai::ctxutil::hip_fail;
+using gpuai::ctxutil::tune_bucket;
+using gpuai::ctxutil::wave_batch;
 
 namespace {
 
@@ -213,11 +236,6 @@ uint32_t grid_for(const mi_ctx *ctx, const mi_tuning &t, uint64_t total) {
   return gpuai::grid_size(need, resident);
 }
 
-uint32_t tune_bucket(uint64_t total) {
-  const uint32_t b = total ? 63u - (uint32_t)__builtin_clzll(total) : 0u;
-  return b < kTuneBuckets ? b : kTuneBuckets - 1u;
-}
-
 // The launch shape of a batch of `total` playouts: the table's entry for its policy and bucket
 // (the faster refill, or refill `only` when it is 0 or 1), else the context's tuning.
 mi_tuning shape_for(const mi_ctx *ctx, uint32_t policy, uint64_t total, int only = -1) {
@@ -229,6 +247,9 @@ mi_tuning shape_for(const mi_ctx *ctx, uint32_t policy, uint64_t total, int only
   }
   return best ? best->tuning : ctx->tuning;
 }
+
+// The statistics' launch shape of such a batch.
+constexpr mi_tuning kWaveShape = {gpuai::kWaveBlock, 0u, MI_REFILL_STATIC, 0u};
 
 void clear_tune_table(mi_ctx *ctx) {
   for (auto &pol : ctx->tune_table)
@@ -243,7 +264,8 @@ int run_kernel(mi_ctx *ctx, uint32_t npos, uint32_t per_pos, uint64_t total, boo
                uint32_t seed, uint32_t epoch, uint32_t policy, bool trace, mi_stats *stats,
                int8_t *winners = nullptr, bool keyed = false, const mi_tuning *shape = nullptr) {
   // the autotuner passes the candidate it measures; every other launch takes its batch's shape
-  const mi_tuning t = shape ? *shape : shape_for(ctx, policy, total);
+  const bool wave = !shape && !trace && wave_batch(ctx, policy, total);
+  const mi_tuning t = shape ? *shape : wave ? kWaveShape : shape_for(ctx, policy, total);
   int rc;
   if ((rc = ensure_host(ctx, ctx->h_back, sizeof(gpuai::WorkWords) + (winners ? total : 0))))
     return rc;
@@ -266,10 +288,12 @@ int run_kernel(mi_ctx *ctx, uint32_t npos, uint32_t per_pos, uint64_t total, boo
   a.order = ctx->ordered ? (const uint32_t *)ctx->order.ptr : nullptr;
   a.ord_offs = ctx->ordered && with_offs ? (const uint32_t *)ctx->ord_offs.ptr : nullptr;
   a.keys = keyed ? (const uint32_t *)ctx->keys.ptr : nullptr;
-  const uint32_t grid = grid_for(ctx, t, total);
+  const uint32_t grid = wave ? (uint32_t)total : grid_for(ctx, t, total);
   MI_HIP(ctx, gpuai::launch_reset(a.work, ctx->stream));
   MI_HIP(ctx, hipEventRecord(ctx->ev_start, ctx->stream));
-  MI_HIP(ctx, gpuai::launch_playouts(a, policy, trace, t.refill, grid, t.block_size, ctx->stream));
+  MI_HIP(ctx, wave ? gpuai::launch_playouts_wave(a, policy, grid, ctx->stream)
+                   : gpuai::launch_playouts(a, policy, trace, t.refill, grid, t.block_size,
+                                            ctx->stream));
   MI_HIP(ctx, hipEventRecord(ctx->ev_stop, ctx->stream));
   gpuai::WorkWords *hw = (gpuai::WorkWords *)ctx->h_back.ptr;
   int8_t *hwin = (int8_t *)ctx->h_back.ptr + sizeof(gpuai::WorkWords);
@@ -283,9 +307,9 @@ int run_kernel(mi_ctx *ctx, uint32_t npos, uint32_t per_pos, uint64_t total, boo
   MI_HIP(ctx, hipEventElapsedTime(&ms, ctx->ev_start, ctx->ev_stop));
   if (stats) {
     stats->playouts = total;
-    stats->plies = w.plies;
+    stats->plies = gpuai::total_plies(w);
     stats->kernel_ms = ms;
-    stats->max_moves = w.max_moves;
+    stats->max_moves = gpuai::longest_list(w);
     stats->grid_blocks = grid;
     stats->block_size = t.block_size;
     stats->refill = t.refill;
@@ -372,7 +396,8 @@ int run_packed(mi_ctx *ctx, const mi_pos *pos, uint32_t npos, const uint32_t *co
   if (keys) std::memcpy(h + L.keys, keys, sizeof(uint32_t) * n);
   std::memset(h + L.work, 0, sizeof(gpuai::WorkWords));
 
-  const mi_tuning t = shape_for(ctx, policy, total);
+  const bool wave = !trace && wave_batch(ctx, policy, total);
+  const mi_tuning t = wave ? kWaveShape : shape_for(ctx, policy, total);
   gpuai::PlayoutArgs a;
   a.pos = ctx->ordered ? nullptr : (const mi_pos *)(d + L.pos);
   a.offs = counts ? (const uint32_t *)(d + L.offs) : nullptr;
@@ -392,10 +417,12 @@ int run_packed(mi_ctx *ctx, const mi_pos *pos, uint32_t npos, const uint32_t *co
   a.work = (gpuai::WorkWords *)(d + L.work);
   a.defer_min = t.defer_min;
   a.desc = nullptr;
-  const uint32_t grid = grid_for(ctx, t, total);
+  const uint32_t grid = wave ? (uint32_t)total : grid_for(ctx, t, total);
   MI_HIP(ctx, hipMemcpyAsync(d, h, L.win, hipMemcpyHostToDevice, ctx->stream));
   MI_HIP(ctx, hipEventRecord(ctx->ev_start, ctx->stream));
-  MI_HIP(ctx, gpuai::launch_playouts(a, policy, trace, t.refill, grid, t.block_size, ctx->stream));
+  MI_HIP(ctx, wave ? gpuai::launch_playouts_wave(a, policy, grid, ctx->stream)
+                   : gpuai::launch_playouts(a, policy, trace, t.refill, grid, t.block_size,
+                                            ctx->stream));
   MI_HIP(ctx, hipEventRecord(ctx->ev_stop, ctx->stream));
   MI_HIP(ctx, hipMemcpyAsync(h + L.work, d + L.work, (back ? L.win + total : L.win) - L.work,
                              hipMemcpyDeviceToHost, ctx->stream));
@@ -420,9 +447,9 @@ int run_packed(mi_ctx *ctx, const mi_pos *pos, uint32_t npos, const uint32_t *co
   MI_HIP(ctx, hipEventElapsedTime(&ms, ctx->ev_start, ctx->ev_stop));
   if (stats) {
     stats->playouts = total;
-    stats->plies = w->plies;
+    stats->plies = gpuai::total_plies(*w);
     stats->kernel_ms = ms;
-    stats->max_moves = w->max_moves;
+    stats->max_moves = gpuai::longest_list(*w);
     stats->grid_blocks = grid;
     stats->block_size = t.block_size;
     stats->refill = t.refill;
@@ -531,6 +558,9 @@ int mi_create(mi_ctx **out, int device, const mi_tuning *tuning) {
       return MI_ERR_INVALID_ARGUMENT;
     }
     ctx->tuning = t;
+    // every field zero but the queue refill: the defaults
+    ctx->shaped = tuning->block_size || tuning->blocks_per_cu || tuning->defer_min ||
+                  tuning->refill != kDefaultTuning.refill;
   }
   hipDeviceProp_t prop;
   if (hipSetDevice(device) != hipSuccess || hipGetDeviceProperties(&prop, device) != hipSuccess ||
@@ -579,6 +609,7 @@ int mi_set_tuning(mi_ctx *ctx, const mi_tuning *tuning) {
   int rc = check_tuning(ctx, t);
   if (rc) return rc;
   ctx->tuning = t;
+  ctx->shaped = true;
   clear_tune_table(ctx);  // an explicit shape holds for every batch size
   return MI_OK;
 }
@@ -777,6 +808,7 @@ int mi_autotune(mi_ctx *ctx, const mi_pos *pos, uint32_t npos, const uint32_t *c
                        max_results, nresults, best_t, best_ms)))
     return rc;
   ctx->tuning = best_t;
+  ctx->shaped = true;
   if (best) *best = best_t;
   return MI_OK;
 }
@@ -991,9 +1023,10 @@ struct mi_graph {
   gpuai::PlayoutArgs args;
   uint32_t block = 0, resident = 0, grid = 0, refill = 0;
   hipEvent_t e0 = nullptr, e1 = nullptr;
-  // a replay launched by mi_graph_launch and not yet finished
+  // a replay launched by mi_graph_launch and not yet finished, and its launch shape
   bool pending = false;
   uint64_t pending_total = 0;
+  uint32_t pending_grid = 0, pending_block = 0, pending_refill = 0;
 };
 
 namespace {
@@ -1132,6 +1165,21 @@ int mi_graph_launch(mi_graph *g, const mi_pos *pos, uint32_t npos, const uint32_
     std::memcpy(h + offs_at, ctx->host_offs.data(), sizeof(uint32_t) * ((size_t)npos + 1));
     if (keys) std::memcpy(h + keys_at, keys, sizeof(uint32_t) * (size_t)npos);
     const size_t out_bytes = sizeof(gpuai::WorkWords) + (size_t)total;
+    if (wave_batch(ctx, g->policy, total)) {  // the graph holds the other kernel: same order, no graph
+      gpuai::PlayoutArgs a = g->args;
+      MI_HIP(ctx, hipEventRecord(g->e0, ctx->stream));
+      MI_HIP(ctx, hipMemcpyAsync(g->d_blob, g->h_blob, in_bytes, hipMemcpyHostToDevice, ctx->stream));
+      MI_HIP(ctx, gpuai::launch_reset(a.work, ctx->stream));
+      MI_HIP(ctx, gpuai::launch_playouts_wave(a, g->policy, (uint32_t)total, ctx->stream));
+      MI_HIP(ctx, hipMemcpyAsync(g->h_out, g->d_out, out_bytes, hipMemcpyDeviceToHost, ctx->stream));
+      MI_HIP(ctx, hipEventRecord(g->e1, ctx->stream));
+      g->pending = true;
+      g->pending_total = total;
+      g->pending_grid = (uint32_t)total;
+      g->pending_block = kWaveShape.block_size;
+      g->pending_refill = kWaveShape.refill;
+      return MI_OK;
+    }
     MI_HIP(ctx, hipGraphExecMemcpyNodeSetParams1D(g->exec, g->n_d2h, g->h_out, g->d_out, out_bytes,
                                                   hipMemcpyDeviceToHost));
     // the batch's shape from the tuning table (the graph's refill policy; both are correct for
@@ -1161,6 +1209,9 @@ int mi_graph_launch(mi_graph *g, const mi_pos *pos, uint32_t npos, const uint32_
   }
   g->pending = true;
   g->pending_total = total;
+  g->pending_grid = g->grid;
+  g->pending_block = g->block;
+  g->pending_refill = g->refill;
   return MI_OK;
 }
 
@@ -1182,12 +1233,12 @@ int mi_graph_finish(mi_graph *g, int8_t *winners, mi_stats *stats) {
     float ms = 0.f;
     MI_HIP(ctx, hipEventElapsedTime(&ms, g->e0, g->e1));
     stats->playouts = total;
-    stats->plies = w->plies;
+    stats->plies = gpuai::total_plies(*w);
     stats->kernel_ms = ms;
-    stats->max_moves = w->max_moves;
-    stats->grid_blocks = g->grid;
-    stats->block_size = g->block;
-    stats->refill = g->refill;
+    stats->max_moves = gpuai::longest_list(*w);
+    stats->grid_blocks = g->pending_grid;
+    stats->block_size = g->pending_block;
+    stats->refill = g->pending_refill;
   }
   return MI_OK;
 }

@@ -1085,6 +1085,69 @@ CK_HD PlyResult ply_random_fast(Lane &L, uint32_t r, uint32_t *list_dig, bool &d
   return res;
 }
 
+// Slots of the moves of largest weight on a ply without longer capture sequences.
+// Single jumps: a move's weight depends only on whether it removes a king and whether a man lands
+// on the far row, so there are four classes (sm + 3p) / (so - (k ? 4 : 1)), each a set of slot
+// bits; the tied best classes give the slots.  Steps: a promotion weighs (sm + 3) / so > sm / so
+// unless so == 0 (all weights +inf).
+CK_HD void best_slots(const Lane &L, const Gen &g, uint32_t t[4]) {
+  const uint32_t sm = material(L.own, L.kings);
+  const uint32_t so = material(L.opp, L.kings);
+  const uint32_t men = L.own & ~L.kings;
+  if (!g.capture) {
+    const uint32_t pa = g.slot[0] & men & ROW6, pb = g.slot[1] & men & ROW6;
+    const bool promo = (pa | pb) && so != 0u;
+    t[0] = promo ? pa : g.slot[0];
+    t[1] = promo ? pb : g.slot[1];
+    t[2] = promo ? 0u : g.slot[2];
+    t[3] = promo ? 0u : g.slot[3];
+    return;
+  }
+  const uint32_t kng = L.own & L.kings;
+  const uint32_t okings = L.opp & L.kings;
+  // origins whose jump in direction d removes a king (the piece one step away in d)
+  const uint32_t kd0 = g.cap[0] & step3(okings), kd1 = g.cap[1] & step2(okings);
+  const uint32_t kd2 = g.cap[2] & step1(okings), kd3 = g.cap[3] & step0(okings);
+  // per slot (a man's slot 0 jumps in direction 1, its slot 1 in direction 0)
+  const uint32_t kc[4] = {g.slot[0] & ((men & kd1) | (kng & kd0)),
+                          g.slot[1] & ((men & kd0) | (kng & kd1)), g.slot[2] & kd2,
+                          g.slot[3] & kd3};
+  const uint32_t pr[4] = {g.slot[0] & men & ROW5, g.slot[1] & men & ROW5, 0u, 0u};
+  uint32_t any[4] = {0u, 0u, 0u, 0u};  // class c = 2 * promotion + king removed
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    any[0] |= g.slot[i] & ~kc[i] & ~pr[i];
+    any[1] |= kc[i] & ~pr[i];
+    any[2] |= pr[i] & ~kc[i];
+    any[3] |= kc[i] & pr[i];
+  }
+  uint32_t cn[4], cd[4];
+#pragma unroll
+  for (int c = 0; c < 4; c++) {
+    cn[c] = sm + ((c & 2) ? 3u : 0u);
+    cd[c] = so - ((c & 1) ? 4u : 1u);  // a class that occurs has that piece to remove
+  }
+  bool have = false;
+  uint32_t bn = 0, bd = 1;
+#pragma unroll
+  for (int c = 0; c < 4; c++) {
+    if (any[c] && (!have || cmp_weight(cn[c], cd[c], bn, bd) > 0)) {
+      bn = cn[c];
+      bd = cd[c];
+      have = true;
+    }
+  }
+  t[0] = t[1] = t[2] = t[3] = 0u;
+#pragma unroll
+  for (int c = 0; c < 4; c++) {
+    if (any[c] && cmp_weight(cn[c], cd[c], bn, bd) == 0) {
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+        t[i] |= ((c & 1) ? kc[i] : g.slot[i] & ~kc[i]) & ((c & 2) ? pr[i] : ~pr[i]);
+    }
+  }
+}
+
 // The heuristic ply after analyse.  WALK = false promises that no capture sequence is longer
 // than one jump (the caller deferred such plies), which drops the tree walks from the code.
 template <bool TRACE, bool WALK, class TAB = Direct>
@@ -1094,58 +1157,9 @@ CK_HD PlyResult heuristic_body(Lane &L, const Gen &g, uint32_t r, uint32_t *list
   const uint32_t sm = material(L.own, L.kings);
   const uint32_t so = material(L.opp, L.kings);
   uint32_t n = 0, ties = 0, bn = 0, bd = 1;
-  uint32_t tslot[4];
   const bool walked = WALK && g.capture && g.multi;  // sequences longer than one jump exist
-  if (g.capture && !walked) {
-    // Single jumps only: a move's weight depends only on whether it removes a king and whether
-    // a man lands on the far row, so there are four classes (sm + 3p) / (so - (k ? 4 : 1)),
-    // each a set of slot bits.  The tied best classes give the slots to choose from.
-    n = slot_count(g.slot);
-    const uint32_t men = L.own & ~L.kings, kng = L.own & L.kings;
-    const uint32_t okings = L.opp & L.kings;
-    // origins whose jump in direction d removes a king (the piece one step away in d)
-    const uint32_t kd0 = g.cap[0] & step3(okings), kd1 = g.cap[1] & step2(okings);
-    const uint32_t kd2 = g.cap[2] & step1(okings), kd3 = g.cap[3] & step0(okings);
-    // per slot (a man's slot 0 jumps in direction 1, its slot 1 in direction 0)
-    const uint32_t kc[4] = {g.slot[0] & ((men & kd1) | (kng & kd0)),
-                            g.slot[1] & ((men & kd0) | (kng & kd1)), g.slot[2] & kd2,
-                            g.slot[3] & kd3};
-    const uint32_t pr[4] = {g.slot[0] & men & ROW5, g.slot[1] & men & ROW5, 0u, 0u};
-    uint32_t any[4] = {0u, 0u, 0u, 0u};  // class c = 2 * promotion + king removed
-#pragma unroll
-    for (int t = 0; t < 4; t++) {
-      any[0] |= g.slot[t] & ~kc[t] & ~pr[t];
-      any[1] |= kc[t] & ~pr[t];
-      any[2] |= pr[t] & ~kc[t];
-      any[3] |= kc[t] & pr[t];
-    }
-    uint32_t cn[4], cd[4];
-#pragma unroll
-    for (int c = 0; c < 4; c++) {
-      cn[c] = sm + ((c & 2) ? 3u : 0u);
-      cd[c] = so - ((c & 1) ? 4u : 1u);  // a class that occurs has that piece to remove
-    }
-    bool have = false;
-#pragma unroll
-    for (int c = 0; c < 4; c++) {
-      if (any[c] && (!have || cmp_weight(cn[c], cd[c], bn, bd) > 0)) {
-        bn = cn[c];
-        bd = cd[c];
-        have = true;
-      }
-    }
-    tslot[0] = tslot[1] = tslot[2] = tslot[3] = 0u;
-#pragma unroll
-    for (int c = 0; c < 4; c++) {
-      if (any[c] && cmp_weight(cn[c], cd[c], bn, bd) == 0) {
-#pragma unroll
-        for (int t = 0; t < 4; t++) {
-          const uint32_t m = ((c & 1) ? kc[t] : g.slot[t] & ~kc[t]) & ((c & 2) ? pr[t] : ~pr[t]);
-          tslot[t] |= m;
-        }
-      }
-    }
-  } else if (g.capture) {
+  SlotWords tw;
+  if (walked) {
     uint32_t o = g.origins;
     uint32_t king = 0;
     auto leaf = [&](uint32_t to, uint32_t removed, uint32_t, uint32_t) {
@@ -1170,17 +1184,8 @@ CK_HD PlyResult heuristic_body(Lane &L, const Gen &g, uint32_t r, uint32_t *list
     }
   } else {
     n = slot_count(g.slot);
-    const uint32_t men = L.own & ~L.kings;
-    uint32_t pa = g.slot[0] & men & ROW6, pb = g.slot[1] & men & ROW6;
-    // a promotion weighs (sm + 3) / so > sm / so unless so == 0 (all weights +inf)
-    bool promo = (pa | pb) && so != 0u;
-    tslot[0] = promo ? pa : g.slot[0];
-    tslot[1] = promo ? pb : g.slot[1];
-    tslot[2] = promo ? 0u : g.slot[2];
-    tslot[3] = promo ? 0u : g.slot[3];
-  }
-  SlotWords tw;
-  if (!walked) {
+    uint32_t tslot[4];
+    best_slots(L, g, tslot);
     tw = slot_words(tslot);
     ties = tw.n;
   }

@@ -41,6 +41,7 @@ struct mi_ctx {
   hipStream_t stream = nullptr;
   hipEvent_t ev_start = nullptr, ev_stop = nullptr;
   mi_tuning tuning = kDefaultTuning;  // the shape of batches whose bucket the table lacks
+  bool shaped = false;  // `tuning` was given or measured: it holds for small batches too
   TuneEntry tune_table[3][kTuneBuckets][2];  // [policy][bucket][refill]
   uint32_t cus = 0, wave = 64, clock_khz = 0;
   gpuai::DevBuf pos, offs, winners, plies, hashes, work, tallies, moves, counts, keys;
@@ -77,6 +78,10 @@ int hip_fail(mi_ctx *ctx, hipError_t e, const char *what);
 int ensure(mi_ctx *ctx, DevBuf &b, size_t bytes);
 // Grows a pinned host buffer to at least `bytes` (the caller's stream must be idle).
 int ensure_host(mi_ctx *ctx, HostBuf &b, size_t bytes);
+// Batch-size bucket of the launch-shape table: floor(log2(total)).
+uint32_t tune_bucket(uint64_t total);
+// Whether a batch runs with one wave per game.
+bool wave_batch(const mi_ctx *ctx, uint32_t policy, uint64_t total);
 }  // namespace ctxutil
 // Looks up the device address of the allocation-free entry point's scratch array for the
 // context's device (once per device; the device must be current).

@@ -29,10 +29,26 @@ struct WorkWords {
   uint32_t pad0[28];
   struct alignas(128) QueueLine {
     uint32_t next;  // next unclaimed slab-local index (wave-level claims)
-    uint32_t pad[31];
+    // the same statistics from kernels whose every wave reports (k_playouts_wave), spread over
+    // the lines
+    uint32_t max_moves;
+    unsigned long long plies;
+    uint32_t pad[28];
   } queue[kSlabs];
 };
 static_assert(sizeof(WorkWords) == 128 * (1 + kSlabs), "header line + one line per slab");
+
+// Statistics of a launch, whichever kernel it ran.
+inline uint64_t total_plies(const WorkWords &w) {
+  uint64_t n = w.plies;
+  for (const auto &q : w.queue) n += q.plies;
+  return n;
+}
+inline uint32_t longest_list(const WorkWords &w) {
+  uint32_t n = w.max_moves;
+  for (const auto &q : w.queue) n = q.max_moves > n ? q.max_moves : n;
+  return n;
+}
 
 // Workgroups of a persistent launch for `need` workgroups' worth of work when `resident` fit on
 // the chip: a multiple of the slab count above it.
@@ -93,6 +109,11 @@ uint32_t playout_lds(uint32_t block);
 hipError_t launch_reset(WorkWords *work, hipStream_t stream);
 hipError_t launch_playouts(const PlayoutArgs &args, uint32_t policy, bool trace, uint32_t refill,
                            uint32_t grid, uint32_t block, hipStream_t stream);
+// One wave per game (wave_playouts.hip): `games` workgroups of kWaveBlock threads.  args.order is
+// not used (every game has a wave of its own); workgroups past the batch's total leave at once.
+constexpr uint32_t kWaveBlock = 64;
+hipError_t launch_playouts_wave(const PlayoutArgs &args, uint32_t policy, uint32_t games,
+                                hipStream_t stream);
 hipError_t launch_gen_moves(const mi_pos *pos, uint32_t npos, mi_move *moves, uint32_t cap,
                             uint32_t *counts, WorkWords *work, hipStream_t stream);
 hipError_t launch_start_positions(uint32_t seed, uint32_t n, uint32_t kmin, uint32_t kmax,

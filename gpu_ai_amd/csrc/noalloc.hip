@@ -147,7 +147,11 @@ __global__ void __launch_bounds__(kPrepThreads)
     }
   }
   if (t == 0u) {
-    for (uint32_t q = 0; q < kSlabs; q++) S->work.queue[q].next = 0u;
+    for (uint32_t q = 0; q < kSlabs; q++) {
+      S->work.queue[q].next = 0u;
+      S->work.queue[q].max_moves = 0u;
+      S->work.queue[q].plies = 0ull;
+    }
     S->work.max_moves = 0u;
     S->work.overflow = 0u;
     S->work.plies = 0ull;
@@ -230,6 +234,10 @@ extern "C" int mi_run_playouts_noalloc(mi_ctx *ctx, const mi_pos *pos, uint32_t 
   a.desc = &S->desc;
   // the grid as mi_run_playouts sizes it; with counts in device memory the total is unknown
   // here, so the whole resident grid runs (waves without work leave at their first refill)
+  if (!counts && gpuai::ctxutil::wave_batch(ctx, policy, uniform_total)) {
+    MI_HIP(ctx, gpuai::launch_playouts_wave(a, policy, (uint32_t)uniform_total, s));
+    return MI_OK;
+  }
   const uint64_t block = ctx->tuning.block_size;
   const uint64_t resident = (uint64_t)ctx->cus * ctx->tuning.blocks_per_cu;
   const uint64_t need = counts ? resident : (uniform_total + block - 1) / block;

@@ -43,7 +43,11 @@ __device__ __forceinline__ bool lane_in(uint64_t mask) {
 }
 
 __global__ void k_reset(WorkWords *work) {
-  if (threadIdx.x < kSlabs) work->queue[threadIdx.x].next = 0;
+  if (threadIdx.x < kSlabs) {
+    work->queue[threadIdx.x].next = 0;
+    work->queue[threadIdx.x].max_moves = 0;
+    work->queue[threadIdx.x].plies = 0ull;
+  }
   if (threadIdx.x == 0) {
     work->max_moves = 0;
     work->overflow = 0;
