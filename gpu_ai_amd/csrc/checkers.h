@@ -1590,6 +1590,34 @@ CK_HD PlyResult ply_noisy_fast(Lane &L, uint32_t r, uint32_t *list_dig, bool &de
   return res;
 }
 
+// Start positions (mi_gen_start_positions): plies of attempt `a` of position i, at most 2^16 (a
+// game ends long before: every capture is irreversible and 50 plies without one are a draw).
+CK_HD Lane start_position() { return lane_from_abs(0x00000FFFu, 0xFFF00000u, 0u, 0u, 0u); }
+CK_HD uint32_t start_plies(uint32_t seed, uint32_t i, uint32_t a, uint32_t kmin, uint32_t span) {
+  uint32_t w[4];
+  philox(0u, a, TAG_START, 1u, seed, i, w);
+  const uint32_t k = kmin + mod_u32(w[0], span);
+  return k < 0x10000u ? k : 0x10000u;
+}
+
+// The common part of a start position's ply: the random ply, but with `stop` the position is left
+// as it is.  res.over: the game is over; deferred: the ply waits for the walk phase.
+template <class TAB>
+CK_HD PlyResult ply_start_fast(Lane &L, uint32_t r, bool stop, bool &deferred, Gen &g,
+                               const TAB &tab) {
+  analyse(L, g);
+  const SlotWords w = slot_words(g.slot);
+  PlyResult res = {w.n, 0u, 0u, 0};
+  res.over = w.n == 0u || L.counter >= 50u;  // (an origin of longer captures has its slot's bit too)
+  deferred = g.multi != 0u && !res.over && !stop;
+  if (deferred || res.over || stop) return res;
+  const uint32_t k = tab.mod(r, w.n);
+  uint32_t sq, sl;
+  select_move(w, L.turn ? w.n - 1u - k : k, sq, sl, tab);
+  play_slot(L, g.capture, sq, sl, tab);
+  return res;
+}
+
 // True when the position is finished (no legal move, or the draw counter reached 50).
 CK_HD bool game_over(const Lane &L) {
   if (L.counter >= 50u) return true;

@@ -38,6 +38,18 @@ struct WorkWords {
 };
 static_assert(sizeof(WorkWords) == 128 * (1 + kSlabs), "header line + one line per slab");
 
+// The position of a lane's game (checkers.h: ck::Lane) as the ABI holds it.
+template <class LANE>
+__device__ __forceinline__ mi_pos packed_position(const LANE &L) {
+  mi_pos q;
+  lane_to_abs(L, q.p1, q.p2, q.kings);
+  q.turn = (uint8_t)L.turn;
+  q.counter = (uint8_t)(L.counter > 255u ? 255u : L.counter);
+  q.pad[0] = 0;
+  q.pad[1] = 0;
+  return q;
+}
+
 // Statistics of a launch, whichever kernel it ran.
 inline uint64_t total_plies(const WorkWords &w) {
   uint64_t n = w.plies;
@@ -116,9 +128,19 @@ hipError_t launch_playouts_wave(const PlayoutArgs &args, uint32_t policy, uint32
                                 hipStream_t stream);
 hipError_t launch_gen_moves(const mi_pos *pos, uint32_t npos, mi_move *moves, uint32_t cap,
                             uint32_t *counts, WorkWords *work, hipStream_t stream);
-hipError_t launch_start_positions(uint32_t seed, uint32_t n, uint32_t kmin, uint32_t kmax,
-                                  uint32_t reject_terminal, mi_pos *out, WorkWords *work,
-                                  hipStream_t stream);
+// Start positions (mi_gen_start_positions), n <= 2^30 of them into `out`: k in [kmin, kmin + span - 1] random
+// plies, with `reject` redrawn where the game is over.  work: reset before the launch; overflow is
+// set where kStartAttempts attempts all ended.
+struct StartArgs {
+  uint32_t seed, n, kmin, span, reject;
+  uint32_t base;   // index of the first position: its stream key
+  uint32_t slots;  // positions a wave works on at a time, 1..64
+  mi_pos *out;
+  WorkWords *work;
+};
+constexpr uint32_t kStartAttempts = 4096;
+constexpr uint32_t kStartBlock = 64;
+hipError_t launch_start_positions(const StartArgs &args, uint32_t grid, hipStream_t stream);
 hipError_t launch_divmod(const uint32_t *r, const uint32_t *n, uint32_t count, uint32_t *q,
                          uint32_t *rem, hipStream_t stream);
 hipError_t launch_copy(const uint4 *src, uint4 *dst, uint64_t n16, hipStream_t stream);

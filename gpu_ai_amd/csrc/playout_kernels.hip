@@ -42,6 +42,10 @@ __device__ __forceinline__ bool lane_in(uint64_t mask) {
   return __builtin_amdgcn_inverse_ballot_w64(mask);
 }
 
+__device__ __forceinline__ uint64_t rotate_right(uint64_t x, uint32_t n) {
+  return x >> n | x << ((64u - n) & 63u);
+}
+
 __global__ void k_reset(WorkWords *work) {
   if (threadIdx.x < kSlabs) {
     work->queue[threadIdx.x].next = 0;
@@ -381,39 +385,193 @@ __global__ void __launch_bounds__(256) k_tally(const int8_t *__restrict__ winner
   }
 }
 
-// One lane per start position (the stream layout of mi_gen_start_positions).
-__global__ void __launch_bounds__(256) k_start_positions(uint32_t seed, uint32_t n, uint32_t kmin,
-                                                         uint32_t kmax, uint32_t reject,
-                                                         mi_pos *__restrict__ out,
-                                                         WorkWords *work) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  ck::Lane L = ck::lane_from_abs(0x00000FFFu, 0xFFF00000u, 0u, 0u, 0u);
-  bool done = false;
-  for (uint32_t attempt = 0; attempt < 4096u && !done; attempt++) {
-    L = ck::lane_from_abs(0x00000FFFu, 0xFFF00000u, 0u, 0u, 0u);
-    uint32_t w[4];
-    ck::philox(0u, attempt, ck::TAG_START, 1u, seed, i, w);
-    const uint32_t k = kmin + ck::mod_u32(w[0], kmax - kmin + 1u);
-    for (uint32_t t = 0; t < k; t++) {
-      if ((t & 3u) == 0u) ck::philox(t >> 2, attempt, ck::TAG_START, 0u, seed, i, w);
-      uint32_t ld;
-      if (ck::ply_random<false>(L, w[t & 3u], &ld).over) break;
+// Start positions (the stream layout of mi_gen_start_positions): lanes play attempts, with
+// k_playouts' word rows and walk phase.  A position takes the first attempt that does not end
+// before its plies are played, and with kmax = 150 more than half of the attempts end: one lane per
+// position would run up to twenty in turn (a call for 262,144 positions took 1.7 ms that way).  So
+// each wave keeps up to a.slots positions open, and lanes that no position needs play the next
+// attempts of the open ones ahead; a position is decided when an attempt is accepted and all
+// before it have ended (1.05 ms, 0.72 of it the kernel; 64 positions 0.27 -> 0.16).
+// Slot q's position is kept by lane q: its attempts before `lo` have ended, those from `hi` on have
+// not begun; bit (attempt mod 64) of marks[q] tells which of those between (at most 64) ended, of
+// marks[64 + q] which were accepted.
+__global__ void __launch_bounds__(64) k_start_positions(StartArgs a) {
+  __shared__ LdsTables tables;
+  __shared__ uint32_t rows[kWordRows * 64u];
+  __shared__ unsigned long long marks[128];  // fails, accepts
+  __shared__ uint32_t decided[64], index[64], next[64], limits[64], list[64];
+  constexpr uint32_t kOpen = 0xFFFFFFFFu;  // in decided[]: no attempt yet
+  const uint32_t lane = threadIdx.x;
+  tables.fill();
+  marks[lane] = marks[64u + lane] = 0ull;
+  decided[lane] = kOpen;
+  __syncthreads();
+  const Lookup tab = {tables};
+  uint32_t *const words = rows + lane;
+  constexpr uint32_t kPly = 64u;  // as in k_playouts
+  // lanes that play an attempt, those of them that wait for the walk phase, and lanes that hold an
+  // accepted attempt's position
+  uint64_t active = 0, deferred = 0, held = 0;
+  uint64_t open = 0;           // slots with a position
+  uint32_t lo = 0, hi = 0;     // of this lane's slot
+  uint32_t slot = 0, i = 0, attempt = 0, ply = 0, limit = 0;
+  ck::Lane L = {0u, 0u, 0u, 0u, 0u};
+  ck::Gen gd;
+  uint32_t since_walk = 0;
+  // (few positions: one slab, since 16 slabs of blocks of kSlabBlock would leave most waves without)
+  const uint32_t nslabs = a.n < 32u * kSlabBlock * kSlabs ? 1u : min(gridDim.x, kSlabs);
+  const uint32_t slab = blockIdx.x % nslabs;
+  bool exhausted = false;
+  for (uint32_t iter = 0;; iter++) {
+    if ((iter & 3u) == 0u) {
+      __syncthreads();  // (one wave: orders the LDS accesses)
+      if (lane_in(open)) {
+        const uint32_t turn = lo & 63u;
+        const uint64_t f = rotate_right(marks[lane], turn);
+        const uint32_t ended = f == ~0ull ? 64u : (uint32_t)__builtin_ctzll(~f);
+        if (ended < 64u && (rotate_right(marks[64u + lane], turn) >> ended & 1u)) {
+          decided[lane] = lo + ended;
+        } else if (ended) {
+          const uint64_t gone = ended == 64u ? ~0ull : (1ull << ended) - 1ull;
+          marks[lane] &= ~rotate_right(gone, (64u - turn) & 63u);
+          lo += ended;
+        }
+      }
+      __syncthreads();
+      {  // a decided position: its attempt's lane writes it, the lanes of later attempts are free
+        const uint32_t by = lane_in(active | held) ? decided[slot] : kOpen;
+        if (by != kOpen && by == attempt) a.out[i] = packed_position(L);
+        const uint64_t gone = __ballot(by != kOpen);
+        active &= ~gone;
+        deferred &= ~gone;
+        held &= ~gone;
+      }
+      {  // close decided slots (a position all of whose attempts ended is reported)
+        const bool lost = lane_in(open) && lo == kStartAttempts;
+        if (lost) atomicOr(&a.work->overflow, 1u);
+        const bool close = lane_in(open) && (lost || decided[lane] != kOpen);
+        if (close) {
+          decided[lane] = kOpen;
+          marks[lane] = marks[64u + lane] = 0ull;
+        }
+        open &= ~__ballot(close);
+      }
+      // Idle lanes go to the open positions without an attempt, then to new positions, then to
+      // further attempts of the open ones: list[] names the slots in that order.
+      const uint64_t idle = ~(active | held);
+      const uint32_t cnt = (uint32_t)__popcll(idle);
+      const uint64_t bare = __ballot(lane_in(open) && lo == hi);
+      uint32_t named = (uint32_t)__popcll(bare);
+      if (lane_in(bare)) {
+        list[lane_rank(bare)] = lane;
+        next[lane] = hi++;
+      }
+      const uint32_t room = a.slots - min(a.slots, (uint32_t)__popcll(open));
+      const uint32_t want = min(cnt - named, room);
+      if (!exhausted && want) {
+        uint32_t c = 0;
+        if (lane == 0u) c = atomicAdd(&a.work->queue[slab].next, want);
+        c = __builtin_amdgcn_readfirstlane(c);
+        const uint32_t rank = lane_rank(~open);
+        const uint32_t at = slab_index(c + rank, slab, nslabs);
+        const bool taken = !lane_in(open) && rank < want && at < a.n;
+        if (taken) {
+          list[named + rank] = lane;
+          index[lane] = at;
+          next[lane] = lo = 0u;
+          hi = 1u;
+        }
+        const uint64_t fresh = __ballot(taken);
+        open |= fresh;
+        named += (uint32_t)__popcll(fresh);
+        exhausted = slab_index(c + want, slab, nslabs) >= a.n;
+      }
+      if (!open) {
+        if (exhausted) break;
+        continue;
+      }
+      const uint32_t spare = cnt - named, nopen = (uint32_t)__popcll(open);
+      const uint32_t ahead = hi;  // the first attempt that a spare lane may take here
+      __syncthreads();
+      const uint32_t rank = lane_rank(idle);
+      bool start = false;
+      if (lane_in(idle) && rank < named) {
+        slot = list[rank];
+        attempt = next[slot];
+        start = true;
+      }
+      if (spare && a.reject) {
+        __syncthreads();
+        const float per = 1.0f / (float)nopen;
+        if (lane_in(open)) {
+          const uint32_t r = lane_rank(open);
+          list[r] = lane;
+          next[lane] = ahead;
+          // spare lanes x = r, r + nopen, ... take attempts ahead, ahead + 1, ...
+          const uint32_t share = r < spare ? (uint32_t)(((float)(spare - 1u - r) + 0.5f) * per) + 1u : 0u;
+          const uint32_t top = min(lo + 64u, kStartAttempts);
+          hi = max(ahead, min(ahead + share, top));
+          limits[lane] = hi;
+        }
+        __syncthreads();
+        if (lane_in(idle) && rank >= named) {
+          const uint32_t x = rank - named;
+          const uint32_t q = (uint32_t)(((float)x + 0.5f) * per);
+          slot = list[x - q * nopen];
+          attempt = next[slot] + q;
+          start = attempt < limits[slot];
+        }
+      }
+      if (start) {
+        i = index[slot];
+        L = ck::start_position();
+        limit = ck::start_plies(a.seed, a.base + i, attempt, a.kmin, a.span) * kPly;
+        ply = 0;
+      }
+      active |= __ballot(start);
+      if (lane_in(active)) {
+        const uint32_t b = (ply / kPly + 3u) >> 2;
+        uint32_t o[4];
+        ck::philox(b, attempt, ck::TAG_START, 0u, a.seed, a.base + i, o);
+        uint32_t *const row = words + (b & 1u) * (4u * 64u);
+#pragma unroll
+        for (uint32_t w = 0; w < 4u; w++) row[w * 64u] = o[w];
+      }
     }
-    done = !reject || !ck::game_over(L);
+    {
+      const bool on = lane_in(active & ~deferred);
+      bool d = false, ended = false, accepted = false;
+      if (on) {
+        const uint32_t r = words[ply & ((kWordRows - 1u) * kPly)];
+        const bool stop = ply == limit;
+        const ck::PlyResult res = ck::ply_start_fast(L, r, stop, d, gd, tab);
+        ended = res.over || stop;
+        accepted = ended && !(res.over && a.reject);
+        if (ended) atomicOr(&marks[accepted ? 64u + slot : slot], 1ull << (attempt & 63u));
+        if (!d) ply += kPly;
+      }
+      deferred |= __ballot(d);
+      active &= ~__ballot(ended);
+      held |= __ballot(accepted);
+    }
+    if (deferred) {
+      const uint32_t nd = (uint32_t)__popcll(deferred);
+      if (nd >= 16u || deferred == active || since_walk >= 8u) {
+        since_walk = 0;
+        if (lane_in(deferred)) {
+          const uint32_t r = words[ply & ((kWordRows - 1u) * kPly)];
+          uint32_t unused = 0;
+          bool deep = false;  // (the game is not over: captures, and the draw count below 50)
+          ck::ply_random_trees<false>(L, gd, r, &unused, deep);
+          if (deep) ck::ply_random_given<false>(L, gd, r, &unused);
+          ply += kPly;
+        }
+        deferred = 0;
+      } else {
+        since_walk++;
+      }
+    }
   }
-  if (!done) atomicOr(&work->overflow, 1u);
-  uint32_t p1, p2, kings;
-  ck::lane_to_abs(L, p1, p2, kings);
-  mi_pos q;
-  q.p1 = p1;
-  q.p2 = p2;
-  q.kings = kings;
-  q.turn = (uint8_t)L.turn;
-  q.counter = (uint8_t)(L.counter > 255u ? 255u : L.counter);
-  q.pad[0] = 0;
-  q.pad[1] = 0;
-  out[i] = q;
 }
 
 __global__ void __launch_bounds__(256) k_divmod(const uint32_t *__restrict__ r,
@@ -521,13 +679,8 @@ hipError_t launch_gen_moves(const mi_pos *pos, uint32_t npos, mi_move *moves, ui
   return hipGetLastError();
 }
 
-hipError_t launch_start_positions(uint32_t seed, uint32_t n, uint32_t kmin, uint32_t kmax,
-                                  uint32_t reject_terminal, mi_pos *out, WorkWords *work,
-                                  hipStream_t stream) {
-  const uint32_t block = 256;
-  const uint32_t grid = (n + block - 1) / block;
-  hipLaunchKernelGGL(k_start_positions, dim3(grid), dim3(block), 0, stream, seed, n, kmin, kmax,
-                     reject_terminal, out, work);
+hipError_t launch_start_positions(const StartArgs &args, uint32_t grid, hipStream_t stream) {
+  hipLaunchKernelGGL(k_start_positions, dim3(grid), dim3(kStartBlock), 0, stream, args);
   return hipGetLastError();
 }
 

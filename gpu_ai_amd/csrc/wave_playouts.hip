@@ -70,8 +70,211 @@ __device__ __forceinline__ uint32_t last_not_above(const uint32_t *values, uint3
   return lo;
 }
 
+// What a lane looks at: its square s and the square's neighbours in directions A = 2h and
+// B = 2h + 1.
+struct Geometry {
+  uint32_t s, h, self;
+  uint32_t stepA, stepB, jumpA, jumpB;  // one step away, where a jump lands (0 off the board)
+  uint32_t wantA, wantB;                // what a valid jump's test yields
+  uint32_t squares;                     // the four squares' numbers (step A, B, jump A, B) in bytes
+  // The factor of r mod n for n = lane: n <= 49, since a step uses one of the board's 49 pairs of
+  // adjacent squares, a single jump one of 36 lines of three, and no two moves of a position share
+  // theirs.
+  uint32_t factor;
+};
+
+__device__ __forceinline__ Geometry geometry(uint32_t lane) {
+  Geometry q;
+  q.s = lane & 31u;
+  q.h = lane >> 5;
+  q.self = ck::bit(q.s);
+  q.stepA = q.h ? ck::step2(q.self) : ck::step0(q.self);
+  q.stepB = q.h ? ck::step3(q.self) : ck::step1(q.self);
+  q.jumpA = q.h ? ck::step2(q.stepA) : ck::step0(q.stepA);
+  q.jumpB = q.h ? ck::step3(q.stepB) : ck::step1(q.stepB);
+  q.wantA = q.jumpA ? q.stepA | q.jumpA : 0xFFFFFFFFu;
+  q.wantB = q.jumpB ? q.stepB | q.jumpB : 0xFFFFFFFFu;
+  q.squares = (31u - __clz(q.stepA | 1u)) | (31u - __clz(q.stepB | 1u)) << 8 |
+              (31u - __clz(q.jumpA | 1u)) << 16 | (31u - __clz(q.jumpB | 1u)) << 24;
+  q.factor = ck::mod_factor(lane);
+  return q;
+}
+
+// A stream of Philox words: that of ply t is word t & 3 of counter (t >> 2, c1, c2, c3).
+struct Stream {
+  uint32_t c1, c2, c3, seed, key;
+};
+
+// Plays a game from L to its end and counts its plies.  The scalar code works with masks (all ones
+// or zero) rather than flags: a flag becomes a pair of scalar registers and back at two or three
+// instructions each, nine cycles apiece where nothing else runs on the SIMD.
 template <uint32_t POLICY>
-__global__ void __launch_bounds__(64) k_playouts_wave(PlayoutArgs a) {
+__device__ __forceinline__ void play(ck::Lane &L, const Geometry &geo, const Stream &st,
+                                     uint32_t &ply, uint32_t &maxn) {
+  const uint32_t lane = geo.h << 5 | geo.s, s = geo.s, h = geo.h, self = geo.self;
+  const uint32_t stepA = geo.stepA, stepB = geo.stepB, jumpA = geo.jumpA, jumpB = geo.jumpB;
+  const uint32_t wantA = geo.wantA, wantB = geo.wantB, squares = geo.squares, factor = geo.factor;
+  uint32_t words = 0;  // this lane's Philox word: that of ply (ply & ~63) + lane
+  ply = 0;
+  auto refresh = [&]() {
+    if ((ply & 63u) == 0u) {
+      uint32_t o[4];
+      ck::philox((ply >> 2) + (lane >> 2), st.c1, st.c2, st.c3, st.seed, st.key, o);
+      const uint32_t w = lane & 3u;
+      words = w == 0u ? o[0] : w == 1u ? o[1] : w == 2u ? o[2] : o[3];
+    }
+  };
+  refresh();
+  // The inner loop plays plies until the game is over or one has longer capture sequences, which
+  // the outer loop plays (a loop of its own keeps the common plies' registers in place: 20% of the
+  // instructions were copies without it).
+  for (;;) {
+    uint64_t jA, jB, m0, m1, longer;
+    uint32_t r;
+    for (;;) {
+      longer = 0;
+      r = lane_value(words, ply & 63u);
+      // squares with a valid jump in A and B, whatever stands on them
+      const uint32_t empty = ~(L.own | L.opp);
+      const uint32_t kng = L.own & L.kings;
+      jA = __ballot(((L.opp & stepA) | (empty & jumpA)) == wantA);
+      jB = __ballot(((L.opp & stepB) | (empty & jumpB)) == wantB);
+      const uint64_t movers = pair(L.own, kng);  // pieces that move in the lanes' directions
+      // the moves' slots in reference order: slots 0 and 2 in m0, 1 and 3 in m1
+      uint32_t cap;  // all ones: captures are mandatory
+      if ((jA | jB) & movers) {
+        cap = 0xFFFFFFFFu;
+        const uint64_t men = L.own & ~L.kings, kings = pair(kng, kng);
+        m0 = (jA & kings) | (jB & men);  // a man's jump in direction 1 comes first
+        m1 = (jB & kings) | (jA & men);
+        // origins of longer sequences: a jump lands where the piece can jump on
+        const uint32_t fwd = lo32(jA) | lo32(jB), any = fwd | hi32(jA) | hi32(jB);
+        const uint64_t fA = __ballot((jumpA & fwd) != 0u), fB = __ballot((jumpB & fwd) != 0u);
+        const uint64_t aA = __ballot((jumpA & any) != 0u), aB = __ballot((jumpB & any) != 0u);
+        longer = (((jA & fA) | (jB & fB)) & men) | (((jA & aA) | (jB & aB)) & kings);
+        if (longer) break;
+      } else {
+        cap = 0u;
+        m0 = __ballot((empty & stepA) != 0u) & movers;
+        m1 = __ballot((empty & stepB) != 0u) & movers;
+      }
+      const uint32_t n = (uint32_t)__popcll(m0) + (uint32_t)__popcll(m1);
+      maxn = n > maxn ? n : maxn;
+      if (n == 0u || L.counter >= 50u) return;  // the game is over
+      uint32_t sq = 0, sl = 0, pick = 1u;  // pick: the word chooses among the moves in m0 and m1
+      uint32_t ties = n, first = 0u;       // first: every weight is +inf, index 0 wins
+      ck::Gen g;
+      if (POLICY != MI_POLICY_RANDOM) g = analysis(jA, jB, m0, m1, 0u, cap & 1u);
+      if (POLICY == MI_POLICY_HEURISTIC) {
+        uint32_t t[4];
+        ck::best_slots(L, g, t);
+        m0 = pair(t[0], t[2]);
+        m1 = pair(t[1], t[3]);
+        ties = (uint32_t)__popcll(m0) + (uint32_t)__popcll(m1);
+      }
+      if (POLICY == MI_POLICY_HEURISTIC_NOISY) {
+        const uint32_t sm = ck::material(L.own, L.kings), so = ck::material(L.opp, L.kings);
+        bool inf = false;
+        if (ck::single_weight(L, g, sm, so, inf)) {
+          first = inf ? 1u : 0u;
+        } else {
+          uint32_t kc[4], prom;
+          ck::weight_classes(L, g, kc, prom);
+          const uint32_t t0 = g.slot[0], t1 = g.slot[1], t2 = g.slot[2], t3 = g.slot[3];
+          // lane m draws for move m (n <= 49); lane (s, h) then takes the draws of its square's
+          // slots 2h and 2h + 1
+          float e0, e1;
+          ck::noise_pair(r, lane >> 1, e0, e1);
+          const float e = (lane & 1u) ? e1 : e0;
+          const uint32_t below = self - 1u;
+          uint32_t at = ck::popc(t0 & below) + ck::popc(t1 & below) + ck::popc(t2 & below) +
+                        ck::popc(t3 & below);
+          const uint32_t a0 = h ? t2 : t0, a1 = h ? t3 : t1;
+          at += h ? ck::getbit(t0, s) + ck::getbit(t1, s) : 0u;
+          const bool on0 = (a0 & self) != 0u, on1 = (a1 & self) != 0u;
+          float v0 = __shfl(e, at & 63u), v1 = __shfl(e, (at + (on0 ? 1u : 0u)) & 63u);
+          const uint32_t promo = (h == 0u && (prom & self)) ? 3u : 0u;
+          const uint32_t k0 = h ? kc[2] : kc[0], k1 = h ? kc[3] : kc[1];
+          const uint32_t d0 = g.capture ? ((k0 & self) ? 4u : 1u) : 0u;
+          const uint32_t d1 = g.capture ? ((k1 & self) ? 4u : 1u) : 0u;
+          {
+#pragma clang fp contract(off)
+            v0 = (float)(sm + promo) / (float)(so - d0) + v0;
+            v1 = (float)(sm + promo) / (float)(so - d1) + v1;
+          }
+          const float ninf = -__builtin_inff();
+          const float best = wave_max(fmaxf(on0 ? v0 : ninf, on1 ? v1 : ninf));
+          const uint64_t b0 = __ballot(on0 && v0 == best), b1 = __ballot(on1 && v1 == best);
+          // the first in reference order: player 2's is the reverse of the order here
+          const uint32_t hit = lo32(b0) | lo32(b1) | hi32(b0) | hi32(b1);
+          sq = L.turn ? 31u - (uint32_t)__builtin_clz(hit) : ck::ctz(hit);
+          const uint32_t on = ck::getbit(lo32(b0), sq) | ck::getbit(lo32(b1), sq) << 1 |
+                              ck::getbit(hi32(b0), sq) << 2 | ck::getbit(hi32(b1), sq) << 3;
+          sl = L.turn ? 31u - (uint32_t)__builtin_clz(on) : ck::ctz(on);
+          pick = 0u;
+        }
+      }
+      uint32_t king;  // all ones: the piece is a king
+      if (pick) {
+        const uint32_t k = first ? 0u : ck::mod_by(r, ties, lane_value(factor, ties));
+        const uint32_t tm = 0u - L.turn;
+        const uint32_t km = (k ^ tm) + (ties & tm);  // player 2: ties - 1 - k
+        // moves on lower squares, per lane of the first half; the last square where they are at most
+        // km holds the move
+        const uint32_t rank = __builtin_amdgcn_mbcnt_lo(
+            lo32(m0), __builtin_amdgcn_mbcnt_lo(
+                          lo32(m1), __builtin_amdgcn_mbcnt_lo(
+                                        hi32(m0), __builtin_amdgcn_mbcnt_lo(hi32(m1), 0u))));
+        sq = 31u - (uint32_t)__builtin_clz(lo32(__ballot(rank <= km)));
+        const uint32_t left = km - lane_value(rank, sq);
+        king = 0u - ck::getbit(L.kings, sq);
+        const uint32_t n0 = ck::getbit(lo32(m0), sq);
+        if (king) {
+          const uint32_t nibble = n0 | ck::getbit(lo32(m1), sq) << 1 |
+                                  ck::getbit(hi32(m0), sq) << 2 | ck::getbit(hi32(m1), sq) << 3;
+          sl = ck::nth_slot(nibble, left);
+        } else {
+          sl = left + 1u - n0;  // slots 0 and 1 alone: slot 1 if it is the second or the only one
+        }
+      } else {
+        king = 0u - ck::getbit(L.kings, sq);
+      }
+      const uint32_t d = sl ^ (cap & ~king & 1u);  // a man's capture slots name directions 1 and 0
+      const uint32_t near = lane_value(squares, sq | (d & 2u) << 4) >> ((d & 1u) * 8u);
+      const uint32_t one = ck::bit(near & 31u);
+      const uint32_t removed = one & cap;
+      const uint32_t flip = ck::bit(sq) | ck::bit((near >> (cap & 16u)) & 31u);
+      const uint32_t own = L.own ^ flip, opp = L.opp & ~removed;
+      const uint32_t kings = (L.kings & ~removed) ^ (flip & (king | ck::ROW7));
+      L.counter = (L.counter + 1u) & ~cap;
+      L.own = ck::brev(opp);
+      L.opp = ck::brev(own);
+      L.kings = ck::brev(kings);
+      L.turn ^= 1u;
+      ply++;
+      refresh();
+    }
+    const ck::Gen g = analysis(jA, jB, m0, m1, longer, 1u);
+    uint32_t unused = 0;
+    ck::PlyResult res;
+    if (POLICY == MI_POLICY_RANDOM) {
+      bool deep = false;
+      res = ck::ply_random_trees<false>(L, g, r, &unused, deep);
+      if (deep) res = ck::ply_random_given<false>(L, g, r, &unused);
+    } else if (POLICY == MI_POLICY_HEURISTIC) {
+      res = ck::ply_heuristic_given<false>(L, g, r, &unused);
+    } else {
+      res = ck::ply_noisy_given<false>(L, g, r, &unused);
+    }
+    maxn = res.n > maxn ? res.n : maxn;
+    if (res.over) return;
+    ply++;
+    refresh();
+  }
+}
+
+template <uint32_t POLICY>
+__global__ void __launch_bounds__(kWaveBlock) k_playouts_wave(PlayoutArgs a) {
   if (a.desc) {  // graph replays and allocation-free launches: the batch lives in device memory
     const LaunchDesc *d = a.desc;
     a.npos = d->npos;
@@ -102,185 +305,10 @@ __global__ void __launch_bounds__(64) k_playouts_wave(PlayoutArgs a) {
   const uint32_t key = a.keys ? uniform(a.keys[p]) : p;
   ck::Lane L = ck::lane_from_abs(uniform(q.p1), uniform(q.p2), uniform(q.kings),
                                  uniform(q.turn), uniform(q.counter));
-  // This lane's square and its neighbours in directions A = 2h and B = 2h + 1: the squares one
-  // step away (0 off the board), the squares a jump lands on, what a valid jump's test yields, and
-  // the four squares' numbers packed into bytes (step A, step B, jump A, jump B).
-  const uint32_t s = lane & 31u, h = lane >> 5, self = ck::bit(s);
-  const uint32_t stepA = h ? ck::step2(self) : ck::step0(self);
-  const uint32_t stepB = h ? ck::step3(self) : ck::step1(self);
-  const uint32_t jumpA = h ? ck::step2(stepA) : ck::step0(stepA);
-  const uint32_t jumpB = h ? ck::step3(stepB) : ck::step1(stepB);
-  const uint32_t wantA = jumpA ? stepA | jumpA : 0xFFFFFFFFu;
-  const uint32_t wantB = jumpB ? stepB | jumpB : 0xFFFFFFFFu;
-  const uint32_t squares = (31u - __clz(stepA | 1u)) | (31u - __clz(stepB | 1u)) << 8 |
-                           (31u - __clz(jumpA | 1u)) << 16 | (31u - __clz(jumpB | 1u)) << 24;
-  // The factor of r mod n, n <= 49: a step uses one of the board's 49 pairs of adjacent squares, a
-  // single jump one of 36 lines of three, and no two moves of one position share theirs.
-  const uint32_t factor = ck::mod_factor(lane);
-
-  // The scalar code below works with masks (all ones or zero) rather than flags: a flag becomes a
-  // pair of scalar registers and back at two or three instructions each, nine cycles apiece where
-  // nothing else runs on the SIMD.
-  uint32_t words = 0;  // this lane's Philox word: that of ply (ply & ~63) + lane
-  uint32_t maxn = 0, ply = 0;
-  auto refresh = [&]() {
-    if ((ply & 63u) == 0u) {
-      uint32_t o[4];
-      ck::philox((ply >> 2) + (lane >> 2), j, ck::TAG_PLAYOUT, a.epoch, a.seed, key, o);
-      const uint32_t w = lane & 3u;
-      words = w == 0u ? o[0] : w == 1u ? o[1] : w == 2u ? o[2] : o[3];
-    }
-  };
-  refresh();
-  // The inner loop plays plies until the game is over or one has longer capture sequences, which
-  // the outer loop plays (a loop of its own keeps the common plies' registers in place).
-  for (;;) {
-   uint64_t jA, jB, m0, m1, longer;
-   uint32_t r;
-   for (;;) {
-    longer = 0;
-    r = lane_value(words, ply & 63u);
-    // squares with a valid jump in A and B, whatever stands on them
-    const uint32_t empty = ~(L.own | L.opp);
-    const uint32_t kng = L.own & L.kings;
-    jA = __ballot(((L.opp & stepA) | (empty & jumpA)) == wantA);
-    jB = __ballot(((L.opp & stepB) | (empty & jumpB)) == wantB);
-    const uint64_t movers = pair(L.own, kng);  // pieces that move in the lanes' directions
-    // the moves' slots in reference order: slots 0 and 2 in m0, 1 and 3 in m1
-    uint32_t cap;  // all ones: captures are mandatory
-    if ((jA | jB) & movers) {
-      cap = 0xFFFFFFFFu;
-      const uint64_t men = L.own & ~L.kings, kings = pair(kng, kng);
-      m0 = (jA & kings) | (jB & men);  // a man's jump in direction 1 comes first
-      m1 = (jB & kings) | (jA & men);
-      // origins of longer sequences: a jump lands where the piece can jump on
-      const uint32_t fwd = lo32(jA) | lo32(jB), any = fwd | hi32(jA) | hi32(jB);
-      const uint64_t fA = __ballot((jumpA & fwd) != 0u), fB = __ballot((jumpB & fwd) != 0u);
-      const uint64_t aA = __ballot((jumpA & any) != 0u), aB = __ballot((jumpB & any) != 0u);
-      longer = (((jA & fA) | (jB & fB)) & men) | (((jA & aA) | (jB & aB)) & kings);
-      if (longer) break;
-    } else {
-      cap = 0u;
-      m0 = __ballot((empty & stepA) != 0u) & movers;
-      m1 = __ballot((empty & stepB) != 0u) & movers;
-    }
-    const uint32_t n = (uint32_t)__popcll(m0) + (uint32_t)__popcll(m1);
-    maxn = n > maxn ? n : maxn;
-    if (n == 0u || L.counter >= 50u) break;  // the game is over
-    uint32_t sq = 0, sl = 0, pick = 1u;  // pick: the word chooses among the moves in m0 and m1
-    uint32_t ties = n, first = 0u;       // first: every weight is +inf, index 0 wins
-    ck::Gen g;
-    if (POLICY != MI_POLICY_RANDOM) g = analysis(jA, jB, m0, m1, 0u, cap & 1u);
-    if (POLICY == MI_POLICY_HEURISTIC) {
-      uint32_t t[4];
-      ck::best_slots(L, g, t);
-      m0 = pair(t[0], t[2]);
-      m1 = pair(t[1], t[3]);
-      ties = (uint32_t)__popcll(m0) + (uint32_t)__popcll(m1);
-    }
-    if (POLICY == MI_POLICY_HEURISTIC_NOISY) {
-      const uint32_t sm = ck::material(L.own, L.kings), so = ck::material(L.opp, L.kings);
-      bool inf = false;
-      if (ck::single_weight(L, g, sm, so, inf)) {
-        first = inf ? 1u : 0u;
-      } else {
-        uint32_t kc[4], prom;
-        ck::weight_classes(L, g, kc, prom);
-        const uint32_t t0 = g.slot[0], t1 = g.slot[1], t2 = g.slot[2], t3 = g.slot[3];
-        // lane m draws for move m (n <= 49); lane (s, h) then takes the draws of its square's
-        // slots 2h and 2h + 1
-        float e0, e1;
-        ck::noise_pair(r, lane >> 1, e0, e1);
-        const float e = (lane & 1u) ? e1 : e0;
-        const uint32_t below = self - 1u;
-        uint32_t at = ck::popc(t0 & below) + ck::popc(t1 & below) + ck::popc(t2 & below) +
-                      ck::popc(t3 & below);
-        const uint32_t a0 = h ? t2 : t0, a1 = h ? t3 : t1;
-        at += h ? ck::getbit(t0, s) + ck::getbit(t1, s) : 0u;
-        const bool on0 = (a0 & self) != 0u, on1 = (a1 & self) != 0u;
-        float v0 = __shfl(e, at & 63u), v1 = __shfl(e, (at + (on0 ? 1u : 0u)) & 63u);
-        const uint32_t promo = (h == 0u && (prom & self)) ? 3u : 0u;
-        const uint32_t k0 = h ? kc[2] : kc[0], k1 = h ? kc[3] : kc[1];
-        const uint32_t d0 = g.capture ? ((k0 & self) ? 4u : 1u) : 0u;
-        const uint32_t d1 = g.capture ? ((k1 & self) ? 4u : 1u) : 0u;
-        {
-#pragma clang fp contract(off)
-          v0 = (float)(sm + promo) / (float)(so - d0) + v0;
-          v1 = (float)(sm + promo) / (float)(so - d1) + v1;
-        }
-        const float ninf = -__builtin_inff();
-        const float best = wave_max(fmaxf(on0 ? v0 : ninf, on1 ? v1 : ninf));
-        const uint64_t b0 = __ballot(on0 && v0 == best), b1 = __ballot(on1 && v1 == best);
-        // the first in reference order: player 2's is the reverse of the order here
-        const uint32_t hit = lo32(b0) | lo32(b1) | hi32(b0) | hi32(b1);
-        sq = L.turn ? 31u - (uint32_t)__builtin_clz(hit) : ck::ctz(hit);
-        const uint32_t on = ck::getbit(lo32(b0), sq) | ck::getbit(lo32(b1), sq) << 1 |
-                            ck::getbit(hi32(b0), sq) << 2 | ck::getbit(hi32(b1), sq) << 3;
-        sl = L.turn ? 31u - (uint32_t)__builtin_clz(on) : ck::ctz(on);
-        pick = 0u;
-      }
-    }
-    uint32_t king;  // all ones: the piece is a king
-    if (pick) {
-      const uint32_t k = first ? 0u : ck::mod_by(r, ties, lane_value(factor, ties));
-      const uint32_t tm = 0u - L.turn;
-      const uint32_t km = (k ^ tm) + (ties & tm);  // player 2: ties - 1 - k
-      // moves on lower squares, per lane of the first half; the last square where they are at most
-      // km holds the move
-      const uint32_t rank = __builtin_amdgcn_mbcnt_lo(
-          lo32(m0), __builtin_amdgcn_mbcnt_lo(
-                        lo32(m1), __builtin_amdgcn_mbcnt_lo(
-                                      hi32(m0), __builtin_amdgcn_mbcnt_lo(hi32(m1), 0u))));
-      sq = 31u - (uint32_t)__builtin_clz(lo32(__ballot(rank <= km)));
-      const uint32_t left = km - lane_value(rank, sq);
-      king = 0u - ck::getbit(L.kings, sq);
-      const uint32_t n0 = ck::getbit(lo32(m0), sq);
-      if (king) {
-        const uint32_t nibble = n0 | ck::getbit(lo32(m1), sq) << 1 |
-                                ck::getbit(hi32(m0), sq) << 2 | ck::getbit(hi32(m1), sq) << 3;
-        sl = ck::nth_slot(nibble, left);
-      } else {
-        sl = left + 1u - n0;  // slots 0 and 1 alone: slot 1 if it is the second or the only one
-      }
-    } else {
-      king = 0u - ck::getbit(L.kings, sq);
-    }
-    const uint32_t d = sl ^ (cap & ~king & 1u);  // a man's capture slots name directions 1 and 0
-    const uint32_t near = lane_value(squares, sq | (d & 2u) << 4) >> ((d & 1u) * 8u);
-    const uint32_t one = ck::bit(near & 31u);
-    const uint32_t removed = one & cap;
-    const uint32_t flip = ck::bit(sq) | ck::bit((near >> (cap & 16u)) & 31u);
-    const uint32_t own = L.own ^ flip, opp = L.opp & ~removed;
-    const uint32_t kings = (L.kings & ~removed) ^ (flip & (king | ck::ROW7));
-    L.counter = (L.counter + 1u) & ~cap;
-    L.own = ck::brev(opp);
-    L.opp = ck::brev(own);
-    L.kings = ck::brev(kings);
-    L.turn ^= 1u;
-    ply++;
-    refresh();
-   }
-   if (!longer) break;
-   const ck::Gen g = analysis(jA, jB, m0, m1, longer, 1u);
-   uint32_t unused = 0;
-   ck::PlyResult res;
-   if (POLICY == MI_POLICY_RANDOM) {
-     bool deep = false;
-     res = ck::ply_random_trees<false>(L, g, r, &unused, deep);
-     if (deep) res = ck::ply_random_given<false>(L, g, r, &unused);
-   } else if (POLICY == MI_POLICY_HEURISTIC) {
-     res = ck::ply_heuristic_given<false>(L, g, r, &unused);
-   } else {
-     res = ck::ply_noisy_given<false>(L, g, r, &unused);
-   }
-   maxn = res.n > maxn ? res.n : maxn;
-   if (res.over) break;
-   ply++;
-   refresh();
-  }
-  const int32_t winner = L.counter < 50u ? (int32_t)(L.turn ^ 1u) : -1;
+  uint32_t ply, maxn = 0;
+  play<POLICY>(L, geometry(lane), {j, ck::TAG_PLAYOUT, a.epoch, a.seed, key}, ply, maxn);
   if (lane == 0u) {
-    a.winners[game] = (int8_t)winner;
+    a.winners[game] = (int8_t)(L.counter < 50u ? (int32_t)(L.turn ^ 1u) : -1);
     WorkWords::QueueLine &line = a.work->queue[game % kSlabs];
     atomicAdd(&line.plies, (unsigned long long)ply);
     atomicMax(&line.max_moves, maxn);
