@@ -28,12 +28,11 @@ struct mi_mlp {
   double beta1 = 0.9, beta2 = 0.999, eps = 1e-8;  // rounded to float where a kernel takes them
   // parameters, Adam moments, gradients (FP32) and BF16 operand copies
   float *w = nullptr, *m = nullptr, *v = nullptr, *g = nullptr;
-  uint16_t *W1t = nullptr, *W2t = nullptr, *W2r = nullptr;
-  // one batch: network outputs, targets, loss; the transposed activations of a training step
-  // ([feature][max_rows]) and its per 32-row block partials of the vector gradients
+  uint16_t *W1f = nullptr, *W2f = nullptr, *W2rf = nullptr;
+  // one batch: network outputs, targets, loss; the activations of a training step in operand order
+  // (max_rows rows) and its per 32-row block partials of the vector gradients
   float *y = nullptr, *targets = nullptr, *loss = nullptr;
-  uint16_t *XT = nullptr, *H1T = nullptr, *dH2T = nullptr, *dH1T = nullptr;
-  float *P = nullptr;  // per 256-row split partials of dW1 and dW2
+  uint16_t *Xf = nullptr, *H1f = nullptr, *dH2f = nullptr, *dH1f = nullptr;
   float *pV = nullptr;
   mi_pos *pos = nullptr;
   // pinned host staging of one batch: positions (max_rows), then values and targets (max_rows
@@ -70,19 +69,18 @@ K::AdamArgs adam_args(mi_mlp *n, uint32_t rows, float lr, float c1, float c2, in
   a.m = n->m;
   a.v = n->v;
   a.grads = n->g;
-  a.XT = n->XT;
-  a.H1T = n->H1T;
-  a.dH2T = n->dH2T;
-  a.dH1T = n->dH1T;
+  a.Xf = n->Xf;
+  a.H1f = n->H1f;
+  a.dH2f = n->dH2f;
+  a.dH1f = n->dH1f;
   a.rows = rows;
-  a.ld = n->max_rows;
-  a.P = n->P;
+  a.slices = n->max_rows / 32u;
   a.splits = (rows + K::kWSplitRows - 1) / K::kWSplitRows;
   a.pV = n->pV;
   a.blocks = rows / K::kTrainRows;
-  a.W1t = n->W1t;
-  a.W2t = n->W2t;
-  a.W2r = n->W2r;
+  a.W1f = n->W1f;
+  a.W2f = n->W2f;
+  a.W2rf = n->W2rf;
   a.lr = lr;
   a.beta1 = (float)n->beta1;
   a.beta2 = (float)n->beta2;
@@ -130,15 +128,15 @@ int upload_params(mi_mlp *n, const float *w) {
   MI_HIP(ctx, K::zero(n->v, MI_MLP_PARAMS, ctx->stream));
   MI_HIP(ctx, K::zero(n->g, MI_MLP_PARAMS, ctx->stream));
   // refresh the BF16 copies without updating (no partials: every gradient reads as 0)
-  MI_HIP(ctx, K::wgrad_adam(adam_args(n, 0, 0.f, 1.f, 1.f, 0), ctx->stream));
+  MI_HIP(ctx, K::update(adam_args(n, 0, 0.f, 1.f, 1.f, 0), ctx->stream));
   MI_HIP(ctx, hipStreamSynchronize(ctx->stream));
   n->step = 0;
   return MI_OK;
 }
 
 // One training step over `rows` rows (count valid): k_train_rows' forward and backward pass to
-// the transposed activations and vector partials, then the weight-gradient partials and Adam
-// (k_wgrad_part, k_adam; when update == 0, only the gradient sums); loss_out (device, may be
+// the activations and vector partials, then the weight gradients and Adam (k_update; when
+// update == 0, only the gradient sums); loss_out (device, may be
 // null) receives the batch loss.  Row r is
 // pos[idx ? idx[r] : r] with target targets[idx ? idx[r] : r].
 int train_rows(mi_mlp *n, const mi_pos *pos, const uint32_t *idx, const float *targets,
@@ -149,18 +147,18 @@ int train_rows(mi_mlp *n, const mi_pos *pos, const uint32_t *idx, const float *t
   ta.idx = idx;
   ta.targets = targets;
   ta.n = count;
-  ta.ld = n->max_rows;
-  ta.W1t = n->W1t;
-  ta.W2t = n->W2t;
-  ta.W2r = n->W2r;
+  ta.slices = n->max_rows / 32u;
+  ta.W1f = n->W1f;
+  ta.W2f = n->W2f;
+  ta.W2rf = n->W2rf;
   ta.b1 = n->w + MI_MLP_OFF_B1;
   ta.b2 = n->w + MI_MLP_OFF_B2;
   ta.w3 = n->w + MI_MLP_OFF_W3;
   ta.b3 = n->w + MI_MLP_OFF_B3;
-  ta.XT = n->XT;
-  ta.H1T = n->H1T;
-  ta.dH2T = n->dH2T;
-  ta.dH1T = n->dH1T;
+  ta.Xf = n->Xf;
+  ta.H1f = n->H1f;
+  ta.dH2f = n->dH2f;
+  ta.dH1f = n->dH1f;
   ta.pV = n->pV;
   MI_HIP(ctx, K::train_rows(ta, rows, ctx->stream));
   // the bias corrections are formed in double precision, as Adam's usual implementations do
@@ -170,7 +168,7 @@ int train_rows(mi_mlp *n, const mi_pos *pos, const uint32_t *idx, const float *t
     c1 = (float)(1.0 / (1.0 - std::pow(n->beta1, (double)n->step)));
     c2 = (float)(1.0 / (1.0 - std::pow(n->beta2, (double)n->step)));
   }
-  MI_HIP(ctx, K::wgrad_adam(adam_args(n, rows, lr, c1, c2, update, loss_out), ctx->stream));
+  MI_HIP(ctx, K::update(adam_args(n, rows, lr, c1, c2, update, loss_out), ctx->stream));
   return MI_OK;
 }
 
@@ -226,18 +224,16 @@ int mi_mlp_create(mi_ctx *ctx, uint32_t max_batch, uint32_t seed, mi_mlp **out) 
   if (e == hipSuccess) e = dev_alloc(n, &n->m, P);
   if (e == hipSuccess) e = dev_alloc(n, &n->v, P);
   if (e == hipSuccess) e = dev_alloc(n, &n->g, P);
-  if (e == hipSuccess) e = dev_alloc(n, &n->W1t, (size_t)128 * 256);
-  if (e == hipSuccess) e = dev_alloc(n, &n->W2t, (size_t)256 * 256);
-  if (e == hipSuccess) e = dev_alloc(n, &n->W2r, (size_t)256 * 256);
+  if (e == hipSuccess) e = dev_alloc(n, &n->W1f, (size_t)128 * 256);
+  if (e == hipSuccess) e = dev_alloc(n, &n->W2f, (size_t)256 * 256);
+  if (e == hipSuccess) e = dev_alloc(n, &n->W2rf, (size_t)256 * 256);
   if (e == hipSuccess) e = dev_alloc(n, &n->y, R);
   if (e == hipSuccess) e = dev_alloc(n, &n->targets, R);
   if (e == hipSuccess) e = dev_alloc(n, &n->loss, 1);
-  if (e == hipSuccess) e = dev_alloc(n, &n->XT, 128 * R);
-  if (e == hipSuccess) e = dev_alloc(n, &n->H1T, 256 * R);
-  if (e == hipSuccess) e = dev_alloc(n, &n->dH2T, 256 * R);
-  if (e == hipSuccess) e = dev_alloc(n, &n->dH1T, 256 * R);
-  if (e == hipSuccess)
-    e = dev_alloc(n, &n->P, ((R + K::kWSplitRows - 1) / K::kWSplitRows) * (size_t)(32768 + 65536));
+  if (e == hipSuccess) e = dev_alloc(n, &n->Xf, 128 * R);
+  if (e == hipSuccess) e = dev_alloc(n, &n->H1f, 256 * R);
+  if (e == hipSuccess) e = dev_alloc(n, &n->dH2f, 256 * R);
+  if (e == hipSuccess) e = dev_alloc(n, &n->dH1f, 256 * R);
   if (e == hipSuccess) e = dev_alloc(n, &n->pV, (R / K::kTrainRows) * K::kVecSlots);
   if (e == hipSuccess) e = dev_alloc(n, &n->pos, R);
   if (e == hipSuccess)
@@ -308,7 +304,7 @@ int mi_mlp_forward(mi_mlp *n, const mi_pos *pos, uint32_t count, float *values) 
   if ((rc = use_device(n))) return rc;
   // one launch: encoding, both hidden layers and the output layer (k_forward)
   if ((rc = upload_positions(n, pos, count))) return rc;
-  MI_HIP(ctx, K::forward(n->pos, count, n->W1t, n->w + MI_MLP_OFF_B1, n->W2t, n->w + MI_MLP_OFF_B2,
+  MI_HIP(ctx, K::forward(n->pos, count, n->W1f, n->w + MI_MLP_OFF_B1, n->W2f, n->w + MI_MLP_OFF_B2,
                          n->w + MI_MLP_OFF_W3, n->w + MI_MLP_OFF_B3, n->y, ctx->stream));
   float *hv = stage_values(n);
   MI_HIP(ctx, hipMemcpyAsync(hv, n->y, sizeof(float) * count, hipMemcpyDeviceToHost, ctx->stream));
