@@ -39,9 +39,10 @@ struct mi_mlp {
   // floats each); copies from and to the caller's pageable buffers go through it, so the DMA
   // transfers need no driver-side staging
   void *h_stage = nullptr;
-  // device-resident training set
-  DevBuf ds_pos, ds_t, ds_perm, ds_loss;
+  // device-resident training set; ds_shuffle: the epoch shuffle's scratch
+  DevBuf ds_pos, ds_t, ds_perm, ds_loss, ds_shuffle;
   uint32_t ds_n = 0;
+  std::vector<uint32_t> host_perm;  // of small sets
   hipEvent_t e0 = nullptr, e1 = nullptr;
   std::vector<void *> allocs;
 };
@@ -172,6 +173,20 @@ int train_rows(mi_mlp *n, const mi_pos *pos, const uint32_t *idx, const float *t
   return MI_OK;
 }
 
+// The order of an epoch over at most this many positions is drawn on the host: four launches take
+// longer than 2 ns a position and one copy (64 positions: 50 against 70 us an epoch; 4099: alike).
+constexpr uint32_t kHostShuffle = 4096;
+
+// Fisher-Yates with Philox key (seed, epoch), counter (c >> 2, 0, 3, 1) (as K::shuffle).
+void host_shuffle(std::vector<uint32_t> &perm, uint32_t seed, uint32_t epoch) {
+  std::iota(perm.begin(), perm.end(), 0u);
+  uint32_t words[4];
+  for (uint32_t i = (uint32_t)perm.size() - 1, c = 0; i > 0; i--, c++) {
+    if ((c & 3) == 0) ck::philox(c >> 2, 0u, ck::TAG_MLP, 1u, seed, epoch, words);
+    std::swap(perm[i], perm[words[c & 3] % (i + 1)]);
+  }
+}
+
 int check_batch(mi_mlp *n, uint32_t count, const void *pos) {
   if (count == 0) return MI_OK;
   if (!pos) return fail(n->ctx, MI_ERR_INVALID_ARGUMENT, "null positions");
@@ -264,7 +279,8 @@ int mi_mlp_destroy(mi_mlp *n) {
   (void)hipStreamSynchronize(n->ctx->stream);
   for (void *p : n->allocs) (void)hipFree(p);
   if (n->h_stage) (void)hipHostFree(n->h_stage);
-  gpuai::DevBuf *bufs[] = {&n->ds_pos, &n->ds_t, &n->ds_perm, &n->ds_loss};
+  gpuai::DevBuf *bufs[] = {&n->ds_pos, &n->ds_t, &n->ds_perm, &n->ds_loss,
+                         &n->ds_shuffle};
   for (auto *b : bufs)
     if (b->ptr) (void)hipFree(b->ptr);
   if (n->e0) (void)hipEventDestroy(n->e0);
@@ -367,6 +383,8 @@ int mi_mlp_set_dataset(mi_mlp *n, const mi_pos *pos, const float *targets, uint3
   if ((rc = ensure(ctx, n->ds_pos, sizeof(mi_pos) * (size_t)std::max<uint32_t>(count, 1)))) return rc;
   if ((rc = ensure(ctx, n->ds_t, sizeof(float) * (size_t)std::max<uint32_t>(count, 1)))) return rc;
   if ((rc = ensure(ctx, n->ds_perm, sizeof(uint32_t) * (size_t)std::max<uint32_t>(count, 1)))) return rc;
+  if ((rc = ensure(ctx, n->ds_shuffle, 4 * sizeof(uint32_t) * (size_t)std::max<uint32_t>(count, 1))))
+    return rc;
   MI_HIP(ctx, hipMemcpyAsync(n->ds_pos.ptr, pos, sizeof(mi_pos) * count, hipMemcpyHostToDevice, ctx->stream));
   MI_HIP(ctx, hipMemcpyAsync(n->ds_t.ptr, targets, sizeof(float) * count, hipMemcpyHostToDevice, ctx->stream));
   MI_HIP(ctx, hipStreamSynchronize(ctx->stream));
@@ -385,18 +403,26 @@ int mi_mlp_train_epoch(mi_mlp *n, uint32_t batch, float lr, uint32_t shuffle_see
   const uint32_t nb = n->ds_n / batch;
   if (nb == 0) return fail(ctx, MI_ERR_INVALID_ARGUMENT, "the dataset holds less than one batch");
   if (int rc0 = use_device(n)) return rc0;
-  // Fisher-Yates with Philox key (shuffle_seed, epoch), counter (i >> 2, 0, 3, 1)
-  std::vector<uint32_t> perm(n->ds_n);
-  std::iota(perm.begin(), perm.end(), 0u);
-  uint32_t words[4];
-  for (uint32_t i = n->ds_n - 1, c = 0; i > 0; i--, c++) {
-    if ((c & 3) == 0) ck::philox(c >> 2, 0u, ck::TAG_MLP, 1u, shuffle_seed, epoch, words);
-    std::swap(perm[i], perm[words[c & 3] % (i + 1)]);
-  }
   int rc;
   if ((rc = ensure(ctx, n->ds_loss, sizeof(float) * nb))) return rc;
-  MI_HIP(ctx, hipMemcpyAsync(n->ds_perm.ptr, perm.data(), sizeof(uint32_t) * n->ds_n,
-                             hipMemcpyHostToDevice, ctx->stream));
+  if (n->ds_n <= kHostShuffle) {
+    std::vector<uint32_t> &perm = n->host_perm;
+    perm.resize(n->ds_n);
+    host_shuffle(perm, shuffle_seed, epoch);
+    MI_HIP(ctx, hipMemcpyAsync(n->ds_perm.ptr, perm.data(), sizeof(uint32_t) * n->ds_n,
+                               hipMemcpyHostToDevice, ctx->stream));
+  } else {
+    K::ShuffleArgs sh;
+    sh.n = n->ds_n;
+    sh.seed = shuffle_seed;
+    sh.epoch = epoch;
+    sh.head = (uint32_t *)n->ds_shuffle.ptr;
+    sh.next = sh.head + (size_t)n->ds_n;
+    sh.target = sh.next + (size_t)n->ds_n;
+    sh.chain = sh.target + (size_t)n->ds_n;
+    sh.order = (uint32_t *)n->ds_perm.ptr;
+    MI_HIP(ctx, K::shuffle(sh, ctx->stream));
+  }
   float *losses = (float *)n->ds_loss.ptr;
   MI_HIP(ctx, hipEventRecord(n->e0, ctx->stream));
   for (uint32_t b = 0; b < nb; b++) {

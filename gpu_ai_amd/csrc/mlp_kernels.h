@@ -59,6 +59,15 @@ hipError_t forward(const mi_pos *pos, uint32_t n, const uint16_t *W1f, const flo
                    hipStream_t stream);
 hipError_t train_rows(const TrainArgs &a, uint32_t rows, hipStream_t stream);
 hipError_t update(const AdamArgs &a, hipStream_t stream);
+
+// The order of an epoch over n >= 1 positions: a Fisher-Yates shuffle drawn from Philox key (seed,
+// epoch), counter (c >> 2, 0, 3, 1).  head, next, target, chain: n words of scratch each.
+struct ShuffleArgs {
+  uint32_t n, seed, epoch;
+  uint32_t *head, *next, *target, *chain;
+  uint32_t *order;
+};
+hipError_t shuffle(const ShuffleArgs &a, hipStream_t stream);
 hipError_t zero(float *p, uint32_t n, hipStream_t stream);
 
 }  // namespace mlp

@@ -21,6 +21,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "checkers.h"
 #include "mlp_kernels.h"
 
 namespace gpuai {
@@ -617,6 +618,64 @@ __global__ void __launch_bounds__(512) k_update(AdamArgs a) {
   adam_step(a, p, g, a.w[p], a.m[p], a.v[p]);
 }
 
+// An epoch's order: the Fisher-Yates shuffle p = 0..n-1, for i = n-1 .. 1 swap(p[i], p[j(i)]) with
+// j(i) = word (n-1-i) of the stream mod (i + 1), computed without running it.  Position i is last
+// touched at its own step, when it takes what stands on j(i).  What stands on position x at step i
+// <= x' was put there by the last step before i that targeted x, that is the smallest i' > i with
+// j(i') = x, and is what stood on i' at that step; without such a step it is x itself.  So with
+// chain(x) = the smallest i' > x with j(i') = x, the value comes from following chain() to its end.
+// The steps that target a position are linked in a list per position (k_shuffle_link; one or two
+// on average, ln n at most positions), chain() is read off the lists (k_shuffle_chain), and every
+// position follows its own (k_shuffle_order).  262,144 positions: 26 us against 0.7 ms on the host with
+// the upload of its result; 8M: 1.2 ms against 38.
+constexpr uint32_t kNone = 0xFFFFFFFFu;
+
+__global__ void __launch_bounds__(256) k_shuffle_clear(uint32_t *head, uint32_t n) {
+  const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+  if (i < n) head[i] = kNone;
+}
+
+// Smallest i' > i in the list of position x, or kNone.
+__device__ __forceinline__ uint32_t step_after(const uint32_t *head, const uint32_t *next, uint32_t x,
+                                               uint32_t i) {
+  uint32_t best = kNone;
+  for (uint32_t k = head[x]; k != kNone; k = next[k])
+    if (k > i && k < best) best = k;
+  return best;
+}
+
+__global__ void __launch_bounds__(256) k_shuffle_link(ShuffleArgs a) {
+  const uint32_t b = blockIdx.x * 256u + threadIdx.x;  // word block: steps n-1-4b .. n-4-4b
+  if (b >= (a.n + 2u) / 4u) return;                    // n - 1 steps
+  uint32_t w[4];
+  ck::philox(b, 0u, ck::TAG_MLP, 1u, a.seed, a.epoch, w);
+#pragma unroll
+  for (uint32_t k = 0; k < 4u; k++) {
+    const uint32_t c = 4u * b + k;
+    if (c + 1u >= a.n) return;
+    const uint32_t i = a.n - 1u - c, j = ck::mod_u32(w[k], i + 1u);
+    a.target[i] = j;
+    a.next[i] = atomicExch(&a.head[j], i);
+  }
+}
+
+__global__ void __launch_bounds__(256) k_shuffle_chain(ShuffleArgs a) {
+  const uint32_t x = blockIdx.x * 256u + threadIdx.x;
+  if (x < a.n) a.chain[x] = step_after(a.head, a.next, x, x);
+}
+
+__global__ void __launch_bounds__(256) k_shuffle_order(ShuffleArgs a) {
+  const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+  if (i >= a.n) return;
+  uint32_t x = i ? a.target[i] : 0u;
+  uint32_t k = step_after(a.head, a.next, x, i);
+  while (k != kNone) {  // (strictly ascending)
+    x = k;
+    k = a.chain[x];
+  }
+  a.order[i] = x;
+}
+
 __global__ void k_zero(float *p, uint32_t n) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = 0.f;
@@ -644,6 +703,16 @@ hipError_t update(const AdamArgs &a, hipStream_t stream) {
       a.splits != (a.rows + kWSplitRows - 1) / kWSplitRows)
     return hipErrorInvalidValue;
   hipLaunchKernelGGL(k_update, dim3(kTiles + kVecWgs), dim3(512), 0, stream, a);
+  return hipGetLastError();
+}
+
+hipError_t shuffle(const ShuffleArgs &a, hipStream_t stream) {
+  if (a.n == 0) return hipErrorInvalidValue;
+  const dim3 block(256), all((a.n + 255u) / 256u), words(((a.n + 2u) / 4u + 255u) / 256u);
+  hipLaunchKernelGGL(k_shuffle_clear, all, block, 0, stream, a.head, a.n);
+  if (a.n > 1u) hipLaunchKernelGGL(k_shuffle_link, words, block, 0, stream, a);
+  hipLaunchKernelGGL(k_shuffle_chain, all, block, 0, stream, a);
+  hipLaunchKernelGGL(k_shuffle_order, all, block, 0, stream, a);
   return hipGetLastError();
 }
 
