@@ -40,7 +40,8 @@ struct TrainArgs {
 // Weight gradients over the step's rows in splits of kWSplitRows, vector gradients from the row
 // pass's partials, and Adam (k_update).  rows = 0 takes every gradient as 0.
 struct AdamArgs {
-  float *w, *m, *v, *grads;
+  float *w, *m, *v;
+  float *grads;      // when set, receives every gradient
   const uint16_t *Xf, *H1f, *dH2f, *dH1f;  // as the row pass wrote them
   uint32_t rows, slices;
   uint32_t splits;   // ceil(rows / kWSplitRows)

@@ -459,7 +459,7 @@ __global__ void __launch_bounds__(512) k_train_rows(TrainArgs a) {
 // beforehand, together with the gradient's partials); returns the new value.
 __device__ __forceinline__ float adam_step(const AdamArgs &a, uint32_t p, float g, float w, float m,
                                            float v) {
-  a.grads[p] = g;
+  if (a.grads) a.grads[p] = g;
   if (a.update) {
     m = a.beta1 * m + a.omb1 * g;
     v = a.beta2 * v + a.omb2 * g * g;
