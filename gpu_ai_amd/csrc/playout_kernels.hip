@@ -8,11 +8,12 @@
 // instructions (every integer instruction, multiplications included, takes four cycles of a SIMD;
 // only reciprocals take longer), so what a ply would compute from small operands -- the factor of
 // r mod n, the j-th slot of a square, a move's masks -- and its Philox words are read from LDS,
-// one issue slot each, and flags of the lanes are wave masks in scalar registers: 355 -> 269
-// vector instructions per wave iteration on random-1024x1024, 0.778 -> 0.615 ms.  Refill policy MI_REFILL_QUEUE claims playout indices for the
-// whole wave in multiples of kChunk from its slab's device counter (one atomic per claim,
-// broadcast with a lane read; slabs are described in kernels.h), MI_REFILL_STATIC strides lanes
-// over the index space without atomics.
+// one issue slot each, flags of the lanes are wave masks in scalar registers (355 -> 269 vector
+// instructions per wave iteration on random-1024x1024, 0.778 -> 0.629 ms), and a walk phase takes
+// every origin's capture tree at once (ck::capture_trees; 0.577 ms).  Refill policy
+// MI_REFILL_QUEUE claims playout indices for the whole wave in multiples of kChunk from its slab's
+// device counter (one atomic per claim, broadcast with a lane read; slabs are described in
+// kernels.h), MI_REFILL_STATIC strides lanes over the index space without atomics.
 #include <hip/hip_runtime.h>
 
 #include "checkers.h"
@@ -99,6 +100,7 @@ __device__ __forceinline__ void locate(const PlayoutArgs &a, uint32_t g, uint32_
 struct LdsTables {
   uint32_t factor[ck::kModMax + 1];
   uint8_t nth[64];
+  uint32_t path[32];
   uint2 move[512];
 
   __device__ void fill() {
@@ -108,6 +110,7 @@ struct LdsTables {
       move[i] = m;
     }
     for (uint32_t i = threadIdx.x; i <= ck::kModMax; i += blockDim.x) factor[i] = ck::mod_factor(i);
+    if (threadIdx.x < 32u) path[threadIdx.x] = ck::path_word(threadIdx.x);
     if (threadIdx.x < 64u) nth[threadIdx.x] = (uint8_t)ck::nth_slot(threadIdx.x >> 2, threadIdx.x & 3u);
   }
 };
@@ -115,6 +118,8 @@ struct LdsTables {
 struct Lookup {
   const LdsTables &t;
   __device__ uint32_t mod(uint32_t r, uint32_t n) const { return ck::mod_by(r, n, t.factor[n]); }
+  __device__ uint32_t kth(uint32_t m, uint32_t j) const { return t.nth[m * 4u + j]; }
+  __device__ uint32_t path(uint32_t i) const { return t.path[i]; }
   __device__ uint32_t nth(uint32_t y, uint32_t j) const { return t.nth[ck::gather4(y) + j]; }
   __device__ void move(uint32_t i, uint32_t &flip, uint32_t &removed) const {
     const uint2 m = t.move[i];
@@ -274,7 +279,7 @@ __global__ void __launch_bounds__(1024) k_playouts(PlayoutArgs a) {
           if (POLICY == MI_POLICY_RANDOM) {
             // capture trees in closed form; the walk only for king trees past two jumps
             bool deep = false;
-            res = ck::ply_random_trees<TRACE>(L, gd, r, &ld, deep);
+            res = ck::ply_random_captures<TRACE>(L, gd, r, &ld, deep, tab);
             if (deep) res = ck::ply_random_given<TRACE>(L, gd, r, &ld);
           }
           else if (POLICY == MI_POLICY_HEURISTIC) res = ck::ply_heuristic_given<TRACE>(L, gd, r, &ld);
@@ -562,7 +567,7 @@ __global__ void __launch_bounds__(64) k_start_positions(StartArgs a) {
           const uint32_t r = words[ply & ((kWordRows - 1u) * kPly)];
           uint32_t unused = 0;
           bool deep = false;  // (the game is not over: captures, and the draw count below 50)
-          ck::ply_random_trees<false>(L, gd, r, &unused, deep);
+          ck::ply_random_captures<false>(L, gd, r, &unused, deep, tab);
           if (deep) ck::ply_random_given<false>(L, gd, r, &unused);
           ply += kPly;
         }
