@@ -1262,81 +1262,86 @@ CK_HD PlyResult ply_random_fast(Lane &L, uint32_t r, uint32_t *list_dig, bool &d
   return res;
 }
 
-// Slots of the moves of largest weight on a ply without longer capture sequences.
-// Single jumps: a move's weight depends only on whether it removes a king and whether a man lands
-// on the far row, so there are four classes (sm + 3p) / (so - (k ? 4 : 1)), each a set of slot
-// bits; the tied best classes give the slots.  Steps: a promotion weighs (sm + 3) / so > sm / so
-// unless so == 0 (all weights +inf).
-CK_HD void best_slots(const Lane &L, const Gen &g, uint32_t t[4]) {
-  const uint32_t sm = material(L.own, L.kings);
-  const uint32_t so = material(L.opp, L.kings);
-  const uint32_t men = L.own & ~L.kings;
-  if (!g.capture) {
-    const uint32_t pa = g.slot[0] & men & ROW6, pb = g.slot[1] & men & ROW6;
-    const bool promo = (pa | pb) && so != 0u;
-    t[0] = promo ? pa : g.slot[0];
-    t[1] = promo ? pb : g.slot[1];
-    t[2] = promo ? 0u : g.slot[2];
-    t[3] = promo ? 0u : g.slot[3];
-    return;
-  }
-  const uint32_t kng = L.own & L.kings;
+// How the weights of a ply's moves differ, where no capture sequence is longer than one jump.  A
+// step weighs sm / so, or (sm + 3) / so when it promotes a man; a jump (sm + 3p) / (so - (k ? 4 : 1))
+// by whether it promotes (p) and removes a king (k).  Most plies' moves all weigh the same, which
+// takes no materials to see: one ply in a thousand has single jumps of several weights (the walk,
+// which computes weights, plays those) and one in 27 steps of two (noisy games from 20 to 60 plies
+// on).  Sorting the moves into weight classes on every ply took a third more cycles than the random
+// ply: heuristic-1024x1024 0.59 ms, now 0.52.
+//
+// Men whose moves in slots 0 and 1 promote.
+CK_HD uint32_t promoting(const Lane &L, const Gen &g) {
+  return L.own & ~L.kings & (g.capture ? ROW5 : ROW6);
+}
+// Whether some moves promote and some do not.
+CK_HD bool some_promote(const Gen &g, uint32_t prom) {
+  const uint32_t men = g.slot[0] | g.slot[1];
+  return (men & prom) && ((men & ~prom) | g.slot[2] | g.slot[3]);
+}
+// Whether some jumps remove a king and some do not.
+CK_HD bool some_take_kings(const Lane &L, const Gen &g) {
   const uint32_t okings = L.opp & L.kings;
-  // origins whose jump in direction d removes a king (the piece one step away in d)
-  const uint32_t kd0 = g.cap[0] & step3(okings), kd1 = g.cap[1] & step2(okings);
-  const uint32_t kd2 = g.cap[2] & step1(okings), kd3 = g.cap[3] & step0(okings);
-  // per slot (a man's slot 0 jumps in direction 1, its slot 1 in direction 0)
-  const uint32_t kc[4] = {g.slot[0] & ((men & kd1) | (kng & kd0)),
-                          g.slot[1] & ((men & kd0) | (kng & kd1)), g.slot[2] & kd2,
-                          g.slot[3] & kd3};
-  const uint32_t pr[4] = {g.slot[0] & men & ROW5, g.slot[1] & men & ROW5, 0u, 0u};
-  uint32_t any[4] = {0u, 0u, 0u, 0u};  // class c = 2 * promotion + king removed
-#pragma unroll
-  for (int i = 0; i < 4; i++) {
-    any[0] |= g.slot[i] & ~kc[i] & ~pr[i];
-    any[1] |= kc[i] & ~pr[i];
-    any[2] |= pr[i] & ~kc[i];
-    any[3] |= kc[i] & pr[i];
-  }
-  uint32_t cn[4], cd[4];
-#pragma unroll
-  for (int c = 0; c < 4; c++) {
-    cn[c] = sm + ((c & 2) ? 3u : 0u);
-    cd[c] = so - ((c & 1) ? 4u : 1u);  // a class that occurs has that piece to remove
-  }
-  bool have = false;
-  uint32_t bn = 0, bd = 1;
-#pragma unroll
-  for (int c = 0; c < 4; c++) {
-    if (any[c] && (!have || cmp_weight(cn[c], cd[c], bn, bd) > 0)) {
-      bn = cn[c];
-      bd = cd[c];
-      have = true;
-    }
-  }
-  t[0] = t[1] = t[2] = t[3] = 0u;
-#pragma unroll
-  for (int c = 0; c < 4; c++) {
-    if (any[c] && cmp_weight(cn[c], cd[c], bn, bd) == 0) {
-#pragma unroll
-      for (int i = 0; i < 4; i++)
-        t[i] |= ((c & 1) ? kc[i] : g.slot[i] & ~kc[i]) & ((c & 2) ? pr[i] : ~pr[i]);
-    }
-  }
+  const uint32_t k0 = step3(okings), k1 = step2(okings);  // next to a king in direction 0, 1
+  // a man's slot 0 jumps in direction 1, its slot 1 in direction 0
+  const uint32_t s0 = (L.kings & k0) | (~L.kings & k1), s1 = (L.kings & k1) | (~L.kings & k0);
+  const uint32_t s2 = step1(okings), s3 = step0(okings);
+  const uint32_t with = (g.slot[0] & s0) | (g.slot[1] & s1) | (g.slot[2] & s2) | (g.slot[3] & s3);
+  const uint32_t without =
+      (g.slot[0] & ~s0) | (g.slot[1] & ~s1) | (g.slot[2] & ~s2) | (g.slot[3] & ~s3);
+  return with && without;
 }
 
-// The heuristic ply after analyse.  WALK = false promises that no capture sequence is longer
-// than one jump (the caller deferred such plies), which drops the tree walks from the code.
-template <bool TRACE, bool WALK, class TAB = Direct>
-CK_HD PlyResult heuristic_body(Lane &L, const Gen &g, uint32_t r, uint32_t *list_dig,
-                               const TAB &tab = TAB()) {
+// The heuristic ply whose moves of largest weight are those of the squares `from` (every move of a
+// square in them).
+template <bool TRACE, class TAB>
+CK_HD PlyResult play_tied(Lane &L, const Gen &g, uint32_t from, uint32_t r, uint32_t *list_dig,
+                          const TAB &tab) {
+  PlyResult res;
+  const uint32_t n = slot_count(g.slot);
+  res.n = n;
+  if (TRACE) *list_dig = list_digest(L, g, n);
+  if (n == 0u || L.counter >= 50u) {
+    res.over = 1u;
+    res.chosen = 0xFFFFu;
+    res.winner = L.counter < 50u ? (int32_t)(L.turn ^ 1u) : -1;
+    return res;
+  }
+  const uint32_t t[4] = {g.slot[0] & from, g.slot[1] & from, g.slot[2] & from, g.slot[3] & from};
+  const SlotWords tw = slot_words(t);
+  const uint32_t k = tab.mod(r, tw.n);
+  res.over = 0u;
+  res.winner = 0;
+  res.chosen = 0u;
+  uint32_t sq, sl;
+  select_move(tw, L.turn ? tw.n - 1u - k : k, sq, sl, tab);
+  if (TRACE) {
+    // reference index: rank of (sq, sl) in the full slot order
+    const uint32_t below = bit(sq) - 1u;
+    uint32_t i = popc(g.slot[0] & below) + popc(g.slot[1] & below) + popc(g.slot[2] & below) +
+                 popc(g.slot[3] & below);
+    for (uint32_t s = 0; s < sl; s++) i += getbit(g.slot[s], sq);
+    res.chosen = L.turn ? n - 1u - i : i;
+  }
+  play_slot(L, g.capture, sq, sl, tab);
+  return res;
+}
+
+// Squares of the steps of largest weight: those that promote, where some do (with no opponent left
+// every weight is +inf).
+CK_HD uint32_t best_steps(const Lane &L, const Gen &g) {
+  const uint32_t prom = promoting(L, g);
+  return some_promote(g, prom) && L.opp ? prom : 0xFFFFFFFFu;
+}
+
+// The heuristic capture ply by the walk.
+template <bool TRACE>
+CK_HD PlyResult heuristic_walk(Lane &L, const Gen &g, uint32_t r, uint32_t *list_dig) {
   PlyResult res;
   const uint32_t sm = material(L.own, L.kings);
   const uint32_t so = material(L.opp, L.kings);
   uint32_t n = 0, ties = 0, bn = 0, bd = 1;
-  const bool walked = WALK && g.capture && g.multi;  // sequences longer than one jump exist
-  SlotWords tw;
-  if (walked) {
+  {
     uint32_t o = g.origins;
     uint32_t king = 0;
     auto leaf = [&](uint32_t to, uint32_t removed, uint32_t, uint32_t) {
@@ -1359,97 +1364,76 @@ CK_HD PlyResult heuristic_body(Lane &L, const Gen &g, uint32_t r, uint32_t *list
       king = getbit(L.kings, s);
       walk(s, king, g.cap, leaf);
     }
-  } else {
-    n = slot_count(g.slot);
-    uint32_t tslot[4];
-    best_slots(L, g, tslot);
-    tw = slot_words(tslot);
-    ties = tw.n;
   }
   res.n = n;
   if (TRACE) *list_dig = list_digest(L, g, n);
-  if (n == 0u || L.counter >= 50u) {
+  if (L.counter >= 50u) {  // (a capture ply always has moves)
     res.over = 1u;
     res.chosen = 0xFFFFu;
-    res.winner = L.counter < 50u ? (int32_t)(L.turn ^ 1u) : -1;
+    res.winner = -1;
     return res;
   }
-  uint32_t k = walked ? mod_small(r, ties) : tab.mod(r, ties);
-  uint32_t km = L.turn ? ties - 1u - k : k;
+  const uint32_t k = mod_small(r, ties);
   res.over = 0u;
   res.winner = 0;
   Choice c = {0u, 0u, 0u};
-  if (walked) {
-    uint32_t o = g.origins;
-    uint32_t king = 0, left = km, idx = 0;
-    bool found = false;
-    auto leaf = [&](uint32_t to, uint32_t removed, uint32_t, uint32_t) {
-      uint32_t num = sm + ((!king && to >= FAR_ROW_FIRST) ? 3u : 0u);
-      uint32_t den = so - material(removed, L.kings);
-      if (cmp_weight(num, den, bn, bd) == 0) {
-        if (left == 0u) {
-          c.to = to;
-          c.removed = removed;
-          found = true;
-          return true;
-        }
-        left--;
+  uint32_t o = g.origins;
+  uint32_t king = 0, left = L.turn ? ties - 1u - k : k, idx = 0;
+  bool found = false;
+  auto leaf = [&](uint32_t to, uint32_t removed, uint32_t, uint32_t) {
+    uint32_t num = sm + ((!king && to >= FAR_ROW_FIRST) ? 3u : 0u);
+    uint32_t den = so - material(removed, L.kings);
+    if (cmp_weight(num, den, bn, bd) == 0) {
+      if (left == 0u) {
+        c.to = to;
+        c.removed = removed;
+        found = true;
+        return true;
       }
-      idx++;
-      return false;
-    };
-    while (o && !found) {
-      uint32_t s = ctz(o);
-      o &= o - 1u;
-      king = getbit(L.kings, s);
-      c.from = s;
-      walk(s, king, g.cap, leaf);
+      left--;
     }
-    // reference index of the chosen move (for the trace record)
-    res.chosen = L.turn ? n - 1u - idx : idx;
-  } else {
-    uint32_t sq, sl;
-    select_move(tw, km, sq, sl, tab);
-    if (TRACE) {
-      // reference index: rank of (sq, sl) in the full slot order
-      uint32_t below = bit(sq) - 1u;
-      uint32_t i = popc(g.slot[0] & below) + popc(g.slot[1] & below) + popc(g.slot[2] & below) +
-                   popc(g.slot[3] & below);
-      for (uint32_t t = 0; t < sl; t++) i += getbit(g.slot[t], sq);
-      res.chosen = L.turn ? n - 1u - i : i;
-    } else {
-      res.chosen = 0u;
-    }
-    play_slot(L, g.capture, sq, sl, tab);
-    return res;
+    idx++;
+    return false;
+  };
+  while (o && !found) {
+    uint32_t s = ctz(o);
+    o &= o - 1u;
+    king = getbit(L.kings, s);
+    c.from = s;
+    walk(s, king, g.cap, leaf);
   }
+  // reference index of the chosen move (for the trace record)
+  res.chosen = L.turn ? n - 1u - idx : idx;
   apply(L, c.from, c.to, c.removed);
   return res;
 }
 
-// Plays one ply of the heuristic policy with word r (src/heuristicPlayout.cpp:20-42 without
-// the noise; ties broken by T[r mod |T|]).
+// The heuristic ply given the position's analysis g (src/heuristicPlayout.cpp:20-42 without the
+// noise; ties broken by T[r mod |T|]).
+template <bool TRACE>
+CK_HD PlyResult ply_heuristic_given(Lane &L, const Gen &g, uint32_t r, uint32_t *list_dig) {
+  if (g.capture) return heuristic_walk<TRACE>(L, g, r, list_dig);
+  return play_tied<TRACE>(L, g, best_steps(L, g), r, list_dig, Direct());
+}
+
+// Plays one ply of the heuristic policy with word r.
 template <bool TRACE>
 CK_HD PlyResult ply_heuristic(Lane &L, uint32_t r, uint32_t *list_dig) {
   Gen g;
   analyse(L, g);
-  return heuristic_body<TRACE, true>(L, g, r, list_dig);
+  return ply_heuristic_given<TRACE>(L, g, r, list_dig);
 }
 
-// The heuristic ply given the position's analysis g.
-template <bool TRACE>
-CK_HD PlyResult ply_heuristic_given(Lane &L, const Gen &g, uint32_t r, uint32_t *list_dig) {
-  return heuristic_body<TRACE, true>(L, g, r, list_dig);
-}
-
-// The common part of a heuristic ply: plays it unless it is a capture ply with a sequence
-// longer than one jump, which is left untouched with `deferred` set (the caller plays it later
-// with ply_heuristic_given, the same word and the analysis left in g).
+// The common part of a heuristic ply: plays it unless it is a capture ply with a sequence longer
+// than one jump or with jumps of several kinds, which is left untouched with `deferred` set (the
+// caller plays it later with ply_heuristic_given, the same word and the analysis left in g).
 template <bool TRACE, class TAB = Direct>
 CK_HD PlyResult ply_heuristic_fast(Lane &L, uint32_t r, uint32_t *list_dig, bool &deferred,
                                    Gen &g, const TAB &tab = TAB()) {
   analyse(L, g);
-  deferred = g.capture && g.multi;
+  const uint32_t prom = promoting(L, g);
+  const bool split = some_promote(g, prom);
+  deferred = g.capture && (g.multi || split || some_take_kings(L, g));
   if (deferred) {
     PlyResult res;
     res.n = 0u;
@@ -1458,7 +1442,7 @@ CK_HD PlyResult ply_heuristic_fast(Lane &L, uint32_t r, uint32_t *list_dig, bool
     res.winner = 0;
     return res;
   }
-  return heuristic_body<TRACE, false>(L, g, r, list_dig, tab);
+  return play_tied<TRACE>(L, g, split && L.opp ? prom : 0xFFFFFFFFu, r, list_dig, tab);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1555,68 +1539,16 @@ CK_HD bool noisy_take(NoisyBest &nb, uint32_t r, float w) {
   return take;
 }
 
-// Weight classes of a ply without longer capture sequences, as slot masks: kc[t] = the move of
-// slot t removes a king, prom = the men whose slot-0/1 move promotes.
-CK_HD void weight_classes(const Lane &L, const Gen &g, uint32_t kc[4], uint32_t &prom) {
-  const uint32_t men = L.own & ~L.kings;
-  kc[0] = kc[1] = kc[2] = kc[3] = 0u;
-  if (g.capture) {
-    const uint32_t kng = L.own & L.kings;
-    const uint32_t okings = L.opp & L.kings;
-    const uint32_t kd0 = g.cap[0] & step3(okings), kd1 = g.cap[1] & step2(okings);
-    kc[0] = g.slot[0] & ((men & kd1) | (kng & kd0));
-    kc[1] = g.slot[1] & ((men & kd0) | (kng & kd1));
-    kc[2] = g.slot[2] & g.cap[2] & step1(okings);
-    kc[3] = g.slot[3] & g.cap[3] & step0(okings);
-  }
-  prom = men & (g.capture ? ROW5 : ROW6);
-}
-
-// Whether every move of such a ply weighs the same; `inf` when that weight is +inf (the mover
-// takes the opponent's last piece, or the opponent has none).
-CK_HD bool single_weight(const Lane &L, const Gen &g, uint32_t sm, uint32_t so, bool &inf) {
-  uint32_t kc[4], prom;
-  weight_classes(L, g, kc, prom);
-  const uint32_t n = slot_count(g.slot);
-  const uint32_t np = popc(g.slot[0] & prom) + popc(g.slot[1] & prom);
-  if (!g.capture) {  // steps: sm / so and, for promotions, (sm + 3) / so
-    inf = so == 0u;
-    return inf || np == 0u || np == n;
-  }
-  // single jumps: (sm + 3p) / (so - (k ? 4 : 1)) over the classes that occur
-  const uint32_t nk = popc(kc[0]) + popc(kc[1]) + popc(kc[2]) + popc(kc[3]);
-  const uint32_t nkp = popc(kc[0] & prom) + popc(kc[1] & prom);
-  const uint32_t cnt[4] = {n - nk - np + nkp, nk - nkp, np - nkp, nkp};
-  bool have = false, same = true;
-  uint32_t bn = 0u, bd = 1u;
-#pragma unroll
-  for (int c = 0; c < 4; c++) {
-    if (!cnt[c]) continue;
-    const uint32_t num = sm + ((c & 2) ? 3u : 0u), den = so - ((c & 1) ? 4u : 1u);
-    if (!have) {
-      bn = num;
-      bd = den;
-      have = true;
-    } else if (cmp_weight(num, den, bn, bd) != 0) {
-      same = false;
-    }
-  }
-  inf = bd == 0u;
-  return same;
-}
-
-// The noisy heuristic ply after analyse (WALK as for heuristic_body).
-template <bool TRACE, bool WALK>
+// The noisy heuristic ply after analyse.
+template <bool TRACE>
 CK_HD PlyResult noisy_body(Lane &L, const Gen &g, uint32_t r, uint32_t *list_dig) {
   PlyResult res;
   const uint32_t sm = material(L.own, L.kings);
   const uint32_t so = material(L.opp, L.kings);
-  const bool walked = WALK && g.capture && g.multi;
   NoisyBest nb = {-__builtin_inff(), 0.0f, 0u, 0u, L.turn};
   Choice c = {0u, 0u, 0u};
   uint32_t n, km;
-  bool single, inf = false;
-  if (!walked) {
+  if (!g.capture) {
     n = slot_count(g.slot);
     if (TRACE) *list_dig = list_digest(L, g, n);
     if (n == 0u || L.counter >= 50u) {
@@ -1626,26 +1558,17 @@ CK_HD PlyResult noisy_body(Lane &L, const Gen &g, uint32_t r, uint32_t *list_dig
       res.winner = L.counter < 50u ? (int32_t)(L.turn ^ 1u) : -1;
       return res;
     }
-    single = single_weight(L, g, sm, so, inf);
-    if (!single) {
-      uint32_t kc[4], prom;
-      weight_classes(L, g, kc, prom);
-      float wc[4];  // by class: bit 0 = a king removed, bit 1 = a man promoted
-#pragma unroll
-      for (int k = 0; k < 4; k++) {
-        const uint32_t num = sm + ((k & 2) ? 3u : 0u);
-        const uint32_t den = so - (g.capture ? ((k & 1) ? 4u : 1u) : 0u);
-        wc[k] = (float)num / (float)den;  // only classes that occur are read
-      }
+    const uint32_t prom = promoting(L, g);
+    if (some_promote(g, prom) && so != 0u) {
+      const float w0 = (float)sm / (float)so, w1 = (float)(sm + 3u) / (float)so;
       uint32_t any = g.slot[0] | g.slot[1] | g.slot[2] | g.slot[3];
       uint32_t bsq = 0u, bsl = 0u;
       while (any) {
         const uint32_t sq = ctz(any);
         any &= any - 1u;
+        const float w = getbit(prom, sq) ? w1 : w0;
         for (uint32_t sl = 0; sl < 4u; sl++) {
           if (!getbit(g.slot[sl], sq)) continue;
-          const uint32_t k = getbit(kc[sl], sq) | ((sl < 2u ? getbit(prom, sq) : 0u) << 1);
-          const float w = k == 0u ? wc[0] : k == 1u ? wc[1] : k == 2u ? wc[2] : wc[3];
           if (noisy_take(nb, r, w)) {
             bsq = sq;
             bsl = sl;
@@ -1655,7 +1578,7 @@ CK_HD PlyResult noisy_body(Lane &L, const Gen &g, uint32_t r, uint32_t *list_dig
       c = slot_choice(L, g, bsq, bsl);
       km = nb.pick;
     } else {
-      const uint32_t k = inf ? 0u : mod_small(r, n);  // reference index
+      const uint32_t k = so == 0u ? 0u : mod_small(r, n);  // reference index
       km = L.turn ? n - 1u - k : k;
       uint32_t sq, sl;
       select_slot(g.slot, km, sq, sl);
@@ -1674,7 +1597,7 @@ CK_HD PlyResult noisy_body(Lane &L, const Gen &g, uint32_t r, uint32_t *list_dig
     // one walk draws for every sequence and notes whether the weights differ at all
     uint32_t o = g.origins;
     uint32_t king = 0, s = 0, fn = 0, fd = 0;
-    single = true;
+    bool single = true;
     auto leaf = [&](uint32_t to, uint32_t removed, uint32_t, uint32_t) {
       const uint32_t num = sm + ((!king && to >= FAR_ROW_FIRST) ? 3u : 0u);
       const uint32_t den = so - material(removed, L.kings);
@@ -1719,13 +1642,13 @@ template <bool TRACE>
 CK_HD PlyResult ply_noisy(Lane &L, uint32_t r, uint32_t *list_dig) {
   Gen g;
   analyse(L, g);
-  return noisy_body<TRACE, true>(L, g, r, list_dig);
+  return noisy_body<TRACE>(L, g, r, list_dig);
 }
 
 // The noisy heuristic ply given the position's analysis g.
 template <bool TRACE>
 CK_HD PlyResult ply_noisy_given(Lane &L, const Gen &g, uint32_t r, uint32_t *list_dig) {
-  return noisy_body<TRACE, true>(L, g, r, list_dig);
+  return noisy_body<TRACE>(L, g, r, list_dig);
 }
 
 // The common part of a noisy heuristic ply: plays it when its moves all weigh the same (and no
@@ -1736,12 +1659,8 @@ CK_HD PlyResult ply_noisy_fast(Lane &L, uint32_t r, uint32_t *list_dig, bool &de
                                const TAB &tab = TAB()) {
   PlyResult res;
   analyse(L, g);
-  const SlotWords w = slot_words(g.slot);
-  const uint32_t n = w.n;
-  bool inf = false;
-  deferred = (g.capture && g.multi) ||
-             (n != 0u && L.counter < 50u &&
-              !single_weight(L, g, material(L.own, L.kings), material(L.opp, L.kings), inf));
+  deferred = (L.opp && some_promote(g, promoting(L, g))) ||
+             (g.capture && (g.multi || some_take_kings(L, g)));
   if (deferred) {
     res.n = 0u;
     res.chosen = 0u;
@@ -1749,6 +1668,8 @@ CK_HD PlyResult ply_noisy_fast(Lane &L, uint32_t r, uint32_t *list_dig, bool &de
     res.winner = 0;
     return res;
   }
+  const SlotWords w = slot_words(g.slot);
+  const uint32_t n = w.n;
   res.n = n;
   if (TRACE) *list_dig = list_digest(L, g, n);
   if (n == 0u || L.counter >= 50u) {
@@ -1757,6 +1678,8 @@ CK_HD PlyResult ply_noisy_fast(Lane &L, uint32_t r, uint32_t *list_dig, bool &de
     res.winner = L.counter < 50u ? (int32_t)(L.turn ^ 1u) : -1;
     return res;
   }
+  // every weight is +inf when no opponent's piece is left after the move: the first move then
+  const bool inf = !(g.capture ? L.opp & (L.opp - 1u) : L.opp);
   const uint32_t k = inf ? 0u : tab.mod(r, n);  // reference index
   uint32_t sq, sl;
   select_move(w, L.turn ? n - 1u - k : k, sq, sl, tab);

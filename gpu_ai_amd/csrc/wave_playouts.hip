@@ -152,7 +152,20 @@ __device__ __forceinline__ void play(ck::Lane &L, const Geometry &geo, const Str
         const uint64_t fA = __ballot((jumpA & fwd) != 0u), fB = __ballot((jumpB & fwd) != 0u);
         const uint64_t aA = __ballot((jumpA & any) != 0u), aB = __ballot((jumpB & any) != 0u);
         longer = (((jA & fA) | (jB & fB)) & men) | (((jA & aA) | (jB & aB)) & kings);
-        if (longer) break;
+        if (POLICY != MI_POLICY_RANDOM) {
+          // jumps of several kinds (some_promote, some_take_kings) are the walk's as well
+          const uint64_t prom = men & ck::ROW5;
+          const uint64_t kinds = m0 | m1;
+          bool mixed = (kinds & prom) && (kinds & ~prom);
+          if (const uint32_t okings = L.opp & L.kings) {
+            const uint64_t kA = __ballot((okings & stepA) != 0u), kB = __ballot((okings & stepB) != 0u);
+            const uint64_t k0 = (kA & kings) | (kB & men), k1 = (kB & kings) | (kA & men);
+            mixed |= ((m0 & k0) | (m1 & k1)) && ((m0 & ~k0) | (m1 & ~k1));
+          }
+          if (longer || mixed) break;
+        } else if (longer) {
+          break;
+        }
       } else {
         cap = 0u;
         m0 = __ballot((empty & stepA) != 0u) & movers;
@@ -163,24 +176,21 @@ __device__ __forceinline__ void play(ck::Lane &L, const Geometry &geo, const Str
       if (n == 0u || L.counter >= 50u) return;  // the game is over
       uint32_t sq = 0, sl = 0, pick = 1u;  // pick: the word chooses among the moves in m0 and m1
       uint32_t ties = n, first = 0u;       // first: every weight is +inf, index 0 wins
-      ck::Gen g;
-      if (POLICY != MI_POLICY_RANDOM) g = analysis(jA, jB, m0, m1, 0u, cap & 1u);
-      if (POLICY == MI_POLICY_HEURISTIC) {
-        uint32_t t[4];
-        ck::best_slots(L, g, t);
-        m0 = pair(t[0], t[2]);
-        m1 = pair(t[1], t[3]);
+      uint64_t prom = 0;  // promoting steps' men, where only some of the steps promote
+      if (POLICY != MI_POLICY_RANDOM) {
+        const uint64_t kinds = m0 | m1, p = L.own & ~L.kings & ck::ROW6 & ~cap;
+        if ((kinds & p) && (kinds & ~p) && L.opp) prom = p;
+      }
+      if (POLICY == MI_POLICY_HEURISTIC && prom) {
+        m0 &= prom;
+        m1 &= prom;
         ties = (uint32_t)__popcll(m0) + (uint32_t)__popcll(m1);
       }
       if (POLICY == MI_POLICY_HEURISTIC_NOISY) {
-        const uint32_t sm = ck::material(L.own, L.kings), so = ck::material(L.opp, L.kings);
-        bool inf = false;
-        if (ck::single_weight(L, g, sm, so, inf)) {
-          first = inf ? 1u : 0u;
+        if (!prom) {
+          first = !(cap ? L.opp & (L.opp - 1u) : L.opp) ? 1u : 0u;
         } else {
-          uint32_t kc[4], prom;
-          ck::weight_classes(L, g, kc, prom);
-          const uint32_t t0 = g.slot[0], t1 = g.slot[1], t2 = g.slot[2], t3 = g.slot[3];
+          const uint32_t t0 = lo32(m0), t1 = lo32(m1), t2 = hi32(m0), t3 = hi32(m1);
           // lane m draws for move m (n <= 49); lane (s, h) then takes the draws of its square's
           // slots 2h and 2h + 1
           float e0, e1;
@@ -193,14 +203,13 @@ __device__ __forceinline__ void play(ck::Lane &L, const Geometry &geo, const Str
           at += h ? ck::getbit(t0, s) + ck::getbit(t1, s) : 0u;
           const bool on0 = (a0 & self) != 0u, on1 = (a1 & self) != 0u;
           float v0 = __shfl(e, at & 63u), v1 = __shfl(e, (at + (on0 ? 1u : 0u)) & 63u);
-          const uint32_t promo = (h == 0u && (prom & self)) ? 3u : 0u;
-          const uint32_t k0 = h ? kc[2] : kc[0], k1 = h ? kc[3] : kc[1];
-          const uint32_t d0 = g.capture ? ((k0 & self) ? 4u : 1u) : 0u;
-          const uint32_t d1 = g.capture ? ((k1 & self) ? 4u : 1u) : 0u;
           {
 #pragma clang fp contract(off)
-            v0 = (float)(sm + promo) / (float)(so - d0) + v0;
-            v1 = (float)(sm + promo) / (float)(so - d1) + v1;
+            const uint32_t sm = ck::material(L.own, L.kings), so = ck::material(L.opp, L.kings);
+            const float w0 = (float)sm / (float)so, w1 = (float)(sm + 3u) / (float)so;
+            const float w = (lo32(prom) & self) && h == 0u ? w1 : w0;
+            v0 = w + v0;
+            v1 = w + v1;
           }
           const float ninf = -__builtin_inff();
           const float best = wave_max(fmaxf(on0 ? v0 : ninf, on1 ? v1 : ninf));
