@@ -1138,7 +1138,7 @@ int mi_graph_create(mi_ctx *ctx, uint32_t max_positions, uint32_t max_playouts, 
   pp.func = const_cast<void *>(gpuai::playout_kernel(policy, g->refill));
   pp.gridDim = dim3(g->grid);
   pp.blockDim = dim3(g->block);
-  pp.sharedMemBytes = gpuai::playout_lds(g->block);
+  pp.sharedMemBytes = gpuai::playout_lds(g->policy, g->block);
   pp.kernelParams = play_args;
   e = hipGraphCreate(&g->graph, 0);
   // The batch's upload is not a node: an asynchronous copy on the stream before each replay
@@ -1222,7 +1222,7 @@ int mi_graph_launch(mi_graph *g, const mi_pos *pos, uint32_t npos, const uint32_
       pp.func = const_cast<void *>(gpuai::playout_kernel(g->policy, g->refill));
       pp.gridDim = dim3(grid);
       pp.blockDim = dim3(t.block_size);
-      pp.sharedMemBytes = gpuai::playout_lds(t.block_size);
+      pp.sharedMemBytes = gpuai::playout_lds(g->policy, t.block_size);
       pp.kernelParams = play_args;
       MI_HIP(ctx, hipGraphExecKernelNodeSetParams(g->exec, g->n_play, &pp));
       g->grid = grid;

@@ -1511,25 +1511,31 @@ CK_HD void noise_pair(uint32_t r, uint32_t j, float &e0, float &e1) {
   e1 = z1 * NOISE_SIGMA;
 }
 
+// The draws of a ply's moves in order, made as they are asked for.
+struct NoiseInOrder {
+  uint32_t r;
+  float spare;  // second draw of the current pair
+  CK_HD float operator()(uint32_t m) {
+    float e;
+    if (m & 1u) return spare;
+    noise_pair(r, m >> 1, e, spare);
+    return e;
+  }
+};
+
 // Running argmax of the noisy weights in mover-frame order.  Player 2's reference order is the
 // reverse, so its first maximum in reference order is the last one here (>=).
 struct NoisyBest {
   float best;
-  float spare;  // second draw of the current pair
-  uint32_t m;   // moves seen
+  uint32_t m;  // moves seen
   uint32_t pick;
   uint32_t rev;
 };
 
-CK_HD bool noisy_take(NoisyBest &nb, uint32_t r, float w) {
+template <class Noise>
+CK_HD bool noisy_take(NoisyBest &nb, float w, Noise &noise) {
 #pragma clang fp contract(off)
-  float e;
-  if ((nb.m & 1u) == 0u) {
-    noise_pair(r, nb.m >> 1, e, nb.spare);
-  } else {
-    e = nb.spare;
-  }
-  const float v = w + e;
+  const float v = w + noise(nb.m);
   const bool take = nb.rev ? v >= nb.best : v > nb.best;
   if (take) {
     nb.best = v;
@@ -1539,97 +1545,109 @@ CK_HD bool noisy_take(NoisyBest &nb, uint32_t r, float w) {
   return take;
 }
 
-// The noisy heuristic ply after analyse.
-template <bool TRACE>
-CK_HD PlyResult noisy_body(Lane &L, const Gen &g, uint32_t r, uint32_t *list_dig) {
+// The noisy capture ply by the walk, its draws from `noise` (NoiseInOrder's interface: asked for
+// moves 0, 1, 2, ... of the ply in turn).
+template <bool TRACE, class Noise>
+CK_HD PlyResult noisy_walk(Lane &L, const Gen &g, uint32_t r, uint32_t *list_dig, Noise &noise) {
   PlyResult res;
+  if (L.counter >= 50u) {
+    res.n = count_walks(L, g);
+    if (TRACE) *list_dig = list_digest(L, g, res.n);
+    res.over = 1u;
+    res.chosen = 0xFFFFu;
+    res.winner = -1;
+    return res;
+  }
   const uint32_t sm = material(L.own, L.kings);
   const uint32_t so = material(L.opp, L.kings);
-  NoisyBest nb = {-__builtin_inff(), 0.0f, 0u, 0u, L.turn};
+  NoisyBest nb = {-__builtin_inff(), 0u, 0u, L.turn};
   Choice c = {0u, 0u, 0u};
-  uint32_t n, km;
-  if (!g.capture) {
-    n = slot_count(g.slot);
-    if (TRACE) *list_dig = list_digest(L, g, n);
-    if (n == 0u || L.counter >= 50u) {
-      res.n = n;
-      res.over = 1u;
-      res.chosen = 0xFFFFu;
-      res.winner = L.counter < 50u ? (int32_t)(L.turn ^ 1u) : -1;
-      return res;
+  // one walk draws for every sequence and notes whether the weights differ at all
+  uint32_t o = g.origins;
+  uint32_t king = 0, s = 0, fn = 0, fd = 0;
+  bool single = true;
+  auto leaf = [&](uint32_t to, uint32_t removed, uint32_t, uint32_t) {
+    const uint32_t num = sm + ((!king && to >= FAR_ROW_FIRST) ? 3u : 0u);
+    const uint32_t den = so - material(removed, L.kings);
+    if (nb.m == 0u) {
+      fn = num;
+      fd = den;
+    } else if (cmp_weight(num, den, fn, fd) != 0) {
+      single = false;
     }
-    const uint32_t prom = promoting(L, g);
-    if (some_promote(g, prom) && so != 0u) {
-      const float w0 = (float)sm / (float)so, w1 = (float)(sm + 3u) / (float)so;
-      uint32_t any = g.slot[0] | g.slot[1] | g.slot[2] | g.slot[3];
-      uint32_t bsq = 0u, bsl = 0u;
-      while (any) {
-        const uint32_t sq = ctz(any);
-        any &= any - 1u;
-        const float w = getbit(prom, sq) ? w1 : w0;
-        for (uint32_t sl = 0; sl < 4u; sl++) {
-          if (!getbit(g.slot[sl], sq)) continue;
-          if (noisy_take(nb, r, w)) {
-            bsq = sq;
-            bsl = sl;
-          }
+    if (noisy_take(nb, (float)num / (float)den, noise)) {
+      c.from = s;
+      c.to = to;
+      c.removed = removed;
+    }
+    return false;
+  };
+  while (o) {
+    s = ctz(o);
+    o &= o - 1u;
+    king = getbit(L.kings, s);
+    walk(s, king, g.cap, leaf);
+  }
+  const uint32_t n = nb.m;
+  uint32_t km = nb.pick;
+  if (single) {
+    const uint32_t k = fd == 0u ? 0u : mod_small(r, n);
+    km = L.turn ? n - 1u - k : k;
+    c = select_walk(L, g, km);
+  }
+  if (TRACE) *list_dig = list_digest(L, g, n);
+  res.n = n;
+  res.over = 0u;
+  res.winner = 0;
+  res.chosen = TRACE ? (L.turn ? n - 1u - km : km) : 0u;
+  apply(L, c.from, c.to, c.removed);
+  return res;
+}
+
+// The noisy heuristic ply given the position's analysis g.
+template <bool TRACE>
+CK_HD PlyResult ply_noisy_given(Lane &L, const Gen &g, uint32_t r, uint32_t *list_dig) {
+  NoiseInOrder noise = {r, 0.0f};
+  if (g.capture) return noisy_walk<TRACE>(L, g, r, list_dig, noise);
+  PlyResult res;
+  const uint32_t n = slot_count(g.slot);
+  if (TRACE) *list_dig = list_digest(L, g, n);
+  res.n = n;
+  if (n == 0u || L.counter >= 50u) {
+    res.over = 1u;
+    res.chosen = 0xFFFFu;
+    res.winner = L.counter < 50u ? (int32_t)(L.turn ^ 1u) : -1;
+    return res;
+  }
+  const uint32_t prom = promoting(L, g);
+  Choice c;
+  uint32_t km;
+  if (L.opp && some_promote(g, prom)) {
+    const uint32_t sm = material(L.own, L.kings), so = material(L.opp, L.kings);
+    const float w0 = (float)sm / (float)so, w1 = (float)(sm + 3u) / (float)so;
+    NoisyBest nb = {-__builtin_inff(), 0u, 0u, L.turn};
+    uint32_t any = g.slot[0] | g.slot[1] | g.slot[2] | g.slot[3];
+    uint32_t bsq = 0u, bsl = 0u;
+    while (any) {
+      const uint32_t sq = ctz(any);
+      any &= any - 1u;
+      for (uint32_t sl = 0; sl < 4u; sl++) {
+        if (!getbit(g.slot[sl], sq)) continue;
+        if (noisy_take(nb, getbit(prom, sq) ? w1 : w0, noise)) {
+          bsq = sq;
+          bsl = sl;
         }
       }
-      c = slot_choice(L, g, bsq, bsl);
-      km = nb.pick;
-    } else {
-      const uint32_t k = so == 0u ? 0u : mod_small(r, n);  // reference index
-      km = L.turn ? n - 1u - k : k;
-      uint32_t sq, sl;
-      select_slot(g.slot, km, sq, sl);
-      c = slot_choice(L, g, sq, sl);
     }
-  } else {
-    if (L.counter >= 50u) {
-      n = count_walks(L, g);
-      if (TRACE) *list_dig = list_digest(L, g, n);
-      res.n = n;
-      res.over = 1u;
-      res.chosen = 0xFFFFu;
-      res.winner = -1;
-      return res;
-    }
-    // one walk draws for every sequence and notes whether the weights differ at all
-    uint32_t o = g.origins;
-    uint32_t king = 0, s = 0, fn = 0, fd = 0;
-    bool single = true;
-    auto leaf = [&](uint32_t to, uint32_t removed, uint32_t, uint32_t) {
-      const uint32_t num = sm + ((!king && to >= FAR_ROW_FIRST) ? 3u : 0u);
-      const uint32_t den = so - material(removed, L.kings);
-      if (nb.m == 0u) {
-        fn = num;
-        fd = den;
-      } else if (cmp_weight(num, den, fn, fd) != 0) {
-        single = false;
-      }
-      if (noisy_take(nb, r, (float)num / (float)den)) {
-        c.from = s;
-        c.to = to;
-        c.removed = removed;
-      }
-      return false;
-    };
-    while (o) {
-      s = ctz(o);
-      o &= o - 1u;
-      king = getbit(L.kings, s);
-      walk(s, king, g.cap, leaf);
-    }
-    n = nb.m;
+    c = slot_choice(L, g, bsq, bsl);
     km = nb.pick;
-    if (single) {
-      const uint32_t k = fd == 0u ? 0u : mod_small(r, n);
-      km = L.turn ? n - 1u - k : k;
-      c = select_walk(L, g, km);
-    }
-    if (TRACE) *list_dig = list_digest(L, g, n);
+  } else {
+    const uint32_t k = L.opp ? mod_small(r, n) : 0u;  // reference index
+    km = L.turn ? n - 1u - k : k;
+    uint32_t sq, sl;
+    select_slot(g.slot, km, sq, sl);
+    c = slot_choice(L, g, sq, sl);
   }
-  res.n = n;
   res.over = 0u;
   res.winner = 0;
   res.chosen = TRACE ? (L.turn ? n - 1u - km : km) : 0u;
@@ -1642,13 +1660,33 @@ template <bool TRACE>
 CK_HD PlyResult ply_noisy(Lane &L, uint32_t r, uint32_t *list_dig) {
   Gen g;
   analyse(L, g);
-  return noisy_body<TRACE>(L, g, r, list_dig);
+  return ply_noisy_given<TRACE>(L, g, r, list_dig);
 }
 
-// The noisy heuristic ply given the position's analysis g.
-template <bool TRACE>
-CK_HD PlyResult ply_noisy_given(Lane &L, const Gen &g, uint32_t r, uint32_t *list_dig) {
-  return noisy_body<TRACE>(L, g, r, list_dig);
+// Steps of two weights by the index of their move (mover-frame order): with the moves from `base`
+// on counted from 0, bit i of the result is set when move i promotes.  Promoting men stand on
+// squares 24 to 27, and 8 squares have at most 32 moves.
+CK_HD uint32_t promoting_moves(const SlotWords &w, uint32_t prom, uint32_t &base) {
+  base = w.n - popc(w.x3);
+  uint32_t bits = 0u, at = 0u;
+#pragma unroll
+  for (uint32_t i = 0; i < 4u; i++) {
+    const uint32_t n = popc(w.x3 & (0x01010101u << i));
+    bits |= getbit(prom, 24u + i) ? ((1u << n) - 1u) << at : 0u;
+    at += n;
+  }
+  return bits;
+}
+
+// A noisy weight and its move as one number: the larger weight is the larger number, of equal ones
+// the first in reference order (rev: player 2's order, the reverse of this one).
+CK_HD uint64_t noisy_key(float v, uint32_t m, uint32_t rev) {
+  const uint32_t b = f32_bits(v);
+  const uint32_t hi = b ^ ((uint32_t)((int32_t)b >> 31) | 0x80000000u);
+  return (uint64_t)hi << 32 | (rev ? m : ~m);
+}
+CK_HD uint32_t noisy_key_move(uint64_t key, uint32_t rev) {
+  return rev ? (uint32_t)key : ~(uint32_t)key;
 }
 
 // The common part of a noisy heuristic ply: plays it when its moves all weigh the same (and no

@@ -116,7 +116,7 @@ struct PlayoutArgs {
 const void *playout_kernel(uint32_t policy, uint32_t refill);
 const void *reset_kernel();
 // Dynamic LDS of a playout launch with workgroups of `block` threads.
-uint32_t playout_lds(uint32_t block);
+uint32_t playout_lds(uint32_t policy, uint32_t block);
 
 hipError_t launch_reset(WorkWords *work, hipStream_t stream);
 hipError_t launch_playouts(const PlayoutArgs &args, uint32_t policy, bool trace, uint32_t refill,

@@ -135,6 +135,130 @@ struct Lookup {
 // the lane has the next four -- it consumes at most one word per iteration.
 constexpr uint32_t kWordRows = 8;
 
+// The noisy heuristic's walk phase draws for the deferred plies of a wave on all of its lanes: a
+// lane's plies need from one draw to twenty-five pairs, some ninety instructions each, and drawn by
+// the deferred lanes for themselves they cost a wave the longest list at every move.  The plies'
+// pairs are numbered through (marks: where each ply's first one lies); a lane takes every 64th,
+// finds its ply by counting marks and, for steps, adds the weights and enters the better of its two
+// moves as the ply's best (promoting_moves says which moves weigh more).  A capture ply is given
+// kDrawn draws for its walk, which seldom has more moves.  noisy-1024x1024: 0.98 -> 0.72 ms (walk
+// phases from 16 deferred plies on).
+constexpr uint32_t kShared = 32;  // plies a walk phase takes
+constexpr uint32_t kDrawn = 4;
+struct NoisyShare {  // of a wave
+  struct Ply {
+    uint32_t r;      // the ply's word
+    uint32_t moves;  // n | base << 8 | turn << 16 | capture << 17
+    uint32_t first;  // its first pair
+    uint32_t promote;
+    float w0, w1;
+  };
+  unsigned long long marks[kShared * 25u / 64u + 1u];  // at most 49 moves each (wave_playouts.hip)
+  unsigned long long best[kShared];
+  float draws[kShared][kDrawn];
+  Ply ply[kShared];
+};
+
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+struct NoiseDrawn {  // kDrawn draws made before, the others as they are asked for
+  const float *drawn;
+  ck::NoiseInOrder rest;
+  __device__ float operator()(uint32_t m) { return m < kDrawn ? drawn[m] : rest(m); }
+};
+
+// The deferred noisy plies `todo` (at most kShared), with the analyses g and the words r.
+template <bool TRACE>
+__device__ __forceinline__ ck::PlyResult noisy_plies(NoisyShare &sh, uint64_t todo, ck::Lane &L,
+                                                     const ck::Gen &g, uint32_t r, uint32_t &ld,
+                                                     const Lookup &tab) {
+  const uint32_t lane = threadIdx.x & 63u;
+  const bool on = lane_in(todo), step = on && !g.capture;
+  const uint32_t rank = lane_rank(todo);
+  ck::SlotWords w = {0u, 0u, 0u, 0u, 0u, 0u, 0u};
+  uint32_t pairs = 0u;
+  if (on) {
+    w = ck::slot_words(g.slot);
+    pairs = g.capture ? kDrawn / 2u : (w.n + 1u) >> 1;
+  }
+  uint32_t first = 0u, total = 0u;  // pairs of the plies before, and of all
+#pragma unroll
+  for (uint32_t b = 0; b < 5u; b++) {
+    const uint64_t m = __ballot(pairs >> b & 1u);
+    first += lane_rank(m) << b;
+    total += (uint32_t)__popcll(m) << b;
+  }
+  if (lane < sizeof(sh.marks) / 8u) sh.marks[lane] = 0ull;
+  wave_lds_fence();
+  if (on) {
+    atomicOr(&sh.marks[first >> 6], 1ull << (first & 63u));
+    NoisyShare::Ply p = {r, 1u << 17, first, 0u, 0.0f, 0.0f};
+    if (step) {
+      uint32_t base;
+      p.promote = ck::promoting_moves(w, ck::promoting(L, g), base);
+      p.moves = w.n | base << 8 | L.turn << 16;
+      const uint32_t sm = ck::material(L.own, L.kings);
+      const float so = (float)ck::material(L.opp, L.kings);
+      p.w0 = (float)sm / so;
+      p.w1 = (float)(sm + 3u) / so;
+    }
+    sh.ply[rank] = p;
+    sh.best[rank] = 0ull;
+  }
+  wave_lds_fence();
+  uint32_t before = 0u;  // plies that begin in earlier rounds
+  for (uint32_t q0 = 0u; q0 < total; q0 += 64u) {
+    const unsigned long long mk = sh.marks[q0 >> 6];
+    const uint32_t at = before + lane_rank(mk) + (uint32_t)(mk >> lane & 1ull) - 1u;
+    before += __builtin_amdgcn_readfirstlane((uint32_t)__popcll(mk));
+    if (q0 + lane < total) {
+      const NoisyShare::Ply p = sh.ply[at];
+      const uint32_t j = q0 + lane - p.first;
+      float e0, e1;
+      ck::noise_pair(p.r, j, e0, e1);
+      if (p.moves >> 17) {
+        sh.draws[at][2u * j] = e0;
+        sh.draws[at][2u * j + 1u] = e1;
+      } else {
+#pragma clang fp contract(off)
+        const uint32_t n = p.moves & 255u, base = p.moves >> 8 & 255u, rev = p.moves >> 16;
+        const uint32_t m = 2u * j;
+        auto weight = [&](uint32_t i) {
+          return i >= base && (p.promote >> ((i - base) & 31u) & 1u) ? p.w1 : p.w0;
+        };
+        const unsigned long long k0 = ck::noisy_key(weight(m) + e0, m, rev);
+        const unsigned long long k1 = ck::noisy_key(weight(m + 1u) + e1, m + 1u, rev);
+        atomicMax(&sh.best[at], m + 1u < n && k1 > k0 ? k1 : k0);
+      }
+    }
+  }
+  wave_lds_fence();
+  ck::PlyResult res = {0u, 0u, 0u, 0};
+  if (step) {
+    const uint32_t n = w.n;
+    res.n = n;
+    if (TRACE) ld = ck::list_digest(L, g, n);
+    if (L.counter >= 50u) {  // (a step of two weights is not the only move)
+      res.over = 1u;
+      res.chosen = 0xFFFFu;
+      res.winner = -1;
+    } else {
+      const uint32_t m = ck::noisy_key_move(sh.best[rank], L.turn);
+      res.chosen = TRACE ? (L.turn ? n - 1u - m : m) : 0u;
+      uint32_t sq, sl;
+      ck::select_move(w, m, sq, sl, tab);
+      ck::play_slot(L, 0u, sq, sl, tab);
+    }
+  } else if (on) {
+    NoiseDrawn noise = {sh.draws[rank], {r, 0.0f}};
+    res = ck::noisy_walk<TRACE>(L, g, r, &ld, noise);
+  }
+  return res;
+}
+
 template <uint32_t POLICY, bool TRACE, uint32_t REFILL>
 __global__ void __launch_bounds__(1024) k_playouts(PlayoutArgs a) {
   if (a.desc) {  // graph replays and allocation-free launches: the batch lives in device memory
@@ -150,12 +274,15 @@ __global__ void __launch_bounds__(1024) k_playouts(PlayoutArgs a) {
     a.keys = d->keys_at ? (const uint32_t *)(base + d->keys_at) : nullptr;
   }
   __shared__ LdsTables tables;
-  extern __shared__ uint32_t wave_words[];  // kWordRows x 64 words per wave
+  // kWordRows x 64 words per wave, then the noisy heuristic's NoisyShare per wave
+  extern __shared__ __align__(8) uint32_t wave_words[];
   tables.fill();
   __syncthreads();
   const Lookup tab = {tables};
   const uint32_t lane = threadIdx.x & 63u;
   uint32_t *const words = wave_words + (threadIdx.x >> 6) * (kWordRows * 64u) + lane;
+  NoisyShare &share =
+      ((NoisyShare *)(wave_words + (blockDim.x >> 6) * (kWordRows * 64u)))[threadIdx.x >> 6];
   const uint32_t nthreads = gridDim.x * blockDim.x;
   // Lanes that hold a game, and those of them whose ply waits for the walk phase.  Wave masks (in
   // scalar registers) rather than per-lane flags: flags changed on divergent paths are kept in
@@ -271,21 +398,26 @@ __global__ void __launch_bounds__(1024) k_playouts(PlayoutArgs a) {
       const uint32_t nd = (uint32_t)__popcll(deferred);
       if (nd >= defer_min || deferred == active || since_walk >= 8u) {
         since_walk = 0;
-        const bool on = lane_in(deferred);
+        uint64_t todo = deferred;
+        if (POLICY == MI_POLICY_HEURISTIC_NOISY && nd > kShared)
+          todo = __ballot(lane_in(deferred) && lane_rank(deferred) < kShared);
+        const bool on = lane_in(todo);
+        const uint32_t r = words[ply & ((kWordRows - 1u) * kPly)];
         ck::PlyResult res = {0u, 0u, 0u, 0};
         uint32_t ld = 0;
-        if (on) {
-          const uint32_t r = words[ply & ((kWordRows - 1u) * kPly)];
+        if (POLICY == MI_POLICY_HEURISTIC_NOISY) {
+          res = noisy_plies<TRACE>(share, todo, L, gd, r, ld, tab);
+        } else if (on) {
           if (POLICY == MI_POLICY_RANDOM) {
             // capture trees in closed form; the walk only for king trees past two jumps
             bool deep = false;
             res = ck::ply_random_captures<TRACE>(L, gd, r, &ld, deep, tab);
             if (deep) res = ck::ply_random_given<TRACE>(L, gd, r, &ld);
+          } else {
+            res = ck::ply_heuristic_given<TRACE>(L, gd, r, &ld);
           }
-          else if (POLICY == MI_POLICY_HEURISTIC) res = ck::ply_heuristic_given<TRACE>(L, gd, r, &ld);
-          else res = ck::ply_noisy_given<TRACE>(L, gd, r, &ld);
         }
-        deferred = 0;
+        deferred &= ~todo;
         decided(on, res, ld);
       } else {
         since_walk++;
@@ -624,7 +756,10 @@ __global__ void __launch_bounds__(256) k_valu_rate(uint32_t iters, uint32_t salt
 
 }  // namespace
 
-uint32_t playout_lds(uint32_t block) { return block / 64u * (kWordRows * 64u * sizeof(uint32_t)); }
+uint32_t playout_lds(uint32_t policy, uint32_t block) {
+  return block / 64u * (uint32_t)(kWordRows * 64u * sizeof(uint32_t) +
+                                  (policy == MI_POLICY_HEURISTIC_NOISY ? sizeof(NoisyShare) : 0u));
+}
 
 namespace {
 
@@ -633,10 +768,10 @@ hipError_t launch_refill(const PlayoutArgs &args, uint32_t refill, uint32_t grid
                          hipStream_t stream) {
   if (refill == MI_REFILL_STATIC)
     hipLaunchKernelGGL((k_playouts<POLICY, TRACE, MI_REFILL_STATIC>), dim3(grid), dim3(block),
-                       playout_lds(block), stream, args);
+                       playout_lds(POLICY, block), stream, args);
   else
     hipLaunchKernelGGL((k_playouts<POLICY, TRACE, MI_REFILL_QUEUE>), dim3(grid), dim3(block),
-                       playout_lds(block), stream, args);
+                       playout_lds(POLICY, block), stream, args);
   return hipGetLastError();
 }
 
