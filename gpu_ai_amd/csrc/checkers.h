@@ -930,11 +930,16 @@ constexpr uint32_t kTreeLeaves = 12;
 struct CaptureTrees {
   uint32_t leaf[kTreeLeaves];
   uint32_t count[4];
+  uint32_t origins, fwd, any, kings;  // squares with a jump ahead and with any; the position's kings
   uint32_t n, deep;
 };
 
 CK_HD void capture_trees(const Lane &L, const Gen &g, CaptureTrees &t) {
   const uint32_t c0 = g.cap[0], c1 = g.cap[1], c2 = g.cap[2], c3 = g.cap[3];
+  t.origins = g.origins;
+  t.fwd = c0 | c1;
+  t.any = t.fwd | c2 | c3;
+  t.kings = L.kings;
   {  // men: a = +7, b = +9
     const uint32_t men = g.origins & ~L.kings, a = men & c1, b = men & c0;
     const uint32_t a7 = c1 >> 7, b7 = c0 >> 7, a9 = c1 >> 9, b9 = c0 >> 9;
@@ -952,7 +957,7 @@ CK_HD void capture_trees(const Lane &L, const Gen &g, CaptureTrees &t) {
     t.leaf[8] = t.leaf[9] = t.leaf[10] = t.leaf[11] = 0u;
   }
   {  // kings
-    const uint32_t kings = g.origins & L.kings, any = c0 | c1 | c2 | c3;
+    const uint32_t kings = g.origins & L.kings;
     const uint32_t cap[4] = {c0, c1, c2, c3};
     auto from = [](uint32_t m, uint32_t d) {  // origins whose jump in direction d lands on m
       return d == 0u ? m >> 9 : d == 1u ? m >> 7 : d == 2u ? m << 7 : m << 9;
@@ -969,7 +974,7 @@ CK_HD void capture_trees(const Lane &L, const Gen &g, CaptureTrees &t) {
     t.deep = 0u;
 #pragma unroll
     for (uint32_t d = 0; d < 4u; d++) {
-      const uint32_t k = kings & cap[d], last = ~from(any, d);
+      const uint32_t k = kings & cap[d], last = ~from(t.any, d);
       t.deep |= k & from(goes_on, d);
       uint32_t i = 3u * d;
 #pragma unroll
@@ -998,10 +1003,9 @@ CK_HD void capture_trees(const Lane &L, const Gen &g, CaptureTrees &t) {
 
 // The k-th move (mover-frame order, k < n).
 template <class TAB>
-CK_HD Choice capture_choice(const Lane &L, const Gen &g, const CaptureTrees &t, uint32_t k,
-                            const TAB &tab) {
+CK_HD Choice capture_choice(const CaptureTrees &t, uint32_t k, const TAB &tab) {
   Choice c;
-  uint32_t o = g.origins;
+  uint32_t o = t.origins;
   for (;;) {
     c.from = ctz(o);
     o &= o - 1u;
@@ -1022,10 +1026,9 @@ CK_HD Choice capture_choice(const Lane &L, const Gen &g, const CaptureTrees &t, 
     at += up ? 4u : 0u;
     k = sub_if(k, below);
   }
-  const uint32_t king = getbit(L.kings, c.from);
+  const uint32_t king = getbit(t.kings, c.from);
   const uint32_t w = tab.path(at + tab.kth(m & 15u, k) + (king << 4));
-  const uint32_t fwd = g.cap[0] | g.cap[1];
-  const uint32_t second = king ? fwd | g.cap[2] | g.cap[3] : fwd, third = king ? 0u : fwd;
+  const uint32_t second = king ? t.any : t.fwd, third = king ? 0u : t.fwd;
   uint32_t x = c.from, go = 1u;
   c.removed = 0u;
 #pragma unroll
@@ -1213,7 +1216,7 @@ CK_HD PlyResult ply_random_captures(Lane &L, const Gen &g, uint32_t r, uint32_t 
   }
   const uint32_t k = tab.mod(r, t.n);
   res.chosen = k;
-  const Choice c = capture_choice(L, g, t, L.turn ? t.n - 1u - k : k, tab);
+  const Choice c = capture_choice(t, L.turn ? t.n - 1u - k : k, tab);
   apply(L, c.from, c.to, c.removed);
   return res;
 }
@@ -1334,36 +1337,39 @@ CK_HD uint32_t best_steps(const Lane &L, const Gen &g) {
   return some_promote(g, prom) && L.opp ? prom : 0xFFFFFFFFu;
 }
 
-// The heuristic capture ply by the walk.
+// The heuristic capture ply by the walk.  The moves of largest weight are kept as they come, up to
+// four of them; only a move beyond those takes a second walk.
 template <bool TRACE>
 CK_HD PlyResult heuristic_walk(Lane &L, const Gen &g, uint32_t r, uint32_t *list_dig) {
   PlyResult res;
   const uint32_t sm = material(L.own, L.kings);
   const uint32_t so = material(L.opp, L.kings);
-  uint32_t n = 0, ties = 0, bn = 0, bd = 1;
-  {
-    uint32_t o = g.origins;
-    uint32_t king = 0;
-    auto leaf = [&](uint32_t to, uint32_t removed, uint32_t, uint32_t) {
-      uint32_t num = sm + ((!king && to >= FAR_ROW_FIRST) ? 3u : 0u);
-      uint32_t den = so - material(removed, L.kings);
-      int c = cmp_weight(num, den, bn, bd);
-      if (c > 0) {
-        bn = num;
-        bd = den;
-        ties = 1u;
-      } else if (c == 0) {
-        ties++;
-      }
-      n++;
-      return false;
-    };
-    while (o) {
-      uint32_t s = ctz(o);
-      o &= o - 1u;
-      king = getbit(L.kings, s);
-      walk(s, king, g.cap, leaf);
+  uint32_t n = 0, ties = 0, bn = 0, bd = 1, from = 0, king = 0;
+  LeafCache lc = {0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u};  // `to` holds to | from << 5 | index << 10
+  auto weight = [&](uint32_t to, uint32_t removed) {
+    const uint32_t num = sm + ((!king && to >= FAR_ROW_FIRST) ? 3u : 0u);
+    const uint32_t den = so - material(removed, L.kings);
+    const int c = cmp_weight(num, den, bn, bd);
+    if (c > 0) {
+      bn = num;
+      bd = den;
     }
+    return c;
+  };
+  auto leaf = [&](uint32_t to, uint32_t removed, uint32_t, uint32_t) {
+    const int c = weight(to, removed);
+    if (c > 0) ties = 0u;
+    if (c >= 0) {
+      cache_put(lc, ties, to | from << 5 | n << 10, removed);
+      ties++;
+    }
+    n++;
+    return false;
+  };
+  for (uint32_t o = g.origins; o; o &= o - 1u) {
+    from = ctz(o);
+    king = getbit(L.kings, from);
+    walk(from, king, g.cap, leaf);
   }
   res.n = n;
   if (TRACE) *list_dig = list_digest(L, g, n);
@@ -1376,35 +1382,30 @@ CK_HD PlyResult heuristic_walk(Lane &L, const Gen &g, uint32_t r, uint32_t *list
   const uint32_t k = mod_small(r, ties);
   res.over = 0u;
   res.winner = 0;
-  Choice c = {0u, 0u, 0u};
-  uint32_t o = g.origins;
-  uint32_t king = 0, left = L.turn ? ties - 1u - k : k, idx = 0;
-  bool found = false;
-  auto leaf = [&](uint32_t to, uint32_t removed, uint32_t, uint32_t) {
-    uint32_t num = sm + ((!king && to >= FAR_ROW_FIRST) ? 3u : 0u);
-    uint32_t den = so - material(removed, L.kings);
-    if (cmp_weight(num, den, bn, bd) == 0) {
-      if (left == 0u) {
-        c.to = to;
-        c.removed = removed;
+  uint32_t left = L.turn ? ties - 1u - k : k, move = 0, removed = 0;
+  if (left < 4u) {
+    cache_get(lc, left, move, removed);
+  } else {
+    uint32_t idx = 0;
+    bool found = false;
+    auto again = [&](uint32_t to, uint32_t rm, uint32_t, uint32_t) {
+      if (weight(to, rm) == 0 && left-- == 0u) {
+        move = to | from << 5 | idx << 10;
+        removed = rm;
         found = true;
-        return true;
       }
-      left--;
+      idx++;
+      return found;
+    };
+    for (uint32_t o = g.origins; o && !found; o &= o - 1u) {
+      from = ctz(o);
+      king = getbit(L.kings, from);
+      walk(from, king, g.cap, again);
     }
-    idx++;
-    return false;
-  };
-  while (o && !found) {
-    uint32_t s = ctz(o);
-    o &= o - 1u;
-    king = getbit(L.kings, s);
-    c.from = s;
-    walk(s, king, g.cap, leaf);
   }
   // reference index of the chosen move (for the trace record)
-  res.chosen = L.turn ? n - 1u - idx : idx;
-  apply(L, c.from, c.to, c.removed);
+  res.chosen = TRACE ? (L.turn ? n - 1u - (move >> 10) : move >> 10) : 0u;
+  apply(L, move >> 5 & 31u, move & 31u, removed);
   return res;
 }
 
@@ -1532,8 +1533,7 @@ struct NoisyBest {
   uint32_t rev;
 };
 
-template <class Noise>
-CK_HD bool noisy_take(NoisyBest &nb, float w, Noise &noise) {
+CK_HD bool noisy_take(NoisyBest &nb, float w, NoiseInOrder &noise) {
 #pragma clang fp contract(off)
   const float v = w + noise(nb.m);
   const bool take = nb.rev ? v >= nb.best : v > nb.best;
@@ -1545,10 +1545,9 @@ CK_HD bool noisy_take(NoisyBest &nb, float w, Noise &noise) {
   return take;
 }
 
-// The noisy capture ply by the walk, its draws from `noise` (NoiseInOrder's interface: asked for
-// moves 0, 1, 2, ... of the ply in turn).
-template <bool TRACE, class Noise>
-CK_HD PlyResult noisy_walk(Lane &L, const Gen &g, uint32_t r, uint32_t *list_dig, Noise &noise) {
+// The noisy capture ply by the walk.
+template <bool TRACE>
+CK_HD PlyResult noisy_walk(Lane &L, const Gen &g, uint32_t r, uint32_t *list_dig) {
   PlyResult res;
   if (L.counter >= 50u) {
     res.n = count_walks(L, g);
@@ -1562,7 +1561,10 @@ CK_HD PlyResult noisy_walk(Lane &L, const Gen &g, uint32_t r, uint32_t *list_dig
   const uint32_t so = material(L.opp, L.kings);
   NoisyBest nb = {-__builtin_inff(), 0u, 0u, L.turn};
   Choice c = {0u, 0u, 0u};
-  // one walk draws for every sequence and notes whether the weights differ at all
+  NoiseInOrder noise = {r, 0.0f};
+  // one walk draws for every sequence and notes whether the weights differ at all; the first four
+  // sequences are kept for a word that chooses among equal weights
+  LeafCache lc = {0u, 0u, 0u, 0u, 0u, 0u, 0u, 0u};
   uint32_t o = g.origins;
   uint32_t king = 0, s = 0, fn = 0, fd = 0;
   bool single = true;
@@ -1575,6 +1577,7 @@ CK_HD PlyResult noisy_walk(Lane &L, const Gen &g, uint32_t r, uint32_t *list_dig
     } else if (cmp_weight(num, den, fn, fd) != 0) {
       single = false;
     }
+    cache_put(lc, nb.m, to | s << 5, removed);
     if (noisy_take(nb, (float)num / (float)den, noise)) {
       c.from = s;
       c.to = to;
@@ -1593,7 +1596,14 @@ CK_HD PlyResult noisy_walk(Lane &L, const Gen &g, uint32_t r, uint32_t *list_dig
   if (single) {
     const uint32_t k = fd == 0u ? 0u : mod_small(r, n);
     km = L.turn ? n - 1u - k : k;
-    c = select_walk(L, g, km);
+    if (km < 4u) {
+      uint32_t move;
+      cache_get(lc, km, move, c.removed);
+      c.from = move >> 5;
+      c.to = move & 31u;
+    } else {
+      c = select_walk(L, g, km);
+    }
   }
   if (TRACE) *list_dig = list_digest(L, g, n);
   res.n = n;
@@ -1607,8 +1617,7 @@ CK_HD PlyResult noisy_walk(Lane &L, const Gen &g, uint32_t r, uint32_t *list_dig
 // The noisy heuristic ply given the position's analysis g.
 template <bool TRACE>
 CK_HD PlyResult ply_noisy_given(Lane &L, const Gen &g, uint32_t r, uint32_t *list_dig) {
-  NoiseInOrder noise = {r, 0.0f};
-  if (g.capture) return noisy_walk<TRACE>(L, g, r, list_dig, noise);
+  if (g.capture) return noisy_walk<TRACE>(L, g, r, list_dig);
   PlyResult res;
   const uint32_t n = slot_count(g.slot);
   if (TRACE) *list_dig = list_digest(L, g, n);
@@ -1626,6 +1635,7 @@ CK_HD PlyResult ply_noisy_given(Lane &L, const Gen &g, uint32_t r, uint32_t *lis
     const uint32_t sm = material(L.own, L.kings), so = material(L.opp, L.kings);
     const float w0 = (float)sm / (float)so, w1 = (float)(sm + 3u) / (float)so;
     NoisyBest nb = {-__builtin_inff(), 0u, 0u, L.turn};
+    NoiseInOrder noise = {r, 0.0f};
     uint32_t any = g.slot[0] | g.slot[1] | g.slot[2] | g.slot[3];
     uint32_t bsq = 0u, bsl = 0u;
     while (any) {

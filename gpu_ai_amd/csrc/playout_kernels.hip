@@ -135,28 +135,36 @@ struct Lookup {
 // the lane has the next four -- it consumes at most one word per iteration.
 constexpr uint32_t kWordRows = 8;
 
-// The noisy heuristic's walk phase draws for the deferred plies of a wave on all of its lanes: a
-// lane's plies need from one draw to twenty-five pairs, some ninety instructions each, and drawn by
-// the deferred lanes for themselves they cost a wave the longest list at every move.  The plies'
-// pairs are numbered through (marks: where each ply's first one lies); a lane takes every 64th,
-// finds its ply by counting marks and, for steps, adds the weights and enters the better of its two
-// moves as the ply's best (promoting_moves says which moves weigh more).  A capture ply is given
-// kDrawn draws for its walk, which seldom has more moves.  noisy-1024x1024: 0.98 -> 0.72 ms (walk
-// phases from 16 deferred plies on).
-constexpr uint32_t kShared = 32;  // plies a walk phase takes
-constexpr uint32_t kDrawn = 4;
-struct NoisyShare {  // of a wave
-  struct Ply {
-    uint32_t r;      // the ply's word
-    uint32_t moves;  // n | base << 8 | turn << 16 | capture << 17
-    uint32_t first;  // its first pair
-    uint32_t promote;
-    float w0, w1;
-  };
-  unsigned long long marks[kShared * 25u / 64u + 1u];  // at most 49 moves each (wave_playouts.hip)
-  unsigned long long best[kShared];
-  float draws[kShared][kDrawn];
-  Ply ply[kShared];
+// The heuristics' walk phases work on all lanes of the wave, whichever wait: the moves of the
+// deferred plies are numbered through and dealt to the lanes, whose best weight per ply is found in
+// LDS.  Done by the waiting lanes for their own plies, the walk over a ply's captures (twice: for
+// the best weight, then for the chosen move) and the draws of its moves (some ninety instructions a
+// pair) cost a wave its longest lists.  noisy-1024x1024: 0.98 ms with both done so, 0.72 with the
+// steps' draws shared, 0.67 with the captures too; heuristic-1024x1024: 0.52 -> 0.475 ms (0.486 by a
+// single walk that keeps the best moves, which plays the long king sequences here).
+constexpr uint32_t kSharedSteps = 32, kSharedCaptures = 16;  // plies a walk phase takes
+union WalkShare {  // of a wave
+  struct {
+    struct Ply {
+      uint32_t r;      // the ply's word
+      uint32_t moves;  // n | base << 8 | turn << 16 (promoting_moves)
+      uint32_t first;  // its first pair of moves
+      uint32_t promote;
+      float w0, w1;
+    } ply[kSharedSteps];
+    unsigned long long best[kSharedSteps];
+    unsigned long long marks[kSharedSteps * 25u / 64u + 1u];  // at most 49 moves each
+  } steps;
+  struct {
+    struct Ply {
+      ck::CaptureTrees trees;  // (deep is not used)
+      uint32_t r, first;
+      uint32_t turn, sm, so;
+    } ply[kSharedCaptures];
+    unsigned long long best[kSharedCaptures];
+    uint2 choice[kSharedCaptures];  // from | to << 8 | move << 16, removed pieces
+    unsigned long long marks;
+  } captures;
 };
 
 __device__ __forceinline__ void wave_lds_fence() {
@@ -164,48 +172,162 @@ __device__ __forceinline__ void wave_lds_fence() {
   __builtin_amdgcn_wave_barrier();
 }
 
-struct NoiseDrawn {  // kDrawn draws made before, the others as they are asked for
-  const float *drawn;
-  ck::NoiseInOrder rest;
-  __device__ float operator()(uint32_t m) { return m < kDrawn ? drawn[m] : rest(m); }
-};
-
-// The deferred noisy plies `todo` (at most kShared), with the analyses g and the words r.
-template <bool TRACE>
-__device__ __forceinline__ ck::PlyResult noisy_plies(NoisyShare &sh, uint64_t todo, ck::Lane &L,
-                                                     const ck::Gen &g, uint32_t r, uint32_t &ld,
-                                                     const Lookup &tab) {
-  const uint32_t lane = threadIdx.x & 63u;
-  const bool on = lane_in(todo), step = on && !g.capture;
-  const uint32_t rank = lane_rank(todo);
-  ck::SlotWords w = {0u, 0u, 0u, 0u, 0u, 0u, 0u};
-  uint32_t pairs = 0u;
-  if (on) {
-    w = ck::slot_words(g.slot);
-    pairs = g.capture ? kDrawn / 2u : (w.n + 1u) >> 1;
-  }
-  uint32_t first = 0u, total = 0u;  // pairs of the plies before, and of all
+// Sum of `count` (below 32) over the lanes before this one, and over all.
+__device__ __forceinline__ uint32_t lanes_before(uint32_t count, uint32_t &total) {
+  uint32_t before = 0u;
+  total = 0u;
 #pragma unroll
   for (uint32_t b = 0; b < 5u; b++) {
-    const uint64_t m = __ballot(pairs >> b & 1u);
-    first += lane_rank(m) << b;
+    const uint64_t m = __ballot(count >> b & 1u);
+    before += lane_rank(m) << b;
     total += (uint32_t)__popcll(m) << b;
   }
+  return before;
+}
+
+// Deferred capture plies (the lanes `todo`, analyses g, words r), a move to a lane; plies with a
+// king sequence past two jumps or more than 31 moves are left to their lane's walk.  Takes the
+// plies that it has not played out of `todo`.
+template <uint32_t POLICY, bool TRACE>
+__device__ __forceinline__ void capture_plies(WalkShare &share, uint64_t &todo, ck::Lane &L,
+                                              const ck::Gen &g, uint32_t r, ck::PlyResult &res,
+                                              uint32_t &ld, const Lookup &tab) {
+  auto &sh = share.captures;
+  const uint32_t lane = threadIdx.x & 63u;
+  uint32_t n = 0u;  // moves to be dealt
+  bool walk = false;
+  ck::CaptureTrees t;
+  if (lane_in(todo)) {
+    ck::capture_trees(L, g, t);
+    walk = t.deep || t.n > 31u;
+    n = walk || L.counter >= 50u ? 0u : t.n;
+  }
+  uint32_t total;
+  const uint32_t first = lanes_before(n, total);
+  const uint64_t dealt = __ballot(n != 0u && first + n <= 64u);
+  const uint32_t rank = lane_rank(dealt);
+  const uint64_t mine = __ballot(lane_in(dealt) && rank < kSharedCaptures);
+  todo &= ~__ballot(n != 0u) | mine;
+  if (lane == 0u) sh.marks = 0ull;
+  wave_lds_fence();
+  if (lane_in(mine)) {
+    atomicOr(&sh.marks, 1ull << first);
+    auto &p = sh.ply[rank];
+    p.trees = t;
+    p.r = r;
+    p.first = first;
+    p.turn = L.turn;
+    p.sm = ck::material(L.own, L.kings);
+    p.so = ck::material(L.opp, L.kings);
+    sh.best[rank] = 0ull;
+  }
+  total = mine ? __builtin_amdgcn_readlane(first + n, 63u - (uint32_t)__builtin_clzll(mine)) : 0u;
+  wave_lds_fence();
+  if (total) {
+    const unsigned long long marks = sh.marks;
+    const bool on = lane < total;
+    const uint32_t at = lane_rank(marks) + (uint32_t)(marks >> lane & 1ull) - 1u;
+    ck::Choice c = {0u, 0u, 0u};
+    uint32_t k = 0u, begin = 0u, moves = 0u, turn = 0u, word = 0u;
+    float w = 0.0f;
+    unsigned long long key = 0ull;
+    if (on) {
+      const auto p = sh.ply[at];
+      begin = p.first;
+      moves = p.trees.n;
+      turn = p.turn;
+      word = p.r;
+      k = lane - begin;
+      c = ck::capture_choice(p.trees, k, tab);
+      const uint32_t king = ck::getbit(p.trees.kings, c.from);
+      const uint32_t num = p.sm + (!king && c.to >= ck::FAR_ROW_FIRST ? 3u : 0u);
+      const uint32_t den = p.so - ck::material(c.removed, p.trees.kings);
+      // Weights are quotients of whole numbers up to 131: those that differ do so by one part in
+      // 17,000 or more, so that rounded they are equal where cmp_weight calls them equal.
+      w = (float)num / (float)den;
+      if (POLICY == MI_POLICY_HEURISTIC) {
+        key = ck::f32_bits(w);
+      } else {
+#pragma clang fp contract(off)
+        float e0, e1;
+        ck::noise_pair(word, k >> 1, e0, e1);
+        key = ck::noisy_key(w + ((k & 1u) ? e1 : e0), k, turn);
+      }
+      atomicMax(&sh.best[at], key);
+    }
+    wave_lds_fence();
+    const unsigned long long best = on ? sh.best[at] : 1ull;
+    // the ply's lanes that hold a move of largest weight (noisy: of the weight of its first move)
+    const float w_first = __shfl(w, (int)begin);
+    const uint64_t same =
+        __ballot(on && (POLICY == MI_POLICY_HEURISTIC ? key == best : w == w_first));
+    const uint32_t all = (1u << moves) - 1u, set = (uint32_t)(same >> begin) & all;
+    bool chosen = false;
+    if (on) {
+      if (POLICY == MI_POLICY_HEURISTIC) {
+        const uint32_t ties = ck::popc(set);
+        const uint32_t i = tab.mod(word, ties);
+        chosen = key == best &&
+                 ck::popc(set & ((1u << k) - 1u)) == (turn ? ties - 1u - i : i);
+      } else if (set == all) {  // one weight: the word chooses, or the first move if it is +inf
+        const uint32_t i = w_first == __builtin_inff() ? 0u : tab.mod(word, moves);
+        chosen = k == (turn ? moves - 1u - i : i);
+      } else {
+        chosen = key == best;
+      }
+    }
+    if (chosen) sh.choice[at] = make_uint2(c.from | c.to << 8 | k << 16, c.removed);
+    wave_lds_fence();
+  }
+  if (lane_in(todo)) {
+    if (walk) {
+      res = POLICY == MI_POLICY_HEURISTIC ? ck::ply_heuristic_given<TRACE>(L, g, r, &ld)
+                                          : ck::ply_noisy_given<TRACE>(L, g, r, &ld);
+    } else {
+      res.n = t.n;
+      if (TRACE) ld = ck::list_digest(L, g, t.n);
+      if (n == 0u) {  // the draw count has run out
+        res.over = 1u;
+        res.chosen = 0xFFFFu;
+        res.winner = -1;
+      } else {
+        const uint2 c = sh.choice[rank];
+        res.chosen = TRACE ? (L.turn ? n - 1u - (c.x >> 16) : c.x >> 16) : 0u;
+        ck::apply(L, c.x & 31u, c.x >> 8 & 31u, c.y);
+      }
+    }
+  }
+  wave_lds_fence();
+}
+
+// Deferred noisy steps of two weights (the lanes `todo`, at most kSharedSteps), a pair of moves to
+// a lane: it draws for both and enters the better one.
+template <bool TRACE>
+__device__ __forceinline__ void noisy_steps(WalkShare &share, uint64_t todo, ck::Lane &L,
+                                            const ck::Gen &g, uint32_t r, ck::PlyResult &res,
+                                            uint32_t &ld, const Lookup &tab) {
+  auto &sh = share.steps;
+  const uint32_t lane = threadIdx.x & 63u;
+  const bool on = lane_in(todo);
+  const uint32_t rank = lane_rank(todo);
+  ck::SlotWords w = {0u, 0u, 0u, 0u, 0u, 0u, 0u};
+  if (on) w = ck::slot_words(g.slot);
+  uint32_t total;
+  const uint32_t first = lanes_before((w.n + 1u) >> 1, total);
   if (lane < sizeof(sh.marks) / 8u) sh.marks[lane] = 0ull;
   wave_lds_fence();
   if (on) {
     atomicOr(&sh.marks[first >> 6], 1ull << (first & 63u));
-    NoisyShare::Ply p = {r, 1u << 17, first, 0u, 0.0f, 0.0f};
-    if (step) {
-      uint32_t base;
-      p.promote = ck::promoting_moves(w, ck::promoting(L, g), base);
-      p.moves = w.n | base << 8 | L.turn << 16;
-      const uint32_t sm = ck::material(L.own, L.kings);
-      const float so = (float)ck::material(L.opp, L.kings);
-      p.w0 = (float)sm / so;
-      p.w1 = (float)(sm + 3u) / so;
-    }
-    sh.ply[rank] = p;
+    auto &p = sh.ply[rank];
+    uint32_t base;
+    p.promote = ck::promoting_moves(w, ck::promoting(L, g), base);
+    p.moves = w.n | base << 8 | L.turn << 16;
+    p.r = r;
+    p.first = first;
+    const uint32_t sm = ck::material(L.own, L.kings);
+    const float so = (float)ck::material(L.opp, L.kings);
+    p.w0 = (float)sm / so;
+    p.w1 = (float)(sm + 3u) / so;
     sh.best[rank] = 0ull;
   }
   wave_lds_fence();
@@ -215,29 +337,22 @@ __device__ __forceinline__ ck::PlyResult noisy_plies(NoisyShare &sh, uint64_t to
     const uint32_t at = before + lane_rank(mk) + (uint32_t)(mk >> lane & 1ull) - 1u;
     before += __builtin_amdgcn_readfirstlane((uint32_t)__popcll(mk));
     if (q0 + lane < total) {
-      const NoisyShare::Ply p = sh.ply[at];
-      const uint32_t j = q0 + lane - p.first;
+#pragma clang fp contract(off)
+      const auto p = sh.ply[at];
+      const uint32_t n = p.moves & 255u, base = p.moves >> 8 & 255u, rev = p.moves >> 16;
+      const uint32_t j = q0 + lane - p.first, m = 2u * j;
       float e0, e1;
       ck::noise_pair(p.r, j, e0, e1);
-      if (p.moves >> 17) {
-        sh.draws[at][2u * j] = e0;
-        sh.draws[at][2u * j + 1u] = e1;
-      } else {
-#pragma clang fp contract(off)
-        const uint32_t n = p.moves & 255u, base = p.moves >> 8 & 255u, rev = p.moves >> 16;
-        const uint32_t m = 2u * j;
-        auto weight = [&](uint32_t i) {
-          return i >= base && (p.promote >> ((i - base) & 31u) & 1u) ? p.w1 : p.w0;
-        };
-        const unsigned long long k0 = ck::noisy_key(weight(m) + e0, m, rev);
-        const unsigned long long k1 = ck::noisy_key(weight(m + 1u) + e1, m + 1u, rev);
-        atomicMax(&sh.best[at], m + 1u < n && k1 > k0 ? k1 : k0);
-      }
+      auto weight = [&](uint32_t i) {
+        return i >= base && (p.promote >> ((i - base) & 31u) & 1u) ? p.w1 : p.w0;
+      };
+      const unsigned long long k0 = ck::noisy_key(weight(m) + e0, m, rev);
+      const unsigned long long k1 = ck::noisy_key(weight(m + 1u) + e1, m + 1u, rev);
+      atomicMax(&sh.best[at], m + 1u < n && k1 > k0 ? k1 : k0);
     }
   }
   wave_lds_fence();
-  ck::PlyResult res = {0u, 0u, 0u, 0};
-  if (step) {
+  if (on) {
     const uint32_t n = w.n;
     res.n = n;
     if (TRACE) ld = ck::list_digest(L, g, n);
@@ -252,11 +367,8 @@ __device__ __forceinline__ ck::PlyResult noisy_plies(NoisyShare &sh, uint64_t to
       ck::select_move(w, m, sq, sl, tab);
       ck::play_slot(L, 0u, sq, sl, tab);
     }
-  } else if (on) {
-    NoiseDrawn noise = {sh.draws[rank], {r, 0.0f}};
-    res = ck::noisy_walk<TRACE>(L, g, r, &ld, noise);
   }
-  return res;
+  wave_lds_fence();
 }
 
 template <uint32_t POLICY, bool TRACE, uint32_t REFILL>
@@ -274,15 +386,15 @@ __global__ void __launch_bounds__(1024) k_playouts(PlayoutArgs a) {
     a.keys = d->keys_at ? (const uint32_t *)(base + d->keys_at) : nullptr;
   }
   __shared__ LdsTables tables;
-  // kWordRows x 64 words per wave, then the noisy heuristic's NoisyShare per wave
+  // kWordRows x 64 words per wave, then the heuristics' WalkShare per wave
   extern __shared__ __align__(8) uint32_t wave_words[];
   tables.fill();
   __syncthreads();
   const Lookup tab = {tables};
   const uint32_t lane = threadIdx.x & 63u;
   uint32_t *const words = wave_words + (threadIdx.x >> 6) * (kWordRows * 64u) + lane;
-  NoisyShare &share =
-      ((NoisyShare *)(wave_words + (blockDim.x >> 6) * (kWordRows * 64u)))[threadIdx.x >> 6];
+  WalkShare &share =
+      ((WalkShare *)(wave_words + (blockDim.x >> 6) * (kWordRows * 64u)))[threadIdx.x >> 6];
   const uint32_t nthreads = gridDim.x * blockDim.x;
   // Lanes that hold a game, and those of them whose ply waits for the walk phase.  Wave masks (in
   // scalar registers) rather than per-lane flags: flags changed on divergent paths are kept in
@@ -399,26 +511,30 @@ __global__ void __launch_bounds__(1024) k_playouts(PlayoutArgs a) {
       if (nd >= defer_min || deferred == active || since_walk >= 8u) {
         since_walk = 0;
         uint64_t todo = deferred;
-        if (POLICY == MI_POLICY_HEURISTIC_NOISY && nd > kShared)
-          todo = __ballot(lane_in(deferred) && lane_rank(deferred) < kShared);
-        const bool on = lane_in(todo);
         const uint32_t r = words[ply & ((kWordRows - 1u) * kPly)];
         ck::PlyResult res = {0u, 0u, 0u, 0};
         uint32_t ld = 0;
-        if (POLICY == MI_POLICY_HEURISTIC_NOISY) {
-          res = noisy_plies<TRACE>(share, todo, L, gd, r, ld, tab);
-        } else if (on) {
-          if (POLICY == MI_POLICY_RANDOM) {
+        if (POLICY == MI_POLICY_RANDOM) {
+          if (lane_in(todo)) {
             // capture trees in closed form; the walk only for king trees past two jumps
             bool deep = false;
             res = ck::ply_random_captures<TRACE>(L, gd, r, &ld, deep, tab);
             if (deep) res = ck::ply_random_given<TRACE>(L, gd, r, &ld);
-          } else {
-            res = ck::ply_heuristic_given<TRACE>(L, gd, r, &ld);
           }
+        } else {
+          uint64_t captures = deferred;
+          if (POLICY == MI_POLICY_HEURISTIC_NOISY) captures &= __ballot(gd.capture != 0u);
+          uint64_t steps = deferred & ~captures;
+          if (captures) capture_plies<POLICY, TRACE>(share, captures, L, gd, r, res, ld, tab);
+          if (POLICY == MI_POLICY_HEURISTIC_NOISY && steps) {
+            if (__popcll(steps) > kSharedSteps)
+              steps = __ballot(lane_in(steps) && lane_rank(steps) < kSharedSteps);
+            noisy_steps<TRACE>(share, steps, L, gd, r, res, ld, tab);
+          }
+          todo = captures | steps;
         }
         deferred &= ~todo;
-        decided(on, res, ld);
+        decided(lane_in(todo), res, ld);
       } else {
         since_walk++;
       }
@@ -758,7 +874,7 @@ __global__ void __launch_bounds__(256) k_valu_rate(uint32_t iters, uint32_t salt
 
 uint32_t playout_lds(uint32_t policy, uint32_t block) {
   return block / 64u * (uint32_t)(kWordRows * 64u * sizeof(uint32_t) +
-                                  (policy == MI_POLICY_HEURISTIC_NOISY ? sizeof(NoisyShare) : 0u));
+                                  (policy == MI_POLICY_RANDOM ? 0u : sizeof(WalkShare)));
 }
 
 namespace {

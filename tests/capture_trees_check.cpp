@@ -48,7 +48,7 @@ int main() {
     most = (long)n > most ? (long)n : most;
     bad += t.n != n;
     for (uint32_t k = 0; k < n && k < t.n && k < 1024u; k++) {
-      const Choice m = capture_choice(L, g, t, k, Direct());
+      const Choice m = capture_choice(t, k, Direct());
       moves++;
       bad += m.from != list[k].from || m.to != list[k].to || m.removed != list[k].removed;
     }
