@@ -315,8 +315,9 @@ CK_HD uint32_t sub_if(uint32_t k, uint32_t c) {
 // hold them in LDS (playout_kernels.hip), where a read costs one issue slot.
 //   mod(r, n)      r mod n, 1 <= n <= kModMax (the moves of four slot masks)
 //   nth(y, j)      the slot of the j-th move of one square: bit 8t of y is set where slot t has one
-//   move(i, f, r)  masks of a move: i = square | slot << 5 | king << 7 | capture << 8; f flips the
-//                  squares it leaves and enters, r holds the piece it removes
+//   move(i, f, r)  masks of a move: i = (square | slot << 5 | king << 7 | capture << 8) << 3; f
+//                  flips the squares it leaves and enters, r holds the piece it removes
+//   slot8(y, j)    the same slot << 8
 //   kth(m, j)      the j-th set bit of the four bits m
 //   path(i)        the steps of a capture sequence: i = leaf | king << 4 (CaptureTrees' leaves)
 constexpr uint32_t kModMax = 128;
@@ -360,12 +361,13 @@ CK_HD uint32_t path_word(uint32_t i) {
 }
 
 struct Direct {
+  CK_HD uint32_t slot8(uint32_t y, uint32_t j) const { return nth(y, j) << 8; }
   CK_HD uint32_t kth(uint32_t m, uint32_t j) const { return nth_slot(m, j); }
   CK_HD uint32_t path(uint32_t i) const { return path_word(i); }
   CK_HD uint32_t mod(uint32_t r, uint32_t n) const { return mod_small(r, n); }
   CK_HD uint32_t nth(uint32_t y, uint32_t j) const { return nth_slot(gather4(y) >> 2, j); }
   CK_HD void move(uint32_t i, uint32_t &flip, uint32_t &removed) const {
-    move_masks(i, flip, removed);
+    move_masks(i >> 3, flip, removed);
   }
 };
 
@@ -382,9 +384,9 @@ CK_HD uint32_t mod_factor(uint32_t n) { return 0xFFFFFFFFu / (n ? n : 1u); }
 // k-th move (0-based) in square-major, slot-minor order.  The word of eight squares that holds it
 // is found from the words' move counts; inside it three steps halve the squares, each counting the
 // moves of the lower half with one popcount and shifting the upper half down where the move lies
-// there.  What is left in bits 0, 8, 16 and 24 are the moves of one square.
+// there.  What is left in bits 0, 8, 16 and 24 are the moves of one square.  sl8: the slot << 8.
 template <class TAB>
-CK_HD void select_move(const SlotWords &w, uint32_t k, uint32_t &sq, uint32_t &sl,
+CK_HD void select_move(const SlotWords &w, uint32_t k, uint32_t &sq, uint32_t &sl8,
                        const TAB &tab) {
   const bool g2 = k >= w.n01;
   const uint32_t lo = g2 ? w.x2 : w.x0, hi = g2 ? w.x3 : w.x1;
@@ -406,11 +408,12 @@ CK_HD void select_move(const SlotWords &w, uint32_t k, uint32_t &sq, uint32_t &s
   x >>= s1;
   k = sub_if(k, c1);
   sq = ((g2 ? 16u : 0u) | (g1 ? 8u : 0u)) | (s4 | s2 | s1);
-  sl = tab.nth(x & 0x01010101u, k);
+  sl8 = tab.slot8(x & 0x01010101u, k);
 }
 
 CK_HD void select_slot(const uint32_t s[4], uint32_t k, uint32_t &sq, uint32_t &sl) {
   select_move(slot_words(s), k, sq, sl, Direct());
+  sl >>= 8;
 }
 
 // ------------------------------------------------------------------------------------------
@@ -485,14 +488,23 @@ CK_HD void apply(Lane &L, uint32_t from, uint32_t to, uint32_t removed) {
   L.turn ^= 1u;
 }
 
-// The move of slot choice (square sq, slot sl), applied (a king is a piece on sq with its bit set:
+// All ones when bit i (< 32) of m is set, else 0.
+CK_HD uint32_t bit_mask(uint32_t m, uint32_t i) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return (uint32_t)__builtin_amdgcn_sbfe((int)m, i, 1u);
+#else
+  return 0u - ((m >> i) & 1u);
+#endif
+}
+
+// The move of slot choice (square sq, slot sl8 >> 8), applied (a king is a piece on sq with its bit set:
 // own holds sq).  A man's entered square on the far row becomes a king; kings hold no empty square,
 // so flipping sets it.
 template <class TAB>
-CK_HD void play_slot(Lane &L, uint32_t capture, uint32_t sq, uint32_t sl, const TAB &tab) {
-  const uint32_t km = 0u - ((L.kings >> sq) & 1u);  // all ones: the piece is a king
+CK_HD void play_slot(Lane &L, uint32_t capture, uint32_t sq, uint32_t sl8, const TAB &tab) {
+  const uint32_t km = bit_mask(L.kings, sq);  // all ones: the piece is a king
   uint32_t flip, removed;
-  tab.move((sq | (sl << 5) | (km & 128u)) + (capture ? 256u : 0u), flip, removed);
+  tab.move((sq << 3) + sl8 + (km & 1024u) + (capture ? 2048u : 0u), flip, removed);
   const uint32_t own = L.own ^ flip;
   const uint32_t opp = L.opp & ~removed;
   const uint32_t kings = (L.kings & ~removed) ^ (flip & (km | ROW7));
@@ -1259,9 +1271,9 @@ CK_HD PlyResult ply_random_fast(Lane &L, uint32_t r, uint32_t *list_dig, bool &d
   res.chosen = k;
   res.over = 0u;
   res.winner = 0;
-  uint32_t sq, sl;
-  select_move(w, L.turn ? n - 1u - k : k, sq, sl, tab);
-  play_slot(L, g.capture, sq, sl, tab);
+  uint32_t sq, sl8;
+  select_move(w, L.turn ? n - 1u - k : k, sq, sl8, tab);
+  play_slot(L, g.capture, sq, sl8, tab);
   return res;
 }
 
@@ -1271,32 +1283,64 @@ CK_HD PlyResult ply_random_fast(Lane &L, uint32_t r, uint32_t *list_dig, bool &d
 // takes no materials to see: one ply in a thousand has single jumps of several weights (the walk,
 // which computes weights, plays those) and one in 27 steps of two (noisy games from 20 to 60 plies
 // on).  Sorting the moves into weight classes on every ply took a third more cycles than the random
-// ply: heuristic-1024x1024 0.59 ms, now 0.52.
+// ply: heuristic-1024x1024 0.59 ms, 0.52 without.
 //
 // Men whose moves in slots 0 and 1 promote.
 CK_HD uint32_t promoting(const Lane &L, const Gen &g) {
   return L.own & ~L.kings & (g.capture ? ROW5 : ROW6);
 }
 // Whether some moves promote and some do not.
-CK_HD bool some_promote(const Gen &g, uint32_t prom) {
+CK_HD void promote_parts(const Gen &g, uint32_t prom, uint32_t &with, uint32_t &without) {
   const uint32_t men = g.slot[0] | g.slot[1];
-  return (men & prom) && ((men & ~prom) | g.slot[2] | g.slot[3]);
+  with = men & prom;
+  without = (men & ~prom) | g.slot[2] | g.slot[3];
 }
-// Whether some jumps remove a king and some do not.
+CK_HD bool some_promote(const Gen &g, uint32_t prom) {
+  uint32_t with, without;
+  promote_parts(g, prom, with, without);
+  return with && without;
+}
+// Whether some jumps remove a king and some do not: the pieces that a jump can remove, by kind.
+CK_HD void king_parts(const Lane &L, const Gen &g, uint32_t &with, uint32_t &without) {
+  const uint32_t kng = L.own & L.kings;
+  const uint32_t jumped = step0(L.own & g.cap[0]) | step1(L.own & g.cap[1]) |
+                          step2(kng & g.cap[2]) | step3(kng & g.cap[3]);
+  with = jumped & L.kings;
+  without = jumped & ~L.kings;
+}
 CK_HD bool some_take_kings(const Lane &L, const Gen &g) {
-  const uint32_t okings = L.opp & L.kings;
-  const uint32_t k0 = step3(okings), k1 = step2(okings);  // next to a king in direction 0, 1
-  // a man's slot 0 jumps in direction 1, its slot 1 in direction 0
-  const uint32_t s0 = (L.kings & k0) | (~L.kings & k1), s1 = (L.kings & k1) | (~L.kings & k0);
-  const uint32_t s2 = step1(okings), s3 = step0(okings);
-  const uint32_t with = (g.slot[0] & s0) | (g.slot[1] & s1) | (g.slot[2] & s2) | (g.slot[3] & s3);
-  const uint32_t without =
-      (g.slot[0] & ~s0) | (g.slot[1] & ~s1) | (g.slot[2] & ~s2) | (g.slot[3] & ~s3);
+  uint32_t with, without;
+  king_parts(L, g, with, without);
   return with && without;
 }
 
-// The heuristic ply whose moves of largest weight are those of the squares `from` (every move of a
-// square in them).
+// The moves of the squares `from` (every move of a square in them).
+CK_HD SlotWords words_from(const Gen &g, uint32_t from) {
+  const uint32_t t[4] = {g.slot[0] & from, g.slot[1] & from, g.slot[2] & from, g.slot[3] & from};
+  return slot_words(t);
+}
+
+// Plays the word's choice among the moves tw, all n moves of the ply being those of g.slot.  Returns
+// its reference index when TRACE.
+template <bool TRACE, class TAB>
+CK_HD uint32_t play_tie(Lane &L, const Gen &g, const SlotWords &tw, uint32_t n, uint32_t r,
+                        const TAB &tab) {
+  const uint32_t k = tab.mod(r, tw.n);
+  uint32_t sq, sl8, chosen = 0u;
+  select_move(tw, L.turn ? tw.n - 1u - k : k, sq, sl8, tab);
+  if (TRACE) {
+    // reference index: rank of the move in the full slot order
+    const uint32_t below = bit(sq) - 1u;
+    uint32_t i = popc(g.slot[0] & below) + popc(g.slot[1] & below) + popc(g.slot[2] & below) +
+                 popc(g.slot[3] & below);
+    for (uint32_t s = 0; s < sl8 >> 8; s++) i += getbit(g.slot[s], sq);
+    chosen = L.turn ? n - 1u - i : i;
+  }
+  play_slot(L, g.capture, sq, sl8, tab);
+  return chosen;
+}
+
+// The heuristic ply whose moves of largest weight are those of the squares `from`.
 template <bool TRACE, class TAB>
 CK_HD PlyResult play_tied(Lane &L, const Gen &g, uint32_t from, uint32_t r, uint32_t *list_dig,
                           const TAB &tab) {
@@ -1310,23 +1354,9 @@ CK_HD PlyResult play_tied(Lane &L, const Gen &g, uint32_t from, uint32_t r, uint
     res.winner = L.counter < 50u ? (int32_t)(L.turn ^ 1u) : -1;
     return res;
   }
-  const uint32_t t[4] = {g.slot[0] & from, g.slot[1] & from, g.slot[2] & from, g.slot[3] & from};
-  const SlotWords tw = slot_words(t);
-  const uint32_t k = tab.mod(r, tw.n);
   res.over = 0u;
   res.winner = 0;
-  res.chosen = 0u;
-  uint32_t sq, sl;
-  select_move(tw, L.turn ? tw.n - 1u - k : k, sq, sl, tab);
-  if (TRACE) {
-    // reference index: rank of (sq, sl) in the full slot order
-    const uint32_t below = bit(sq) - 1u;
-    uint32_t i = popc(g.slot[0] & below) + popc(g.slot[1] & below) + popc(g.slot[2] & below) +
-                 popc(g.slot[3] & below);
-    for (uint32_t s = 0; s < sl; s++) i += getbit(g.slot[s], sq);
-    res.chosen = L.turn ? n - 1u - i : i;
-  }
-  play_slot(L, g.capture, sq, sl, tab);
+  res.chosen = play_tie<TRACE>(L, g, words_from(g, from), n, r, tab);
   return res;
 }
 
@@ -1729,12 +1759,12 @@ CK_HD PlyResult ply_noisy_fast(Lane &L, uint32_t r, uint32_t *list_dig, bool &de
   // every weight is +inf when no opponent's piece is left after the move: the first move then
   const bool inf = !(g.capture ? L.opp & (L.opp - 1u) : L.opp);
   const uint32_t k = inf ? 0u : tab.mod(r, n);  // reference index
-  uint32_t sq, sl;
-  select_move(w, L.turn ? n - 1u - k : k, sq, sl, tab);
+  uint32_t sq, sl8;
+  select_move(w, L.turn ? n - 1u - k : k, sq, sl8, tab);
   res.over = 0u;
   res.winner = 0;
   res.chosen = k;
-  play_slot(L, g.capture, sq, sl, tab);
+  play_slot(L, g.capture, sq, sl8, tab);
   return res;
 }
 
@@ -1746,24 +1776,6 @@ CK_HD uint32_t start_plies(uint32_t seed, uint32_t i, uint32_t a, uint32_t kmin,
   philox(0u, a, TAG_START, 1u, seed, i, w);
   const uint32_t k = kmin + mod_u32(w[0], span);
   return k < 0x10000u ? k : 0x10000u;
-}
-
-// The common part of a start position's ply: the random ply, but with `stop` the position is left
-// as it is.  res.over: the game is over; deferred: the ply waits for the walk phase.
-template <class TAB>
-CK_HD PlyResult ply_start_fast(Lane &L, uint32_t r, bool stop, bool &deferred, Gen &g,
-                               const TAB &tab) {
-  analyse(L, g);
-  const SlotWords w = slot_words(g.slot);
-  PlyResult res = {w.n, 0u, 0u, 0};
-  res.over = w.n == 0u || L.counter >= 50u;  // (an origin of longer captures has its slot's bit too)
-  deferred = g.multi != 0u && !res.over && !stop;
-  if (deferred || res.over || stop) return res;
-  const uint32_t k = tab.mod(r, w.n);
-  uint32_t sq, sl;
-  select_move(w, L.turn ? w.n - 1u - k : k, sq, sl, tab);
-  play_slot(L, g.capture, sq, sl, tab);
-  return res;
 }
 
 // True when the position is finished (no legal move, or the draw counter reached 50).

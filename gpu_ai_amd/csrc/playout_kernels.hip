@@ -9,8 +9,10 @@
 // only reciprocals take longer), so what a ply would compute from small operands -- the factor of
 // r mod n, the j-th slot of a square, a move's masks -- and its Philox words are read from LDS,
 // one issue slot each, flags of the lanes are wave masks in scalar registers (355 -> 269 vector
-// instructions per wave iteration on random-1024x1024, 0.778 -> 0.629 ms), and a walk phase takes
-// every origin's capture tree at once (ck::capture_trees; 0.577 ms).  Refill policy
+// instructions per wave iteration on random-1024x1024, 0.778 -> 0.629 ms), a walk phase takes
+// every origin's capture tree at once (ck::capture_trees; 0.577 ms), and all lanes look at their
+// position, whatever they hold, so that which of them wait, play or are done are comparisons
+// straight into wave masks instead of flags carried out of branches (0.525 ms).  Refill policy
 // MI_REFILL_QUEUE claims playout indices for the whole wave in multiples of kChunk from its slab's
 // device counter (one atomic per claim, broadcast with a lane read; slabs are described in
 // kernels.h), MI_REFILL_STATIC strides lanes over the index space without atomics.
@@ -99,6 +101,7 @@ __device__ __forceinline__ void locate(const PlayoutArgs &a, uint32_t g, uint32_
 // The lane logic's lookups (ck::Direct's functions) from LDS, filled once per workgroup.
 struct LdsTables {
   uint32_t factor[ck::kModMax + 1];
+  uint16_t nth8[64];  // a slot << 8
   uint8_t nth[64];
   uint32_t path[32];
   uint2 move[512];
@@ -111,7 +114,11 @@ struct LdsTables {
     }
     for (uint32_t i = threadIdx.x; i <= ck::kModMax; i += blockDim.x) factor[i] = ck::mod_factor(i);
     if (threadIdx.x < 32u) path[threadIdx.x] = ck::path_word(threadIdx.x);
-    if (threadIdx.x < 64u) nth[threadIdx.x] = (uint8_t)ck::nth_slot(threadIdx.x >> 2, threadIdx.x & 3u);
+    if (threadIdx.x < 64u) {
+      const uint32_t sl = ck::nth_slot(threadIdx.x >> 2, threadIdx.x & 3u);
+      nth[threadIdx.x] = (uint8_t)sl;
+      nth8[threadIdx.x] = (uint16_t)(sl << 8);
+    }
   }
 };
 
@@ -120,9 +127,11 @@ struct Lookup {
   __device__ uint32_t mod(uint32_t r, uint32_t n) const { return ck::mod_by(r, n, t.factor[n]); }
   __device__ uint32_t kth(uint32_t m, uint32_t j) const { return t.nth[m * 4u + j]; }
   __device__ uint32_t path(uint32_t i) const { return t.path[i]; }
-  __device__ uint32_t nth(uint32_t y, uint32_t j) const { return t.nth[ck::gather4(y) + j]; }
+  __device__ uint32_t slot8(uint32_t y, uint32_t j) const {  // bytes weigh 4, 8, 16 and 32
+    return t.nth8[__builtin_amdgcn_udot4(y, 0x20100804u, j, false)];
+  }
   __device__ void move(uint32_t i, uint32_t &flip, uint32_t &removed) const {
-    const uint2 m = t.move[i];
+    const uint2 m = *(const uint2 *)((const char *)t.move + i);
     flip = m.x;
     removed = m.y;
   }
@@ -363,9 +372,9 @@ __device__ __forceinline__ void noisy_steps(WalkShare &share, uint64_t todo, ck:
     } else {
       const uint32_t m = ck::noisy_key_move(sh.best[rank], L.turn);
       res.chosen = TRACE ? (L.turn ? n - 1u - m : m) : 0u;
-      uint32_t sq, sl;
-      ck::select_move(w, m, sq, sl, tab);
-      ck::play_slot(L, 0u, sq, sl, tab);
+      uint32_t sq, sl8;
+      ck::select_move(w, m, sq, sl8, tab);
+      ck::play_slot(L, 0u, sq, sl8, tab);
     }
   }
   wave_lds_fence();
@@ -396,16 +405,14 @@ __global__ void __launch_bounds__(1024) k_playouts(PlayoutArgs a) {
   WalkShare &share =
       ((WalkShare *)(wave_words + (blockDim.x >> 6) * (kWordRows * 64u)))[threadIdx.x >> 6];
   const uint32_t nthreads = gridDim.x * blockDim.x;
-  // Lanes that hold a game, and those of them whose ply waits for the walk phase.  Wave masks (in
-  // scalar registers) rather than per-lane flags: flags changed on divergent paths are kept in
-  // vector registers, a dozen instructions per ply.
-  uint64_t active = 0, deferred = 0;
+  // Lanes that hold a game.  A wave mask (in scalar registers) rather than a per-lane flag: flags
+  // changed on divergent paths are kept in vector registers, a dozen instructions per ply.
+  uint64_t active = 0;
   // ply counts in units of kPly, the row stride of `words`: a word's row offset is one mask away
   constexpr uint32_t kPly = 64u;
   uint32_t g = 0, p = 0, j = 0, ply = 0, h = 0, maxn = 0;
   uint32_t plies_acc = 0;  // a lane's plies of a launch stay far below 2^32 (2^31 playouts in all)
   ck::Lane L = {0u, 0u, 0u, 0u, 0u};
-  ck::Gen gd;  // the analysis of a deferred ply, kept for its walk (saves a second analyse)
   // wave-uniform refill and deferral state: the reservation [res_next, res_end) is slab-local in
   // slab `slab`
   uint32_t res_next = 0, res_end = 0, since_walk = 0;
@@ -415,23 +422,17 @@ __global__ void __launch_bounds__(1024) k_playouts(PlayoutArgs a) {
   uint32_t static_next = blockIdx.x * blockDim.x + threadIdx.x;
   const uint32_t defer_min = a.defer_min;
 
-  // Plies were decided on the lanes `on`: their game is over, or its move has been played.
-  auto decided = [&](bool on, const ck::PlyResult &res, uint32_t ld) {
-    if (on) {
-      if (TRACE) h = ck::hash_step(h, ck::ply_record(ld, res.n, res.chosen));
-      maxn = res.n > maxn ? res.n : maxn;
-    }
-    const bool over = on && res.over;
-    if (over) {
-      a.winners[g] = (int8_t)res.winner;
+  // Games that are over on the lanes `over`.
+  auto ended = [&](uint64_t over, int32_t winner) {
+    if (lane_in(over)) {
+      a.winners[g] = (int8_t)winner;
       if (TRACE) {
         if (a.plies) a.plies[g] = ply / kPly;
         if (a.hashes) a.hashes[g] = h;
       }
       plies_acc += ply / kPly;
     }
-    if (on) ply += kPly;  // (of no account once the game is over)
-    active &= ~__ballot(over);
+    active &= ~over;
   };
 
   for (uint32_t iter = 0;; iter++) {
@@ -490,21 +491,53 @@ __global__ void __launch_bounds__(1024) k_playouts(PlayoutArgs a) {
         for (uint32_t w = 0; w < 4u; w++) row[w * 64u] = o[w];
       }
     }
-    // common part of the ply; plies with longer captures (for the noisy heuristic also those whose
-    // moves weigh differently) wait for the walk phase, where they take the same word again
+    // The common part of the ply: every lane looks at its position (an idle lane's or a waiting
+    // one's yields what it did before), and those that can play do.  Plies with longer captures,
+    // for the heuristics also those whose moves weigh differently, wait for the walk phase, where
+    // they take the same word.
+    ck::Gen gen;
+    ck::analyse(L, gen);
+    uint64_t deferred = active & __ballot(gen.multi != 0u);
+    uint32_t from = 0xFFFFFFFFu;  // heuristic: squares of the moves of largest weight
+    if (POLICY != MI_POLICY_RANDOM) {
+      const uint32_t prom = ck::promoting(L, gen);
+      uint32_t pw, po, kw, ko;
+      ck::promote_parts(gen, prom, pw, po);
+      ck::king_parts(L, gen, kw, ko);
+      const uint64_t split = __ballot(pw != 0u) & __ballot(po != 0u) & __ballot(L.opp != 0u);
+      deferred |= active & __ballot(kw != 0u) & __ballot(ko != 0u);
+      deferred |= active & (POLICY == MI_POLICY_HEURISTIC_NOISY
+                                ? split : split & __ballot(gen.origins != 0u));
+      if (lane_in(split)) from = prom;
+    }
     {
-      const bool on = lane_in(active & ~deferred);
-      bool d = false;
-      ck::PlyResult res = {0u, 0u, 0u, 0};
-      uint32_t ld = 0;
-      if (on) {
+      const ck::SlotWords w = POLICY == MI_POLICY_HEURISTIC ? ck::words_from(gen, from)
+                                                            : ck::slot_words(gen.slot);
+      const uint32_t n = POLICY == MI_POLICY_HEURISTIC ? ck::slot_count(gen.slot) : w.n;
+      const uint64_t can = active & ~deferred;
+      const uint64_t go = can & __ballot(w.n != 0u) & __ballot(L.counter < 50u);
+      // (a waiting ply has no fewer moves than first jumps, an idle lane's last game had these)
+      maxn = n > maxn ? n : maxn;
+      uint32_t ld = 0u, chosen = 0xFFFFu;
+      if (TRACE && lane_in(can)) ld = ck::list_digest(L, gen, n);
+      if (lane_in(go)) {
         const uint32_t r = words[ply & ((kWordRows - 1u) * kPly)];
-        if (POLICY == MI_POLICY_RANDOM) res = ck::ply_random_fast<TRACE>(L, r, &ld, d, gd, tab);
-        else if (POLICY == MI_POLICY_HEURISTIC) res = ck::ply_heuristic_fast<TRACE>(L, r, &ld, d, gd, tab);
-        else res = ck::ply_noisy_fast<TRACE>(L, r, &ld, d, gd, tab);
+        if (POLICY == MI_POLICY_HEURISTIC) {
+          chosen = ck::play_tie<TRACE>(L, gen, w, n, r, tab);
+        } else {
+          chosen = tab.mod(r, w.n);
+          // with no opponent's piece left after the move every noisy weight is +inf: the first move
+          if (POLICY == MI_POLICY_HEURISTIC_NOISY &&
+              !(gen.capture ? L.opp & (L.opp - 1u) : L.opp))
+            chosen = 0u;
+          uint32_t sq, sl8;
+          ck::select_move(w, L.turn ? w.n - 1u - chosen : chosen, sq, sl8, tab);
+          ck::play_slot(L, gen.capture, sq, sl8, tab);
+        }
+        ply += kPly;
       }
-      deferred |= __ballot(on && d);
-      decided(on && !d, res, ld);
+      if (TRACE && lane_in(can)) h = ck::hash_step(h, ck::ply_record(ld, n, chosen));
+      if (can & ~go) ended(can & ~go, L.counter < 50u ? (int32_t)(L.turn ^ 1u) : -1);
     }
     if (deferred) {
       const uint32_t nd = (uint32_t)__popcll(deferred);
@@ -518,23 +551,28 @@ __global__ void __launch_bounds__(1024) k_playouts(PlayoutArgs a) {
           if (lane_in(todo)) {
             // capture trees in closed form; the walk only for king trees past two jumps
             bool deep = false;
-            res = ck::ply_random_captures<TRACE>(L, gd, r, &ld, deep, tab);
-            if (deep) res = ck::ply_random_given<TRACE>(L, gd, r, &ld);
+            res = ck::ply_random_captures<TRACE>(L, gen, r, &ld, deep, tab);
+            if (deep) res = ck::ply_random_given<TRACE>(L, gen, r, &ld);
           }
         } else {
           uint64_t captures = deferred;
-          if (POLICY == MI_POLICY_HEURISTIC_NOISY) captures &= __ballot(gd.capture != 0u);
+          if (POLICY == MI_POLICY_HEURISTIC_NOISY) captures &= __ballot(gen.capture != 0u);
           uint64_t steps = deferred & ~captures;
-          if (captures) capture_plies<POLICY, TRACE>(share, captures, L, gd, r, res, ld, tab);
+          if (captures) capture_plies<POLICY, TRACE>(share, captures, L, gen, r, res, ld, tab);
           if (POLICY == MI_POLICY_HEURISTIC_NOISY && steps) {
             if (__popcll(steps) > kSharedSteps)
               steps = __ballot(lane_in(steps) && lane_rank(steps) < kSharedSteps);
-            noisy_steps<TRACE>(share, steps, L, gd, r, res, ld, tab);
+            noisy_steps<TRACE>(share, steps, L, gen, r, res, ld, tab);
           }
           todo = captures | steps;
         }
-        deferred &= ~todo;
-        decided(lane_in(todo), res, ld);
+        if (lane_in(todo)) {
+          if (TRACE) h = ck::hash_step(h, ck::ply_record(ld, res.n, res.chosen));
+          maxn = res.n > maxn ? res.n : maxn;
+        }
+        const uint64_t over = todo & __ballot(res.over != 0u);
+        if (over) ended(over, res.winner);
+        if (lane_in(todo)) ply += kPly;
       } else {
         since_walk++;
       }
@@ -662,14 +700,12 @@ __global__ void __launch_bounds__(64) k_start_positions(StartArgs a) {
   const Lookup tab = {tables};
   uint32_t *const words = rows + lane;
   constexpr uint32_t kPly = 64u;  // as in k_playouts
-  // lanes that play an attempt, those of them that wait for the walk phase, and lanes that hold an
-  // accepted attempt's position
-  uint64_t active = 0, deferred = 0, held = 0;
+  // lanes that play an attempt, and lanes that hold an accepted attempt's position
+  uint64_t active = 0, held = 0;
   uint64_t open = 0;           // slots with a position
   uint32_t lo = 0, hi = 0;     // of this lane's slot
   uint32_t slot = 0, i = 0, attempt = 0, ply = 0, limit = 0;
   ck::Lane L = {0u, 0u, 0u, 0u, 0u};
-  ck::Gen gd;
   uint32_t since_walk = 0;
   // (few positions: one slab, since 16 slabs of blocks of kSlabBlock would leave most waves without)
   const uint32_t nslabs = a.n < 32u * kSlabBlock * kSlabs ? 1u : min(gridDim.x, kSlabs);
@@ -696,7 +732,6 @@ __global__ void __launch_bounds__(64) k_start_positions(StartArgs a) {
         if (by != kOpen && by == attempt) a.out[i] = packed_position(L);
         const uint64_t gone = __ballot(by != kOpen);
         active &= ~gone;
-        deferred &= ~gone;
         held &= ~gone;
       }
       {  // close decided slots (a position all of whose attempts ended is reported)
@@ -791,35 +826,42 @@ __global__ void __launch_bounds__(64) k_start_positions(StartArgs a) {
         for (uint32_t w = 0; w < 4u; w++) row[w * 64u] = o[w];
       }
     }
-    {
-      const bool on = lane_in(active & ~deferred);
-      bool d = false, ended = false, accepted = false;
-      if (on) {
-        const uint32_t r = words[ply & ((kWordRows - 1u) * kPly)];
-        const bool stop = ply == limit;
-        const ck::PlyResult res = ck::ply_start_fast(L, r, stop, d, gd, tab);
-        ended = res.over || stop;
-        accepted = ended && !(res.over && a.reject);
-        if (ended) atomicOr(&marks[accepted ? 64u + slot : slot], 1ull << (attempt & 63u));
-        if (!d) ply += kPly;
-      }
-      deferred |= __ballot(d);
-      active &= ~__ballot(ended);
-      held |= __ballot(accepted);
+    // The common part of the ply, as in k_playouts; a position at its limit is left as it is.
+    ck::Gen gen;
+    ck::analyse(L, gen);
+    const ck::SlotWords w = ck::slot_words(gen.slot);
+    const uint64_t stop = __ballot(ply == limit);
+    // (an origin of longer captures has its slot's bit too)
+    const uint64_t over = ~(__ballot(w.n != 0u) & __ballot(L.counter < 50u));
+    const uint64_t done = active & (stop | over);
+    const uint64_t deferred = active & ~done & __ballot(gen.multi != 0u);
+    const uint64_t go = active & ~done & ~deferred;
+    const uint32_t r = words[ply & ((kWordRows - 1u) * kPly)];
+    if (lane_in(go)) {
+      const uint32_t k = tab.mod(r, w.n);
+      uint32_t sq, sl8;
+      ck::select_move(w, L.turn ? w.n - 1u - k : k, sq, sl8, tab);
+      ck::play_slot(L, gen.capture, sq, sl8, tab);
+      ply += kPly;
+    }
+    if (done) {
+      const uint64_t accepted = a.reject ? done & ~over : done;
+      if (lane_in(done))
+        atomicOr(&marks[lane_in(accepted) ? 64u + slot : slot], 1ull << (attempt & 63u));
+      active &= ~done;
+      held |= accepted;
     }
     if (deferred) {
       const uint32_t nd = (uint32_t)__popcll(deferred);
       if (nd >= 16u || deferred == active || since_walk >= 8u) {
         since_walk = 0;
         if (lane_in(deferred)) {
-          const uint32_t r = words[ply & ((kWordRows - 1u) * kPly)];
           uint32_t unused = 0;
           bool deep = false;  // (the game is not over: captures, and the draw count below 50)
-          ck::ply_random_captures<false>(L, gd, r, &unused, deep, tab);
-          if (deep) ck::ply_random_given<false>(L, gd, r, &unused);
+          ck::ply_random_captures<false>(L, gen, r, &unused, deep, tab);
+          if (deep) ck::ply_random_given<false>(L, gen, r, &unused);
           ply += kPly;
         }
-        deferred = 0;
       } else {
         since_walk++;
       }
