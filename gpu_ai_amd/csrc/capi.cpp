@@ -71,17 +71,27 @@ uint32_t tune_bucket(uint64_t total) {
   return b < kTuneBuckets ? b : kTuneBuckets - 1u;
 }
 
+mi_tuning batch_shape(const mi_ctx *ctx, uint64_t total) {
+  mi_tuning t = ctx->tuning;
+  const uint64_t lanes = 64u * (uint64_t)ctx->cus;  // of a wave per CU
+  if (ctx->shaped || total <= 4u * lanes) return t;
+  const uint64_t waves = (total + lanes - 1u) / lanes;
+  t.block_size = 64u * (uint32_t)(total >= 32u * lanes ? 16u : waves < 12u ? waves : 12u);
+  t.blocks_per_cu = 1u;
+  return t;
+}
+
 // Whether a batch of `total` playouts runs with one wave per game (k_playouts_wave).  A small batch
-// lasts as long as its longest game: 0.41-0.66 us per ply with a wave of its own (random, noisy)
-// against 1.0-2.3 us in a wave of 64 games, but a game costs a whole wave's instructions, so from
+// lasts as long as its longest game: 0.41-0.65 us per ply with a wave of its own (random, noisy)
+// against 0.9-1.5 us in a wave of 64 games, but a game costs a whole wave's instructions, so from
 // some size on the lanes win.  Kernel ms, one wave per game / one lane per game, 256 CUs:
-//   playouts       256          4,096        8,192        16,384       32,768
-//   random     .060 / .140  .088 / .148  .120 / .144  .170 / .146  .278 / .166
-//   heuristic  .062 / .213  .105 / .206  .145 / .199  .217 / .202  .352 / .208
-//   noisy      .079 / .395  .124 / .331  .174 / .319  .238 / .330  .393 / .333
+//   playouts       256          4,096        8,192        12,288       16,384
+//   random     .074 / .129  .106 / .121  .142 / .128  .160 / .133  .195 / .135
+//   heuristic  .082 / .149  .125 / .139  .163 / .142  .191 / .149  .224 / .151
+//   noisy      .089 / .208  .133 / .185  .168 / .186  .202 / .185  .233 / .185
 // A context that was given a launch shape, or has measured one for the batch's size, uses it.
 bool wave_batch(const mi_ctx *ctx, uint32_t policy, uint64_t total) {
-  if (ctx->shaped || total > (uint64_t)ctx->cus * (policy == MI_POLICY_HEURISTIC_NOISY ? 64u : 32u))
+  if (ctx->shaped || total > (uint64_t)ctx->cus * (policy == MI_POLICY_HEURISTIC_NOISY ? 32u : 16u))
     return false;
   const TuneEntry *e = ctx->tune_table[policy][tune_bucket(total)];
   return e[0].kernel_ms < 0.f && e[1].kernel_ms < 0.f;
@@ -245,7 +255,7 @@ mi_tuning shape_for(const mi_ctx *ctx, uint32_t policy, uint64_t total, int only
     if (e[r].kernel_ms < 0.f || (only >= 0 && r != only)) continue;
     if (!best || e[r].kernel_ms < best->kernel_ms) best = &e[r];
   }
-  return best ? best->tuning : ctx->tuning;
+  return best ? best->tuning : gpuai::ctxutil::batch_shape(ctx, total);
 }
 
 // The statistics' launch shape of such a batch.

@@ -23,8 +23,8 @@ struct HostBuf {
 }  // namespace gpuai
 
 // Default launch shape: 64-thread blocks, 12 per CU (3 waves per SIMD), queue refill, defer_min
-// 16.  Among the fastest shapes for a 1M-playout batch, and a small batch spreads over many CUs
-// instead of sharing a few SIMDs.
+// 16.  A small batch spreads over many CUs this way instead of sharing a few SIMDs; larger ones take
+// batch_shape's.
 constexpr mi_tuning kDefaultTuning = {64u, 12u, MI_REFILL_QUEUE, 16u};
 
 // Launch-shape table: the fastest shape the autotuner measured for a policy, a batch-size bucket
@@ -80,6 +80,14 @@ int ensure(mi_ctx *ctx, DevBuf &b, size_t bytes);
 int ensure_host(mi_ctx *ctx, HostBuf &b, size_t bytes);
 // Batch-size bucket of the launch-shape table: floor(log2(total)).
 uint32_t tune_bucket(uint64_t total);
+// The launch shape of a batch of `total` playouts that the table has none for: the context's, when
+// one was given.  Otherwise a workgroup per CU with the waves that the batch fills, up to 12 (3 a
+// SIMD), and 16 from two games a lane on: waves of a workgroup hand their last games over to each
+// other (playout_kernels.hip), and 16 hide each other's latencies better but have more last games.
+// Against 64x12, in ms: 1024x1024 0.546 -> 0.480 with 16 waves (0.499 with 12), 64x4096 0.243 ->
+// 0.210 with 12 (0.216 with 16), 65536x256 4.76 -> 4.45 with 16 (4.77 with 12).  Up to four waves a CU there is nothing to hand
+// over, and 64-thread blocks it is.
+mi_tuning batch_shape(const mi_ctx *ctx, uint64_t total);
 // Whether a batch runs with one wave per game.
 bool wave_batch(const mi_ctx *ctx, uint32_t policy, uint64_t total);
 }  // namespace ctxutil

@@ -232,17 +232,18 @@ extern "C" int mi_run_playouts_noalloc(mi_ctx *ctx, const mi_pos *pos, uint32_t 
   a.work = &S->work;
   a.defer_min = ctx->tuning.defer_min;
   a.desc = &S->desc;
-  // the grid as mi_run_playouts sizes it; with counts in device memory the total is unknown
-  // here, so the whole resident grid runs (waves without work leave at their first refill)
+  // the shape and grid as mi_run_playouts sizes them; with counts in device memory the total is
+  // unknown here, so a whole resident grid of small workgroups runs (waves without work leave at
+  // their first refill, and a small batch is not left on a few CUs)
   if (!counts && gpuai::ctxutil::wave_batch(ctx, policy, uniform_total)) {
     MI_HIP(ctx, gpuai::launch_playouts_wave(a, policy, (uint32_t)uniform_total, s));
     return MI_OK;
   }
-  const uint64_t block = ctx->tuning.block_size;
-  const uint64_t resident = (uint64_t)ctx->cus * ctx->tuning.blocks_per_cu;
+  const mi_tuning t = counts ? ctx->tuning : gpuai::ctxutil::batch_shape(ctx, uniform_total);
+  const uint64_t block = t.block_size;
+  const uint64_t resident = (uint64_t)ctx->cus * t.blocks_per_cu;
   const uint64_t need = counts ? resident : (uniform_total + block - 1) / block;
   const uint32_t grid = gpuai::grid_size(need, resident);
-  MI_HIP(ctx, gpuai::launch_playouts(a, policy, false, ctx->tuning.refill, grid, (uint32_t)block,
-                                     s));
+  MI_HIP(ctx, gpuai::launch_playouts(a, policy, false, t.refill, grid, (uint32_t)block, s));
   return MI_OK;
 }

@@ -45,6 +45,12 @@ __device__ __forceinline__ bool lane_in(uint64_t mask) {
   return __builtin_amdgcn_inverse_ballot_w64(mask);
 }
 
+__device__ __forceinline__ uint64_t uniform64(uint64_t x) {
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)x);
+  const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(x >> 32));
+  return (uint64_t)hi << 32 | lo;
+}
+
 __device__ __forceinline__ uint64_t rotate_right(uint64_t x, uint32_t n) {
   return x >> n | x << ((64u - n) & 63u);
 }
@@ -380,6 +386,40 @@ __device__ __forceinline__ void noisy_steps(WalkShare &share, uint64_t todo, ck:
   wave_lds_fence();
 }
 
+// The waves of a workgroup hand their last games over.  Once no playout is left to claim, a wave's
+// games end one after the other while an iteration costs the same to its last one: on
+// random-64x4096 72% of all wave iterations had 18 of 64 lanes playing.  A wave with at most half of
+// its lanes playing therefore asks for games (its bit in `asking`) or, where another wave asks,
+// leaves it its own and ends.  The giver takes the other's bit back, writes the games over its own
+// Philox words, which it needs no more, and then sets the other's entry in `given`; a wave whose bit
+// was taken so does not end before it has its games, and the giver writes them without waiting for
+// anything.  Games leave a SIMD that has several waves for one with no more (wave w of a workgroup
+// runs on SIMD w & 3): what is saved is the turns that waves of a SIMD wait for each other.  Up to
+// four waves have a SIMD each and nothing to save (there the checks alone took 21000x3 from 133 to
+// 150 us).  random-1024x1024 0.525 -> 0.48 ms, random-64x4096 0.232 -> 0.21 ms with 16 and 12 waves
+// in a workgroup per CU against as many workgroups of one wave.
+struct Handover {
+  uint32_t asking;     // a bit per wave
+  uint32_t alive;      // waves that play
+  uint32_t given[16];  // games handed to a wave << 8 | giver + 1
+};
+
+__device__ __forceinline__ uint32_t lds_value(const uint32_t &x) {
+  return __builtin_amdgcn_readfirstlane(
+      __hip_atomic_load(&x, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP));
+}
+// Clears the bits in a word; returns what it held.
+__device__ __forceinline__ uint32_t lds_take(uint32_t &x, uint32_t bits) {
+  uint32_t old = 0u;
+  if ((threadIdx.x & 63u) == 0u)
+    old = __hip_atomic_fetch_and(&x, ~bits, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP);
+  return __builtin_amdgcn_readfirstlane(old);
+}
+__device__ __forceinline__ void lds_set(uint32_t &x, uint32_t bits) {
+  if ((threadIdx.x & 63u) == 0u)
+    __hip_atomic_fetch_or(&x, bits, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
 template <uint32_t POLICY, bool TRACE, uint32_t REFILL>
 __global__ void __launch_bounds__(1024) k_playouts(PlayoutArgs a) {
   if (a.desc) {  // graph replays and allocation-free launches: the batch lives in device memory
@@ -397,10 +437,17 @@ __global__ void __launch_bounds__(1024) k_playouts(PlayoutArgs a) {
   __shared__ LdsTables tables;
   // kWordRows x 64 words per wave, then the heuristics' WalkShare per wave
   extern __shared__ __align__(8) uint32_t wave_words[];
+  __shared__ Handover handover;
   tables.fill();
+  if (threadIdx.x < 16u) handover.given[threadIdx.x] = 0u;
+  if (threadIdx.x == 0u) {
+    handover.asking = 0u;
+    handover.alive = (1u << (blockDim.x >> 6)) - 1u;
+  }
   __syncthreads();
   const Lookup tab = {tables};
   const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   uint32_t *const words = wave_words + (threadIdx.x >> 6) * (kWordRows * 64u) + lane;
   WalkShare &share =
       ((WalkShare *)(wave_words + (blockDim.x >> 6) * (kWordRows * 64u)))[threadIdx.x >> 6];
@@ -422,6 +469,40 @@ __global__ void __launch_bounds__(1024) k_playouts(PlayoutArgs a) {
   uint32_t static_next = blockIdx.x * blockDim.x + threadIdx.x;
   const uint32_t defer_min = a.defer_min;
 
+  // A game on its way to another wave: word w of the game in place i is games[w * 32 + i].
+  auto give = [&](uint32_t *games, uint32_t i) {
+    games[i] = L.own;
+    games[32u + i] = L.opp;
+    games[64u + i] = L.kings;
+    games[96u + i] = L.turn | L.counter << 1;
+    games[128u + i] = g;
+    games[160u + i] = p;
+    games[192u + i] = j;
+    games[224u + i] = ply;
+    if (TRACE) games[256u + i] = h;
+  };
+  auto receive = [&](const uint32_t *games, uint32_t i) {
+    L.own = games[i];
+    L.opp = games[32u + i];
+    L.kings = games[64u + i];
+    L.turn = games[96u + i] & 1u;
+    L.counter = games[96u + i] >> 1;
+    g = games[128u + i];
+    p = games[160u + i];
+    j = games[192u + i];
+    ply = games[224u + i];
+    if (TRACE) h = games[256u + i];
+  };
+  // The next four words' block b of the lanes' streams.
+  auto generate = [&](uint32_t b) {
+    uint32_t o[4];
+    ck::philox(b, j, ck::TAG_PLAYOUT, a.epoch, a.seed, p, o);
+    uint32_t *const row = words + (b & 1u) * (4u * 64u);
+#pragma unroll
+    for (uint32_t w = 0; w < 4u; w++) row[w * 64u] = o[w];
+  };
+  uint32_t asks = 0u;  // this wave's bit in handover.asking was set and no games came yet
+
   // Games that are over on the lanes `over`.
   auto ended = [&](uint64_t over, int32_t winner) {
     if (lane_in(over)) {
@@ -435,146 +516,189 @@ __global__ void __launch_bounds__(1024) k_playouts(PlayoutArgs a) {
     active &= ~over;
   };
 
-  for (uint32_t iter = 0;; iter++) {
-    if ((iter & 3u) == 0u) {
-      bool start = false;
-      if (REFILL == MI_REFILL_STATIC) {
-        if (!lane_in(active) && static_next < a.total) {
-          g = static_next;
-          static_next += nthreads;
+  for (;;) {
+    bool start = false;
+    if (REFILL == MI_REFILL_STATIC) {
+      if (!lane_in(active) && static_next < a.total) {
+        g = static_next;
+        static_next += nthreads;
+        start = true;
+      }
+    } else if (!exhausted && ~active) {
+      const uint64_t idle = ~active;
+      const uint32_t cnt = (uint32_t)__popcll(idle);
+      const uint32_t rank = lane_rank(idle);  // of an idle lane among the idle lanes
+      const uint32_t avail = res_end - res_next;
+      uint32_t c = 0;
+      // the new claim covers every idle lane that the old one cannot
+      const uint32_t want = avail < cnt ? ((cnt - avail + kChunk - 1u) / kChunk) * kChunk : 0u;
+      if (avail < cnt) {
+        if (lane == 0u) c = atomicAdd(&a.work->queue[slab].next, want);
+        c = __builtin_amdgcn_readfirstlane(c);
+      }
+      if (lane_in(idle)) {
+        const uint32_t idx =
+            slab_index(rank < avail ? res_next + rank : c + (rank - avail), slab, nslabs);
+        if (idx < a.total) {
+          g = idx;
           start = true;
         }
-      } else if (!exhausted && ~active) {
-        const uint64_t idle = ~active;
-        const uint32_t cnt = (uint32_t)__popcll(idle);
-        const uint32_t rank = lane_rank(idle);  // of an idle lane among the idle lanes
-        const uint32_t avail = res_end - res_next;
-        uint32_t c = 0;
-        // the new claim covers every idle lane that the old one cannot
-        const uint32_t want = avail < cnt ? ((cnt - avail + kChunk - 1u) / kChunk) * kChunk : 0u;
-        if (avail < cnt) {
-          if (lane == 0u) c = atomicAdd(&a.work->queue[slab].next, want);
-          c = __builtin_amdgcn_readfirstlane(c);
-        }
-        if (lane_in(idle)) {
-          const uint32_t idx =
-              slab_index(rank < avail ? res_next + rank : c + (rank - avail), slab, nslabs);
-          if (idx < a.total) {
-            g = idx;
-            start = true;
-          }
-        }
-        if (avail < cnt) {
-          res_next = c + (cnt - avail);
-          res_end = c + want;
-        } else {
-          res_next += cnt;
-        }
-        if (slab_index(res_next, slab, nslabs) >= a.total) exhausted = true;  // slab dry
       }
-      if (start) {
-        mi_pos q;
-        locate(a, g, p, j, g, q);  // from here on g is the playout's result slot
-        if (a.keys) p = a.keys[p];  // from here on p is the stream key
-        L = ck::lane_from_abs(q.p1, q.p2, q.kings, q.turn, q.counter);
-        ply = 0;
-        h = 0;
-      }
-      active |= __ballot(start);
-      if (!active) break;
-      if (lane_in(active)) {
-        const uint32_t b = (ply / kPly + 3u) >> 2;
-        uint32_t o[4];
-        ck::philox(b, j, ck::TAG_PLAYOUT, a.epoch, a.seed, p, o);
-        uint32_t *const row = words + (b & 1u) * (4u * 64u);
-#pragma unroll
-        for (uint32_t w = 0; w < 4u; w++) row[w * 64u] = o[w];
-      }
-    }
-    // The common part of the ply: every lane looks at its position (an idle lane's or a waiting
-    // one's yields what it did before), and those that can play do.  Plies with longer captures,
-    // for the heuristics also those whose moves weigh differently, wait for the walk phase, where
-    // they take the same word.
-    ck::Gen gen;
-    ck::analyse(L, gen);
-    uint64_t deferred = active & __ballot(gen.multi != 0u);
-    uint32_t from = 0xFFFFFFFFu;  // heuristic: squares of the moves of largest weight
-    if (POLICY != MI_POLICY_RANDOM) {
-      const uint32_t prom = ck::promoting(L, gen);
-      uint32_t pw, po, kw, ko;
-      ck::promote_parts(gen, prom, pw, po);
-      ck::king_parts(L, gen, kw, ko);
-      const uint64_t split = __ballot(pw != 0u) & __ballot(po != 0u) & __ballot(L.opp != 0u);
-      deferred |= active & __ballot(kw != 0u) & __ballot(ko != 0u);
-      deferred |= active & (POLICY == MI_POLICY_HEURISTIC_NOISY
-                                ? split : split & __ballot(gen.origins != 0u));
-      if (lane_in(split)) from = prom;
-    }
-    {
-      const ck::SlotWords w = POLICY == MI_POLICY_HEURISTIC ? ck::words_from(gen, from)
-                                                            : ck::slot_words(gen.slot);
-      const uint32_t n = POLICY == MI_POLICY_HEURISTIC ? ck::slot_count(gen.slot) : w.n;
-      const uint64_t can = active & ~deferred;
-      const uint64_t go = can & __ballot(w.n != 0u) & __ballot(L.counter < 50u);
-      // (a waiting ply has no fewer moves than first jumps, an idle lane's last game had these)
-      maxn = n > maxn ? n : maxn;
-      uint32_t ld = 0u, chosen = 0xFFFFu;
-      if (TRACE && lane_in(can)) ld = ck::list_digest(L, gen, n);
-      if (lane_in(go)) {
-        const uint32_t r = words[ply & ((kWordRows - 1u) * kPly)];
-        if (POLICY == MI_POLICY_HEURISTIC) {
-          chosen = ck::play_tie<TRACE>(L, gen, w, n, r, tab);
-        } else {
-          chosen = tab.mod(r, w.n);
-          // with no opponent's piece left after the move every noisy weight is +inf: the first move
-          if (POLICY == MI_POLICY_HEURISTIC_NOISY &&
-              !(gen.capture ? L.opp & (L.opp - 1u) : L.opp))
-            chosen = 0u;
-          uint32_t sq, sl8;
-          ck::select_move(w, L.turn ? w.n - 1u - chosen : chosen, sq, sl8, tab);
-          ck::play_slot(L, gen.capture, sq, sl8, tab);
-        }
-        ply += kPly;
-      }
-      if (TRACE && lane_in(can)) h = ck::hash_step(h, ck::ply_record(ld, n, chosen));
-      if (can & ~go) ended(can & ~go, L.counter < 50u ? (int32_t)(L.turn ^ 1u) : -1);
-    }
-    if (deferred) {
-      const uint32_t nd = (uint32_t)__popcll(deferred);
-      if (nd >= defer_min || deferred == active || since_walk >= 8u) {
-        since_walk = 0;
-        uint64_t todo = deferred;
-        const uint32_t r = words[ply & ((kWordRows - 1u) * kPly)];
-        ck::PlyResult res = {0u, 0u, 0u, 0};
-        uint32_t ld = 0;
-        if (POLICY == MI_POLICY_RANDOM) {
-          if (lane_in(todo)) {
-            // capture trees in closed form; the walk only for king trees past two jumps
-            bool deep = false;
-            res = ck::ply_random_captures<TRACE>(L, gen, r, &ld, deep, tab);
-            if (deep) res = ck::ply_random_given<TRACE>(L, gen, r, &ld);
-          }
-        } else {
-          uint64_t captures = deferred;
-          if (POLICY == MI_POLICY_HEURISTIC_NOISY) captures &= __ballot(gen.capture != 0u);
-          uint64_t steps = deferred & ~captures;
-          if (captures) capture_plies<POLICY, TRACE>(share, captures, L, gen, r, res, ld, tab);
-          if (POLICY == MI_POLICY_HEURISTIC_NOISY && steps) {
-            if (__popcll(steps) > kSharedSteps)
-              steps = __ballot(lane_in(steps) && lane_rank(steps) < kSharedSteps);
-            noisy_steps<TRACE>(share, steps, L, gen, r, res, ld, tab);
-          }
-          todo = captures | steps;
-        }
-        if (lane_in(todo)) {
-          if (TRACE) h = ck::hash_step(h, ck::ply_record(ld, res.n, res.chosen));
-          maxn = res.n > maxn ? res.n : maxn;
-        }
-        const uint64_t over = todo & __ballot(res.over != 0u);
-        if (over) ended(over, res.winner);
-        if (lane_in(todo)) ply += kPly;
+      if (avail < cnt) {
+        res_next = c + (cnt - avail);
+        res_end = c + want;
       } else {
-        since_walk++;
+        res_next += cnt;
+      }
+      if (slab_index(res_next, slab, nslabs) >= a.total) exhausted = true;  // slab dry
+    }
+    if (start) {
+      mi_pos q;
+      locate(a, g, p, j, g, q);  // from here on g is the playout's result slot
+      if (a.keys) p = a.keys[p];  // from here on p is the stream key
+      L = ck::lane_from_abs(q.p1, q.p2, q.kings, q.turn, q.counter);
+      ply = 0;
+      h = 0;
+    }
+    active |= __ballot(start);
+    const bool dry = REFILL == MI_REFILL_STATIC ? !__ballot(static_next < a.total) : exhausted;
+    uint32_t leaves = 0u;  // this wave's games, if any, go to another one
+    if (blockDim.x > 256u && dry && (uint32_t)__popcll(active) <= 32u) {
+      const uint32_t me = 1u << wave;
+      uint32_t games = 0u;
+      if (asks) games = lds_value(handover.given[wave]);
+      if (asks && !games && !active && !(lds_take(handover.asking, me) & me)) {
+        // a giver took the bit: it writes its games now
+        while (!(games = lds_value(handover.given[wave]))) __builtin_amdgcn_s_sleep(1);
+      }
+      if (games) {
+        asks = 0u;
+        if (lane == 0u) handover.given[wave] = 0u;
+        const uint32_t *from = wave_words + ((games & 255u) - 1u) * (kWordRows * 64u);
+        const uint32_t rank = lane_rank(~active);
+        const bool take = !lane_in(active) && rank < games >> 8;
+        if (take) {
+          receive(from, rank);
+          generate(ply / kPly >> 2);
+        }
+        active |= __ballot(take);
+      } else if (active) {
+        // another wave that asks, on a SIMD that is no busier than this one's
+        const uint32_t alive = lds_value(handover.alive);
+        auto load = [alive](uint32_t w) { return __builtin_popcount(alive >> (w & 3u) & 0x1111u); };
+        uint32_t others = load(wave) < 2u ? 0u : lds_value(handover.asking) & ~me, to = 0u;
+        for (; others; others &= others - 1u) {
+          to = (uint32_t)__builtin_ctz(others);
+          if (load(to) <= load(wave)) break;
+        }
+        if (others && (!asks || (lds_take(handover.asking, me) & me))) {
+          asks = 0u;
+          if (lds_take(handover.asking, 1u << to) >> to & 1u) {
+            if (lane_in(active)) give(words - lane, lane_rank(active));
+            if (lane == 0u)
+              __hip_atomic_store(&handover.given[to], (uint32_t)__popcll(active) << 8 | (wave + 1u),
+                                 __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+            leaves = 1u;
+          }
+        } else if (!others && !asks) {
+          asks = 1u;
+          lds_set(handover.asking, me);
+        }
+      }
+      if (leaves || !active) lds_take(handover.alive, me);
+    }
+    // (uniform, but not to the compiler: the branches above hold divergent ones)
+    active = uniform64(active);
+    asks = __builtin_amdgcn_readfirstlane(asks);
+    if (__builtin_amdgcn_readfirstlane(leaves) || !active) break;
+    if (lane_in(active)) generate((ply / kPly + 3u) >> 2);
+#pragma unroll 1
+    for (uint32_t step = 0; step < 4u; step++) {
+      // The common part of the ply: every lane looks at its position (an idle lane's or a waiting
+      // one's yields what it did before), and those that can play do.  Plies with longer captures,
+      // for the heuristics also those whose moves weigh differently, wait for the walk phase, where
+      // they take the same word.
+      ck::Gen gen;
+      ck::analyse(L, gen);
+      uint64_t deferred = active & __ballot(gen.multi != 0u);
+      uint32_t from = 0xFFFFFFFFu;  // heuristic: squares of the moves of largest weight
+      if (POLICY != MI_POLICY_RANDOM) {
+        const uint32_t prom = ck::promoting(L, gen);
+        uint32_t pw, po, kw, ko;
+        ck::promote_parts(gen, prom, pw, po);
+        ck::king_parts(L, gen, kw, ko);
+        const uint64_t split = __ballot(pw != 0u) & __ballot(po != 0u) & __ballot(L.opp != 0u);
+        deferred |= active & __ballot(kw != 0u) & __ballot(ko != 0u);
+        deferred |= active & (POLICY == MI_POLICY_HEURISTIC_NOISY
+                                  ? split : split & __ballot(gen.origins != 0u));
+        if (lane_in(split)) from = prom;
+      }
+      {
+        const ck::SlotWords w = POLICY == MI_POLICY_HEURISTIC ? ck::words_from(gen, from)
+                                                              : ck::slot_words(gen.slot);
+        const uint32_t n = POLICY == MI_POLICY_HEURISTIC ? ck::slot_count(gen.slot) : w.n;
+        const uint64_t can = active & ~deferred;
+        const uint64_t go = can & __ballot(w.n != 0u) & __ballot(L.counter < 50u);
+        // (a waiting ply has no fewer moves than first jumps, an idle lane's last game had these)
+        maxn = n > maxn ? n : maxn;
+        uint32_t ld = 0u, chosen = 0xFFFFu;
+        if (TRACE && lane_in(can)) ld = ck::list_digest(L, gen, n);
+        if (lane_in(go)) {
+          const uint32_t r = words[ply & ((kWordRows - 1u) * kPly)];
+          if (POLICY == MI_POLICY_HEURISTIC) {
+            chosen = ck::play_tie<TRACE>(L, gen, w, n, r, tab);
+          } else {
+            chosen = tab.mod(r, w.n);
+            // with no opponent's piece left after the move every noisy weight is +inf: move 0
+            if (POLICY == MI_POLICY_HEURISTIC_NOISY &&
+                !(gen.capture ? L.opp & (L.opp - 1u) : L.opp))
+              chosen = 0u;
+            uint32_t sq, sl8;
+            ck::select_move(w, L.turn ? w.n - 1u - chosen : chosen, sq, sl8, tab);
+            ck::play_slot(L, gen.capture, sq, sl8, tab);
+          }
+          ply += kPly;
+        }
+        if (TRACE && lane_in(can)) h = ck::hash_step(h, ck::ply_record(ld, n, chosen));
+        if (can & ~go) ended(can & ~go, L.counter < 50u ? (int32_t)(L.turn ^ 1u) : -1);
+      }
+      if (deferred) {
+        const uint32_t nd = (uint32_t)__popcll(deferred);
+        if (nd >= defer_min || deferred == active || since_walk >= 8u) {
+          since_walk = 0;
+          uint64_t todo = deferred;
+          const uint32_t r = words[ply & ((kWordRows - 1u) * kPly)];
+          ck::PlyResult res = {0u, 0u, 0u, 0};
+          uint32_t ld = 0;
+          if (POLICY == MI_POLICY_RANDOM) {
+            if (lane_in(todo)) {
+              // capture trees in closed form; the walk only for king trees past two jumps
+              bool deep = false;
+              res = ck::ply_random_captures<TRACE>(L, gen, r, &ld, deep, tab);
+              if (deep) res = ck::ply_random_given<TRACE>(L, gen, r, &ld);
+            }
+          } else {
+            uint64_t captures = deferred;
+            if (POLICY == MI_POLICY_HEURISTIC_NOISY) captures &= __ballot(gen.capture != 0u);
+            uint64_t steps = deferred & ~captures;
+            if (captures) capture_plies<POLICY, TRACE>(share, captures, L, gen, r, res, ld, tab);
+            if (POLICY == MI_POLICY_HEURISTIC_NOISY && steps) {
+              if (__popcll(steps) > kSharedSteps)
+                steps = __ballot(lane_in(steps) && lane_rank(steps) < kSharedSteps);
+              noisy_steps<TRACE>(share, steps, L, gen, r, res, ld, tab);
+            }
+            todo = captures | steps;
+          }
+          if (lane_in(todo)) {
+            if (TRACE) h = ck::hash_step(h, ck::ply_record(ld, res.n, res.chosen));
+            maxn = res.n > maxn ? res.n : maxn;
+          }
+          const uint64_t over = todo & __ballot(res.over != 0u);
+          if (over) ended(over, res.winner);
+          if (lane_in(todo)) ply += kPly;
+        } else {
+          since_walk++;
+        }
       }
     }
   }
@@ -711,159 +835,160 @@ __global__ void __launch_bounds__(64) k_start_positions(StartArgs a) {
   const uint32_t nslabs = a.n < 32u * kSlabBlock * kSlabs ? 1u : min(gridDim.x, kSlabs);
   const uint32_t slab = blockIdx.x % nslabs;
   bool exhausted = false;
-  for (uint32_t iter = 0;; iter++) {
-    if ((iter & 3u) == 0u) {
-      __syncthreads();  // (one wave: orders the LDS accesses)
+  for (;;) {
+    __syncthreads();  // (one wave: orders the LDS accesses)
+    if (lane_in(open)) {
+      const uint32_t turn = lo & 63u;
+      const uint64_t f = rotate_right(marks[lane], turn);
+      const uint32_t ended = f == ~0ull ? 64u : (uint32_t)__builtin_ctzll(~f);
+      if (ended < 64u && (rotate_right(marks[64u + lane], turn) >> ended & 1u)) {
+        decided[lane] = lo + ended;
+      } else if (ended) {
+        const uint64_t gone = ended == 64u ? ~0ull : (1ull << ended) - 1ull;
+        marks[lane] &= ~rotate_right(gone, (64u - turn) & 63u);
+        lo += ended;
+      }
+    }
+    __syncthreads();
+    {  // a decided position: its attempt's lane writes it, the lanes of later attempts are free
+      const uint32_t by = lane_in(active | held) ? decided[slot] : kOpen;
+      if (by != kOpen && by == attempt) a.out[i] = packed_position(L);
+      const uint64_t gone = __ballot(by != kOpen);
+      active &= ~gone;
+      held &= ~gone;
+    }
+    {  // close decided slots (a position all of whose attempts ended is reported)
+      const bool lost = lane_in(open) && lo == kStartAttempts;
+      if (lost) atomicOr(&a.work->overflow, 1u);
+      const bool close = lane_in(open) && (lost || decided[lane] != kOpen);
+      if (close) {
+        decided[lane] = kOpen;
+        marks[lane] = marks[64u + lane] = 0ull;
+      }
+      open &= ~__ballot(close);
+    }
+    // Idle lanes go to the open positions without an attempt, then to new positions, then to
+    // further attempts of the open ones: list[] names the slots in that order.
+    const uint64_t idle = ~(active | held);
+    const uint32_t cnt = (uint32_t)__popcll(idle);
+    const uint64_t bare = __ballot(lane_in(open) && lo == hi);
+    uint32_t named = (uint32_t)__popcll(bare);
+    if (lane_in(bare)) {
+      list[lane_rank(bare)] = lane;
+      next[lane] = hi++;
+    }
+    const uint32_t room = a.slots - min(a.slots, (uint32_t)__popcll(open));
+    const uint32_t want = min(cnt - named, room);
+    if (!exhausted && want) {
+      uint32_t c = 0;
+      if (lane == 0u) c = atomicAdd(&a.work->queue[slab].next, want);
+      c = __builtin_amdgcn_readfirstlane(c);
+      const uint32_t rank = lane_rank(~open);
+      const uint32_t at = slab_index(c + rank, slab, nslabs);
+      const bool taken = !lane_in(open) && rank < want && at < a.n;
+      if (taken) {
+        list[named + rank] = lane;
+        index[lane] = at;
+        next[lane] = lo = 0u;
+        hi = 1u;
+      }
+      const uint64_t fresh = __ballot(taken);
+      open |= fresh;
+      named += (uint32_t)__popcll(fresh);
+      exhausted = slab_index(c + want, slab, nslabs) >= a.n;
+    }
+    if (!open) {
+      if (exhausted) break;
+      continue;
+    }
+    const uint32_t spare = cnt - named, nopen = (uint32_t)__popcll(open);
+    const uint32_t ahead = hi;  // the first attempt that a spare lane may take here
+    __syncthreads();
+    const uint32_t rank = lane_rank(idle);
+    bool start = false;
+    if (lane_in(idle) && rank < named) {
+      slot = list[rank];
+      attempt = next[slot];
+      start = true;
+    }
+    if (spare && a.reject) {
+      __syncthreads();
+      const float per = 1.0f / (float)nopen;
       if (lane_in(open)) {
-        const uint32_t turn = lo & 63u;
-        const uint64_t f = rotate_right(marks[lane], turn);
-        const uint32_t ended = f == ~0ull ? 64u : (uint32_t)__builtin_ctzll(~f);
-        if (ended < 64u && (rotate_right(marks[64u + lane], turn) >> ended & 1u)) {
-          decided[lane] = lo + ended;
-        } else if (ended) {
-          const uint64_t gone = ended == 64u ? ~0ull : (1ull << ended) - 1ull;
-          marks[lane] &= ~rotate_right(gone, (64u - turn) & 63u);
-          lo += ended;
-        }
+        const uint32_t r = lane_rank(open);
+        list[r] = lane;
+        next[lane] = ahead;
+        // spare lanes x = r, r + nopen, ... take attempts ahead, ahead + 1, ...
+        const uint32_t share = r < spare ? (uint32_t)(((float)(spare - 1u - r) + 0.5f) * per) + 1u : 0u;
+        const uint32_t top = min(lo + 64u, kStartAttempts);
+        hi = max(ahead, min(ahead + share, top));
+        limits[lane] = hi;
       }
       __syncthreads();
-      {  // a decided position: its attempt's lane writes it, the lanes of later attempts are free
-        const uint32_t by = lane_in(active | held) ? decided[slot] : kOpen;
-        if (by != kOpen && by == attempt) a.out[i] = packed_position(L);
-        const uint64_t gone = __ballot(by != kOpen);
-        active &= ~gone;
-        held &= ~gone;
+      if (lane_in(idle) && rank >= named) {
+        const uint32_t x = rank - named;
+        const uint32_t q = (uint32_t)(((float)x + 0.5f) * per);
+        slot = list[x - q * nopen];
+        attempt = next[slot] + q;
+        start = attempt < limits[slot];
       }
-      {  // close decided slots (a position all of whose attempts ended is reported)
-        const bool lost = lane_in(open) && lo == kStartAttempts;
-        if (lost) atomicOr(&a.work->overflow, 1u);
-        const bool close = lane_in(open) && (lost || decided[lane] != kOpen);
-        if (close) {
-          decided[lane] = kOpen;
-          marks[lane] = marks[64u + lane] = 0ull;
-        }
-        open &= ~__ballot(close);
-      }
-      // Idle lanes go to the open positions without an attempt, then to new positions, then to
-      // further attempts of the open ones: list[] names the slots in that order.
-      const uint64_t idle = ~(active | held);
-      const uint32_t cnt = (uint32_t)__popcll(idle);
-      const uint64_t bare = __ballot(lane_in(open) && lo == hi);
-      uint32_t named = (uint32_t)__popcll(bare);
-      if (lane_in(bare)) {
-        list[lane_rank(bare)] = lane;
-        next[lane] = hi++;
-      }
-      const uint32_t room = a.slots - min(a.slots, (uint32_t)__popcll(open));
-      const uint32_t want = min(cnt - named, room);
-      if (!exhausted && want) {
-        uint32_t c = 0;
-        if (lane == 0u) c = atomicAdd(&a.work->queue[slab].next, want);
-        c = __builtin_amdgcn_readfirstlane(c);
-        const uint32_t rank = lane_rank(~open);
-        const uint32_t at = slab_index(c + rank, slab, nslabs);
-        const bool taken = !lane_in(open) && rank < want && at < a.n;
-        if (taken) {
-          list[named + rank] = lane;
-          index[lane] = at;
-          next[lane] = lo = 0u;
-          hi = 1u;
-        }
-        const uint64_t fresh = __ballot(taken);
-        open |= fresh;
-        named += (uint32_t)__popcll(fresh);
-        exhausted = slab_index(c + want, slab, nslabs) >= a.n;
-      }
-      if (!open) {
-        if (exhausted) break;
-        continue;
-      }
-      const uint32_t spare = cnt - named, nopen = (uint32_t)__popcll(open);
-      const uint32_t ahead = hi;  // the first attempt that a spare lane may take here
-      __syncthreads();
-      const uint32_t rank = lane_rank(idle);
-      bool start = false;
-      if (lane_in(idle) && rank < named) {
-        slot = list[rank];
-        attempt = next[slot];
-        start = true;
-      }
-      if (spare && a.reject) {
-        __syncthreads();
-        const float per = 1.0f / (float)nopen;
-        if (lane_in(open)) {
-          const uint32_t r = lane_rank(open);
-          list[r] = lane;
-          next[lane] = ahead;
-          // spare lanes x = r, r + nopen, ... take attempts ahead, ahead + 1, ...
-          const uint32_t share = r < spare ? (uint32_t)(((float)(spare - 1u - r) + 0.5f) * per) + 1u : 0u;
-          const uint32_t top = min(lo + 64u, kStartAttempts);
-          hi = max(ahead, min(ahead + share, top));
-          limits[lane] = hi;
-        }
-        __syncthreads();
-        if (lane_in(idle) && rank >= named) {
-          const uint32_t x = rank - named;
-          const uint32_t q = (uint32_t)(((float)x + 0.5f) * per);
-          slot = list[x - q * nopen];
-          attempt = next[slot] + q;
-          start = attempt < limits[slot];
-        }
-      }
-      if (start) {
-        i = index[slot];
-        L = ck::start_position();
-        limit = ck::start_plies(a.seed, a.base + i, attempt, a.kmin, a.span) * kPly;
-        ply = 0;
-      }
-      active |= __ballot(start);
-      if (lane_in(active)) {
-        const uint32_t b = (ply / kPly + 3u) >> 2;
-        uint32_t o[4];
-        ck::philox(b, attempt, ck::TAG_START, 0u, a.seed, a.base + i, o);
-        uint32_t *const row = words + (b & 1u) * (4u * 64u);
+    }
+    if (start) {
+      i = index[slot];
+      L = ck::start_position();
+      limit = ck::start_plies(a.seed, a.base + i, attempt, a.kmin, a.span) * kPly;
+      ply = 0;
+    }
+    active |= __ballot(start);
+    if (lane_in(active)) {
+      const uint32_t b = (ply / kPly + 3u) >> 2;
+      uint32_t o[4];
+      ck::philox(b, attempt, ck::TAG_START, 0u, a.seed, a.base + i, o);
+      uint32_t *const row = words + (b & 1u) * (4u * 64u);
 #pragma unroll
-        for (uint32_t w = 0; w < 4u; w++) row[w * 64u] = o[w];
+      for (uint32_t w = 0; w < 4u; w++) row[w * 64u] = o[w];
+    }
+#pragma unroll 1
+    for (uint32_t step = 0; step < 4u; step++) {
+      // The common part of the ply, as in k_playouts; a position at its limit is left as it is.
+      ck::Gen gen;
+      ck::analyse(L, gen);
+      const ck::SlotWords w = ck::slot_words(gen.slot);
+      const uint64_t stop = __ballot(ply == limit);
+      // (an origin of longer captures has its slot's bit too)
+      const uint64_t over = ~(__ballot(w.n != 0u) & __ballot(L.counter < 50u));
+      const uint64_t done = active & (stop | over);
+      const uint64_t deferred = active & ~done & __ballot(gen.multi != 0u);
+      const uint64_t go = active & ~done & ~deferred;
+      const uint32_t r = words[ply & ((kWordRows - 1u) * kPly)];
+      if (lane_in(go)) {
+        const uint32_t k = tab.mod(r, w.n);
+        uint32_t sq, sl8;
+        ck::select_move(w, L.turn ? w.n - 1u - k : k, sq, sl8, tab);
+        ck::play_slot(L, gen.capture, sq, sl8, tab);
+        ply += kPly;
       }
-    }
-    // The common part of the ply, as in k_playouts; a position at its limit is left as it is.
-    ck::Gen gen;
-    ck::analyse(L, gen);
-    const ck::SlotWords w = ck::slot_words(gen.slot);
-    const uint64_t stop = __ballot(ply == limit);
-    // (an origin of longer captures has its slot's bit too)
-    const uint64_t over = ~(__ballot(w.n != 0u) & __ballot(L.counter < 50u));
-    const uint64_t done = active & (stop | over);
-    const uint64_t deferred = active & ~done & __ballot(gen.multi != 0u);
-    const uint64_t go = active & ~done & ~deferred;
-    const uint32_t r = words[ply & ((kWordRows - 1u) * kPly)];
-    if (lane_in(go)) {
-      const uint32_t k = tab.mod(r, w.n);
-      uint32_t sq, sl8;
-      ck::select_move(w, L.turn ? w.n - 1u - k : k, sq, sl8, tab);
-      ck::play_slot(L, gen.capture, sq, sl8, tab);
-      ply += kPly;
-    }
-    if (done) {
-      const uint64_t accepted = a.reject ? done & ~over : done;
-      if (lane_in(done))
-        atomicOr(&marks[lane_in(accepted) ? 64u + slot : slot], 1ull << (attempt & 63u));
-      active &= ~done;
-      held |= accepted;
-    }
-    if (deferred) {
-      const uint32_t nd = (uint32_t)__popcll(deferred);
-      if (nd >= 16u || deferred == active || since_walk >= 8u) {
-        since_walk = 0;
-        if (lane_in(deferred)) {
-          uint32_t unused = 0;
-          bool deep = false;  // (the game is not over: captures, and the draw count below 50)
-          ck::ply_random_captures<false>(L, gen, r, &unused, deep, tab);
-          if (deep) ck::ply_random_given<false>(L, gen, r, &unused);
-          ply += kPly;
+      if (done) {
+        const uint64_t accepted = a.reject ? done & ~over : done;
+        if (lane_in(done))
+          atomicOr(&marks[lane_in(accepted) ? 64u + slot : slot], 1ull << (attempt & 63u));
+        active &= ~done;
+        held |= accepted;
+      }
+      if (deferred) {
+        const uint32_t nd = (uint32_t)__popcll(deferred);
+        if (nd >= 16u || deferred == active || since_walk >= 8u) {
+          since_walk = 0;
+          if (lane_in(deferred)) {
+            uint32_t unused = 0;
+            bool deep = false;  // (the game is not over: captures, and the draw count below 50)
+            ck::ply_random_captures<false>(L, gen, r, &unused, deep, tab);
+            if (deep) ck::ply_random_given<false>(L, gen, r, &unused);
+            ply += kPly;
+          }
+        } else {
+          since_walk++;
         }
-      } else {
-        since_walk++;
       }
     }
   }

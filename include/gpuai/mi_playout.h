@@ -105,9 +105,10 @@ typedef struct mi_tune_result {
 typedef struct mi_ctx mi_ctx;
 
 /* Creates a context on HIP device `device`.  `tuning` may be NULL (or have zero fields) for the
- * default launch shape: 64-thread blocks, 12 per CU, queue refill, defer_min 16.  No
- * counterpart in the reference, whose drivers allocate on every call
- * (src/singlePlayout.cu:76-84). */
+ * defaults: queue refill, defer_min 16, and the shape each batch takes by its size (up to four
+ * waves a CU 64-thread blocks, beyond that one workgroup per CU of up to 16 waves; mi_get_tuning
+ * reports 64-thread blocks, 12 per CU).  No counterpart in the reference, whose drivers allocate
+ * on every call (src/singlePlayout.cu:76-84). */
 int mi_create(mi_ctx **ctx, int device, const mi_tuning *tuning);
 int mi_destroy(mi_ctx *ctx);
 const char *mi_strerror(int code);
@@ -185,7 +186,7 @@ int mi_gen_start_positions(mi_ctx *ctx, uint32_t seed, uint32_t n, uint32_t kmin
  * and graph replays then launch each batch with its bucket's shape (graph replays: the fastest of
  * the graph's refill policy), and batches whose bucket has no entry with the context's tuning.
  * mi_set_tuning empties the table.  Until a context is given a shape (mi_create, mi_set_tuning,
- * mi_autotune), batches of up to 32 playouts per compute unit (64 for the noisy heuristic) whose
+ * mi_autotune), batches of up to 16 playouts per compute unit (32 for the noisy heuristic) whose
  * bucket has no entry run with one wave per game instead of one lane per game (stats: 64-thread
  * blocks, one per playout, MI_REFILL_STATIC; the same winners).  The allocation-free entry point
  * uses the context's tuning, or one wave per game where it knows the batch's size (counts ==
