@@ -82,16 +82,16 @@ mi_tuning batch_shape(const mi_ctx *ctx, uint64_t total) {
 }
 
 // Whether a batch of `total` playouts runs with one wave per game (k_playouts_wave).  A small batch
-// lasts as long as its longest game: 0.41-0.65 us per ply with a wave of its own (random, noisy)
+// lasts as long as its longest game: 0.33-0.47 us per ply with a wave of its own (random, noisy)
 // against 0.9-1.5 us in a wave of 64 games, but a game costs a whole wave's instructions, so from
 // some size on the lanes win.  Kernel ms, one wave per game / one lane per game, 256 CUs:
 //   playouts       256          4,096        8,192        12,288       16,384
-//   random     .074 / .129  .106 / .121  .142 / .128  .160 / .133  .195 / .135
-//   heuristic  .082 / .149  .125 / .139  .163 / .142  .191 / .149  .224 / .151
-//   noisy      .089 / .208  .133 / .185  .168 / .186  .202 / .185  .233 / .185
+//   random     .053 / .130  .081 / .121  .113 / .128  .139 / .133  .160 / .135
+//   heuristic  .054 / .150  .096 / .140  .134 / .142  .171 / .151  .200 / .151
+//   noisy      .066 / .213  .113 / .188  .150 / .185  .184 / .186  .225 / .187
 // A context that was given a launch shape, or has measured one for the batch's size, uses it.
 bool wave_batch(const mi_ctx *ctx, uint32_t policy, uint64_t total) {
-  if (ctx->shaped || total > (uint64_t)ctx->cus * (policy == MI_POLICY_HEURISTIC_NOISY ? 32u : 16u))
+  if (ctx->shaped || total > (uint64_t)ctx->cus * (policy == MI_POLICY_HEURISTIC_NOISY ? 48u : 32u))
     return false;
   const TuneEntry *e = ctx->tune_table[policy][tune_bucket(total)];
   return e[0].kernel_ms < 0.f && e[1].kernel_ms < 0.f;

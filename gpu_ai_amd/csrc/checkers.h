@@ -1525,9 +1525,10 @@ CK_HD void normal_pair(uint32_t a, uint32_t b, float &z0, float &z1) {
       1.0f + x2 * (-0.5f + x2 * (4.16666667e-2f + x2 * (-1.38888889e-3f +
                                                         x2 * (2.48015873e-5f +
                                                               x2 * -2.75573192e-7f))));
-  const uint32_t q = b >> 30;
-  const float c = q == 0u ? cs : q == 1u ? -sn : q == 2u ? -cs : sn;
-  const float t = q == 0u ? sn : q == 1u ? cs : q == 2u ? -sn : -cs;
+  // by quadrant: (cs, sn), (-sn, cs), (-cs, -sn), (sn, -cs)
+  const uint32_t q = b >> 30, odd = 0u - (q & 1u), bc = f32_bits(cs), bs = f32_bits(sn);
+  const float c = f32_from_bits(((bc & ~odd) | (bs & odd)) ^ ((q ^ (q >> 1)) << 31));
+  const float t = f32_from_bits(((bs & ~odd) | (bc & odd)) ^ ((q >> 1) << 31));
   z0 = rad * c;
   z1 = rad * t;
 }

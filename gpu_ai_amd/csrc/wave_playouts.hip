@@ -7,9 +7,14 @@
 // lanes: lane (s, h) looks at square s in directions 2h and 2h + 1, comparisons collect each
 // direction's squares as wave masks, and ranks of moves are counts of mask bits below a lane.  A
 // ply takes about a hundred instructions, so the longest game ends several times sooner; per
-// game they are spent by a whole wave, so large batches stay with k_playouts (wave_batch_limit).
-// Plies with capture sequences longer than one jump (3%) run the lane logic of checkers.h on the
-// uniform position.
+// game they are spent by a whole wave, so large batches stay with k_playouts (ctxutil::wave_batch).
+// Plies with capture sequences longer than one jump (3%) go through the capture trees of checkers.h
+// (random: on the uniform position; the heuristics: a move to a lane).
+//
+// The position stays in scalar registers only where no branch on a lane's own value joins the loop
+// that carries it, and the loop that plays has one exit: with a select chain over the Philox words
+// (a branch to the compiler) and three exits a ply took 465 ns in a wave alone on its SIMD, with
+// neither 336, and 256 playouts 56 us instead of 77.
 #include <hip/hip_runtime.h>
 
 #include "checkers.h"
@@ -47,11 +52,85 @@ __device__ __forceinline__ ck::Gen analysis(uint64_t jA, uint64_t jB, uint64_t m
   return g;
 }
 
-// Largest float over the wave.
-__device__ __forceinline__ float wave_max(float x) {
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) x = fmaxf(x, __shfl_xor(x, off));
-  return x;
+// A float's place in the order of floats, as an integer.
+__device__ __forceinline__ int32_t ordered(float x) {
+  const int32_t b = (int32_t)ck::f32_bits(x);
+  return b ^ (b >> 31 & 0x7FFFFFFF);
+}
+
+// Largest value over the wave: rotations within the rows of 16 lanes, then a lane of each row.
+template <int ROTATE>
+__device__ __forceinline__ int32_t row_max(int32_t x) {
+  return max(x, __builtin_amdgcn_update_dpp(x, x, 0x120 + ROTATE, 0xF, 0xF, false));
+}
+__device__ __forceinline__ int32_t wave_max(int32_t x) {
+  x = row_max<1>(row_max<2>(row_max<4>(row_max<8>(x))));
+  const int32_t a = (int32_t)lane_value((uint32_t)x, 0u), b = (int32_t)lane_value((uint32_t)x, 16u);
+  const int32_t c = (int32_t)lane_value((uint32_t)x, 32u), d = (int32_t)lane_value((uint32_t)x, 48u);
+  return max(max(a, b), max(c, d));
+}
+
+// A capture ply of the heuristics, a move to a lane: it decodes its move from the ply's capture
+// trees and weighs it (noisy: draws for it).  Leaves the position as it is and returns false where a
+// king has three jumps or more, or there are more than 64 moves.  Against the walk, which goes through
+// them one after the other: 421 -> 389 ns a ply over all of 256 heuristic games.
+template <uint32_t POLICY>
+__device__ __forceinline__ bool capture_ply(ck::Lane &L, const ck::Gen &g, uint32_t r, uint32_t lane,
+                                            ck::PlyResult &res) {
+  ck::CaptureTrees t;
+  ck::capture_trees(L, g, t);
+  if (t.deep || t.n > 64u) return false;
+  res = {t.n, 0u, 0u, 0};
+  if (L.counter >= 50u) {
+    res.over = 1u;
+    res.winner = -1;
+    return true;
+  }
+  const uint32_t sm = ck::material(L.own, L.kings), so = ck::material(L.opp, L.kings);
+  const bool on = lane < t.n;
+  ck::Choice c = {0u, 0u, 0u};
+  float w = 0.0f;
+  int32_t v = (int32_t)0x80000000;
+  if (on) {
+    c = ck::capture_choice(t, lane, ck::Direct());
+    const bool promotes = !ck::getbit(L.kings, c.from) && c.to >= ck::FAR_ROW_FIRST;
+    // (as whole numbers these quotients are equal or differ by more than their rounding)
+    w = (float)(sm + (promotes ? 3u : 0u)) / (float)(so - ck::material(c.removed, L.kings));
+    v = ordered(w);
+    if (POLICY == MI_POLICY_HEURISTIC_NOISY) {
+#pragma clang fp contract(off)
+      float e0, e1;
+      ck::noise_pair(r, lane >> 1, e0, e1);
+      v = ordered(w + ((lane & 1u) ? e1 : e0));
+    }
+  }
+  // lanes whose moves the word chooses among; none: the best draw, the first in reference order
+  const int32_t best = wave_max(v);
+  uint64_t among = __ballot(on && v == best);
+  uint32_t pick = 0u;
+  bool word = true;
+  if (POLICY == MI_POLICY_HEURISTIC_NOISY) {
+    const float w0 = ck::f32_from_bits(lane_value(ck::f32_bits(w), 0u));
+    const uint64_t all = __ballot(on);
+    word = __ballot(on && w == w0) == all;
+    if (word) among = all;
+    else pick = L.turn ? 63u - (uint32_t)__builtin_clzll(among) : (uint32_t)__builtin_ctzll(among);
+    if (word && w0 == __builtin_inff()) {  // every weight is +inf: the first move
+      pick = L.turn ? t.n - 1u : 0u;
+      word = false;
+    }
+  }
+  if (word) {
+    const uint32_t ties = (uint32_t)__popcll(among);
+    const uint32_t i = ck::mod_small(r, ties);
+    const uint32_t km = L.turn ? ties - 1u - i : i;
+    const uint32_t rank = __builtin_amdgcn_mbcnt_hi(hi32(among),
+                                                    __builtin_amdgcn_mbcnt_lo(lo32(among), 0u));
+    // the last lane with at most km of them below it that is one of them
+    pick = 63u - (uint32_t)__builtin_clzll(__ballot(rank <= km) & among);
+  }
+  ck::apply(L, lane_value(c.from, pick), lane_value(c.to, pick), lane_value(c.removed, pick));
+  return true;
 }
 
 // Index of the last of n >= 1 ascending values that is <= g (values[0] <= g), by the whole wave:
@@ -100,6 +179,18 @@ __device__ __forceinline__ Geometry geometry(uint32_t lane) {
   return q;
 }
 
+// Slot of the j-th set bit of a nibble, at bit 8 * (nibble & 7) + 2 j: nibbles below 8, and the rest.
+constexpr uint64_t nth_table(uint32_t from) {
+  uint64_t t = 0;
+  for (uint32_t n = 0; n < 8u; n++) {
+    uint32_t j = 0;
+    for (uint32_t s = 0; s < 4u; s++)
+      if ((n + from) >> s & 1u) t |= (uint64_t)s << (8u * n + 2u * j++);
+  }
+  return t;
+}
+constexpr uint64_t kNthLow = nth_table(0u), kNthHigh = nth_table(8u);
+
 // A stream of Philox words: that of ply t is word t & 3 of counter (t >> 2, c1, c2, c3).
 struct Stream {
   uint32_t c1, c2, c3, seed, key;
@@ -120,19 +211,24 @@ __device__ __forceinline__ void play(ck::Lane &L, const Geometry &geo, const Str
     if ((ply & 63u) == 0u) {
       uint32_t o[4];
       ck::philox((ply >> 2) + (lane >> 2), st.c1, st.c2, st.c3, st.seed, st.key, o);
-      const uint32_t w = lane & 3u;
-      words = w == 0u ? o[0] : w == 1u ? o[1] : w == 2u ? o[2] : o[3];
+      // (by masks: a chain of selects becomes a branch on the lane, and what the loop carries past
+      // it is no longer known to be uniform)
+      const uint32_t odd = 0u - (lane & 1u), high = 0u - (lane >> 1 & 1u);
+      words = (((o[0] & ~odd) | (o[1] & odd)) & ~high) | (((o[2] & ~odd) | (o[3] & odd)) & high);
     }
   };
   refresh();
   // The inner loop plays plies until the game is over or one has longer capture sequences, which
   // the outer loop plays (a loop of its own keeps the common plies' registers in place: 20% of the
-  // instructions were copies without it).
+  // instructions were copies without it; it has one exit, since each further one costs every ply
+  // the flags that tell them apart).
   for (;;) {
     uint64_t jA, jB, m0, m1, longer;
     uint32_t r;
+    bool walk;  // the ply is the walk's
     for (;;) {
       longer = 0;
+      walk = false;
       r = lane_value(words, ply & 63u);
       // squares with a valid jump in A and B, whatever stands on them
       const uint32_t empty = ~(L.own | L.opp);
@@ -162,18 +258,17 @@ __device__ __forceinline__ void play(ck::Lane &L, const Geometry &geo, const Str
             const uint64_t k0 = (kA & kings) | (kB & men), k1 = (kB & kings) | (kA & men);
             mixed |= ((m0 & k0) | (m1 & k1)) && ((m0 & ~k0) | (m1 & ~k1));
           }
-          if (longer || mixed) break;
-        } else if (longer) {
-          break;
+          walk = mixed;
         }
+        walk |= longer != 0;
       } else {
         cap = 0u;
         m0 = __ballot((empty & stepA) != 0u) & movers;
         m1 = __ballot((empty & stepB) != 0u) & movers;
       }
       const uint32_t n = (uint32_t)__popcll(m0) + (uint32_t)__popcll(m1);
-      maxn = n > maxn ? n : maxn;
-      if (n == 0u || L.counter >= 50u) return;  // the game is over
+      maxn = n > maxn ? n : maxn;  // (a ply of the walk's has no fewer moves than first jumps)
+      if (walk || n == 0u || L.counter >= 50u) break;
       uint32_t sq = 0, sl = 0, pick = 1u;  // pick: the word chooses among the moves in m0 and m1
       uint32_t ties = n, first = 0u;       // first: every weight is +inf, index 0 wins
       uint64_t prom = 0;  // promoting steps' men, where only some of the steps promote
@@ -211,9 +306,10 @@ __device__ __forceinline__ void play(ck::Lane &L, const Geometry &geo, const Str
             v0 = w + v0;
             v1 = w + v1;
           }
-          const float ninf = -__builtin_inff();
-          const float best = wave_max(fmaxf(on0 ? v0 : ninf, on1 ? v1 : ninf));
-          const uint64_t b0 = __ballot(on0 && v0 == best), b1 = __ballot(on1 && v1 == best);
+          const int32_t i0 = on0 ? ordered(v0) : (int32_t)0x80000000;
+          const int32_t i1 = on1 ? ordered(v1) : (int32_t)0x80000000;
+          const int32_t best = wave_max(max(i0, i1));
+          const uint64_t b0 = __ballot(i0 == best), b1 = __ballot(i1 == best);
           // the first in reference order: player 2's is the reverse of the order here
           const uint32_t hit = lo32(b0) | lo32(b1) | hi32(b0) | hi32(b1);
           sq = L.turn ? 31u - (uint32_t)__builtin_clz(hit) : ck::ctz(hit);
@@ -239,9 +335,11 @@ __device__ __forceinline__ void play(ck::Lane &L, const Geometry &geo, const Str
         king = 0u - ck::getbit(L.kings, sq);
         const uint32_t n0 = ck::getbit(lo32(m0), sq);
         if (king) {
-          const uint32_t nibble = n0 | ck::getbit(lo32(m1), sq) << 1 |
-                                  ck::getbit(hi32(m0), sq) << 2 | ck::getbit(hi32(m1), sq) << 3;
-          sl = ck::nth_slot(nibble, left);
+          // slots 0 and 2 are bits 0 and 32 of m0 >> sq, 1 and 3 of m1 >> sq
+          const uint64_t two = (m0 >> sq & 0x100000001ull) | (m1 >> sq & 0x100000001ull) << 1;
+          const uint32_t nibble = lo32(two) | hi32(two) << 2;
+          // entry (nibble, left) of a table of the left-th set bits, two bits each
+          sl = (uint32_t)((nibble & 8u ? kNthHigh : kNthLow) >> ((nibble * 8u + left * 2u) & 63u)) & 3u;
         } else {
           sl = left + 1u - n0;  // slots 0 and 1 alone: slot 1 if it is the second or the only one
         }
@@ -263,6 +361,7 @@ __device__ __forceinline__ void play(ck::Lane &L, const Geometry &geo, const Str
       ply++;
       refresh();
     }
+    if (!walk) return;  // the game is over
     const ck::Gen g = analysis(jA, jB, m0, m1, longer, 1u);
     uint32_t unused = 0;
     ck::PlyResult res;
@@ -270,10 +369,9 @@ __device__ __forceinline__ void play(ck::Lane &L, const Geometry &geo, const Str
       bool deep = false;
       res = ck::ply_random_trees<false>(L, g, r, &unused, deep);
       if (deep) res = ck::ply_random_given<false>(L, g, r, &unused);
-    } else if (POLICY == MI_POLICY_HEURISTIC) {
-      res = ck::ply_heuristic_given<false>(L, g, r, &unused);
-    } else {
-      res = ck::ply_noisy_given<false>(L, g, r, &unused);
+    } else if (!capture_ply<POLICY>(L, g, r, lane, res)) {
+      res = POLICY == MI_POLICY_HEURISTIC ? ck::ply_heuristic_given<false>(L, g, r, &unused)
+                                          : ck::ply_noisy_given<false>(L, g, r, &unused);
     }
     maxn = res.n > maxn ? res.n : maxn;
     if (res.over) return;

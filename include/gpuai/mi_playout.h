@@ -186,7 +186,7 @@ int mi_gen_start_positions(mi_ctx *ctx, uint32_t seed, uint32_t n, uint32_t kmin
  * and graph replays then launch each batch with its bucket's shape (graph replays: the fastest of
  * the graph's refill policy), and batches whose bucket has no entry with the context's tuning.
  * mi_set_tuning empties the table.  Until a context is given a shape (mi_create, mi_set_tuning,
- * mi_autotune), batches of up to 16 playouts per compute unit (32 for the noisy heuristic) whose
+ * mi_autotune), batches of up to 32 playouts per compute unit (48 for the noisy heuristic) whose
  * bucket has no entry run with one wave per game instead of one lane per game (stats: 64-thread
  * blocks, one per playout, MI_REFILL_STATIC; the same winners).  The allocation-free entry point
  * uses the context's tuning, or one wave per game where it knows the batch's size (counts ==

@@ -59,3 +59,17 @@ def test_deferred_plies(shaped, oracle, policy, kind, block, per_cu, refill, def
     assert np.array_equal(res.winners, w)
     assert res.stats["plies"] == int(tr["plies"].sum(dtype=np.uint64))
     assert res.stats["max_moves"] == int(tr["max_n"].max())
+
+
+@pytest.mark.parametrize("policy", [POLICY_RANDOM, POLICY_HEURISTIC, POLICY_HEURISTIC_NOISY])
+@pytest.mark.parametrize("kind", ["steps", "captures"])
+def test_the_same_with_a_wave_per_game(oracle, policy, kind):
+    pos = boards(oracle.start_positions(1, 1, 0, 1, False).dtype, 300, kind)
+    with Engine(0) as eng:
+        print(f"[gpu] a wave per game: {kind}, policy {policy}", file=sys.stderr, flush=True)
+        res = eng.run_playouts(pos, per_pos=25, seed=6, epoch=7, policy=policy)
+    assert res.stats["grid_blocks"] == 300 * 25
+    w, tr = oracle.run_playouts(pos, per_pos=25, seed=6, epoch=7, policy=policy)
+    assert np.array_equal(res.winners, w)
+    assert res.stats["plies"] == int(tr["plies"].sum(dtype=np.uint64))
+    assert res.stats["max_moves"] == int(tr["max_n"].max())

@@ -35,7 +35,7 @@ def positions(oracle, n: int, seed: int) -> np.ndarray:
 
 
 @pytest.mark.parametrize("policy", POLICIES)
-@pytest.mark.parametrize("n,per", [(1, 1), (1, 3), (63, 1), (65, 7), (700, 4), (255, 16), (3000, 1)])
+@pytest.mark.parametrize("n,per", [(1, 1), (1, 3), (63, 1), (65, 7), (700, 4), (257, 16), (3000, 1)])
 def test_uniform_counts(fresh, oracle, policy, n, per):
     pos = positions(oracle, n, 500 + n)
     announce(f"one wave per game: {n} x {per}, policy {policy}")
@@ -48,7 +48,7 @@ def test_uniform_counts(fresh, oracle, policy, n, per):
 
 
 @pytest.mark.parametrize("policy", POLICIES)
-@pytest.mark.parametrize("n", [1, 64, 65, 2600])
+@pytest.mark.parametrize("n", [1, 64, 65, 4097])
 def test_uneven_keyed_graph_and_noalloc(fresh, oracle, policy, n):
     pos = positions(oracle, n, 900 + n)
     rng = np.random.default_rng(n)
@@ -72,7 +72,7 @@ def test_uneven_keyed_graph_and_noalloc(fresh, oracle, policy, n):
 @pytest.mark.parametrize("policy", POLICIES)
 def test_route_ends_at_its_limit(fresh, oracle, policy):
     """The last size with one wave per game and the first with one lane per game: the same games."""
-    limit = fresh.device_info()["compute_units"] * (32 if policy == POLICY_HEURISTIC_NOISY else 16)
+    limit = fresh.device_info()["compute_units"] * (48 if policy == POLICY_HEURISTIC_NOISY else 32)
     pos = positions(oracle, limit + 1, 41)
     announce(f"{limit} and {limit + 1} playouts, policy {policy}")
     a = fresh.run_playouts(pos[:limit], per_pos=1, seed=8, epoch=2, policy=policy)
