@@ -20,6 +20,7 @@
 
 #include "checkers.h"
 #include "kernels.h"
+#include "wave_play.h"
 
 namespace gpuai {
 
@@ -43,6 +44,10 @@ __device__ __forceinline__ uint32_t lane_rank(uint64_t mask) {
 // Whether this lane is in a wave mask.
 __device__ __forceinline__ bool lane_in(uint64_t mask) {
   return __builtin_amdgcn_inverse_ballot_w64(mask);
+}
+
+__device__ __forceinline__ uint32_t uniform(uint32_t x) {
+  return __builtin_amdgcn_readfirstlane(x);
 }
 
 __device__ __forceinline__ uint64_t uniform64(uint64_t x) {
@@ -386,6 +391,22 @@ __device__ __forceinline__ void noisy_steps(WalkShare &share, uint64_t todo, ck:
   wave_lds_fence();
 }
 
+// A wave's last game is played by the whole wave (wave_play.h), at 0.33 us a ply instead of 0.85:
+// 21000x3 0.137 -> 0.129 ms, random-64x4096 0.213 -> 0.203.  With two such games the second one
+// waits for the first and nothing is gained over playing both in their lanes (0.133, 0.210).
+struct LastGame {
+  int32_t winner;
+  uint32_t plies, longest;
+};
+template <uint32_t POLICY>
+__device__ __forceinline__ LastGame last_game(ck::Lane L, uint32_t ply, uint32_t lane,
+                                              const wave::Stream &stream) {
+  LastGame end = {0, ply, 0u};
+  wave::play<POLICY>(L, wave::geometry(lane), stream, end.plies, end.longest);
+  end.winner = L.counter < 50u ? (int32_t)(L.turn ^ 1u) : -1;
+  return end;
+}
+
 // The waves of a workgroup hand their last games over.  Once no playout is left to claim, a wave's
 // games end one after the other while an iteration costs the same to its last one: on
 // random-64x4096 72% of all wave iterations had 18 of 64 lanes playing.  A wave with at most half of
@@ -495,8 +516,11 @@ __global__ void __launch_bounds__(1024) k_playouts(PlayoutArgs a) {
   };
   // The next four words' block b of the lanes' streams.
   auto generate = [&](uint32_t b) {
-    uint32_t o[4];
-    ck::philox(b, j, ck::TAG_PLAYOUT, a.epoch, a.seed, p, o);
+    uint32_t o[4], seed = a.seed;
+    // (the rounds' keys are ten additions; kept for the whole loop they do not fit the scalar
+    // registers and come back by lane reads)
+    asm volatile("" : "+s"(seed));
+    ck::philox(b, j, ck::TAG_PLAYOUT, a.epoch, seed, p, o);
     uint32_t *const row = words + (b & 1u) * (4u * 64u);
 #pragma unroll
     for (uint32_t w = 0; w < 4u; w++) row[w * 64u] = o[w];
@@ -610,7 +634,12 @@ __global__ void __launch_bounds__(1024) k_playouts(PlayoutArgs a) {
     // (uniform, but not to the compiler: the branches above hold divergent ones)
     active = uniform64(active);
     asks = __builtin_amdgcn_readfirstlane(asks);
-    if (__builtin_amdgcn_readfirstlane(leaves) || !active) break;
+    if (__builtin_amdgcn_readfirstlane(leaves)) active = 0;
+    if (!active) break;
+    // the last game of a wave that nobody will give any is played below
+    if (!TRACE && !(active & (active - 1ull)) && uniform(dry) &&
+        (!asks || (lds_take(handover.asking, 1u << wave) >> wave & 1u)))
+      break;
     if (lane_in(active)) generate((ply / kPly + 3u) >> 2);
 #pragma unroll 1
     for (uint32_t step = 0; step < 4u; step++) {
@@ -700,6 +729,18 @@ __global__ void __launch_bounds__(1024) k_playouts(PlayoutArgs a) {
           since_walk++;
         }
       }
+    }
+  }
+  if (!TRACE && active) {
+    const uint32_t from = (uint32_t)__builtin_ctzll(active);
+    auto of = [from](uint32_t x) { return wave::lane_value(x, from); };
+    const LastGame end = last_game<POLICY>(
+        {of(L.own), of(L.opp), of(L.kings), of(L.turn), of(L.counter)}, of(ply) / kPly, lane,
+        {of(j), ck::TAG_PLAYOUT, a.epoch, a.seed, of(p)});
+    maxn = end.longest > maxn ? end.longest : maxn;
+    if (lane == from) {
+      a.winners[g] = (int8_t)end.winner;
+      plies_acc += end.plies;
     }
   }
   // statistics: per wave, then per workgroup in LDS, then one device atomic each (device atomics
