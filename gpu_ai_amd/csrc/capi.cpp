@@ -715,17 +715,17 @@ int mi_gen_start_positions(mi_ctx *ctx, uint32_t seed, uint32_t n, uint32_t kmin
     return fail(ctx, MI_ERR_INVALID_ARGUMENT, "kmax - kmin + 1 exceeds 2^32 - 1");
   if (hipSetDevice(ctx->device) != hipSuccess) return fail(ctx, MI_ERR_DEVICE, "hipSetDevice failed");
   int rc;
-  // work words and positions in one block: one copy brings both back, through its pinned mirror
-  // while that stays within the staging limit (262,144 positions: 1.10 -> 1.05 ms a call against
-  // two copies to pageable memory, 30,000: 0.57 -> 0.39 ms)
+  // Within the staging limit the kernel writes the positions, each once, to the pinned mirror of the
+  // work words (262,144 positions: 895 -> 830 us a call against device memory and a copy of 75 us
+  // behind the kernel); beyond it they go to device memory and are copied out.
   const size_t bytes = sizeof(mi_pos) * (size_t)n;
   const bool back = bytes <= kPinnedMax;
-  if ((rc = ensure(ctx, ctx->batch, sizeof(gpuai::WorkWords) + bytes))) return rc;
+  if ((rc = ensure(ctx, ctx->batch, sizeof(gpuai::WorkWords) + (back ? 0 : bytes)))) return rc;
   if ((rc = ensure_host(ctx, ctx->h_batch, sizeof(gpuai::WorkWords) + (back ? bytes : 0)))) return rc;
   ctx->staged = false;
   gpuai::WorkWords *work = (gpuai::WorkWords *)ctx->batch.ptr;
-  mi_pos *d_out = (mi_pos *)(work + 1);
-  const gpuai::WorkWords *h_work = (const gpuai::WorkWords *)ctx->h_batch.ptr;
+  gpuai::WorkWords *h_work = (gpuai::WorkWords *)ctx->h_batch.ptr;
+  mi_pos *to = (mi_pos *)((back ? h_work : work) + 1);
   // in pieces of 2^30 positions, which the kernel's claims can count in 32 bits
   constexpr uint32_t kPiece = 1u << 30;
   uint32_t overflow = 0;
@@ -737,15 +737,14 @@ int mi_gen_start_positions(mi_ctx *ctx, uint32_t seed, uint32_t n, uint32_t kmin
     a.kmin = kmin;
     a.span = kmax - kmin + 1u;
     a.reject = reject_terminal;
-    a.out = d_out + at;
+    a.out = to + at;
     a.work = work;
     MI_HIP(ctx, gpuai::launch_reset(work, ctx->stream));
     // few positions: as many waves as positions, whose lanes play attempts ahead
     const uint32_t grid = gpuai::grid_size(a.n, (uint64_t)ctx->cus * kDefaultTuning.blocks_per_cu);
     a.slots = std::min(64u, (a.n + grid - 1u) / grid);
     MI_HIP(ctx, gpuai::launch_start_positions(a, grid, ctx->stream));
-    MI_HIP(ctx, hipMemcpyAsync(ctx->h_batch.ptr, work, sizeof(*work) + (back ? bytes : 0),
-                               hipMemcpyDeviceToHost, ctx->stream));
+    MI_HIP(ctx, hipMemcpyAsync(h_work, work, sizeof(*work), hipMemcpyDeviceToHost, ctx->stream));
     if (!back)
       MI_HIP(ctx, hipMemcpyAsync(out + at, a.out, sizeof(mi_pos) * (size_t)a.n,
                                  hipMemcpyDeviceToHost, ctx->stream));
@@ -753,7 +752,7 @@ int mi_gen_start_positions(mi_ctx *ctx, uint32_t seed, uint32_t n, uint32_t kmin
     overflow |= h_work->overflow;
     if (n - at <= kPiece) break;
   }
-  if (back) std::memcpy(out, h_work + 1, bytes);
+  if (back) std::memcpy(out, to, bytes);
   if (overflow) return fail(ctx, MI_ERR_INVALID_ARGUMENT, "no unfinished position in 4096 attempts");
   return MI_OK;
 }
