@@ -71,10 +71,12 @@ uint32_t tune_bucket(uint64_t total) {
   return b < kTuneBuckets ? b : kTuneBuckets - 1u;
 }
 
-mi_tuning batch_shape(const mi_ctx *ctx, uint64_t total) {
+mi_tuning batch_shape(const mi_ctx *ctx, uint32_t policy, uint64_t total) {
   mi_tuning t = ctx->tuning;
+  if (ctx->shaped) return t;
+  if (policy == MI_POLICY_HEURISTIC_NOISY) t.defer_min = 24u;
   const uint64_t lanes = 64u * (uint64_t)ctx->cus;  // of a wave per CU
-  if (ctx->shaped || total <= 4u * lanes) return t;
+  if (total <= 4u * lanes) return t;
   const uint64_t waves = (total + lanes - 1u) / lanes;
   t.block_size = 64u * (uint32_t)(total >= 32u * lanes ? 16u : waves < 12u ? waves : 12u);
   t.blocks_per_cu = 1u;
@@ -255,7 +257,7 @@ mi_tuning shape_for(const mi_ctx *ctx, uint32_t policy, uint64_t total, int only
     if (e[r].kernel_ms < 0.f || (only >= 0 && r != only)) continue;
     if (!best || e[r].kernel_ms < best->kernel_ms) best = &e[r];
   }
-  return best ? best->tuning : gpuai::ctxutil::batch_shape(ctx, total);
+  return best ? best->tuning : gpuai::ctxutil::batch_shape(ctx, policy, total);
 }
 
 // The statistics' launch shape of such a batch.
@@ -770,8 +772,8 @@ int tune_sweep(mi_ctx *ctx, uint32_t npos, uint32_t per_pos, uint64_t total, boo
   // 3 and 4 waves per SIMD are the fast ones on random-1024x1024 (more lanes in flight lengthen
   // the end of a batch, fewer leave the SIMDs short of waves to issue from)
   const uint32_t waves_per_simd[] = {1u, 2u, 3u, 4u, 8u};
-  // 32 for the noisy heuristic, whose deferred plies make the draws: 1.07 against 1.16-1.19 ms
-  // at 16 on noisy-1024x1024 (the other policies gain nothing past 16)
+  // 32 for the noisy heuristic, whose deferred plies make the draws: 0.546 against 0.564 ms at 16
+  // on noisy-1024x1024 (the other policies gain nothing past 16)
   const uint32_t defers[] = {1u, 8u, 16u, 32u};
   mi_tuning refill_best[2] = {};
   float refill_ms[2] = {3.0e38f, 3.0e38f};

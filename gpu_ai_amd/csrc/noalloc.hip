@@ -230,7 +230,7 @@ extern "C" int mi_run_playouts_noalloc(mi_ctx *ctx, const mi_pos *pos, uint32_t 
   a.plies = nullptr;
   a.hashes = nullptr;
   a.work = &S->work;
-  a.defer_min = ctx->tuning.defer_min;
+  a.defer_min = 0;
   a.desc = &S->desc;
   // the shape and grid as mi_run_playouts sizes them; with counts in device memory the total is
   // unknown here, so a whole resident grid of small workgroups runs (waves without work leave at
@@ -239,7 +239,8 @@ extern "C" int mi_run_playouts_noalloc(mi_ctx *ctx, const mi_pos *pos, uint32_t 
     MI_HIP(ctx, gpuai::launch_playouts_wave(a, policy, (uint32_t)uniform_total, s));
     return MI_OK;
   }
-  const mi_tuning t = counts ? ctx->tuning : gpuai::ctxutil::batch_shape(ctx, uniform_total);
+  const mi_tuning t = gpuai::ctxutil::batch_shape(ctx, policy, counts ? 0u : uniform_total);
+  a.defer_min = t.defer_min;
   const uint64_t block = t.block_size;
   const uint64_t resident = (uint64_t)ctx->cus * t.blocks_per_cu;
   const uint64_t need = counts ? resident : (uniform_total + block - 1) / block;

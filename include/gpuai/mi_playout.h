@@ -105,10 +105,10 @@ typedef struct mi_tune_result {
 typedef struct mi_ctx mi_ctx;
 
 /* Creates a context on HIP device `device`.  `tuning` may be NULL (or have zero fields) for the
- * defaults: queue refill, defer_min 16, and the shape each batch takes by its size (up to four
- * waves a CU 64-thread blocks, beyond that one workgroup per CU of up to 16 waves; mi_get_tuning
- * reports 64-thread blocks, 12 per CU).  No counterpart in the reference, whose drivers allocate
- * on every call (src/singlePlayout.cu:76-84). */
+ * defaults: queue refill, defer_min 16 (noisy heuristic 24), and the shape each batch takes by its
+ * size (up to four waves a CU 64-thread blocks, beyond that one workgroup per CU of up to 16 waves;
+ * mi_get_tuning reports 64-thread blocks, 12 per CU, defer_min 16).  No counterpart in the
+ * reference, whose drivers allocate on every call (src/singlePlayout.cu:76-84). */
 int mi_create(mi_ctx **ctx, int device, const mi_tuning *tuning);
 int mi_destroy(mi_ctx *ctx);
 const char *mi_strerror(int code);
