@@ -1055,7 +1055,7 @@ struct mi_graph {
   size_t out_bytes = 0;
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
-  hipGraphNode_t n_reset = nullptr, n_play = nullptr, n_d2h = nullptr;
+  hipGraphNode_t n_stage = nullptr, n_play = nullptr, n_d2h = nullptr;
   // the playout node's arguments and launch shape, fixed at creation except for the grid, which
   // each replay sizes to its batch (a small batch spread over every CU, as mi_run_playouts does)
   gpuai::PlayoutArgs args;
@@ -1106,6 +1106,7 @@ int mi_graph_create(mi_ctx *ctx, uint32_t max_positions, uint32_t max_playouts, 
     return fail(ctx, MI_ERR_INVALID_ARGUMENT, "too many positions for one graph batch");
   }
   g->out_bytes = sizeof(gpuai::WorkWords) + (size_t)max_playouts;
+  g->blob_bytes = (g->blob_bytes + 15u) & ~(size_t)15u;  // whole words of k_stage
   hipError_t e = hipHostMalloc(&g->h_blob, g->blob_bytes, hipHostMallocDefault);
   if (e == hipSuccess) e = hipHostMalloc(&g->h_out, g->out_bytes, hipHostMallocDefault);
   if (e == hipSuccess) e = hipMalloc(&g->d_blob, g->blob_bytes);
@@ -1136,14 +1137,14 @@ int mi_graph_create(mi_ctx *ctx, uint32_t max_positions, uint32_t max_playouts, 
   g->refill = t.refill;
   g->resident = ctx->cus * t.blocks_per_cu;
   g->grid = grid_for(ctx, t, max_playouts);
-  void *reset_args[] = {&work};
+  void *stage_args[] = {&g->h_blob, &g->d_blob, &work};
   void *play_args[] = {&a};
   hipKernelNodeParams rp;
   std::memset(&rp, 0, sizeof(rp));
-  rp.func = const_cast<void *>(gpuai::reset_kernel());
-  rp.gridDim = dim3(1);
-  rp.blockDim = dim3(64);
-  rp.kernelParams = reset_args;
+  rp.func = const_cast<void *>(gpuai::stage_kernel());
+  rp.gridDim = dim3(gpuai::kStageGrid);
+  rp.blockDim = dim3(gpuai::kStageBlock);
+  rp.kernelParams = stage_args;
   hipKernelNodeParams pp;
   std::memset(&pp, 0, sizeof(pp));
   pp.func = const_cast<void *>(gpuai::playout_kernel(policy, g->refill));
@@ -1152,10 +1153,10 @@ int mi_graph_create(mi_ctx *ctx, uint32_t max_positions, uint32_t max_playouts, 
   pp.sharedMemBytes = gpuai::playout_lds(g->policy, g->block);
   pp.kernelParams = play_args;
   e = hipGraphCreate(&g->graph, 0);
-  // The batch's upload is not a node: an asynchronous copy on the stream before each replay
-  // moves a 64k-leaf batch (1.3 MB) in ~40 us, a memcpy node took ~320 us.
-  if (e == hipSuccess) e = hipGraphAddKernelNode(&g->n_reset, g->graph, nullptr, 0, &rp);
-  if (e == hipSuccess) e = hipGraphAddKernelNode(&g->n_play, g->graph, &g->n_reset, 1, &pp);
+  // The batch's upload is a kernel node that reads as much of the pinned blob as its description
+  // says (k_stage; a memcpy node of 1.3 MB took 320 us).
+  if (e == hipSuccess) e = hipGraphAddKernelNode(&g->n_stage, g->graph, nullptr, 0, &rp);
+  if (e == hipSuccess) e = hipGraphAddKernelNode(&g->n_play, g->graph, &g->n_stage, 1, &pp);
   if (e == hipSuccess)
     e = hipGraphAddMemcpyNode1D(&g->n_d2h, g->graph, &g->n_play, 1, g->h_out, g->d_out,
                                 g->out_bytes, hipMemcpyDeviceToHost);
@@ -1190,6 +1191,7 @@ int mi_graph_launch(mi_graph *g, const mi_pos *pos, uint32_t npos, const uint32_
     const size_t keys_at = offs_at + sizeof(uint32_t) * ((size_t)npos + 1);
     const size_t in_bytes = keys_at + (keys ? sizeof(uint32_t) * (size_t)npos : 0);
     std::memset(d, 0, sizeof(*d));
+    d->words = (uint32_t)((in_bytes + 15u) / 16u);
     d->npos = npos;
     d->total = (uint32_t)total;
     d->seed = seed;
@@ -1206,8 +1208,7 @@ int mi_graph_launch(mi_graph *g, const mi_pos *pos, uint32_t npos, const uint32_
     if (wave_batch(ctx, g->policy, total)) {  // the graph holds the other kernel: same order, no graph
       gpuai::PlayoutArgs a = g->args;
       MI_HIP(ctx, hipEventRecord(g->e0, ctx->stream));
-      MI_HIP(ctx, hipMemcpyAsync(g->d_blob, g->h_blob, in_bytes, hipMemcpyHostToDevice, ctx->stream));
-      MI_HIP(ctx, gpuai::launch_reset(a.work, ctx->stream));
+      MI_HIP(ctx, gpuai::launch_stage(d, (gpuai::LaunchDesc *)g->d_blob, a.work, ctx->stream));
       MI_HIP(ctx, gpuai::launch_playouts_wave(a, g->policy, (uint32_t)total, ctx->stream));
       MI_HIP(ctx, hipMemcpyAsync(g->h_out, g->d_out, out_bytes, hipMemcpyDeviceToHost, ctx->stream));
       MI_HIP(ctx, hipEventRecord(g->e1, ctx->stream));
@@ -1241,7 +1242,6 @@ int mi_graph_launch(mi_graph *g, const mi_pos *pos, uint32_t npos, const uint32_
       g->resident = ctx->cus * t.blocks_per_cu;
     }
     MI_HIP(ctx, hipEventRecord(g->e0, ctx->stream));
-    MI_HIP(ctx, hipMemcpyAsync(g->d_blob, g->h_blob, in_bytes, hipMemcpyHostToDevice, ctx->stream));
     MI_HIP(ctx, hipGraphLaunch(g->exec, ctx->stream));
     MI_HIP(ctx, hipEventRecord(g->e1, ctx->stream));
   }

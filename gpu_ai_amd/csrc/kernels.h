@@ -79,10 +79,11 @@ struct LaunchDesc {
   uint32_t epoch;
   uint32_t ordered;  // 0: the hand-out order of the arguments is ignored (positions in index order)
   // Byte offsets from this description of the batch's sections when they follow it in one
-  // block of device memory (graph replays pack positions, offsets and keys behind it, so that one
-  // copy of the used prefix uploads a batch); 0: the pointer of the arguments (keys: none).
+  // block of device memory (graph replays pack positions, offsets and keys behind it, so that
+  // k_stage uploads a batch in one piece); 0: the pointer of the arguments (keys: none).
   uint32_t pos_at, offs_at, keys_at;
-  uint32_t pad[8];
+  uint32_t words;  // 16-byte words of the description and its sections (launch_stage)
+  uint32_t pad[7];
 };
 
 struct PlayoutArgs {
@@ -114,11 +115,15 @@ struct PlayoutArgs {
 
 // Kernel entry of the playout kernel for a policy and refill policy (graph construction).
 const void *playout_kernel(uint32_t policy, uint32_t refill);
-const void *reset_kernel();
+// The upload of a packed batch (k_stage) as a graph node.
+const void *stage_kernel();
+constexpr uint32_t kStageBlock = 256, kStageGrid = 128;
 // Dynamic LDS of a playout launch with workgroups of `block` threads.
 uint32_t playout_lds(uint32_t policy, uint32_t block);
 
 hipError_t launch_reset(WorkWords *work, hipStream_t stream);
+// Copies a packed batch from pinned host memory and clears the work words.
+hipError_t launch_stage(const LaunchDesc *from, LaunchDesc *to, WorkWords *work, hipStream_t stream);
 hipError_t launch_playouts(const PlayoutArgs &args, uint32_t policy, bool trace, uint32_t refill,
                            uint32_t grid, uint32_t block, hipStream_t stream);
 // One wave per game (wave_playouts.hip): `games` workgroups of kWaveBlock threads.  args.order is
