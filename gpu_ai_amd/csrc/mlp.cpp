@@ -41,8 +41,9 @@ struct mi_mlp {
   // copied. The gradients of 4096 with the copies of the batch, the gradients and the loss took
   // 86 us, without 54.
   void *h_stage = nullptr;
-  // device-resident training set; ds_shuffle: the epoch shuffle's scratch
-  DevBuf ds_pos, ds_t, ds_perm, ds_loss, ds_shuffle;
+  // device-resident training set; ds_shuffle: the epoch shuffle's scratch, ds_rows: the set in the
+  // epoch's order (positions, then targets)
+  DevBuf ds_pos, ds_t, ds_rows, ds_loss, ds_shuffle;
   uint32_t ds_n = 0;
   std::vector<uint32_t> host_perm;  // of small sets
   hipEvent_t e0 = nullptr, e1 = nullptr;
@@ -144,15 +145,12 @@ int upload_params(mi_mlp *n, const float *w) {
 // One training step over `rows` rows (count valid): k_train_rows' forward and backward pass to
 // the activations and vector partials, then the weight gradients and Adam (k_update; when
 // update == 0, only the gradient sums).  loss_out receives the batch loss and
-// `grads` every gradient (either may be null; device or pinned host memory).  Row r is
-// pos[idx ? idx[r] : r] with target targets[idx ? idx[r] : r].
-int train_rows(mi_mlp *n, const mi_pos *pos, const uint32_t *idx, const float *targets,
-               uint32_t count, uint32_t rows, float lr, int update, float *loss_out,
-               float *grads = nullptr) {
+// `grads` every gradient (either may be null; device or pinned host memory).
+int train_rows(mi_mlp *n, const mi_pos *pos, const float *targets, uint32_t count, uint32_t rows,
+               float lr, int update, float *loss_out, float *grads = nullptr) {
   mi_ctx *ctx = n->ctx;
   K::TrainArgs ta = {};
   ta.pos = pos;
-  ta.idx = idx;
   ta.targets = targets;
   ta.n = count;
   ta.slices = n->max_rows / 32u;
@@ -270,7 +268,7 @@ int mi_mlp_destroy(mi_mlp *n) {
   (void)hipStreamSynchronize(n->ctx->stream);
   for (void *p : n->allocs) (void)hipFree(p);
   if (n->h_stage) (void)hipHostFree(n->h_stage);
-  gpuai::DevBuf *bufs[] = {&n->ds_pos, &n->ds_t, &n->ds_perm, &n->ds_loss,
+  gpuai::DevBuf *bufs[] = {&n->ds_pos, &n->ds_t, &n->ds_rows, &n->ds_loss,
                          &n->ds_shuffle};
   for (auto *b : bufs)
     if (b->ptr) (void)hipFree(b->ptr);
@@ -329,7 +327,7 @@ static int grad_common(mi_mlp *n, const mi_pos *pos, const float *targets, uint3
   std::memcpy(stage_pos(n), pos, sizeof(mi_pos) * count);
   std::memcpy(stage_targets(n), targets, sizeof(float) * count);
   float *hg = stage_params(n, 0);
-  if ((rc = train_rows(n, stage_pos(n), nullptr, stage_targets(n), count, round64(count), lr, update,
+  if ((rc = train_rows(n, stage_pos(n), stage_targets(n), count, round64(count), lr, update,
                        stage_loss(n), grads ? hg : nullptr)))
     return rc;
   MI_HIP(ctx, hipStreamSynchronize(ctx->stream));
@@ -369,7 +367,9 @@ int mi_mlp_set_dataset(mi_mlp *n, const mi_pos *pos, const float *targets, uint3
   if ((rc = use_device(n))) return rc;
   if ((rc = ensure(ctx, n->ds_pos, sizeof(mi_pos) * (size_t)std::max<uint32_t>(count, 1)))) return rc;
   if ((rc = ensure(ctx, n->ds_t, sizeof(float) * (size_t)std::max<uint32_t>(count, 1)))) return rc;
-  if ((rc = ensure(ctx, n->ds_perm, sizeof(uint32_t) * (size_t)std::max<uint32_t>(count, 1)))) return rc;
+  if ((rc = ensure(ctx, n->ds_rows,
+                   (sizeof(mi_pos) + sizeof(float)) * (size_t)std::max<uint32_t>(count, 1))))
+    return rc;
   if ((rc = ensure(ctx, n->ds_shuffle, 4 * sizeof(uint32_t) * (size_t)std::max<uint32_t>(count, 1))))
     return rc;
   MI_HIP(ctx, hipMemcpyAsync(n->ds_pos.ptr, pos, sizeof(mi_pos) * count, hipMemcpyHostToDevice, ctx->stream));
@@ -392,30 +392,33 @@ int mi_mlp_train_epoch(mi_mlp *n, uint32_t batch, float lr, uint32_t shuffle_see
   if (int rc0 = use_device(n)) return rc0;
   int rc;
   if ((rc = ensure(ctx, n->ds_loss, sizeof(float) * nb))) return rc;
+  K::ShuffleArgs sh;
+  sh.n = n->ds_n;
+  sh.seed = shuffle_seed;
+  sh.epoch = epoch;
+  sh.head = (uint32_t *)n->ds_shuffle.ptr;
+  sh.next = sh.head + (size_t)n->ds_n;
+  sh.target = sh.next + (size_t)n->ds_n;
+  sh.chain = sh.target + (size_t)n->ds_n;
+  sh.pos = (const mi_pos *)n->ds_pos.ptr;
+  sh.targets = (const float *)n->ds_t.ptr;
+  sh.rows = (mi_pos *)n->ds_rows.ptr;
+  sh.row_targets = (float *)(sh.rows + (size_t)n->ds_n);
   if (n->ds_n <= kHostShuffle) {
     std::vector<uint32_t> &perm = n->host_perm;
     perm.resize(n->ds_n);
     host_shuffle(perm, shuffle_seed, epoch);
-    MI_HIP(ctx, hipMemcpyAsync(n->ds_perm.ptr, perm.data(), sizeof(uint32_t) * n->ds_n,
+    MI_HIP(ctx, hipMemcpyAsync(sh.head, perm.data(), sizeof(uint32_t) * n->ds_n,
                                hipMemcpyHostToDevice, ctx->stream));
+    MI_HIP(ctx, K::shuffle_take(sh, sh.head, ctx->stream));
   } else {
-    K::ShuffleArgs sh;
-    sh.n = n->ds_n;
-    sh.seed = shuffle_seed;
-    sh.epoch = epoch;
-    sh.head = (uint32_t *)n->ds_shuffle.ptr;
-    sh.next = sh.head + (size_t)n->ds_n;
-    sh.target = sh.next + (size_t)n->ds_n;
-    sh.chain = sh.target + (size_t)n->ds_n;
-    sh.order = (uint32_t *)n->ds_perm.ptr;
     MI_HIP(ctx, K::shuffle(sh, ctx->stream));
   }
   float *losses = (float *)n->ds_loss.ptr;
   MI_HIP(ctx, hipEventRecord(n->e0, ctx->stream));
   for (uint32_t b = 0; b < nb; b++) {
-    const uint32_t *idx = (const uint32_t *)n->ds_perm.ptr + (size_t)b * batch;
-    if ((rc = train_rows(n, (const mi_pos *)n->ds_pos.ptr, idx, (const float *)n->ds_t.ptr, batch,
-                         batch, lr, 1, losses + b)))
+    const size_t at = (size_t)b * batch;
+    if ((rc = train_rows(n, sh.rows + at, sh.row_targets + at, batch, batch, lr, 1, losses + b)))
       return rc;
   }
   MI_HIP(ctx, hipEventRecord(n->e1, ctx->stream));

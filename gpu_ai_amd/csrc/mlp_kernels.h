@@ -21,13 +21,11 @@ constexpr uint32_t kWSplitRows = 128;
 // loss 769.
 constexpr uint32_t kVecSlots = 1024;
 
-// One training step's row pass (k_train_rows), kTrainRows rows per workgroup: row r < n is
-// pos[idx ? idx[r] : r] with target targets[idx ? idx[r] : r]; rows n and up (to the multiple
-// of kTrainRows) are padding.  Writes the activations and their gradients in operand order
+// One training step's row pass (k_train_rows), kTrainRows rows per workgroup: row r < n is pos[r]
+// with target targets[r]; rows n and up (to the multiple of kTrainRows) are padding.  Writes the activations and their gradients in operand order
 // (mlp_kernels.hip) and block b's vector partials at pV + b * kVecSlots.
 struct TrainArgs {
   const mi_pos *pos;
-  const uint32_t *idx;
   const float *targets;
   uint32_t n;
   uint32_t slices;  // 32-row slices per 16 features of the operands (>= rows / 32)
@@ -66,9 +64,14 @@ hipError_t update(const AdamArgs &a, hipStream_t stream);
 struct ShuffleArgs {
   uint32_t n, seed, epoch;
   uint32_t *head, *next, *target, *chain;
-  uint32_t *order;
+  const mi_pos *pos;      // the dataset
+  const float *targets;
+  mi_pos *rows;           // receive it in the epoch's order
+  float *row_targets;
 };
 hipError_t shuffle(const ShuffleArgs &a, hipStream_t stream);
+// The epoch's order given (device memory).
+hipError_t shuffle_take(const ShuffleArgs &a, const uint32_t *order, hipStream_t stream);
 hipError_t zero(float *p, uint32_t n, hipStream_t stream);
 
 }  // namespace mlp

@@ -183,7 +183,7 @@ __global__ void __launch_bounds__(512) k_forward(const mi_pos *pos, uint32_t n,
 }
 
 // ---------------------------------------------------------------------------------------------
-// Training.  Row r of the batch is pos[idx ? idx[r] : r] with target targets[idx ? idx[r] : r];
+// Training.  Row r of the batch is pos[r] with target targets[r];
 // rows n and up (to the multiple of kTrainRows) are padding: zero inputs and no loss.  The
 // arithmetic: H1 = bf(relu(X W1 + b1)), H2 = bf(relu(H1 W2 + b2)), y = tanh(H2 . w3 + b3),
 // dz = 2 (y - t)(1 - y^2) / n, dH2 = bf(dz w3) where H2 > 0, dH1 = bf(dH2 W2^T) where H1 > 0;
@@ -221,27 +221,25 @@ __global__ void __launch_bounds__(512) k_train_rows(TrainArgs a) {
   // same time, and the rotation spreads their requests over different lines of L2
   const int cw = ((wave + (int)blockIdx.x) & 7) * 32;
   // Loads, issued before any is used, in an order that lets each wait cover only what it needs --
-  // loads complete in issue order as far as the wait counter goes: the dataset index of this
-  // thread's row (threads 0..127: row t/4, plane t%4), the wave's W1 operands, the position and
-  // target the index points to, then the W2 operands of both directions and the biases.  The
-  // empty asm statements keep the compiler from reordering the groups.
+  // loads complete in issue order as far as the wait counter goes: the position and target of this
+  // thread's row (threads 0..127: row t/4, plane t%4), the wave's W1 operands, then the W2 operands
+  // of both directions and the biases.  The empty asm statements keep the compiler from reordering
+  // the groups.
   const int erow = t >> 2;
   const bool encodes = t < 4 * KR, evalid = r0 + erow < a.n;
-  uint32_t esrc = min(r0 + erow, a.n - 1u);
-  if (encodes && a.idx) esrc = a.idx[esrc];
-  __asm__ volatile("" ::: "memory");
-  bf16x8 w1p[4][2], w2p[8][2], w2rp[8][2];  // this wave's weights: [slice][column tile]
-#pragma unroll
-  for (int s = 0; s < 4; s++)
-#pragma unroll
-    for (int c = 0; c < 2; c++) w1p[s][c] = fragment(a.W1f, cw / 16 + c, 4, s, lane);
-  __asm__ volatile("" ::: "memory");
+  const uint32_t esrc = min(r0 + erow, a.n - 1u);
   mi_pos epos = {};
   float tgt = 0.f;
   if (encodes) {
     epos = a.pos[esrc];
     tgt = a.targets[esrc];
   }
+  __asm__ volatile("" ::: "memory");
+  bf16x8 w1p[4][2], w2p[8][2], w2rp[8][2];  // this wave's weights: [slice][column tile]
+#pragma unroll
+  for (int s = 0; s < 4; s++)
+#pragma unroll
+    for (int c = 0; c < 2; c++) w1p[s][c] = fragment(a.W1f, cw / 16 + c, 4, s, lane);
   __asm__ volatile("" ::: "memory");
 #pragma unroll
   for (int s = 0; s < 8; s++)
@@ -626,8 +624,10 @@ __global__ void __launch_bounds__(512) k_update(AdamArgs a) {
 // chain(x) = the smallest i' > x with j(i') = x, the value comes from following chain() to its end.
 // The steps that target a position are linked in a list per position (k_shuffle_link; one or two
 // on average, ln n at most positions), chain() is read off the lists (k_shuffle_chain), and every
-// position follows its own (k_shuffle_order).  262,144 positions: 26 us against 0.7 ms on the host with
-// the upload of its result; 8M: 1.2 ms against 38.
+// position follows its own (k_shuffle_order), which copies what it finds into the epoch's order, so
+// that the steps read consecutive rows.  262,144 positions: 26 us against 0.7 ms on the host with
+// the upload of its result; 8M: 1.2 ms against 38.  A
+// step of 4096 rows takes 19.7 us from consecutive rows, 20.2 when it looks the order up itself.
 constexpr uint32_t kNone = 0xFFFFFFFFu;
 
 __global__ void __launch_bounds__(256) k_shuffle_clear(uint32_t *head, uint32_t n) {
@@ -673,7 +673,16 @@ __global__ void __launch_bounds__(256) k_shuffle_order(ShuffleArgs a) {
     x = k;
     k = a.chain[x];
   }
-  a.order[i] = x;
+  a.rows[i] = a.pos[x];
+  a.row_targets[i] = a.targets[x];
+}
+
+// The same from an order made on the host.
+__global__ void __launch_bounds__(256) k_shuffle_take(ShuffleArgs a, const uint32_t *order) {
+  const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+  if (i >= a.n) return;
+  a.rows[i] = a.pos[order[i]];
+  a.row_targets[i] = a.targets[order[i]];
 }
 
 __global__ void k_zero(float *p, uint32_t n) {
@@ -713,6 +722,11 @@ hipError_t shuffle(const ShuffleArgs &a, hipStream_t stream) {
   if (a.n > 1u) hipLaunchKernelGGL(k_shuffle_link, words, block, 0, stream, a);
   hipLaunchKernelGGL(k_shuffle_chain, all, block, 0, stream, a);
   hipLaunchKernelGGL(k_shuffle_order, all, block, 0, stream, a);
+  return hipGetLastError();
+}
+
+hipError_t shuffle_take(const ShuffleArgs &a, const uint32_t *order, hipStream_t stream) {
+  hipLaunchKernelGGL(k_shuffle_take, dim3((a.n + 255u) / 256u), dim3(256), 0, stream, a, order);
   return hipGetLastError();
 }
 
