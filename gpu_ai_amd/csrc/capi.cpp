@@ -742,8 +742,12 @@ int mi_gen_start_positions(mi_ctx *ctx, uint32_t seed, uint32_t n, uint32_t kmin
     a.out = to + at;
     a.work = work;
     MI_HIP(ctx, gpuai::launch_reset(work, ctx->stream));
-    // few positions: as many waves as positions, whose lanes play attempts ahead
-    const uint32_t grid = gpuai::grid_size(a.n, (uint64_t)ctx->cus * kDefaultTuning.blocks_per_cu);
+    // Few positions: as many waves as positions, whose lanes play attempts ahead, up to one a SIMD,
+    // where a wave issues alone (16,000 positions of 0-10 / 20-60 / 40-150 plies, us a call: 53 / 121 /
+    // 301, with three a SIMD 61 / 143 / 305).  More positions than those have lanes: two a SIMD
+    // (262,144: 327 / 521 / 1207; one 334 / 583 / 1541, three 330 / 524 / 1215).
+    const uint64_t simds = 4ull * ctx->cus;
+    const uint32_t grid = gpuai::grid_size(a.n, a.n <= 64u * simds ? simds : 2u * simds);
     a.slots = std::min(64u, (a.n + grid - 1u) / grid);
     MI_HIP(ctx, gpuai::launch_start_positions(a, grid, ctx->stream));
     MI_HIP(ctx, hipMemcpyAsync(h_work, work, sizeof(*work), hipMemcpyDeviceToHost, ctx->stream));

@@ -21,3 +21,13 @@ def test_start_positions_match_oracle(engine, oracle, n, kmin, kmax, reject):
     got = engine.start_positions(11 + n, n, kmin, kmax, reject_terminal=reject)
     want = oracle.start_positions(11 + n, n, kmin, kmax, reject_terminal=reject)
     assert got.tobytes() == want.tobytes()
+
+
+# around one and two waves a SIMD (1024 and 2048), and around 64 positions for each of their waves:
+# dealt out to the slots up to 131,072 positions, claimed from a queue beyond
+@pytest.mark.parametrize("n", [1023, 1025, 65537, 131071, 131072, 131073])
+def test_start_positions_dealt_and_claimed(engine, oracle, n):
+    print(f"[gpu] {n} start positions", file=sys.stderr, flush=True)
+    got = engine.start_positions(n, n, 0, 60, reject_terminal=True)
+    want = oracle.start_positions(n, n, 0, 60, reject_terminal=True)
+    assert got.tobytes() == want.tobytes()
