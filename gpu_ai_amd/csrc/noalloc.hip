@@ -234,7 +234,8 @@ extern "C" int mi_run_playouts_noalloc(mi_ctx *ctx, const mi_pos *pos, uint32_t 
   a.desc = &S->desc;
   // the shape and grid as mi_run_playouts sizes them; with counts in device memory the total is
   // unknown here, so a whole resident grid of small workgroups runs (waves without work leave at
-  // their first refill, and a small batch is not left on a few CUs)
+  // their first refill, and a small batch is not left on a few CUs; of a game per wave at most each
+  // wave plays one)
   if (!counts && gpuai::ctxutil::wave_batch(ctx, policy, uniform_total)) {
     MI_HIP(ctx, gpuai::launch_playouts_wave(a, policy, (uint32_t)uniform_total, s));
     return MI_OK;

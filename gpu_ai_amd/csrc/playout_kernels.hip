@@ -455,7 +455,10 @@ __device__ __forceinline__ void lds_set(uint32_t &x, uint32_t bits) {
     __hip_atomic_fetch_or(&x, bits, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-template <uint32_t POLICY, bool TRACE, uint32_t REFILL>
+// FEW: for launches of single-wave workgroups whose number of games the host does not know: a batch
+// with at most a game for each wave is played as such (300 positions, 1191 random games by counts in
+// device memory 182 -> 104 us; as a branch of the other launches' kernel it cost those 1%).
+template <uint32_t POLICY, bool TRACE, uint32_t REFILL, bool FEW = false>
 __global__ void __launch_bounds__(1024) k_playouts(PlayoutArgs a) {
   if (a.desc) {  // graph replays and allocation-free launches: the batch lives in device memory
     const LaunchDesc *d = a.desc;
@@ -553,7 +556,24 @@ __global__ void __launch_bounds__(1024) k_playouts(PlayoutArgs a) {
     }
     active &= ~over;
   };
+  // The game in g from its start.
+  auto begin = [&]() {
+    mi_pos q;
+    locate(a, g, p, j, g, q);  // from here on g is the playout's result slot
+    if (a.keys) p = a.keys[p];  // from here on p is the stream key
+    L = ck::lane_from_abs(q.p1, q.p2, q.kings, q.turn, q.counter);
+    ply = 0;
+    h = 0;
+  };
 
+  if (FEW && a.total <= gridDim.x) {  // each game is its wave's last one from the start
+    exhausted = true;
+    if (blockIdx.x < a.total) {
+      g = blockIdx.x;
+      if (lane == 0u) begin();
+      active = 1u;
+    }
+  }
   for (;;) {
     bool start = false;
     if (REFILL == MI_REFILL_STATIC) {
@@ -590,14 +610,7 @@ __global__ void __launch_bounds__(1024) k_playouts(PlayoutArgs a) {
       }
       if (slab_index(res_next, slab, nslabs) >= a.total) exhausted = true;  // slab dry
     }
-    if (start) {
-      mi_pos q;
-      locate(a, g, p, j, g, q);  // from here on g is the playout's result slot
-      if (a.keys) p = a.keys[p];  // from here on p is the stream key
-      L = ck::lane_from_abs(q.p1, q.p2, q.kings, q.turn, q.counter);
-      ply = 0;
-      h = 0;
-    }
+    if (start) begin();
     active |= __ballot(start);
     const bool dry = REFILL == MI_REFILL_STATIC ? !__ballot(static_next < a.total) : exhausted;
     uint32_t leaves = 0u;  // this wave's games, if any, go to another one
@@ -1115,6 +1128,9 @@ hipError_t launch_refill(const PlayoutArgs &args, uint32_t refill, uint32_t grid
                          hipStream_t stream) {
   if (refill == MI_REFILL_STATIC)
     hipLaunchKernelGGL((k_playouts<POLICY, TRACE, MI_REFILL_STATIC>), dim3(grid), dim3(block),
+                       playout_lds(POLICY, block), stream, args);
+  else if (!TRACE && args.desc && args.offs && block == 64u)
+    hipLaunchKernelGGL((k_playouts<POLICY, false, MI_REFILL_QUEUE, !TRACE>), dim3(grid), dim3(block),
                        playout_lds(POLICY, block), stream, args);
   else
     hipLaunchKernelGGL((k_playouts<POLICY, TRACE, MI_REFILL_QUEUE>), dim3(grid), dim3(block),
