@@ -365,6 +365,7 @@ int mi_mlp_set_dataset(mi_mlp *n, const mi_pos *pos, const float *targets, uint3
   ctx->last_error.clear();
   int rc;
   if ((rc = use_device(n))) return rc;
+  n->ds_n = 0;  // the buffers go one by one: a call that fails leaves no set
   if ((rc = ensure(ctx, n->ds_pos, sizeof(mi_pos) * (size_t)std::max<uint32_t>(count, 1)))) return rc;
   if ((rc = ensure(ctx, n->ds_t, sizeof(float) * (size_t)std::max<uint32_t>(count, 1)))) return rc;
   if ((rc = ensure(ctx, n->ds_rows,

@@ -66,7 +66,8 @@ int mi_mlp_adam_state(mi_mlp *mlp, float *m, float *v, uint32_t *step);
 
 /* Device-resident training set (positions and targets copied once), and one epoch over it in
  * batches of `batch` (a multiple of 64, <= max_batch) in an order drawn from Philox key
- * (shuffle_seed, epoch), counter (i >> 2, 0, 3, 1); a trailing partial batch is dropped.
+ * (shuffle_seed, epoch), counter (i >> 2, 0, 3, 1); a trailing partial batch is dropped.  A set
+ * that device memory cannot hold leaves the network without one.
  * mean_loss receives the mean of the batch losses; ms the device time of the epoch. */
 int mi_mlp_set_dataset(mi_mlp *mlp, const mi_pos *pos, const float *targets, uint32_t n);
 int mi_mlp_train_epoch(mi_mlp *mlp, uint32_t batch, float lr, uint32_t shuffle_seed,
