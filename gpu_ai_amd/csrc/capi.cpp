@@ -570,9 +570,7 @@ int mi_create(mi_ctx **out, int device, const mi_tuning *tuning) {
       return MI_ERR_INVALID_ARGUMENT;
     }
     ctx->tuning = t;
-    // every field zero but the queue refill: the defaults
-    ctx->shaped = tuning->block_size || tuning->blocks_per_cu || tuning->defer_min ||
-                  tuning->refill != kDefaultTuning.refill;
+    ctx->shaped = !is_default(t);
   }
   hipDeviceProp_t prop;
   if (hipSetDevice(device) != hipSuccess || hipGetDeviceProperties(&prop, device) != hipSuccess ||
@@ -621,7 +619,7 @@ int mi_set_tuning(mi_ctx *ctx, const mi_tuning *tuning) {
   int rc = check_tuning(ctx, t);
   if (rc) return rc;
   ctx->tuning = t;
-  ctx->shaped = true;
+  ctx->shaped = !is_default(t);
   clear_tune_table(ctx);  // an explicit shape holds for every batch size
   return MI_OK;
 }

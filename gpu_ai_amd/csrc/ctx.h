@@ -27,6 +27,14 @@ struct HostBuf {
 // batch_shape's.
 constexpr mi_tuning kDefaultTuning = {64u, 12u, MI_REFILL_QUEUE, 16u};
 
+// Whether a tuning asks for the defaults: a program that saves a context's tuning and sets it again
+// later gets its routes by size back.
+constexpr bool is_default(const mi_tuning &t) {
+  return t.block_size == kDefaultTuning.block_size &&
+         t.blocks_per_cu == kDefaultTuning.blocks_per_cu && t.refill == kDefaultTuning.refill &&
+         t.defer_min == kDefaultTuning.defer_min;
+}
+
 // Launch-shape table: the fastest shape the autotuner measured for a policy, a batch-size bucket
 // (floor(log2(playouts))) and a refill policy; kernel_ms < 0 marks an empty entry.
 constexpr uint32_t kTuneBuckets = 32;
@@ -41,7 +49,7 @@ struct mi_ctx {
   hipStream_t stream = nullptr;
   hipEvent_t ev_start = nullptr, ev_stop = nullptr;
   mi_tuning tuning = kDefaultTuning;  // the shape of batches whose bucket the table lacks
-  bool shaped = false;  // `tuning` was given or measured: it holds for small batches too
+  bool shaped = false;  // `tuning` was given or measured: it holds for every size
   TuneEntry tune_table[3][kTuneBuckets][2];  // [policy][bucket][refill]
   uint32_t cus = 0, wave = 64, clock_khz = 0;
   gpuai::DevBuf pos, offs, winners, plies, hashes, work, tallies, moves, counts, keys;

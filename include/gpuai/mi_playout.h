@@ -115,7 +115,8 @@ const char *mi_strerror(int code);
 /* Text of the last error raised on this context (empty if none). */
 const char *mi_last_error(const mi_ctx *ctx);
 /* Sets the launch shape, for every batch size: the launch-shape table (see mi_autotune) is
- * emptied.  Zero fields take the defaults of mi_create. */
+ * emptied.  Zero fields take the values that mi_get_tuning reports for the defaults of mi_create, and
+ * a tuning that has all of those values sets these defaults: batches take their shape by size again. */
 int mi_set_tuning(mi_ctx *ctx, const mi_tuning *tuning);
 int mi_get_tuning(const mi_ctx *ctx, mi_tuning *tuning);
 /* Device facts: compute units, wave size, clock in kHz. */

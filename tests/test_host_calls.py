@@ -49,3 +49,7 @@ def check(tmp_path_factory):
 def test_a_set_that_does_not_fit_leaves_none(check):
     out = check("dataset_check.cpp")
     assert "failed allocations 4, null arguments 0, mismatches 0" in out, out
+
+
+def test_default_tuning_is_by_size(check):
+    assert "mismatches 0" in check("tuning_check.cpp")
