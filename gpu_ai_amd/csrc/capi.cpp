@@ -72,8 +72,8 @@ uint32_t tune_bucket(uint64_t total) {
 }
 
 mi_tuning batch_shape(const mi_ctx *ctx, uint32_t policy, uint64_t total) {
-  mi_tuning t = ctx->tuning;
-  if (ctx->shaped) return t;
+  if (ctx->shaped || (!total && !is_default(ctx->tuning))) return ctx->tuning;
+  mi_tuning t = kDefaultTuning;
   if (policy == MI_POLICY_HEURISTIC_NOISY) t.defer_min = 24u;
   const uint64_t lanes = 64u * (uint64_t)ctx->cus;  // of a wave per CU
   if (total <= 4u * lanes) return t;
@@ -83,7 +83,17 @@ mi_tuning batch_shape(const mi_ctx *ctx, uint32_t policy, uint64_t total) {
   return t;
 }
 
-// Whether a batch of `total` playouts runs with one wave per game (k_playouts_wave).  A small batch
+mi_tuning shape_for(const mi_ctx *ctx, uint32_t policy, uint64_t total, int only) {
+  const TuneEntry *e = ctx->tune_table[policy][tune_bucket(total)];
+  const TuneEntry *best = nullptr;
+  for (int r = 0; r < 2; r++) {
+    if (e[r].kernel_ms < 0.f || (only >= 0 && r != only)) continue;
+    if (!best || e[r].kernel_ms < best->kernel_ms) best = &e[r];
+  }
+  return best ? best->tuning : batch_shape(ctx, policy, total);
+}
+
+// The largest batch that may run with one wave per game (k_playouts_wave).  A small batch
 // lasts as long as its longest game: 0.33-0.47 us per ply with a wave of its own (random, noisy)
 // against 0.9-1.5 us in a wave of 64 games, but a game costs a whole wave's instructions, so from
 // some size on the lanes win.  Kernel ms, one wave per game / one lane per game, 256 CUs:
@@ -91,12 +101,19 @@ mi_tuning batch_shape(const mi_ctx *ctx, uint32_t policy, uint64_t total) {
 //   random     .053 / .130  .081 / .121  .113 / .128  .139 / .133  .160 / .135
 //   heuristic  .054 / .150  .096 / .140  .134 / .142  .171 / .151  .200 / .151
 //   noisy      .066 / .213  .113 / .188  .150 / .185  .184 / .186  .225 / .187
-// A context that was given a launch shape, or has measured one for the batch's size, uses it.
-bool wave_batch(const mi_ctx *ctx, uint32_t policy, uint64_t total) {
-  if (ctx->shaped || total > (uint64_t)ctx->cus * (policy == MI_POLICY_HEURISTIC_NOISY ? 48u : 32u))
-    return false;
+static uint32_t wave_limit(const mi_ctx *ctx, uint32_t policy) {
+  return ctx->cus * (policy == MI_POLICY_HEURISTIC_NOISY ? 48u : 32u);
+}
+
+// A tuning run measures both for the sizes below the limit, and its bucket takes the faster one;
+// without, a context that was given a launch shape uses it.
+bool wave_batch(const mi_ctx *ctx, uint32_t policy, uint64_t total, int only) {
+  if (total > wave_limit(ctx, policy)) return false;
   const TuneEntry *e = ctx->tune_table[policy][tune_bucket(total)];
-  return e[0].kernel_ms < 0.f && e[1].kernel_ms < 0.f;
+  if (e[0].wave_ms < 0.f) return !ctx->shaped;
+  for (int r = 0; r < 2; r++)
+    if ((only < 0 || r == only) && e[r].kernel_ms <= e[r].wave_ms) return false;
+  return true;
 }
 
 }  // namespace ctxutil
@@ -107,6 +124,7 @@ using gpuai::ctxutil::ensure;
 using gpuai::ctxutil::ensure_host;
 using gpuai::ctxutil::fail;
 using gpuai::ctxutil::hip_fail;
+using gpuai::ctxutil::shape_for;
 using gpuai::ctxutil::tune_bucket;
 using gpuai::ctxutil::wave_batch;
 
@@ -248,20 +266,25 @@ uint32_t grid_for(const mi_ctx *ctx, const mi_tuning &t, uint64_t total) {
   return gpuai::grid_size(need, resident);
 }
 
-// The launch shape of a batch of `total` playouts: the table's entry for its policy and bucket
-// (the faster refill, or refill `only` when it is 0 or 1), else the context's tuning.
-mi_tuning shape_for(const mi_ctx *ctx, uint32_t policy, uint64_t total, int only = -1) {
-  const TuneEntry *e = ctx->tune_table[policy][tune_bucket(total)];
-  const TuneEntry *best = nullptr;
-  for (int r = 0; r < 2; r++) {
-    if (e[r].kernel_ms < 0.f || (only >= 0 && r != only)) continue;
-    if (!best || e[r].kernel_ms < best->kernel_ms) best = &e[r];
-  }
-  return best ? best->tuning : gpuai::ctxutil::batch_shape(ctx, policy, total);
+// One wave per game in statistics and among tuning results: no workgroups per CU, each game has its
+// own.
+constexpr mi_tuning kWaveShape = {gpuai::kWaveBlock, 0u, MI_REFILL_STATIC, 0u};
+
+mi_tuning wave_shape(uint32_t refill) {
+  mi_tuning t = kWaveShape;
+  t.refill = refill;
+  return t;
 }
 
-// The statistics' launch shape of such a batch.
-constexpr mi_tuning kWaveShape = {gpuai::kWaveBlock, 0u, MI_REFILL_STATIC, 0u};
+// An entry of the table as its refill policy's batches run.
+TuneEntry fastest(const TuneEntry &e) {
+  TuneEntry f = e;
+  if (e.wave_ms >= 0.f && e.wave_ms < e.kernel_ms) {
+    f.tuning = wave_shape(e.tuning.refill);
+    f.kernel_ms = e.wave_ms;
+  }
+  return f;
+}
 
 void clear_tune_table(mi_ctx *ctx) {
   for (auto &pol : ctx->tune_table)
@@ -276,7 +299,7 @@ int run_kernel(mi_ctx *ctx, uint32_t npos, uint32_t per_pos, uint64_t total, boo
                uint32_t seed, uint32_t epoch, uint32_t policy, bool trace, mi_stats *stats,
                int8_t *winners = nullptr, bool keyed = false, const mi_tuning *shape = nullptr) {
   // the autotuner passes the candidate it measures; every other launch takes its batch's shape
-  const bool wave = !shape && !trace && wave_batch(ctx, policy, total);
+  const bool wave = shape ? !shape->blocks_per_cu : !trace && wave_batch(ctx, policy, total);
   const mi_tuning t = shape ? *shape : wave ? kWaveShape : shape_for(ctx, policy, total);
   int rc;
   if ((rc = ensure_host(ctx, ctx->h_back, sizeof(gpuai::WorkWords) + (winners ? total : 0))))
@@ -764,12 +787,13 @@ int mi_gen_start_positions(mi_ctx *ctx, uint32_t seed, uint32_t n, uint32_t kmin
 namespace {
 
 // Measures every candidate launch shape on the uploaded batch -- workgroup sizes 64..1024, 1..8
-// resident waves per SIMD, both refill policies, deferral thresholds 1, 8, 16 and 32 -- `reps`
-// launches each (median kernel time), records the fastest of each refill policy in the tuning
-// table's entry for the batch's policy and size bucket, and returns the fastest overall.
+// resident waves per SIMD, both refill policies, deferral thresholds 1, 8, 16 and 32, and for small
+// batches one wave per game -- `reps` launches each (median kernel time), records the fastest of
+// each refill policy in the tuning table's entry for the batch's policy and size bucket, and
+// returns the fastest overall and the fastest with one lane per game.
 int tune_sweep(mi_ctx *ctx, uint32_t npos, uint32_t per_pos, uint64_t total, bool with_offs,
                uint32_t policy, uint32_t reps, mi_tune_result *results, uint32_t max_results,
-               uint32_t *nresults, mi_tuning &best_t, float &best_ms) {
+               uint32_t *nresults, mi_tuning &best_t, float &best_ms, mi_tuning &lanes_t) {
   const uint32_t blocks[] = {64u, 128u, 192u, 256u, 512u, 768u, 1024u};
   // 3 and 4 waves per SIMD are the fast ones on random-1024x1024 (more lanes in flight lengthen
   // the end of a batch, fewer leave the SIMDs short of waves to issue from)
@@ -778,8 +802,30 @@ int tune_sweep(mi_ctx *ctx, uint32_t npos, uint32_t per_pos, uint64_t total, boo
   // on noisy-1024x1024 (the other policies gain nothing past 16)
   const uint32_t defers[] = {1u, 8u, 16u, 32u};
   mi_tuning refill_best[2] = {};
-  float refill_ms[2] = {3.0e38f, 3.0e38f};
+  float refill_ms[2] = {3.0e38f, 3.0e38f}, wave_ms = -1.f;
   uint32_t n = 0;
+  // the median kernel time of a candidate, which is listed
+  auto measure = [&](const mi_tuning &t, float &med) {
+    std::vector<float> ms;
+    for (uint32_t r = 0; r < reps; r++) {
+      mi_stats st;
+      const int rc = run_kernel(ctx, npos, per_pos, total, with_offs, 0x7A5Eu, 0xFFFF0000u + r,
+                                policy, false, &st, nullptr, false, &t);
+      if (rc) return rc;
+      ms.push_back(st.kernel_ms);
+    }
+    std::sort(ms.begin(), ms.end());
+    med = ms[ms.size() / 2];
+    return (int)MI_OK;
+  };
+  auto list = [&](const mi_tuning &t, float med) {
+    if (results && n < max_results) {
+      results[n].tuning = t;
+      results[n].kernel_ms = med;
+      results[n].playouts_per_s = (float)((double)total / (med * 1e-3));
+    }
+    n++;
+  };
   for (uint32_t refill = 0; refill < 2; refill++) {
     for (uint32_t b : blocks) {
       for (uint32_t w : waves_per_simd) {
@@ -788,22 +834,9 @@ int tune_sweep(mi_ctx *ctx, uint32_t npos, uint32_t per_pos, uint64_t total, boo
           if ((b / 64u) > waves_per_cu) continue;  // a block larger than the residency
           if ((waves_per_cu * 64u) % b) continue;  // whole blocks only
           const mi_tuning t = {b, waves_per_cu * 64u / b, refill, dm};
-          std::vector<float> ms;
-          for (uint32_t r = 0; r < reps; r++) {
-            mi_stats st;
-            const int rc = run_kernel(ctx, npos, per_pos, total, with_offs, 0x7A5Eu,
-                                      0xFFFF0000u + r, policy, false, &st, nullptr, false, &t);
-            if (rc) return rc;
-            ms.push_back(st.kernel_ms);
-          }
-          std::sort(ms.begin(), ms.end());
-          const float med = ms[ms.size() / 2];
-          if (results && n < max_results) {
-            results[n].tuning = t;
-            results[n].kernel_ms = med;
-            results[n].playouts_per_s = (float)((double)total / (med * 1e-3));
-          }
-          n++;
+          float med;
+          if (const int rc = measure(t, med)) return rc;
+          list(t, med);
           if (med < refill_ms[refill]) {
             refill_ms[refill] = med;
             refill_best[refill] = t;
@@ -812,15 +845,23 @@ int tune_sweep(mi_ctx *ctx, uint32_t npos, uint32_t per_pos, uint64_t total, boo
       }
     }
   }
+  if (total <= gpuai::ctxutil::wave_limit(ctx, policy)) {
+    // a game has its wave under either refill policy, so each has the candidate
+    if (const int rc = measure(kWaveShape, wave_ms)) return rc;
+    for (uint32_t refill = 0; refill < 2; refill++) list(wave_shape(refill), wave_ms);
+  }
   TuneEntry *e = ctx->tune_table[policy][tune_bucket(total)];
   for (int r = 0; r < 2; r++) {
     e[r].tuning = refill_best[r];
     e[r].kernel_ms = refill_ms[r];
+    e[r].wave_ms = wave_ms;
     e[r].playouts = (uint32_t)total;
   }
   const int r = refill_ms[1] < refill_ms[0] ? 1 : 0;
-  best_t = refill_best[r];
-  best_ms = refill_ms[r];
+  lanes_t = refill_best[r];
+  const TuneEntry best = fastest(e[0]).kernel_ms <= fastest(e[1]).kernel_ms ? fastest(e[0]) : fastest(e[1]);
+  best_t = best.tuning;
+  best_ms = best.kernel_ms;
   if (nresults) *nresults = n;
   return MI_OK;
 }
@@ -842,13 +883,13 @@ int mi_autotune(mi_ctx *ctx, const mi_pos *pos, uint32_t npos, const uint32_t *c
   if (hipSetDevice(ctx->device) != hipSuccess) return fail(ctx, MI_ERR_DEVICE, "hipSetDevice failed");
   if ((rc = upload_batch(ctx, pos, npos, counts, total))) return rc;
   ctx->staged = false;
-  mi_tuning best_t = ctx->tuning;
+  mi_tuning best_t, lanes_t;
   float best_ms = 0.f;
   if ((rc = tune_sweep(ctx, npos, per_pos, total, counts != nullptr, policy, reps, results,
-                       max_results, nresults, best_t, best_ms)))
+                       max_results, nresults, best_t, best_ms, lanes_t)))
     return rc;
-  ctx->tuning = best_t;
-  ctx->shaped = true;
+  ctx->tuning = lanes_t;
+  ctx->shaped = false;
   if (best) *best = best_t;
   return MI_OK;
 }
@@ -873,9 +914,10 @@ int mi_autotune_sizes(mi_ctx *ctx, const mi_pos *pos, uint32_t npos, uint32_t po
     if ((rc = plan_batch(ctx, pos, n, nullptr, per, total))) return rc;
     if ((rc = upload_batch(ctx, pos, n, nullptr, total))) return rc;
     ctx->staged = false;
-    mi_tuning t = ctx->tuning;
+    mi_tuning t, lanes_t;
     float ms = 0.f;
-    if ((rc = tune_sweep(ctx, n, per, total, false, policy, reps, nullptr, 0, nullptr, t, ms)))
+    if ((rc = tune_sweep(ctx, n, per, total, false, policy, reps, nullptr, 0, nullptr, t, ms,
+                         lanes_t)))
       return rc;
     if (best) {
       best[i].policy = policy;
@@ -894,7 +936,7 @@ int mi_get_tuning_table(const mi_ctx *ctx, mi_tune_entry *out, uint32_t cap, uin
   for (uint32_t pol = 0; pol <= MI_POLICY_HEURISTIC_NOISY; pol++)
     for (uint32_t b = 0; b < kTuneBuckets; b++)
       for (uint32_t r = 0; r < 2; r++) {
-        const TuneEntry &e = ctx->tune_table[pol][b][r];
+        const TuneEntry e = fastest(ctx->tune_table[pol][b][r]);
         if (e.kernel_ms < 0.f) continue;
         if (n < cap) {
           out[n].policy = pol;
@@ -1207,7 +1249,7 @@ int mi_graph_launch(mi_graph *g, const mi_pos *pos, uint32_t npos, const uint32_
     std::memcpy(h + offs_at, ctx->host_offs.data(), sizeof(uint32_t) * ((size_t)npos + 1));
     if (keys) std::memcpy(h + keys_at, keys, sizeof(uint32_t) * (size_t)npos);
     const size_t out_bytes = sizeof(gpuai::WorkWords) + (size_t)total;
-    if (wave_batch(ctx, g->policy, total)) {  // the graph holds the other kernel: same order, no graph
+    if (wave_batch(ctx, g->policy, total, (int)g->refill)) {  // the graph holds the other kernel: same order, no graph
       gpuai::PlayoutArgs a = g->args;
       MI_HIP(ctx, hipEventRecord(g->e0, ctx->stream));
       MI_HIP(ctx, gpuai::launch_stage(d, (gpuai::LaunchDesc *)g->d_blob, a.work, ctx->stream));
@@ -1218,7 +1260,7 @@ int mi_graph_launch(mi_graph *g, const mi_pos *pos, uint32_t npos, const uint32_
       g->pending_total = total;
       g->pending_grid = (uint32_t)total;
       g->pending_block = kWaveShape.block_size;
-      g->pending_refill = kWaveShape.refill;
+      g->pending_refill = g->refill;
       return MI_OK;
     }
     MI_HIP(ctx, hipGraphExecMemcpyNodeSetParams1D(g->exec, g->n_d2h, g->h_out, g->d_out, out_bytes,

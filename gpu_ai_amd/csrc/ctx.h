@@ -39,8 +39,9 @@ constexpr bool is_default(const mi_tuning &t) {
 // (floor(log2(playouts))) and a refill policy; kernel_ms < 0 marks an empty entry.
 constexpr uint32_t kTuneBuckets = 32;
 struct TuneEntry {
-  mi_tuning tuning = {0u, 0u, 0u, 0u};
+  mi_tuning tuning = {0u, 0u, 0u, 0u};  // of one lane per game
   float kernel_ms = -1.f;
+  float wave_ms = -1.f;   // the same batch with one wave per game; < 0: not measured (too large)
   uint32_t playouts = 0;  // size of the batch it was measured on
 };
 
@@ -48,8 +49,8 @@ struct mi_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
   hipEvent_t ev_start = nullptr, ev_stop = nullptr;
-  mi_tuning tuning = kDefaultTuning;  // the shape of batches whose bucket the table lacks
-  bool shaped = false;  // `tuning` was given or measured: it holds for every size
+  mi_tuning tuning = kDefaultTuning;  // as given, or the fastest of mi_autotune's batch
+  bool shaped = false;  // `tuning` was given: batches of every size take it unless the table has theirs
   TuneEntry tune_table[3][kTuneBuckets][2];  // [policy][bucket][refill]
   uint32_t cus = 0, wave = 64, clock_khz = 0;
   gpuai::DevBuf pos, offs, winners, plies, hashes, work, tallies, moves, counts, keys;
@@ -96,10 +97,15 @@ uint32_t tune_bucket(uint64_t total);
 // 0.210 with 12 (0.216 with 16), 65536x256 4.76 -> 4.45 with 16 (4.77 with 12).  Up to four waves a CU there is nothing to hand
 // over, and 64-thread blocks it is.  The noisy heuristic waits for 24 plies: its walk phases cost
 // much the same for any number of them (noisy-1024x1024 0.582, 0.564, 0.552, 0.539 and 0.546 ms at
-// 12, 16, 20, 24 and 32; the other policies are level from 16 on).
+// 12, 16, 20, 24 and 32; the other policies are level from 16 on).  What mi_autotune measured on one
+// batch holds for that batch's bucket: at 65,536 random playouts the shape of 1,048,576 takes 0.203
+// ms, the size's own 0.139.  total 0: the size is not known here, and the context's tuning it is.
 mi_tuning batch_shape(const mi_ctx *ctx, uint32_t policy, uint64_t total);
-// Whether a batch runs with one wave per game.
-bool wave_batch(const mi_ctx *ctx, uint32_t policy, uint64_t total);
+// The launch shape of a batch with one lane per game: the table's entry for its policy and bucket
+// (the faster refill, or refill `only` when it is 0 or 1), else batch_shape's.
+mi_tuning shape_for(const mi_ctx *ctx, uint32_t policy, uint64_t total, int only = -1);
+// Whether a batch runs with one wave per game instead (`only` as for shape_for).
+bool wave_batch(const mi_ctx *ctx, uint32_t policy, uint64_t total, int only = -1);
 }  // namespace ctxutil
 // Looks up the device address of the allocation-free entry point's scratch array for the
 // context's device (once per device; the device must be current).

@@ -240,7 +240,8 @@ extern "C" int mi_run_playouts_noalloc(mi_ctx *ctx, const mi_pos *pos, uint32_t 
     MI_HIP(ctx, gpuai::launch_playouts_wave(a, policy, (uint32_t)uniform_total, s));
     return MI_OK;
   }
-  const mi_tuning t = gpuai::ctxutil::batch_shape(ctx, policy, counts ? 0u : uniform_total);
+  const mi_tuning t = counts ? gpuai::ctxutil::batch_shape(ctx, policy, 0u)
+                             : gpuai::ctxutil::shape_for(ctx, policy, uniform_total);
   a.defer_min = t.defer_min;
   const uint64_t block = t.block_size;
   const uint64_t resident = (uint64_t)ctx->cus * t.blocks_per_cu;

@@ -179,23 +179,29 @@ int mi_gen_start_positions(mi_ctx *ctx, uint32_t seed, uint32_t n, uint32_t kmin
  * drivers by a runtime model of the batch size, src/playout.cpp:80-166).  Runs the given batch
  * under every candidate launch shape -- workgroup sizes 64..1024, 1..8 resident waves per SIMD
  * (which sets the playouts each lane runs), both refill policies and deferral thresholds 1, 8, 16
- * and 32 -- `reps` times each and takes the one with the smallest median kernel time.
+ * and 32, for small batches also one wave per game -- `reps` times each and takes the one with the smallest median kernel time.
  *
  * The context keeps a launch-shape table: per policy, batch-size bucket (batches of 2^b to
  * 2^(b+1) - 1 playouts) and refill policy, the fastest shape measured.  Every tuning run records
  * its batch's bucket there; mi_run_playouts (and the keyed, traced, tally and staged launches)
  * and graph replays then launch each batch with its bucket's shape (graph replays: the fastest of
- * the graph's refill policy), and batches whose bucket has no entry with the context's tuning.
- * mi_set_tuning empties the table.  Until a context is given a shape (mi_create, mi_set_tuning,
- * mi_autotune), batches of up to 32 playouts per compute unit (48 for the noisy heuristic) whose
- * bucket has no entry run with one wave per game instead of one lane per game (stats: 64-thread
- * blocks, one per playout, MI_REFILL_STATIC; the same winners).  The allocation-free entry point
- * uses the context's tuning, or one wave per game where it knows the batch's size (counts ==
- * NULL) and the same rule asks for it.
+ * the graph's refill policy).  Batches whose bucket has no entry take the shape that the context was
+ * given (mi_create, mi_set_tuning) or, without one, the shape of their size.  mi_set_tuning empties
+ * the table.
  *
- * mi_autotune tunes on one batch and also makes the winner the context's tuning.  `results` (may
- * be NULL) receives up to `max_results` candidates; `nresults` the number measured; `best` (may
- * be NULL) the winner. */
+ * Small batches, of up to 32 playouts per compute unit (48 for the noisy heuristic), can also run
+ * with one wave per game instead of one lane per game (the same winners; not traced launches).  They
+ * do on a context that was given no shape, unless a tuning run measured a lane's shape faster for
+ * their bucket; a tuning run lists it, once per refill policy, as blocks_per_cu 0 (64-thread blocks,
+ * defer_min 0).  The statistics then say 64-thread blocks, one per playout, and MI_REFILL_STATIC
+ * (graph replays: the graph's refill policy).
+ *
+ * The allocation-free entry point takes the same routes where it knows the batch's size (counts ==
+ * NULL), else the context's tuning.
+ *
+ * mi_autotune tunes on one batch and also makes the fastest shape with one lane per game the
+ * context's tuning, in place of a shape that it was given.  `results` (may be NULL) receives up to `max_results` candidates; `nresults` the
+ * number measured; `best` (may be NULL) the winner. */
 int mi_autotune(mi_ctx *ctx, const mi_pos *pos, uint32_t npos, const uint32_t *counts,
                 uint32_t per_pos, uint32_t policy, uint32_t reps, mi_tune_result *results,
                 uint32_t max_results, uint32_t *nresults, mi_tuning *best);

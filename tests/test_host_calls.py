@@ -51,5 +51,5 @@ def test_a_set_that_does_not_fit_leaves_none(check):
     assert "failed allocations 4, null arguments 0, mismatches 0" in out, out
 
 
-def test_default_tuning_is_by_size(check):
+def test_routes_of_shaped_and_tuned_contexts(check):
     assert "mismatches 0" in check("tuning_check.cpp")
