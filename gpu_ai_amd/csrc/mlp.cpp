@@ -411,12 +411,13 @@ int mi_mlp_train_epoch(mi_mlp *n, uint32_t batch, float lr, uint32_t shuffle_see
     host_shuffle(perm, shuffle_seed, epoch);
     MI_HIP(ctx, hipMemcpyAsync(sh.head, perm.data(), sizeof(uint32_t) * n->ds_n,
                                hipMemcpyHostToDevice, ctx->stream));
+    MI_HIP(ctx, hipEventRecord(n->e0, ctx->stream));
     MI_HIP(ctx, K::shuffle_take(sh, sh.head, ctx->stream));
   } else {
+    MI_HIP(ctx, hipEventRecord(n->e0, ctx->stream));
     MI_HIP(ctx, K::shuffle(sh, ctx->stream));
   }
   float *losses = (float *)n->ds_loss.ptr;
-  MI_HIP(ctx, hipEventRecord(n->e0, ctx->stream));
   for (uint32_t b = 0; b < nb; b++) {
     const size_t at = (size_t)b * batch;
     if ((rc = train_rows(n, sh.rows + at, sh.row_targets + at, batch, batch, lr, 1, losses + b)))

@@ -68,7 +68,8 @@ int mi_mlp_adam_state(mi_mlp *mlp, float *m, float *v, uint32_t *step);
  * batches of `batch` (a multiple of 64, <= max_batch) in an order drawn from Philox key
  * (shuffle_seed, epoch), counter (i >> 2, 0, 3, 1); a trailing partial batch is dropped.  A set
  * that device memory cannot hold leaves the network without one.
- * mean_loss receives the mean of the batch losses; ms the device time of the epoch. */
+ * mean_loss receives the mean of the batch losses; ms the device time of the epoch: the rows put in
+ * order (drawn on the host for up to 4096 positions, else on the device), then the steps. */
 int mi_mlp_set_dataset(mi_mlp *mlp, const mi_pos *pos, const float *targets, uint32_t n);
 int mi_mlp_train_epoch(mi_mlp *mlp, uint32_t batch, float lr, uint32_t shuffle_seed,
                        uint32_t epoch, float *mean_loss, float *ms);

@@ -53,3 +53,7 @@ def test_a_set_that_does_not_fit_leaves_none(check):
 
 def test_routes_of_shaped_and_tuned_contexts(check):
     assert "mismatches 0" in check("tuning_check.cpp")
+
+
+def test_the_time_of_an_epoch_is_all_of_it(check):
+    assert "mismatches 0" in check("epoch_check.cpp")
