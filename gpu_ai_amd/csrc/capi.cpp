@@ -30,6 +30,8 @@ int fail(mi_ctx *ctx, int code, const std::string &msg) {
 int hip_fail(mi_ctx *ctx, hipError_t e, const char *what) {
   std::string msg = std::string(what) + ": " + hipGetErrorString(e);
   int code = (e == hipErrorOutOfMemory) ? MI_ERR_OUT_OF_MEMORY : MI_ERR_DEVICE;
+  // reported here: the next launch asks the runtime for its last error and would be told of this one
+  (void)hipGetLastError();
   return fail(ctx, code, msg);
 }
 

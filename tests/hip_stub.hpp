@@ -20,6 +20,7 @@ namespace stub {
 
 int allocations_left = -1;          // device allocations until one fails; < 0: none fails
 std::set<void *> live;              // device allocations
+hipError_t last = hipSuccess;       // what hipGetLastError returns next, a launch too
 std::vector<std::string> calls;     // launches, event records and copies, in order
 // the last playout launch: threads a workgroup, workgroups, one wave per game or not
 uint32_t block = 0, grid = 0;
@@ -37,6 +38,11 @@ inline void need(std::initializer_list<const void *> ptrs) {
 
 extern "C" {
 
+hipError_t hipGetLastError(void) {
+  const hipError_t e = stub::last;
+  stub::last = hipSuccess;
+  return e;
+}
 hipError_t hipGetDeviceCount(int *n) {
   *n = 1;
   return hipSuccess;
@@ -52,7 +58,7 @@ hipError_t hipGetDevicePropertiesR0600(hipDeviceProp_tR0600 *p, int) {
 const char *hipGetErrorString(hipError_t e) { return e == hipErrorOutOfMemory ? "out of memory" : "error"; }
 hipError_t hipMalloc(void **p, size_t bytes) {
   *p = nullptr;
-  if (stub::allocations_left == 0) return hipErrorOutOfMemory;
+  if (stub::allocations_left == 0) return stub::last = hipErrorOutOfMemory;
   if (stub::allocations_left > 0) stub::allocations_left--;
   *p = std::calloc(bytes, 1);
   stub::live.insert(*p);
@@ -152,11 +158,11 @@ const void *stage_kernel() { return "stage"; }
 const void *playout_kernel(uint32_t, uint32_t) { return "playouts"; }
 hipError_t launch_reset(WorkWords *work, hipStream_t) {
   stub::need({work});
-  return hipSuccess;
+  return hipGetLastError();
 }
 hipError_t launch_stage(const LaunchDesc *from, LaunchDesc *to, WorkWords *work, hipStream_t) {
   stub::need({from, to, work});
-  return hipSuccess;
+  return hipGetLastError();
 }
 hipError_t launch_playouts(const PlayoutArgs &, uint32_t, bool, uint32_t, uint32_t grid,
                            uint32_t block, hipStream_t) {
@@ -164,58 +170,58 @@ hipError_t launch_playouts(const PlayoutArgs &, uint32_t, bool, uint32_t, uint32
   stub::block = block;
   stub::grid = grid;
   stub::wave = false;
-  return hipSuccess;
+  return hipGetLastError();
 }
 hipError_t launch_playouts_wave(const PlayoutArgs &, uint32_t, uint32_t games, hipStream_t) {
   stub::calls.push_back("playouts");
   stub::block = kWaveBlock;
   stub::grid = games;
   stub::wave = true;
-  return hipSuccess;
+  return hipGetLastError();
 }
 hipError_t launch_gen_moves(const mi_pos *, uint32_t, mi_move *, uint32_t, uint32_t *, WorkWords *,
                             hipStream_t) {
-  return hipSuccess;
+  return hipGetLastError();
 }
-hipError_t launch_start_positions(const StartArgs &, uint32_t, hipStream_t) { return hipSuccess; }
+hipError_t launch_start_positions(const StartArgs &, uint32_t, hipStream_t) { return hipGetLastError(); }
 hipError_t launch_divmod(const uint32_t *, const uint32_t *, uint32_t, uint32_t *, uint32_t *,
                          hipStream_t) {
-  return hipSuccess;
+  return hipGetLastError();
 }
-hipError_t launch_copy(const uint4 *, uint4 *, uint64_t, hipStream_t) { return hipSuccess; }
+hipError_t launch_copy(const uint4 *, uint4 *, uint64_t, hipStream_t) { return hipGetLastError(); }
 hipError_t launch_valu_rate(uint32_t, uint32_t, uint32_t *, uint32_t, hipStream_t) {
-  return hipSuccess;
+  return hipGetLastError();
 }
 hipError_t launch_tally(const int8_t *, const uint32_t *, uint32_t, uint32_t, uint32_t *,
                         hipStream_t) {
-  return hipSuccess;
+  return hipGetLastError();
 }
 
 namespace mlp {
 hipError_t forward(const mi_pos *, uint32_t, const uint16_t *, const float *, const uint16_t *,
                    const float *, const float *, const float *, float *, hipStream_t) {
-  return hipSuccess;
+  return hipGetLastError();
 }
 hipError_t train_rows(const TrainArgs &a, uint32_t, hipStream_t) {
   stub::need({a.pos, a.targets, a.Xf, a.H1f, a.dH2f, a.dH1f, a.pV});
   stub::calls.push_back("train_rows");
-  return hipSuccess;
+  return hipGetLastError();
 }
 hipError_t update(const AdamArgs &, hipStream_t) {
   stub::calls.push_back("update");
-  return hipSuccess;
+  return hipGetLastError();
 }
 hipError_t shuffle(const ShuffleArgs &a, hipStream_t) {
   stub::need({a.head, a.next, a.target, a.chain, a.pos, a.targets, a.rows, a.row_targets});
   stub::calls.push_back("shuffle");
-  return hipSuccess;
+  return hipGetLastError();
 }
 hipError_t shuffle_take(const ShuffleArgs &a, const uint32_t *order, hipStream_t) {
   stub::need({order, a.pos, a.targets, a.rows, a.row_targets});
   stub::calls.push_back("take");
-  return hipSuccess;
+  return hipGetLastError();
 }
-hipError_t zero(float *, uint32_t, hipStream_t) { return hipSuccess; }
+hipError_t zero(float *, uint32_t, hipStream_t) { return hipGetLastError(); }
 }  // namespace mlp
 
 }  // namespace gpuai
