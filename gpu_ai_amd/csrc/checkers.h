@@ -25,9 +25,14 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "gpuai/mi_playout.h"
+
 #define CK_HD __host__ __device__ __forceinline__
 
 namespace ck {
+
+constexpr uint32_t RANDOM = MI_POLICY_RANDOM, HEURISTIC = MI_POLICY_HEURISTIC,
+                   NOISY = MI_POLICY_HEURISTIC_NOISY;
 
 // ------------------------------------------------------------------------------------------
 // bit helpers
@@ -1233,50 +1238,6 @@ CK_HD PlyResult ply_random_captures(Lane &L, const Gen &g, uint32_t r, uint32_t 
   return res;
 }
 
-// Plays one ply of the random policy with word r.
-template <bool TRACE>
-CK_HD PlyResult ply_random(Lane &L, uint32_t r, uint32_t *list_dig) {
-  Gen g;
-  analyse(L, g);
-  return ply_random_given<TRACE>(L, g, r, list_dig);
-}
-
-// The common part of a random ply: plays it unless it is a capture ply with a multi-jump origin,
-// in which case the position is left untouched and `deferred` is returned set (the caller plays
-// it later with ply_random_given, the same word and the analysis left in g).
-template <bool TRACE, class TAB = Direct>
-CK_HD PlyResult ply_random_fast(Lane &L, uint32_t r, uint32_t *list_dig, bool &deferred, Gen &g,
-                                const TAB &tab = TAB()) {
-  analyse(L, g);
-  PlyResult res;
-  deferred = g.multi != 0u;
-  if (deferred) {
-    res.n = 0u;
-    res.chosen = 0u;
-    res.over = 0u;
-    res.winner = 0;
-    return res;
-  }
-  const SlotWords w = slot_words(g.slot);
-  const uint32_t n = w.n;
-  res.n = n;
-  if (TRACE) *list_dig = list_digest(L, g, n);
-  if (n == 0u || L.counter >= 50u) {
-    res.over = 1u;
-    res.chosen = 0xFFFFu;
-    res.winner = L.counter < 50u ? (int32_t)(L.turn ^ 1u) : -1;
-    return res;
-  }
-  const uint32_t k = tab.mod(r, n);
-  res.chosen = k;
-  res.over = 0u;
-  res.winner = 0;
-  uint32_t sq, sl8;
-  select_move(w, L.turn ? n - 1u - k : k, sq, sl8, tab);
-  play_slot(L, g.capture, sq, sl8, tab);
-  return res;
-}
-
 // How the weights of a ply's moves differ, where no capture sequence is longer than one jump.  A
 // step weighs sm / so, or (sm + 3) / so when it promotes a man; a jump (sm + 3p) / (so - (k ? 4 : 1))
 // by whether it promotes (p) and removes a king (k).  Most plies' moves all weigh the same, which
@@ -1308,12 +1269,6 @@ CK_HD void king_parts(const Lane &L, const Gen &g, uint32_t &with, uint32_t &wit
   with = jumped & L.kings;
   without = jumped & ~L.kings;
 }
-CK_HD bool some_take_kings(const Lane &L, const Gen &g) {
-  uint32_t with, without;
-  king_parts(L, g, with, without);
-  return with && without;
-}
-
 // The moves of the squares `from` (every move of a square in them).
 CK_HD SlotWords words_from(const Gen &g, uint32_t from) {
   const uint32_t t[4] = {g.slot[0] & from, g.slot[1] & from, g.slot[2] & from, g.slot[3] & from};
@@ -1338,6 +1293,96 @@ CK_HD uint32_t play_tie(Lane &L, const Gen &g, const SlotWords &tw, uint32_t n, 
   }
   play_slot(L, g.capture, sq, sl8, tab);
   return chosen;
+}
+
+// The common part of a ply, as the lanes of k_playouts play it and the host checks do.  What lanes do
+// is told by masks: of a wave on the device (the kernel's own), of the one lane on the host.
+struct OneLane {
+  typedef uint32_t Mask;
+  CK_HD static Mask where(bool x) { return x ? 1u : 0u; }
+  CK_HD static bool in(Mask m) { return m != 0u; }
+};
+
+// The lanes of `active` whose ply waits for the walk phase: plies with capture sequences longer than
+// one jump, for the heuristics also those whose moves weigh differently (but for the argmax
+// heuristic's steps).  from: squares of the moves of largest weight (heuristic).
+template <uint32_t POLICY, class WAVE>
+CK_HD typename WAVE::Mask waiting(const Lane &L, const Gen &g, typename WAVE::Mask active,
+                                  uint32_t &from) {
+  typename WAVE::Mask waits = active & WAVE::where(g.multi != 0u);
+  from = 0xFFFFFFFFu;
+  if (POLICY != RANDOM) {
+    const uint32_t prom = promoting(L, g);
+    uint32_t pw, po, kw, ko;
+    promote_parts(g, prom, pw, po);
+    king_parts(L, g, kw, ko);
+    const typename WAVE::Mask split =
+        WAVE::where(pw != 0u) & WAVE::where(po != 0u) & WAVE::where(L.opp != 0u);
+    waits |= active & WAVE::where(kw != 0u) & WAVE::where(ko != 0u);
+    waits |= active & (POLICY == NOISY ? split : split & WAVE::where(g.origins != 0u));
+    if (WAVE::in(split)) from = prom;
+  }
+  return waits;
+}
+
+// The moves that the ply's word chooses among (all of them but for the argmax heuristic), and the
+// number of all moves, of a ply that does not wait.
+template <uint32_t POLICY>
+CK_HD SlotWords common_moves(const Gen &g, uint32_t from, uint32_t &n) {
+  const SlotWords w = POLICY == HEURISTIC ? words_from(g, from) : slot_words(g.slot);
+  n = POLICY == HEURISTIC ? slot_count(g.slot) : w.n;
+  return w;
+}
+
+// Plays the choice of word r among the moves w (there are some, and the draw count has not run out);
+// returns its reference index (argmax heuristic: when TRACE).
+template <uint32_t POLICY, bool TRACE, class TAB>
+CK_HD uint32_t play_common(Lane &L, const Gen &g, const SlotWords &w, uint32_t n, uint32_t r,
+                           const TAB &tab) {
+  if (POLICY == HEURISTIC) return play_tie<TRACE>(L, g, w, n, r, tab);
+  uint32_t chosen = tab.mod(r, w.n);
+  // with no opponent's piece left after the move every noisy weight is +inf: move 0
+  if (POLICY == NOISY && !(g.capture ? L.opp & (L.opp - 1u) : L.opp)) chosen = 0u;
+  uint32_t sq, sl8;
+  select_move(w, L.turn ? w.n - 1u - chosen : chosen, sq, sl8, tab);
+  play_slot(L, g.capture, sq, sl8, tab);
+  return chosen;
+}
+
+// All of it for one lane: plays the ply, or leaves the position as it is with `deferred` set.
+template <uint32_t POLICY, bool TRACE, class TAB>
+CK_HD PlyResult ply_common(Lane &L, uint32_t r, uint32_t *list_dig, bool &deferred, Gen &g,
+                           const TAB &tab) {
+  PlyResult res = {0u, 0u, 0u, 0};
+  uint32_t from;
+  analyse(L, g);
+  deferred = waiting<POLICY, OneLane>(L, g, 1u, from) != 0u;
+  if (deferred) return res;
+  const SlotWords w = common_moves<POLICY>(g, from, res.n);
+  if (TRACE) *list_dig = list_digest(L, g, res.n);
+  if (w.n != 0u && L.counter < 50u) {
+    res.chosen = play_common<POLICY, TRACE>(L, g, w, res.n, r, tab);
+  } else {
+    res.over = 1u;
+    res.chosen = 0xFFFFu;
+    res.winner = L.counter < 50u ? (int32_t)(L.turn ^ 1u) : -1;
+  }
+  return res;
+}
+template <bool TRACE, class TAB = Direct>
+CK_HD PlyResult ply_random_fast(Lane &L, uint32_t r, uint32_t *list_dig, bool &deferred, Gen &g,
+                                const TAB &tab = TAB()) {
+  return ply_common<RANDOM, TRACE>(L, r, list_dig, deferred, g, tab);
+}
+template <bool TRACE, class TAB = Direct>
+CK_HD PlyResult ply_heuristic_fast(Lane &L, uint32_t r, uint32_t *list_dig, bool &deferred, Gen &g,
+                                   const TAB &tab = TAB()) {
+  return ply_common<HEURISTIC, TRACE>(L, r, list_dig, deferred, g, tab);
+}
+template <bool TRACE, class TAB = Direct>
+CK_HD PlyResult ply_noisy_fast(Lane &L, uint32_t r, uint32_t *list_dig, bool &deferred, Gen &g,
+                               const TAB &tab = TAB()) {
+  return ply_common<NOISY, TRACE>(L, r, list_dig, deferred, g, tab);
 }
 
 // The heuristic ply whose moves of largest weight are those of the squares `from`.
@@ -1445,35 +1490,6 @@ template <bool TRACE>
 CK_HD PlyResult ply_heuristic_given(Lane &L, const Gen &g, uint32_t r, uint32_t *list_dig) {
   if (g.capture) return heuristic_walk<TRACE>(L, g, r, list_dig);
   return play_tied<TRACE>(L, g, best_steps(L, g), r, list_dig, Direct());
-}
-
-// Plays one ply of the heuristic policy with word r.
-template <bool TRACE>
-CK_HD PlyResult ply_heuristic(Lane &L, uint32_t r, uint32_t *list_dig) {
-  Gen g;
-  analyse(L, g);
-  return ply_heuristic_given<TRACE>(L, g, r, list_dig);
-}
-
-// The common part of a heuristic ply: plays it unless it is a capture ply with a sequence longer
-// than one jump or with jumps of several kinds, which is left untouched with `deferred` set (the
-// caller plays it later with ply_heuristic_given, the same word and the analysis left in g).
-template <bool TRACE, class TAB = Direct>
-CK_HD PlyResult ply_heuristic_fast(Lane &L, uint32_t r, uint32_t *list_dig, bool &deferred,
-                                   Gen &g, const TAB &tab = TAB()) {
-  analyse(L, g);
-  const uint32_t prom = promoting(L, g);
-  const bool split = some_promote(g, prom);
-  deferred = g.capture && (g.multi || split || some_take_kings(L, g));
-  if (deferred) {
-    PlyResult res;
-    res.n = 0u;
-    res.chosen = 0u;
-    res.over = 0u;
-    res.winner = 0;
-    return res;
-  }
-  return play_tied<TRACE>(L, g, split && L.opp ? prom : 0xFFFFFFFFu, r, list_dig, tab);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1696,14 +1712,6 @@ CK_HD PlyResult ply_noisy_given(Lane &L, const Gen &g, uint32_t r, uint32_t *lis
   return res;
 }
 
-// Plays one ply of the noisy heuristic with word r.
-template <bool TRACE>
-CK_HD PlyResult ply_noisy(Lane &L, uint32_t r, uint32_t *list_dig) {
-  Gen g;
-  analyse(L, g);
-  return ply_noisy_given<TRACE>(L, g, r, list_dig);
-}
-
 // Steps of two weights by the index of their move (mover-frame order): with the moves from `base`
 // on counted from 0, bit i of the result is set when move i promotes.  Promoting men stand on
 // squares 24 to 27, and 8 squares have at most 32 moves.
@@ -1730,43 +1738,61 @@ CK_HD uint32_t noisy_key_move(uint64_t key, uint32_t rev) {
   return rev ? (uint32_t)key : ~(uint32_t)key;
 }
 
-// The common part of a noisy heuristic ply: plays it when its moves all weigh the same (and no
-// capture sequence is longer than one jump), else leaves it untouched with `deferred` set, for
-// ply_noisy_given with the same word and the analysis left in g.
-template <bool TRACE, class TAB = Direct>
-CK_HD PlyResult ply_noisy_fast(Lane &L, uint32_t r, uint32_t *list_dig, bool &deferred, Gen &g,
-                               const TAB &tab = TAB()) {
-  PlyResult res;
-  analyse(L, g);
-  deferred = (L.opp && some_promote(g, promoting(L, g))) ||
-             (g.capture && (g.multi || some_take_kings(L, g)));
-  if (deferred) {
-    res.n = 0u;
-    res.chosen = 0u;
-    res.over = 0u;
-    res.winner = 0;
-    return res;
+// The walk phase of k_playouts for the heuristics, as its lanes take it by turns: a move of a capture
+// ply, weighed.  w is its weight, key orders the ply's moves (noisy: with move k's draw).
+//
+// Weights are quotients of whole numbers up to 131: those that differ do so by one part in 17,000
+// or more, so that rounded they are equal where cmp_weight calls them equal.
+template <uint32_t POLICY, class TAB>
+CK_HD Choice weigh_capture(const CaptureTrees &t, uint32_t k, uint32_t sm, uint32_t so, uint32_t turn,
+                           uint32_t r, const TAB &tab, float &w, uint64_t &key) {
+  const Choice c = capture_choice(t, k, tab);
+  const uint32_t king = getbit(t.kings, c.from);
+  const uint32_t num = sm + (!king && c.to >= FAR_ROW_FIRST ? 3u : 0u);
+  const uint32_t den = so - material(c.removed, t.kings);
+  w = (float)num / (float)den;
+  if (POLICY == HEURISTIC) {
+    key = f32_bits(w);
+  } else {
+#pragma clang fp contract(off)
+    float e0, e1;
+    noise_pair(r, k >> 1, e0, e1);
+    key = noisy_key(w + ((k & 1u) ? e1 : e0), k, turn);
   }
-  const SlotWords w = slot_words(g.slot);
-  const uint32_t n = w.n;
-  res.n = n;
-  if (TRACE) *list_dig = list_digest(L, g, n);
-  if (n == 0u || L.counter >= 50u) {
-    res.over = 1u;
-    res.chosen = 0xFFFFu;
-    res.winner = L.counter < 50u ? (int32_t)(L.turn ^ 1u) : -1;
-    return res;
+  return c;
+}
+
+// Whether move k of a capture ply of n < 32 moves is the one played.  best: it has the largest key;
+// set: the moves that have it, or (noisy) those that weigh as much as the first move, w_first.
+template <uint32_t POLICY, class TAB>
+CK_HD bool plays_capture(uint32_t k, uint32_t n, bool best, uint32_t set, float w_first, uint32_t turn,
+                         uint32_t r, const TAB &tab) {
+  if (POLICY == HEURISTIC) {
+    const uint32_t ties = popc(set);
+    const uint32_t i = tab.mod(r, ties);
+    return best && popc(set & ((1u << k) - 1u)) == (turn ? ties - 1u - i : i);
   }
-  // every weight is +inf when no opponent's piece is left after the move: the first move then
-  const bool inf = !(g.capture ? L.opp & (L.opp - 1u) : L.opp);
-  const uint32_t k = inf ? 0u : tab.mod(r, n);  // reference index
-  uint32_t sq, sl8;
-  select_move(w, L.turn ? n - 1u - k : k, sq, sl8, tab);
-  res.over = 0u;
-  res.winner = 0;
-  res.chosen = k;
-  play_slot(L, g.capture, sq, sl8, tab);
-  return res;
+  if (set == (1u << n) - 1u) {  // one weight: the word chooses, or the first move if it is +inf
+    const uint32_t i = w_first == __builtin_inff() ? 0u : tab.mod(r, n);
+    return k == (turn ? n - 1u - i : i);
+  }
+  return best;
+}
+
+// The larger key of moves 2j and 2j + 1 of noisy steps (n of them) that weigh w1 where they promote
+// (promoting_moves) and w0 where they don't.
+CK_HD uint64_t steps_key(uint32_t r, uint32_t j, uint32_t n, uint32_t base, uint32_t promote, float w0,
+                         float w1, uint32_t turn) {
+#pragma clang fp contract(off)
+  const uint32_t m = 2u * j;
+  float e0, e1;
+  noise_pair(r, j, e0, e1);
+  auto weight = [&](uint32_t i) {
+    return i >= base && (promote >> ((i - base) & 31u) & 1u) ? w1 : w0;
+  };
+  const uint64_t k0 = noisy_key(weight(m) + e0, m, turn);
+  const uint64_t k1 = noisy_key(weight(m + 1u) + e1, m + 1u, turn);
+  return m + 1u < n && k1 > k0 ? k1 : k0;
 }
 
 // Start positions (mi_gen_start_positions): plies of attempt `a` of position i, at most 2^16 (a

@@ -46,6 +46,13 @@ __device__ __forceinline__ bool lane_in(uint64_t mask) {
   return __builtin_amdgcn_inverse_ballot_w64(mask);
 }
 
+// The lanes of the wave in the lane logic that it shares with the host (ck::OneLane).
+struct WaveLanes {
+  typedef uint64_t Mask;
+  static __device__ __forceinline__ Mask where(bool x) { return __ballot(x); }
+  static __device__ __forceinline__ bool in(Mask m) { return lane_in(m); }
+};
+
 __device__ __forceinline__ uint32_t uniform(uint32_t x) {
   return __builtin_amdgcn_readfirstlane(x);
 }
@@ -272,21 +279,9 @@ __device__ __forceinline__ void capture_plies(WalkShare &share, uint64_t &todo, 
       turn = p.turn;
       word = p.r;
       k = lane - begin;
-      c = ck::capture_choice(p.trees, k, tab);
-      const uint32_t king = ck::getbit(p.trees.kings, c.from);
-      const uint32_t num = p.sm + (!king && c.to >= ck::FAR_ROW_FIRST ? 3u : 0u);
-      const uint32_t den = p.so - ck::material(c.removed, p.trees.kings);
-      // Weights are quotients of whole numbers up to 131: those that differ do so by one part in
-      // 17,000 or more, so that rounded they are equal where cmp_weight calls them equal.
-      w = (float)num / (float)den;
-      if (POLICY == MI_POLICY_HEURISTIC) {
-        key = ck::f32_bits(w);
-      } else {
-#pragma clang fp contract(off)
-        float e0, e1;
-        ck::noise_pair(word, k >> 1, e0, e1);
-        key = ck::noisy_key(w + ((k & 1u) ? e1 : e0), k, turn);
-      }
+      uint64_t order;
+      c = ck::weigh_capture<POLICY>(p.trees, k, p.sm, p.so, turn, word, tab, w, order);
+      key = order;
       atomicMax(&sh.best[at], key);
     }
     wave_lds_fence();
@@ -295,21 +290,10 @@ __device__ __forceinline__ void capture_plies(WalkShare &share, uint64_t &todo, 
     const float w_first = __shfl(w, (int)begin);
     const uint64_t same =
         __ballot(on && (POLICY == MI_POLICY_HEURISTIC ? key == best : w == w_first));
-    const uint32_t all = (1u << moves) - 1u, set = (uint32_t)(same >> begin) & all;
+    const uint32_t set = (uint32_t)(same >> begin) & ((1u << moves) - 1u);
     bool chosen = false;
-    if (on) {
-      if (POLICY == MI_POLICY_HEURISTIC) {
-        const uint32_t ties = ck::popc(set);
-        const uint32_t i = tab.mod(word, ties);
-        chosen = key == best &&
-                 ck::popc(set & ((1u << k) - 1u)) == (turn ? ties - 1u - i : i);
-      } else if (set == all) {  // one weight: the word chooses, or the first move if it is +inf
-        const uint32_t i = w_first == __builtin_inff() ? 0u : tab.mod(word, moves);
-        chosen = k == (turn ? moves - 1u - i : i);
-      } else {
-        chosen = key == best;
-      }
-    }
+    if (on)
+      chosen = ck::plays_capture<POLICY>(k, moves, key == best, set, w_first, turn, word, tab);
     if (chosen) sh.choice[at] = make_uint2(c.from | c.to << 8 | k << 16, c.removed);
     wave_lds_fence();
   }
@@ -371,18 +355,11 @@ __device__ __forceinline__ void noisy_steps(WalkShare &share, uint64_t todo, ck:
     const uint32_t at = before + lane_rank(mk) + (uint32_t)(mk >> lane & 1ull) - 1u;
     before += __builtin_amdgcn_readfirstlane((uint32_t)__popcll(mk));
     if (q0 + lane < total) {
-#pragma clang fp contract(off)
       const auto p = sh.ply[at];
-      const uint32_t n = p.moves & 255u, base = p.moves >> 8 & 255u, rev = p.moves >> 16;
-      const uint32_t j = q0 + lane - p.first, m = 2u * j;
-      float e0, e1;
-      ck::noise_pair(p.r, j, e0, e1);
-      auto weight = [&](uint32_t i) {
-        return i >= base && (p.promote >> ((i - base) & 31u) & 1u) ? p.w1 : p.w0;
-      };
-      const unsigned long long k0 = ck::noisy_key(weight(m) + e0, m, rev);
-      const unsigned long long k1 = ck::noisy_key(weight(m + 1u) + e1, m + 1u, rev);
-      atomicMax(&sh.best[at], m + 1u < n && k1 > k0 ? k1 : k0);
+      const unsigned long long key =
+          ck::steps_key(p.r, q0 + lane - p.first, p.moves & 255u, p.moves >> 8 & 255u, p.promote,
+                        p.w0, p.w1, p.moves >> 16);
+      atomicMax(&sh.best[at], key);
     }
   }
   wave_lds_fence();
@@ -671,28 +648,15 @@ __global__ void __launch_bounds__(1024) k_playouts(PlayoutArgs a) {
 #pragma unroll 1
     for (uint32_t step = 0; step < 4u; step++) {
       // The common part of the ply: every lane looks at its position (an idle lane's or a waiting
-      // one's yields what it did before), and those that can play do.  Plies with longer captures,
-      // for the heuristics also those whose moves weigh differently, wait for the walk phase, where
-      // they take the same word.
+      // one's yields what it did before), and those that can play do.  The others wait for the walk
+      // phase, where they take the same word.
       ck::Gen gen;
       ck::analyse(L, gen);
-      uint64_t deferred = active & __ballot(gen.multi != 0u);
-      uint32_t from = 0xFFFFFFFFu;  // heuristic: squares of the moves of largest weight
-      if (POLICY != MI_POLICY_RANDOM) {
-        const uint32_t prom = ck::promoting(L, gen);
-        uint32_t pw, po, kw, ko;
-        ck::promote_parts(gen, prom, pw, po);
-        ck::king_parts(L, gen, kw, ko);
-        const uint64_t split = __ballot(pw != 0u) & __ballot(po != 0u) & __ballot(L.opp != 0u);
-        deferred |= active & __ballot(kw != 0u) & __ballot(ko != 0u);
-        deferred |= active & (POLICY == MI_POLICY_HEURISTIC_NOISY
-                                  ? split : split & __ballot(gen.origins != 0u));
-        if (lane_in(split)) from = prom;
-      }
+      uint32_t from;
+      const uint64_t deferred = ck::waiting<POLICY, WaveLanes>(L, gen, active, from);
       {
-        const ck::SlotWords w = POLICY == MI_POLICY_HEURISTIC ? ck::words_from(gen, from)
-                                                              : ck::slot_words(gen.slot);
-        const uint32_t n = POLICY == MI_POLICY_HEURISTIC ? ck::slot_count(gen.slot) : w.n;
+        uint32_t n;
+        const ck::SlotWords w = ck::common_moves<POLICY>(gen, from, n);
         const uint64_t can = active & ~deferred;
         const uint64_t go = can & __ballot(w.n != 0u) & __ballot(L.counter < 50u);
         // (a waiting ply has no fewer moves than first jumps, an idle lane's last game had these)
@@ -701,18 +665,7 @@ __global__ void __launch_bounds__(1024) k_playouts(PlayoutArgs a) {
         if (TRACE && lane_in(can)) ld = ck::list_digest(L, gen, n);
         if (lane_in(go)) {
           const uint32_t r = words[ply & ((kWordRows - 1u) * kPly)];
-          if (POLICY == MI_POLICY_HEURISTIC) {
-            chosen = ck::play_tie<TRACE>(L, gen, w, n, r, tab);
-          } else {
-            chosen = tab.mod(r, w.n);
-            // with no opponent's piece left after the move every noisy weight is +inf: move 0
-            if (POLICY == MI_POLICY_HEURISTIC_NOISY &&
-                !(gen.capture ? L.opp & (L.opp - 1u) : L.opp))
-              chosen = 0u;
-            uint32_t sq, sl8;
-            ck::select_move(w, L.turn ? w.n - 1u - chosen : chosen, sq, sl8, tab);
-            ck::play_slot(L, gen.capture, sq, sl8, tab);
-          }
+          chosen = ck::play_common<POLICY, TRACE>(L, gen, w, n, r, tab);
           ply += kPly;
         }
         if (TRACE && lane_in(can)) h = ck::hash_step(h, ck::ply_record(ld, n, chosen));

@@ -227,7 +227,7 @@ __device__ __forceinline__ void play(ck::Lane &L, const Geometry &geo, const Str
         const uint64_t aA = __ballot((jumpA & any) != 0u), aB = __ballot((jumpB & any) != 0u);
         longer = (((jA & fA) | (jB & fB)) & men) | (((jA & aA) | (jB & aB)) & kings);
         if (POLICY != MI_POLICY_RANDOM) {
-          // jumps of several kinds (some_promote, some_take_kings) are the walk's as well
+          // jumps of several kinds (as in ck::waiting) are the walk's as well
           const uint64_t prom = men & ck::ROW5;
           const uint64_t kinds = m0 | m1;
           bool mixed = (kinds & prom) && (kinds & ~prom);
