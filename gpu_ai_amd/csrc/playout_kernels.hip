@@ -855,8 +855,7 @@ __global__ void __launch_bounds__(64) k_start_positions(StartArgs a) {
   // Where the slots hold all positions a wave takes its own at once: claims on one counter go one by
   // one, some 20 ns each (3,000 positions of no ply by as many waves: 90 -> 29 us a call).
   const bool dealt = (uint64_t)gridDim.x * a.slots >= a.n;
-  // (few positions: one slab, since 16 slabs of blocks of kSlabBlock would leave most waves without)
-  const uint32_t nslabs = a.n < 32u * kSlabBlock * kSlabs ? 1u : min(gridDim.x, kSlabs);
+  const uint32_t nslabs = min(gridDim.x, kSlabs);
   const uint32_t slab = blockIdx.x % nslabs;
   bool exhausted = false;
   for (;;) {
