@@ -322,7 +322,7 @@ def bench_value(args) -> int:
                         "after_epochs": epochs + args.warmup},
         "roofline": {"bound": "mfma", "achieved": round(achieved / 1e12, 3), "peak": 2500.0,
                      "unit": "TFLOP/s", "frac": round(achieved / 2.5e15, 5), "traffic": None,
-                     "kernel": "training step (k_train_rows, k_update)",
+                     "kernel": "training step (k_train_rows, k_update; its share of k_shuffle_*)",
                      "flops_per_step": flops, "device_us_per_step": round(device_s / steps * 1e6, 2)},
     }
     print(json.dumps(line), flush=True)

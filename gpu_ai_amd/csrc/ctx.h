@@ -65,8 +65,8 @@ struct mi_ctx {
   // stream is idle.
   gpuai::HostBuf h_in, h_back;
   // the packed batch of mi_run_playouts (inputs | work words | winners in one device block and
-  // its pinned mirror, one copy each way); used and released only by that route, which waits
-  // for its stream before it returns
+  // its pinned mirror, one copy each way), and the work words and results of start positions; both
+  // wait for the stream before they return
   gpuai::DevBuf batch;
   gpuai::HostBuf h_batch;
   // staged batch
@@ -94,8 +94,8 @@ uint32_t tune_bucket(uint64_t total);
 // SIMD), and 16 from two games a lane on: waves of a workgroup hand their last games over to each
 // other (playout_kernels.hip), and 16 hide each other's latencies better but have more last games.
 // Against 64x12, in ms: 1024x1024 0.546 -> 0.480 with 16 waves (0.499 with 12), 64x4096 0.243 ->
-// 0.210 with 12 (0.216 with 16), 65536x256 4.76 -> 4.45 with 16 (4.77 with 12).  Up to four waves a CU there is nothing to hand
-// over, and 64-thread blocks it is.  The noisy heuristic waits for 24 plies: its walk phases cost
+// 0.210 with 12 (0.216 with 16), 65536x256 4.76 -> 4.45 with 16 (4.77 with 12).  Up to four waves a CU
+// there is nothing to hand over, and 64-thread blocks it is.  The noisy heuristic waits for 24 plies: its walk phases cost
 // much the same for any number of them (noisy-1024x1024 0.582, 0.564, 0.552, 0.539 and 0.546 ms at
 // 12, 16, 20, 24 and 32; the other policies are level from 16 on).  What mi_autotune measured on one
 // batch holds for that batch's bucket: at 65,536 random playouts the shape of 1,048,576 takes 0.203

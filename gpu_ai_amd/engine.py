@@ -336,7 +336,8 @@ class Engine:
 
     def autotune(self, pos, per_pos: int | None = None, counts=None, policy: int = POLICY_RANDOM,
                  reps: int = 3) -> tuple[dict, list[dict]]:
-        """Sweeps launch shapes on this batch; the fastest becomes the context's tuning."""
+        """Sweeps launch shapes on this batch, for a small one also one wave per game (blocks_per_cu
+        0); batches of its bucket take the fastest."""
         pos = as_positions(pos)
         c, pp, _ = self._counts(len(pos), per_pos, counts)
         res = (MiTuneResult * 256)()
@@ -396,8 +397,8 @@ class Engine:
 
 
 class GraphBatch:
-    """A hipGraph of (reset, persistent playout kernel, copy out) replayed per batch, after an
-    asynchronous copy of the batch; the playout node's grid is sized to each batch."""
+    """A hipGraph of (upload from pinned memory, persistent playout kernel, copy out) replayed per
+    batch; the playout node's shape and grid follow each batch."""
 
     def __init__(self, engine: Engine, max_positions: int, max_playouts: int, policy: int):
         self.engine = engine

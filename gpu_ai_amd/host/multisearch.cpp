@@ -54,8 +54,8 @@ namespace {
 
 // The launch shapes for the searches' batches: the context's launch-shape table filled for every
 // size an iteration's batch can take -- one search's `initial` trials, doubling up to `maxBatch`
-// (every search at its largest iteration) -- tuned on batches of the roots; or the context's
-// default shape.  Returns the shape of the largest batch (reported with the results).
+// (every search at its largest iteration) -- tuned on batches of the roots; or the sizes' own
+// shapes.  Returns the shape of the largest batch (reported with the results).
 mi_tuning tuneSearches(mi_ctx *ctx, const MultiSearchConfig &cfg, const std::vector<mi_pos> &roots,
                        uint64_t maxBatch) {
   mi_tuning t = {};

@@ -52,8 +52,8 @@ struct MultiSearchConfig {
   uint32_t policy = MI_POLICY_RANDOM;
   MultiSearchMode mode = MultiSearchMode::GRAPH;
   uint32_t groups = 2;           // pipelined mode: groups of searches (device streams)
-  // launch shape from the autotuner (mi_autotune on every root with `initial` playouts, before
-  // the timed search; the shape changes no result), else the library's default
+  // launch shapes from the autotuner (mi_autotune_sizes on the roots, for every size that an
+  // iteration's batch can take, before the timed search; no shape changes a result), else the library's
   bool autotune = true;
   int device = 0;
   std::function<void(const MultiSearchBatch &)> hook;  // test hook: every batch (may be empty)

@@ -67,7 +67,7 @@ typedef struct gpuai_multisearch_config {
   uint32_t mode;          /* 0 graph replay, 1 one plain launch, 2 one launch per search,
                              3 graph replays of `groups` groups overlapped with the host's work */
   uint32_t groups;        /* pipelined mode: groups of searches, one stream each (2) */
-  uint32_t autotune;      /* 1: launch shape from mi_autotune before the search, 0: default */
+  uint32_t autotune;      /* 1: launch shapes tuned before the search, 0: defaults */
   gpuai_batch_hook hook;  /* called with every device batch (may be NULL) */
   void *hook_user;
   uint32_t *budgets;      /* out (may be NULL): each search's playout budget */

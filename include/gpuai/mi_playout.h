@@ -200,8 +200,8 @@ int mi_gen_start_positions(mi_ctx *ctx, uint32_t seed, uint32_t n, uint32_t kmin
  * NULL), else the context's tuning.
  *
  * mi_autotune tunes on one batch and also makes the fastest shape with one lane per game the
- * context's tuning, in place of a shape that it was given.  `results` (may be NULL) receives up to `max_results` candidates; `nresults` the
- * number measured; `best` (may be NULL) the winner. */
+ * context's tuning, in place of a shape that it was given.  `results` (may be NULL) receives up to
+ * `max_results` candidates; `nresults` the number measured; `best` (may be NULL) the winner. */
 int mi_autotune(mi_ctx *ctx, const mi_pos *pos, uint32_t npos, const uint32_t *counts,
                 uint32_t per_pos, uint32_t policy, uint32_t reps, mi_tune_result *results,
                 uint32_t max_results, uint32_t *nresults, mi_tuning *best);
@@ -228,14 +228,14 @@ int mi_get_tuning_table(const mi_ctx *ctx, mi_tune_entry *out, uint32_t cap, uin
 
 /* Graph-replayed batches for search loops (no counterpart in the reference, which launches,
  * copies and frees per call).  mi_graph_create fixes the capacities and builds one hipGraph for
- * the context's stream: a reset kernel, the persistent playout kernel (the launch shape of a full
- * batch, whose refill policy the graph keeps; each replay takes its batch's shape from the
- * launch-shape table, see mi_autotune, and its grid is sized to the batch), and the copy of the
- * winners back to pinned memory.
+ * the context's stream: a kernel that reads the batch from pinned memory and clears the counters, the
+ * persistent playout kernel (the launch shape of a full batch, whose refill policy the graph keeps;
+ * each replay takes its batch's shape, see mi_autotune, and its grid is sized to the batch), and
+ * the copy of the winners back to pinned memory.
  * mi_graph_run packs the batch (seed, epoch, positions, playout offsets and, when keys is not
- * NULL, stream keys) into pinned memory, copies it to the device with one asynchronous copy on
- * the stream, replays the graph and returns the winners as mi_run_playouts_keyed would (same
- * streams).  kernel_ms in the stats is the device time of the upload and the replay.  A graph is
+ * NULL, stream keys) into pinned memory, replays the graph -- or, for a batch with one wave per game,
+ * launches the same kernels of its own -- and returns the winners as mi_run_playouts_keyed would
+ * (same streams).  kernel_ms in the stats is the device time of the upload and the replay.  A graph is
  * used by one thread at a time and must be destroyed before its context. */
 typedef struct mi_graph mi_graph;
 int mi_graph_create(mi_ctx *ctx, uint32_t max_positions, uint32_t max_playouts, uint32_t policy,
