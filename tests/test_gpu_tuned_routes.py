@@ -33,11 +33,11 @@ def test_sizes_of_a_tuned_context(oracle, policy):
             w, _ = oracle.run_playouts(pos, counts=counts, seed=4, epoch=2, policy=policy, traces=False)
             assert np.array_equal(r.winners, w), total
         assert eng.run_playouts(pos, per_pos=256, policy=policy).stats["block_size"] == best["block_size"]
-        announce("mi_autotune_sizes 64, 1024, 4096")
-        for e in eng.autotune_sizes(pos, [64, 1024, 4096], policy=policy, reps=3):
-            # a wave per game is two to four times as fast at 64 games, and a third at 4096
+        announce("mi_autotune_sizes 64, 1024, 2048")
+        for e in eng.autotune_sizes(pos, [64, 1024, 2048], policy=policy, reps=3):
+            # a wave per game takes less than three fifths of the time at all of these
             assert e["blocks_per_cu"] == 0 and e["block_size"] == 64, e
-        for total in (64, 1500, 4096):
+        for total in (64, 1500, 2048):
             counts = np.full(1024, total // 1024, np.uint32)
             counts[:total % 1024] += 1
             r = eng.run_playouts(pos, counts=counts, seed=5, epoch=3, policy=policy)
