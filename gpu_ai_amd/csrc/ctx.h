@@ -95,11 +95,12 @@ uint32_t tune_bucket(uint64_t total);
 // other (playout_kernels.hip), and 16 hide each other's latencies better but have more last games.
 // Against 64x12, in ms: 1024x1024 0.546 -> 0.480 with 16 waves (0.499 with 12), 64x4096 0.243 ->
 // 0.210 with 12 (0.216 with 16), 65536x256 4.76 -> 4.45 with 16 (4.77 with 12).  Up to four waves a CU
-// there is nothing to hand over, and 64-thread blocks it is.  The noisy heuristic waits for 24 plies: its walk phases cost
-// much the same for any number of them (noisy-1024x1024 0.582, 0.564, 0.552, 0.539 and 0.546 ms at
-// 12, 16, 20, 24 and 32; the other policies are level from 16 on).  What mi_autotune measured on one
-// batch holds for that batch's bucket: at 65,536 random playouts the shape of 1,048,576 takes 0.203
-// ms, the size's own 0.139.  total 0: the size is not known here, and the context's tuning it is.
+// there is nothing to hand over, and 64-thread blocks it is.  The noisy heuristic waits for 24 plies:
+// its walk phases cost much the same for any number of them (noisy-1024x1024 0.582, 0.564, 0.552,
+// 0.539 and 0.546 ms at 12, 16, 20, 24 and 32; the other policies are level from 16 on).  What
+// mi_autotune measured on one batch holds for that batch's bucket: at 65,536 random playouts the shape
+// of 1,048,576 takes 0.203 ms, the size's own 0.139.  total 0: the size is not known here, and the
+// context's tuning it is.
 mi_tuning batch_shape(const mi_ctx *ctx, uint32_t policy, uint64_t total);
 // The launch shape of a batch with one lane per game: the table's entry for its policy and bucket
 // (the faster refill, or refill `only` when it is 0 or 1), else batch_shape's.
